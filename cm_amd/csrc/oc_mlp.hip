@@ -4,6 +4,7 @@
 // an answer is accepted only by the Newton solve's own FP64 residual test.
 #include <algorithm>
 #include <cmath>
+#include <cstring>
 #include <vector>
 
 #include "oc_internal.h"
@@ -364,6 +365,446 @@ __global__ void __launch_bounds__(256) warm_apply_pressure_kernel(int nq, int nl
     }
 }
 
+// ---- fused network -------------------------------------------------------------
+// Networks of up to kFusedLayers linear layers no wider than kFusedMax run
+// whole per row tile: a block of four waves takes 32 kRT rows through every
+// layer with the activations in LDS, so only the inputs and outputs (and, for
+// training, the pre-activations and activations the backward pass reads) pass
+// through memory.  Bound by the FP32 matrix rate and the GELU beside it.
+// Each wave owns 32 columns of a layer for all the block's rows: its slice of
+// W stays in registers, the rows come from LDS as 16-byte reads (stride 132
+// floats: 16 rows cover the banks once), and mfma_f32_32x32x2 (153 of 157
+// TFLOP/s, against 126 for 16x16x4) takes them in the order k = 8 s + 4 h + t of
+// instruction t, h the wave half.  Measured, 9 -> 4 x 128 -> 4: 274,625 rows
+// 1.14 ms in ten GEMM and bias/GELU passes, 0.31 ms here (90 TFLOP/s; 0.39 with
+// 128 rows per block and two blocks per CU, where the GELU and the slice loads
+// of one block find too little beside them); forward, backward and weight
+// gradients of 4,096 rows 3.72 ms, 0.082 ms here.  Against 64 bits the outputs
+// are off by 5e-8 to 9e-8 (1.5e-7 before), the gradient by 6e-8 to 1.1e-7 (8e-8
+// to 2.9e-7 before).
+constexpr int kFusedMax = 128, kFusedLayers = 16, kFusedStride = kFusedMax + 4;
+typedef float f32x16 __attribute__((ext_vector_type(16)));
+
+// E(x) = erfc(|x| / sqrt 2) = 2^(|x| Q(|x|)), with Q a degree-8 minimax fit of
+// log2(E) / |x| on [0, 9] (iteratively reweighted least squares against the
+// exact function; 4.4e-9 in E / 2), |x| held at 9.5 beyond, where E < 1e-20.
+// GELU is x E / 2 for x < 0, where 1 + erf would cancel, and x (1 - E / 2)
+// otherwise: one polynomial and one exp2 for every lane, where erff's two ranges
+// both run in a mixed wave.  In FP32 against 64 bits its error is at most
+// 6.8e-8 |x| on [-12, 12], 2.4e-8 rms (0.5 x (1 + erff): 1.1e-7 |x|, 3.4e-8).
+// The bf16 layers keep erff: a last-bit change there flips bf16 roundings.
+__device__ __forceinline__ float half_tail(float x)  // E / 2
+{
+    const float a = fminf(fabsf(x), 9.5f);
+    float q = 2.671841628e-07f;
+    q = fmaf(q, a, -6.325424692e-06f);
+    q = fmaf(q, a, 5.781458822e-05f);
+    q = fmaf(q, a, -2.369977883e-04f);
+    q = fmaf(q, a, -5.822885578e-05f);
+    q = fmaf(q, a, 6.994748488e-03f);
+    q = fmaf(q, a, -5.246420577e-02f);
+    q = fmaf(q, a, -4.592151344e-01f);
+    q = fmaf(q, a, -1.151104689e+00f);
+    return __builtin_amdgcn_exp2f(fmaf(a, q, -1.0f));
+}
+__device__ __forceinline__ float gelu_exp2(float x)
+{
+    const float e = half_tail(x);
+    return x * (x < 0.0f ? e : 1.0f - e);
+}
+// Phi(x) + x phi(x)
+__device__ __forceinline__ float gelu_grad_exp2(float x)
+{
+    const float e = half_tail(x);
+    const float phi = 0.39894228040143268f * __builtin_amdgcn_exp2f(-0.72134752044448170f * x * x);
+    return fmaf(x, phi, x < 0.0f ? e : 1.0f - e);
+}
+
+struct FusedNet {
+    int layers;
+    int in[kFusedLayers], out[kFusedLayers];
+    int w[kFusedLayers], b[kFusedLayers];  // offsets into the parameters
+};
+struct FusedBuffers {
+    float *pre[kFusedLayers], *act[kFusedLayers], *dz[kFusedLayers];
+};
+
+// row of accumulator register r of a 32x32 tile in this lane (column lane % 32)
+__device__ __forceinline__ int tile_row(int lane, int r) { return 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3); }
+
+// Operand slices in the order the waves load them: for layer l, column tile w
+// and step s, lane i's four values M(8 s + 4 h + t, 32 w + i % 32), h = i / 32,
+// zero outside the layer, so a wave reads 1 KiB in one piece.  Read from the
+// parameters themselves, the 32 rows a load touches lie 512 bytes apart: that
+// took 6 us a layer (4,096 rows), most of the kernel.  M = W^T for the forward
+// product (M(k, col) = W[col][k]), W for the backward one (kTransposed).
+constexpr int kSliceSteps = kFusedMax / 8, kSliceLayer = 4 * kSliceSteps * 64;  // float4 per layer
+
+template <bool kTransposed>
+__global__ void __launch_bounds__(256) pack_slices_kernel(FusedNet net, const float *__restrict__ params,
+                                                         float4 *__restrict__ slices)
+{
+    const int q = blockIdx.x * 256 + threadIdx.x;
+    if (q >= net.layers * kSliceLayer) return;
+    const int l = q / kSliceLayer, lane = q & 63, s = (q >> 6) % kSliceSteps, w = (q >> 6) / kSliceSteps % 4;
+    const int K = kTransposed ? net.out[l] : net.in[l], N = kTransposed ? net.in[l] : net.out[l];
+    const int col = 32 * w + (lane & 31), k0 = 8 * s + 4 * (lane >> 5);
+    const float *W = params + net.w[l];
+    float v[4];
+#pragma unroll
+    for (int t = 0; t < 4; ++t)
+        v[t] = (col < N && k0 + t < K) ? (kTransposed ? W[(k0 + t) * N + col] : W[col * K + k0 + t]) : 0.f;
+    slices[q] = make_float4(v[0], v[1], v[2], v[3]);
+}
+
+// this wave's slice of layer l, and its registers
+__device__ __forceinline__ const float4 *slice_of(const float4 *__restrict__ slices, int l, int wave, int lane)
+{
+    return slices + l * kSliceLayer + wave * (kSliceSteps * 64) + lane;
+}
+__device__ __forceinline__ void load_slice(const float4 *__restrict__ slices, int l, int wave, int lane, float4 (&b)[16])
+{
+    const float4 *p = slice_of(slices, l, wave, lane);
+#pragma unroll
+    for (int s = 0; s < kSliceSteps; ++s) b[s] = p[64 * s];
+}
+
+// One k-step of eight: two accumulators take turns, the row tiles' or, with one
+// row tile, those of the even and odd products, so that a product does not wait
+// for the one before it.
+template <int kRT>
+__device__ __forceinline__ void tile_step(const float4 (&a)[kRT], const float4 &b, f32x16 (&acc)[2])
+{
+    const float4 a0 = a[0], a1 = a[kRT - 1];
+    acc[0] = __builtin_amdgcn_mfma_f32_32x32x2f32(a0.x, b.x, acc[0], 0, 0, 0);
+    if (kRT == 2) acc[1] = __builtin_amdgcn_mfma_f32_32x32x2f32(a1.x, b.x, acc[1], 0, 0, 0);
+    if (kRT == 2) acc[0] = __builtin_amdgcn_mfma_f32_32x32x2f32(a0.y, b.y, acc[0], 0, 0, 0);
+    acc[1] = __builtin_amdgcn_mfma_f32_32x32x2f32(a1.y, b.y, acc[1], 0, 0, 0);
+    acc[0] = __builtin_amdgcn_mfma_f32_32x32x2f32(a0.z, b.z, acc[0], 0, 0, 0);
+    if (kRT == 2) acc[1] = __builtin_amdgcn_mfma_f32_32x32x2f32(a1.z, b.z, acc[1], 0, 0, 0);
+    if (kRT == 2) acc[0] = __builtin_amdgcn_mfma_f32_32x32x2f32(a0.w, b.w, acc[0], 0, 0, 0);
+    acc[1] = __builtin_amdgcn_mfma_f32_32x32x2f32(a1.w, b.w, acc[1], 0, 0, 0);
+}
+
+// acc[rt] = rows 32 rt .. +31 of the LDS tile (first K columns, zero padded to
+// a multiple of eight) times this wave's slice.  K > 120 takes the slice from
+// registers (b) and reads a step's rows under the products of the step before;
+// fewer columns read both step by step (a loop over b would keep it in memory).
+template <int kRT>
+__device__ __forceinline__ void tile_product(const float (*H)[kFusedStride], int K, int lane, const float4 (&b)[16],
+                                             const float4 *__restrict__ slice, f32x16 (&acc)[2])
+{
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) acc[i][r] = 0.f;
+    const float *h0 = &H[lane & 31][4 * (lane >> 5)];
+    auto rows = [&](int s, float4(&a)[kRT]) {
+#pragma unroll
+        for (int rt = 0; rt < kRT; ++rt) a[rt] = *reinterpret_cast<const float4 *>(h0 + 32 * rt * kFusedStride + 8 * s);
+    };
+    if (K > 120) {
+        float4 a[2][kRT];
+        rows(0, a[0]);
+#pragma unroll
+        for (int s = 0; s < kSliceSteps; ++s) {
+            if (s + 1 < kSliceSteps) rows(s + 1, a[(s + 1) & 1]);
+            tile_step<kRT>(a[s & 1], b[s], acc);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    } else {
+#pragma unroll 1
+        for (int s = 0; 8 * s < K; ++s) {
+            float4 a[kRT];
+            rows(s, a);
+            const float4 bs = slice[64 * s];
+            tile_step<kRT>(a, bs, acc);
+        }
+    }
+    if (kRT == 1) acc[0] += acc[1];
+}
+
+// y = network(x): x is normalised on the way in when shift is given (and, with
+// kTrain, kept as act[0] with every layer's pre-activation and activation)
+template <int kRT, bool kTrain>
+__global__ void __launch_bounds__(256, kRT == 2 ? 4 : 2)
+mlp_fused_forward_kernel(int n, FusedNet net, const float *__restrict__ params,
+                         const float4 *__restrict__ slices, const float *__restrict__ x,
+                         const float *__restrict__ shift, const float *__restrict__ scale, FusedBuffers buf,
+                         float *__restrict__ y)
+{
+    constexpr int kRows = 32 * kRT;
+    __shared__ __align__(16) float H[kRows][kFusedStride];
+    __shared__ __align__(16) float s_last[8][kFusedMax];
+    const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+    const int row0 = blockIdx.x * kRows;
+    {
+        const int K = net.in[net.layers - 1], N = net.out[net.layers - 1];
+        if (N <= 8) {
+            const float *W = params + net.w[net.layers - 1];
+            for (int q = t; q < N * kFusedMax; q += 256) {
+                const int o = q / kFusedMax, k = q % kFusedMax;
+                s_last[o][k] = k < K ? W[o * K + k] : 0.f;
+            }
+        }
+    }
+    {
+        const int K = net.in[0], Kp = (K + 7) & ~7;
+        for (int q = t; q < kRows * Kp; q += 256) {
+            const int r = q / Kp, k = q % Kp;
+            float v = 0.f;
+            if (row0 + r < n && k < K) {
+                v = x[static_cast<int64_t>(row0 + r) * K + k];
+                if (shift) {
+                    v = (v - shift[k]) * scale[k];
+                    if (kTrain) buf.act[0][static_cast<int64_t>(row0 + r) * K + k] = v;
+                }
+            }
+            H[r][k] = v;
+        }
+    }
+    const int col = 32 * wave + (lane & 31);
+    // one row tile (few blocks, nothing beside them on the CU): a layer's slice
+    // is loaded under the whole of the layer before it.  Two row tiles leave
+    // that to the other three blocks on the CU.
+    constexpr bool kAhead = kRT == 1;
+    float4 b[16], next[16];
+    if (kAhead) load_slice(slices, 0, wave, lane, next);
+    __syncthreads();
+    for (int l = 0; l < net.layers; ++l) {
+        const int K = net.in[l], N = net.out[l];
+        const bool last = l + 1 == net.layers;
+        const float *bias = params + net.b[l];
+        if (last && N <= 8) {
+            // few outputs: kParts threads share a row's sum over k, the
+            // weights in LDS (staged with the first layer)
+            constexpr int kParts = 256 / kRows;
+            const int r = t / kParts, part = t % kParts;
+            float acc[8];
+#pragma unroll
+            for (int o = 0; o < 8; ++o) acc[o] = 0.f;
+            for (int k = 4 * part; k < K; k += 4 * kParts) {
+                const float4 h = *reinterpret_cast<const float4 *>(&H[r][k]);
+#pragma unroll
+                for (int o = 0; o < 8; ++o) {
+                    if (o >= N) break;
+                    const float4 w = *reinterpret_cast<const float4 *>(&s_last[o][k]);
+                    acc[o] = fmaf(h.w, w.w, fmaf(h.z, w.z, fmaf(h.y, w.y, fmaf(h.x, w.x, acc[o]))));
+                }
+            }
+#pragma unroll
+            for (int o = 0; o < 8; ++o) {
+#pragma unroll
+                for (int sh = kParts / 2; sh > 0; sh >>= 1) acc[o] += __shfl_xor(acc[o], sh);
+                if (o < N && part == 0 && row0 + r < n) y[static_cast<int64_t>(row0 + r) * N + o] = acc[o] + bias[o];
+            }
+            break;
+        }
+        const bool active = 32 * wave < N;  // whole waves
+        f32x16 acc[2];
+        if (kAhead) {
+#pragma unroll
+            for (int s = 0; s < 16; ++s) b[s] = next[s];
+            if (!last) load_slice(slices, l + 1, wave, lane, next);
+        } else {
+            load_slice(slices, l, wave, lane, b);
+        }
+        if (active) tile_product<kRT>(H, K, lane, b, slice_of(slices, l, wave, lane), acc);
+        __syncthreads();  // the layer's input is read
+        if (active) {
+            const float bc = col < N ? bias[col] : 0.f;
+            const bool full = row0 + kRows <= n && 32 * wave + 32 <= N;  // every row and column exists
+            const int64_t g0 = static_cast<int64_t>(row0) * N + col;
+#pragma unroll
+            for (int rt = 0; rt < kRT; ++rt) {
+                float z[16], hv[16];
+#pragma unroll
+                for (int r = 0; r < 16; ++r) z[r] = acc[rt][r] + bc;
+                if (!last) {
+                    // values before stores: sixteen independent GELU chains
+#pragma unroll
+                    for (int r = 0; r < 16; ++r) hv[r] = gelu_exp2(z[r]);
+#pragma unroll
+                    for (int r = 0; r < 16; ++r) H[32 * rt + tile_row(lane, r)][col] = col < N ? hv[r] : 0.f;
+                }
+                if (!kTrain && !last) continue;
+                float *p0 = last ? y : buf.pre[l], *p1 = last ? nullptr : buf.act[l + 1];
+                if (full) {
+#pragma unroll
+                    for (int r = 0; r < 16; ++r) {
+                        const int64_t g = g0 + static_cast<int64_t>(32 * rt + tile_row(lane, r)) * N;
+                        p0[g] = z[r];
+                        if (!last) p1[g] = hv[r];
+                    }
+                } else {
+#pragma unroll
+                    for (int r = 0; r < 16; ++r) {
+                        const int row = 32 * rt + tile_row(lane, r);
+                        if (row0 + row >= n || col >= N) continue;
+                        const int64_t g = g0 + static_cast<int64_t>(row) * N;
+                        p0[g] = z[r];
+                        if (!last) p1[g] = hv[r];
+                    }
+                }
+            }
+        }
+        __syncthreads();
+    }
+}
+
+// dZ of every layer from the outputs y and targets tt, and per-block partial
+// sums of (y - tt)^2: the same tiles as the forward pass, going back
+template <int kRT>
+__global__ void __launch_bounds__(256, kRT == 2 ? 3 : 2)
+mlp_fused_backward_kernel(int n, FusedNet net, const float4 *__restrict__ slices,
+                          const float *__restrict__ y, const float *__restrict__ tt, FusedBuffers buf, float *__restrict__ partial)
+{
+    constexpr int kRows = 32 * kRT;
+    __shared__ __align__(16) float H[kRows][kFusedStride];
+    __shared__ float s_sum[4];
+    const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+    const int row0 = blockIdx.x * kRows, L = net.layers;
+    {
+        const int N = net.out[L - 1], Np = (N + 7) & ~7;
+        const float count = static_cast<float>(static_cast<int64_t>(n) * N);
+        float sum = 0.f;
+        for (int q = t; q < kRows * Np; q += 256) {
+            const int r = q / Np, o = q % Np;
+            float v = 0.f;
+            if (row0 + r < n && o < N) {
+                const int64_t g = static_cast<int64_t>(row0 + r) * N + o;
+                const float d = y[g] - tt[g];
+                sum += d * d;
+                v = 2.0f * d / count;
+                buf.dz[L - 1][g] = v;
+            }
+            H[r][o] = v;
+        }
+#pragma unroll
+        for (int sh = 32; sh > 0; sh >>= 1) sum += __shfl_xor(sum, sh);
+        if (lane == 0) s_sum[wave] = sum;
+    }
+    __syncthreads();
+    if (t == 0) partial[blockIdx.x] = (s_sum[0] + s_sum[1]) + (s_sum[2] + s_sum[3]);
+    const int col = 32 * wave + (lane & 31);
+    constexpr bool kAhead = kRT == 1;
+    float4 b[16], next[16];
+    if (kAhead && L > 1) load_slice(slices, L - 1, wave, lane, next);
+    for (int l = L - 1; l > 0; --l) {
+        const int K = net.out[l], N = net.in[l];
+        const bool active = 32 * wave < N;  // whole waves
+        f32x16 acc[2];
+        if (kAhead) {
+#pragma unroll
+            for (int s = 0; s < 16; ++s) b[s] = next[s];
+            if (l > 1) load_slice(slices, l - 1, wave, lane, next);
+        } else {
+            load_slice(slices, l, wave, lane, b);
+        }
+        if (active) tile_product<kRT>(H, K, lane, b, slice_of(slices, l, wave, lane), acc);
+        __syncthreads();
+        if (active) {
+            const float *pre = buf.pre[l - 1];
+            float *dz = buf.dz[l - 1];
+            const int cc = min(col, N - 1);
+#pragma unroll
+            for (int rt = 0; rt < kRT; ++rt) {
+                float z[16], v[16];
+#pragma unroll
+                for (int r = 0; r < 16; ++r)  // clamped rows: loads without branches
+                    z[r] = pre[static_cast<int64_t>(min(row0 + 32 * rt + tile_row(lane, r), n - 1)) * N + cc];
+#pragma unroll
+                for (int r = 0; r < 16; ++r) v[r] = acc[rt][r] * gelu_grad_exp2(z[r]);
+#pragma unroll
+                for (int r = 0; r < 16; ++r) {
+                    const int row = 32 * rt + tile_row(lane, r);
+                    const bool in = row0 + row < n && col < N;
+                    H[row][col] = in ? v[r] : 0.f;
+                    if (in) dz[static_cast<int64_t>(row0 + row) * N + col] = v[r];
+                }
+            }
+        }
+        __syncthreads();
+    }
+}
+
+// Weight and bias gradients, dW_l = dZ_l^T act_l and db_l = column sums of
+// dZ_l: block (split, l) sums its share of the rows into its own copy of the
+// parameter layout.  As single 128 x 128 products these ran on four blocks with
+// the rows in series: 3.1 of the 3.7 ms of a 4,096-row gradient, 0.021 ms here.  The rows are the long dimension (a 128 x 128 product over
+// thousands of them), so they are split until the blocks fill the chip, and
+// both operands go from memory straight into registers: a lane's values of one
+// row are 32 consecutive columns.  Wave w owns columns 32 w .. of act_l.
+__global__ void __launch_bounds__(256, 2)
+mlp_weight_gradient_kernel(int n, int chunk, FusedNet net, FusedBuffers buf, int64_t n_params,
+                           float *__restrict__ partial)
+{
+    const int t = threadIdx.x, lane = t & 63, wave = t >> 6, c = lane & 31, h = lane >> 5;
+    const int l = blockIdx.y, K = net.in[l], N = net.out[l];
+    if (32 * wave >= K) return;  // whole waves, no barrier below
+    const float *dz = buf.dz[l], *act = buf.act[l];
+    const int i = 32 * wave + c;
+    const int64_t r1 = min(static_cast<int64_t>(n), static_cast<int64_t>(blockIdx.x + 1) * chunk);
+    f32x16 acc[4];
+    double sum[4];  // bias gradients: long sums of one sign, in 64 bits
+#pragma unroll
+    for (int rt = 0; rt < 4; ++rt) {
+        sum[rt] = 0.0;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) acc[rt][r] = 0.f;
+    }
+    constexpr int kU = 4;  // pairs of rows in flight
+    for (int64_t r0 = static_cast<int64_t>(blockIdx.x) * chunk; r0 < r1; r0 += 2 * kU) {
+        float a[kU][4], b[kU];
+#pragma unroll
+        for (int u = 0; u < kU; ++u) {  // clamped addresses, zeros selected below
+            const int64_t r = min(r0 + 2 * u + h, r1 - 1);
+            b[u] = act[r * K + min(i, K - 1)];
+#pragma unroll
+            for (int rt = 0; rt < 4; ++rt) a[u][rt] = dz[r * N + min(32 * rt + c, N - 1)];
+        }
+#pragma unroll
+        for (int u = 0; u < kU; ++u) {
+            const bool in = r0 + 2 * u + h < r1;
+            b[u] = in && i < K ? b[u] : 0.f;
+#pragma unroll
+            for (int rt = 0; rt < 4; ++rt) a[u][rt] = in && 32 * rt + c < N ? a[u][rt] : 0.f;
+        }
+#pragma unroll
+        for (int u = 0; u < kU; ++u)
+#pragma unroll
+            for (int rt = 0; rt < 4; ++rt) {
+                if (32 * rt >= N) continue;
+                acc[rt] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[u][rt], b[u], acc[rt], 0, 0, 0);
+                if (wave == 0) sum[rt] += static_cast<double>(a[u][rt]);
+            }
+    }
+    float *out = partial + static_cast<int64_t>(blockIdx.x) * n_params;
+#pragma unroll
+    for (int rt = 0; rt < 4; ++rt) {
+        if (32 * rt >= N) continue;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+            const int o = 32 * rt + tile_row(lane, r);
+            if (o < N && i < K) out[net.w[l] + o * K + i] = acc[rt][r];
+        }
+        const double both = sum[rt] + __shfl_xor(sum[rt], 32);
+        if (wave == 0 && h == 0 && 32 * rt + c < N) out[net.b[l] + 32 * rt + c] = static_cast<float>(both);
+    }
+}
+
+// grads = the splits' partial gradients added in order
+__global__ void __launch_bounds__(256) gradient_sum_kernel(int64_t n_params, int splits,
+                                                          const float *__restrict__ partial, float *__restrict__ grads)
+{
+    const int64_t p = blockIdx.x * static_cast<int64_t>(blockDim.x) + threadIdx.x;
+    if (p >= n_params) return;
+    double acc = 0.0;
+#pragma unroll 8
+    for (int s = 0; s < splits; ++s) acc += static_cast<double>(partial[s * n_params + p]);
+    grads[p] = static_cast<float>(acc);
+}
+
 unsigned blocks_for(int64_t n) { return static_cast<unsigned>(std::max<int64_t>(1, std::min<int64_t>((n + 255) / 256, 4096))); }
 
 }  // namespace
@@ -375,16 +816,22 @@ struct Mlp {
     int64_t n_params = 0;
     DevBuf<float> params, grads, adam_m, adam_v, shift, scale;
     int adam_t = 0;
-    int capacity = 0;
+    int capacity = 0, layer_capacity = 0;
     std::vector<DevBuf<float>> pre, act;  // pre[l]: n x out_l ; act[l]: n x in_l (act[0] = input)
     DevBuf<float> dY, dA, dB, partial, out;
+    // the fused network's dZ of every layer and the splits' partial gradients,
+    // and the host arrays' device copies of one call (grown, kept)
+    std::vector<DevBuf<float>> dz;
+    DevBuf<float> gpartial, raw;
+    int train_capacity = 0;
     DevBuf<float> data_x, data_t;
     DevBuf<double> dload;  // per-mesh load increments of the last warm start
     int n_data = 0;
     // inference precision (OC_FP32 or OC_BF16); bf16 weights are converted
     // from params whenever params changed since the last conversion
     int infer_precision = OC_FP32;
-    uint64_t params_version = 1, bf16_version = 0;
+    uint64_t params_version = 1, bf16_version = 0, slices_version = 0, back_slices_version = 0;
+    DevBuf<float> slices;
     DevBuf<uint16_t> wbf, xb, hb0, hb1;
     std::vector<int64_t> wbf_off;
     int bf_capacity = 0;
@@ -392,23 +839,167 @@ struct Mlp {
 
     int layers() const { return static_cast<int>(in_dim.size()); }
 
+    // the fused kernels serve this network
+    bool fused() const
+    {
+        return layers() <= kFusedLayers && std::max(n_in, std::max(n_hidden, n_out)) <= kFusedMax;
+    }
+    FusedNet fused_net() const
+    {
+        FusedNet f{};
+        f.layers = layers();
+        for (int l = 0; l < layers(); ++l) {
+            f.in[l] = in_dim[l];
+            f.out[l] = out_dim[l];
+            f.w[l] = static_cast<int>(w_off[l]);
+            f.b[l] = static_cast<int>(b_off[l]);
+        }
+        return f;
+    }
+    FusedBuffers fused_buffers() const
+    {
+        FusedBuffers f{};
+        for (int l = 0; l < layers(); ++l) {
+            f.pre[l] = pre[l].ptr;
+            f.act[l] = act[l].ptr;
+            f.dz[l] = static_cast<size_t>(l) < dz.size() ? dz[l].ptr : nullptr;
+        }
+        return f;
+    }
+
+    // input and output rows; every layer's arrays where inference needs them
     int ensure_capacity(int n)
     {
-        if (n <= capacity) return OC_NO_ERROR;
         const int L = layers();
         pre.resize(L);
         act.resize(L);
+        if (n > capacity) {
+            capacity = 0;
+            OC_CHECK(act[0].alloc(static_cast<size_t>(n) * n_in));
+            OC_CHECK(out.alloc(static_cast<size_t>(n) * n_out));
+            if (!partial.ptr) OC_CHECK(partial.alloc(4096));
+            capacity = n;
+        }
+        const bool per_layer = !fused() || infer_precision == OC_BF16_HIDDEN;
+        return per_layer ? ensure_layers(n) : OC_NO_ERROR;
+    }
+    int ensure_layers(int n)
+    {
+        if (n <= layer_capacity) return OC_NO_ERROR;
+        layer_capacity = 0;
+        const int L = layers();
         for (int l = 0; l < L; ++l) {
             OC_CHECK(pre[l].alloc(static_cast<size_t>(n) * out_dim[l]));
-            OC_CHECK(act[l].alloc(static_cast<size_t>(n) * in_dim[l]));
+            if (l > 0) OC_CHECK(act[l].alloc(static_cast<size_t>(n) * in_dim[l]));
         }
-        int wmax = std::max(n_hidden, std::max(n_in, n_out));
-        OC_CHECK(dY.alloc(static_cast<size_t>(n) * wmax));
-        OC_CHECK(dA.alloc(static_cast<size_t>(n) * wmax));
-        OC_CHECK(dB.alloc(static_cast<size_t>(n) * wmax));
-        OC_CHECK(out.alloc(static_cast<size_t>(n) * n_out));
-        OC_CHECK(partial.alloc(4096));
-        capacity = n;
+        layer_capacity = n;
+        return OC_NO_ERROR;
+    }
+    // what a gradient of n rows needs beside them
+    int ensure_training(int n)
+    {
+        OC_CHECK(ensure_capacity(n));
+        OC_CHECK(ensure_layers(n));
+        if (fused()) {
+            const size_t blocks = (static_cast<size_t>(n) + 31) / 32;
+            if (partial.n < blocks) OC_CHECK(partial.alloc(blocks));
+            const size_t gp = static_cast<size_t>(gradient_splits(n)) * n_params;
+            if (gpartial.n < gp) OC_CHECK(gpartial.alloc(gp));
+        }
+        if (n <= train_capacity) return OC_NO_ERROR;
+        train_capacity = 0;
+        const int L = layers();
+        if (fused()) {
+            dz.resize(L);
+            for (int l = 0; l < L; ++l) OC_CHECK(dz[l].alloc(static_cast<size_t>(n) * out_dim[l]));
+        } else {
+            const int wmax = std::max(n_hidden, std::max(n_in, n_out));
+            OC_CHECK(dY.alloc(static_cast<size_t>(n) * wmax));
+            OC_CHECK(dA.alloc(static_cast<size_t>(n) * wmax));
+            OC_CHECK(dB.alloc(static_cast<size_t>(n) * wmax));
+        }
+        train_capacity = n;
+        return OC_NO_ERROR;
+    }
+    // rows per block of the weight gradient: 64 fill the chip from a few
+    // thousand rows on (five layers x 64 splits), and 64 splits at most bound
+    // the partial gradients
+    static int gradient_chunk(int n) { return std::max(64, ((n + 63) / 64 + 1) & ~1); }
+    static int gradient_splits(int n) { return (n + gradient_chunk(n) - 1) / gradient_chunk(n); }
+
+    // Host arrays of a call: up to kPinnedBytes in all go through one pinned
+    // buffer of the network and asynchronous copies on the library stream (two
+    // pageable copies each way cost a 4,096-sample gradient 70 us beside 82 us
+    // of kernels); larger ones are copied as they are.  The device copy and the
+    // pinned buffer are grown and kept.
+    static constexpr size_t kPinnedBytes = size_t(4) << 20;
+    char *pinned = nullptr;
+    size_t pinned_n = 0;
+    bool pinned_busy = false;  // a copy out of it is queued (a call that failed before its fetch leaves it so)
+    Mlp() = default;
+    Mlp(const Mlp &) = delete;
+    Mlp &operator=(const Mlp &) = delete;
+    ~Mlp()
+    {
+        if (pinned) (void)hipHostFree(pinned);
+    }
+    int ensure_pinned(size_t bytes)
+    {
+        if (bytes <= pinned_n) return OC_NO_ERROR;
+        if (pinned) (void)hipHostFree(pinned);
+        pinned = nullptr;
+        pinned_n = 0;
+        void *p = nullptr;
+        OC_HIP_CHECK(hipHostMalloc(&p, bytes, hipHostMallocDefault));
+        pinned = static_cast<char *>(p);
+        pinned_n = bytes;
+        return OC_NO_ERROR;
+    }
+    // a (na floats), then b (nb floats) into raw
+    int stage(const float *a, size_t na, const float *b, size_t nb)
+    {
+        Runtime &rt = runtime();
+        const size_t bytes = (na + nb) * sizeof(float);
+        if (raw.n < na + nb) {
+            OC_HIP_CHECK(hipStreamSynchronize(rt.stream));
+            OC_CHECK(raw.alloc(na + nb));
+        }
+        if (bytes <= kPinnedBytes) {
+            if (pinned_busy) OC_HIP_CHECK(hipStreamSynchronize(rt.stream));
+            OC_CHECK(ensure_pinned(bytes));
+            std::memcpy(pinned, a, na * sizeof(float));
+            if (nb) std::memcpy(pinned + na * sizeof(float), b, nb * sizeof(float));
+            pinned_busy = true;
+            OC_HIP_CHECK(hipMemcpyAsync(raw.ptr, pinned, bytes, hipMemcpyHostToDevice, rt.stream));
+            return OC_NO_ERROR;
+        }
+        OC_HIP_CHECK(hipStreamSynchronize(rt.stream));  // kernels in flight may read the last call's
+        OC_HIP_CHECK(hipMemcpy(raw.ptr, a, na * sizeof(float), hipMemcpyHostToDevice));
+        if (nb) OC_HIP_CHECK(hipMemcpy(raw.ptr + na, b, nb * sizeof(float), hipMemcpyHostToDevice));
+        return OC_NO_ERROR;
+    }
+    // device arrays a (na floats) and b to the host, after everything queued;
+    // synchronises, so the pinned buffer is free again
+    int fetch(float *a, const float *a_dev, size_t na, float *b, const float *b_dev, size_t nb)
+    {
+        Runtime &rt = runtime();
+        const size_t bytes = (na + nb) * sizeof(float);
+        if (bytes <= kPinnedBytes) {
+            if (bytes > pinned_n) OC_HIP_CHECK(hipStreamSynchronize(rt.stream));  // its copy may be in flight
+            OC_CHECK(ensure_pinned(bytes));
+            OC_HIP_CHECK(hipMemcpyAsync(pinned, a_dev, na * sizeof(float), hipMemcpyDeviceToHost, rt.stream));
+            if (nb)
+                OC_HIP_CHECK(hipMemcpyAsync(pinned + na * sizeof(float), b_dev, nb * sizeof(float),
+                                            hipMemcpyDeviceToHost, rt.stream));
+            OC_HIP_CHECK(hipStreamSynchronize(rt.stream));
+            pinned_busy = false;
+            std::memcpy(a, pinned, na * sizeof(float));
+            if (nb) std::memcpy(b, pinned + na * sizeof(float), nb * sizeof(float));
+            return OC_NO_ERROR;
+        }
+        OC_HIP_CHECK(hipStreamSynchronize(rt.stream));
+        OC_HIP_CHECK(hipMemcpy(a, a_dev, na * sizeof(float), hipMemcpyDeviceToHost));
+        if (nb) OC_HIP_CHECK(hipMemcpy(b, b_dev, nb * sizeof(float), hipMemcpyDeviceToHost));
         return OC_NO_ERROR;
     }
 
@@ -421,10 +1012,70 @@ struct Mlp {
         return OC_NO_ERROR;
     }
 
-    // act[0] must hold the normalised input; result in pre[L-1]
-    int forward(int n)
+    const float4 *forward_slices() const { return reinterpret_cast<const float4 *>(slices.ptr); }
+    size_t slice_count() const { return static_cast<size_t>(layers()) * kSliceLayer; }
+    // the operand slices of the current parameters; the backward pass's follow
+    // the forward pass's
+    int pack_slices(bool train)
+    {
+        Runtime &rt = runtime();
+        if (!slices.ptr) OC_CHECK(slices.alloc(2 * 4 * slice_count()));
+        float4 *p = reinterpret_cast<float4 *>(slices.ptr);
+        const unsigned blocks = static_cast<unsigned>((slice_count() + 255) / 256);
+        if (slices_version != params_version) {
+            pack_slices_kernel<false><<<blocks, 256, 0, rt.stream>>>(fused_net(), params.ptr, p);
+            OC_HIP_CHECK(hipGetLastError());
+            slices_version = params_version;
+        }
+        if (train && back_slices_version != params_version) {
+            pack_slices_kernel<true><<<blocks, 256, 0, rt.stream>>>(fused_net(), params.ptr, p + slice_count());
+            OC_HIP_CHECK(hipGetLastError());
+            back_slices_version = params_version;
+        }
+        return OC_NO_ERROR;
+    }
+
+    // One launch for the whole network (the fused kernels' limits).  64 rows
+    // per block read each weight slice once per 64 rows; below two blocks per CU
+    // of them, 32-row blocks spread the rows over twice as many CUs.
+    template <bool kTrain>
+    int launch_fused(int n, const float *x, const float *sh, const float *sc)
+    {
+        Runtime &rt = runtime();
+        OC_CHECK(pack_slices(kTrain));
+        if (static_cast<int64_t>(n) >= static_cast<int64_t>(rt.num_cus) * 2 * 64)
+            mlp_fused_forward_kernel<2, kTrain><<<static_cast<unsigned>((n + 63) / 64), 256, 0, rt.stream>>>(
+                n, fused_net(), params.ptr, forward_slices(), x, sh, sc, fused_buffers(), out.ptr);
+        else
+            mlp_fused_forward_kernel<1, kTrain><<<static_cast<unsigned>((n + 31) / 32), 256, 0, rt.stream>>>(
+                n, fused_net(), params.ptr, forward_slices(), x, sh, sc, fused_buffers(), out.ptr);
+        OC_HIP_CHECK(hipGetLastError());
+        return OC_NO_ERROR;
+    }
+
+    // FP32 outputs in `out` from n rows of raw (sh and sc given) or normalised
+    // inputs x; the layer-by-layer path keeps every layer's arrays, the fused
+    // one only with `train`
+    int forward(int n, const float *x, const float *sh, const float *sc, bool train)
     {
         KernelTimer timer("mlp_forward");
+        if (fused()) return train ? launch_fused<true>(n, x, sh, sc) : launch_fused<false>(n, x, sh, sc);
+        if (sh) OC_CHECK(normalise(n, x));
+        return forward_layers(n);
+    }
+    // act[0] = (x - shift) * scale
+    int normalise(int n, const float *x)
+    {
+        normalise_kernel<<<static_cast<unsigned>((n + 255) / 256), 256, 0, runtime().stream>>>(n, n_in, x, shift.ptr,
+                                                                                              scale.ptr, act[0].ptr);
+        OC_HIP_CHECK(hipGetLastError());
+        return OC_NO_ERROR;
+    }
+
+    // networks wider than the fused kernels take: act[0] holds the normalised
+    // input; one GEMM and one bias/GELU pass per layer
+    int forward_layers(int n)
+    {
         const int L = layers();
         Runtime &rt = runtime();
         for (int l = 0; l < L; ++l) {
@@ -501,7 +1152,7 @@ struct Mlp {
     {
         KernelTimer timer("mlp_forward_bf16_hidden");
         const int L = layers();
-        if (L < 3) return forward(n);
+        if (L < 3) return forward(n, act[0].ptr, nullptr, nullptr, false);
         Runtime &rt = runtime();
         OC_CHECK(prepare_bf16(n));
         auto fp32_layer = [&](int l, const float *in, float *h, int act) -> int {
@@ -533,11 +1184,12 @@ struct Mlp {
         return fp32_layer(L - 1, act[L - 1].ptr, out.ptr, 0);
     }
 
-    int infer(int n)
+    // outputs of n rows of raw (sh and sc given) or normalised inputs
+    int infer(int n, const float *x, const float *sh, const float *sc)
     {
-        if (infer_precision == OC_BF16) return forward_bf16(n);
-        if (infer_precision == OC_BF16_HIDDEN) return forward_bf16_hidden(n);
-        return forward(n);
+        if (infer_precision == OC_FP32) return forward(n, x, sh, sc, false);
+        if (sh) OC_CHECK(normalise(n, x));
+        return infer_precision == OC_BF16 ? forward_bf16(n) : forward_bf16_hidden(n);
     }
 
     // after forward(n) with targets T on device: gradients into grads, loss partials into partial
@@ -546,6 +1198,27 @@ struct Mlp {
         KernelTimer timer("mlp_backward");
         const int L = layers();
         Runtime &rt = runtime();
+        if (fused()) {
+            // row tiles as the forward pass, then the split weight gradients
+            const bool big = static_cast<int64_t>(n) >= static_cast<int64_t>(rt.num_cus) * 2 * 64;
+            const int rows = big ? 64 : 32, blocks = (n + rows - 1) / rows;
+            if (big)
+                mlp_fused_backward_kernel<2><<<static_cast<unsigned>(blocks), 256, 0, rt.stream>>>(
+                    n, fused_net(), forward_slices() + slice_count(), out.ptr, T, fused_buffers(), partial.ptr);
+            else
+                mlp_fused_backward_kernel<1><<<static_cast<unsigned>(blocks), 256, 0, rt.stream>>>(
+                    n, fused_net(), forward_slices() + slice_count(), out.ptr, T, fused_buffers(), partial.ptr);
+            OC_HIP_CHECK(hipGetLastError());
+            const int splits = gradient_splits(n);
+            mlp_weight_gradient_kernel<<<dim3(splits, L), 256, 0, rt.stream>>>(n, gradient_chunk(n), fused_net(),
+                                                                              fused_buffers(), n_params, gpartial.ptr);
+            OC_HIP_CHECK(hipGetLastError());
+            gradient_sum_kernel<<<static_cast<unsigned>((n_params + 255) / 256), 256, 0, rt.stream>>>(
+                n_params, splits, gpartial.ptr, grads.ptr);
+            OC_HIP_CHECK(hipGetLastError());
+            *n_partials = blocks;
+            return OC_NO_ERROR;
+        }
         const int64_t cnt = static_cast<int64_t>(n) * n_out;
         const unsigned nb = std::min<unsigned>(blocks_for(cnt), 1024);
         mse_kernel<<<nb, 256, 0, rt.stream>>>(cnt, out.ptr, T, dY.ptr, partial.ptr);
@@ -717,15 +1390,9 @@ int oc_mlp_forward(oc_mlp mlp, int n, const float *x, float *y)
     if (!mlp || !x || !y || n < 1) return set_error(OC_ERR_INVALID_ARGUMENT, "oc_mlp_forward: invalid arguments");
     Mlp &m = mlp->m;
     OC_CHECK(m.ensure_capacity(n));
-    Runtime &rt = runtime();
-    DevBuf<float> raw;
-    OC_CHECK(raw.upload(x, static_cast<size_t>(n) * m.n_in));
-    normalise_kernel<<<blocks_for(n), 256, 0, rt.stream>>>(n, m.n_in, raw.ptr, m.shift.ptr, m.scale.ptr, m.act[0].ptr);
-    OC_HIP_CHECK(hipGetLastError());
-    OC_CHECK(m.infer(n));
-    OC_HIP_CHECK(hipStreamSynchronize(rt.stream));
-    OC_HIP_CHECK(hipMemcpy(y, m.out.ptr, sizeof(float) * n * m.n_out, hipMemcpyDeviceToHost));
-    return OC_NO_ERROR;
+    OC_CHECK(m.stage(x, static_cast<size_t>(n) * m.n_in, nullptr, 0));
+    OC_CHECK(m.infer(n, m.raw.ptr, m.shift.ptr, m.scale.ptr));
+    return m.fetch(y, m.out.ptr, static_cast<size_t>(n) * m.n_out, nullptr, nullptr, 0);
 }
 
 int oc_mlp_gradient(oc_mlp mlp, int n, const float *x, const float *t, float *loss, float *gradient)
@@ -734,23 +1401,17 @@ int oc_mlp_gradient(oc_mlp mlp, int n, const float *x, const float *t, float *lo
     if (!mlp || !x || !t || !loss || !gradient || n < 1)
         return set_error(OC_ERR_INVALID_ARGUMENT, "oc_mlp_gradient: invalid arguments");
     Mlp &m = mlp->m;
-    OC_CHECK(m.ensure_capacity(n));
-    Runtime &rt = runtime();
-    DevBuf<float> raw, tt;
-    OC_CHECK(raw.upload(x, static_cast<size_t>(n) * m.n_in));
-    OC_CHECK(tt.upload(t, static_cast<size_t>(n) * m.n_out));
-    normalise_kernel<<<blocks_for(n), 256, 0, rt.stream>>>(n, m.n_in, raw.ptr, m.shift.ptr, m.scale.ptr, m.act[0].ptr);
-    OC_HIP_CHECK(hipGetLastError());
-    OC_CHECK(m.forward(n));
+    OC_CHECK(m.ensure_training(n));
+    const size_t nx = static_cast<size_t>(n) * m.n_in;
+    OC_CHECK(m.stage(x, nx, t, static_cast<size_t>(n) * m.n_out));
+    OC_CHECK(m.forward(n, m.raw.ptr, m.shift.ptr, m.scale.ptr, true));
     int np = 0;
-    OC_CHECK(m.backward(n, tt.ptr, &np));
-    OC_HIP_CHECK(hipStreamSynchronize(rt.stream));
+    OC_CHECK(m.backward(n, m.raw.ptr + nx, &np));
     std::vector<float> part(np);
-    OC_HIP_CHECK(hipMemcpy(part.data(), m.partial.ptr, sizeof(float) * np, hipMemcpyDeviceToHost));
+    OC_CHECK(m.fetch(gradient, m.grads.ptr, static_cast<size_t>(m.n_params), part.data(), m.partial.ptr, part.size()));
     double acc = 0.0;
     for (float v : part) acc += v;
     *loss = static_cast<float>(acc / (static_cast<double>(n) * m.n_out));
-    OC_HIP_CHECK(hipMemcpy(gradient, m.grads.ptr, sizeof(float) * m.n_params, hipMemcpyDeviceToHost));
     return OC_NO_ERROR;
 }
 
@@ -771,9 +1432,9 @@ int oc_mlp_train(oc_mlp mlp, int steps, int batch, float learning_rate, unsigned
     if (!mlp || steps < 1 || batch < 1 || !mean_loss) return set_error(OC_ERR_INVALID_ARGUMENT, "oc_mlp_train: invalid arguments");
     Mlp &m = mlp->m;
     if (m.n_data < 1) return set_error(OC_ERR_INVALID_ARGUMENT, "oc_mlp_train: no dataset");
-    OC_CHECK(m.ensure_capacity(batch));
+    OC_CHECK(m.ensure_training(batch));
     Runtime &rt = runtime();
-    DevBuf<float> bt, losses;
+    DevBuf<float> bt;
     OC_CHECK(bt.alloc(static_cast<size_t>(batch) * m.n_out));
     std::vector<float> part;
     double total = 0.0;
@@ -782,7 +1443,7 @@ int oc_mlp_train(oc_mlp mlp, int steps, int batch, float learning_rate, unsigned
                                                                       m.data_x.ptr, m.data_t.ptr, m.shift.ptr,
                                                                       m.scale.ptr, m.act[0].ptr, bt.ptr);
         OC_HIP_CHECK(hipGetLastError());
-        OC_CHECK(m.forward(batch));
+        OC_CHECK(m.forward(batch, m.act[0].ptr, nullptr, nullptr, true));
         int np = 0;
         OC_CHECK(m.backward(batch, bt.ptr, &np));
         OC_CHECK(m.adam(learning_rate));
@@ -832,7 +1493,7 @@ int oc_mlp_warm_start_batch(oc_mlp mlp, oc_equations_set h, const double *load_i
                                                                 m.dload.ptr, s.node_mat.ptr, m.shift.ptr, m.scale.ptr,
                                                                 m.act[0].ptr);
     OC_HIP_CHECK(hipGetLastError());
-    OC_CHECK(m.infer(nq));
+    OC_CHECK(m.infer(nq, m.act[0].ptr, nullptr, nullptr));
     warm_apply_kernel<<<blocks_for(nq), 256, 0, rt.stream>>>(nq, m.out.ptr, m.n_out, M, s.q_off.ptr, m.dload.ptr,
                                                              s.free_mask.ptr, s.dofs.ptr);
     OC_HIP_CHECK(hipGetLastError());
