@@ -31,12 +31,6 @@ __global__ void __launch_bounds__(256) axpby_kernel(int n, double a, const doubl
         y[i] = a * x[i] + b * y[i];
 }
 
-__global__ void __launch_bounds__(256) copy_scale_kernel(int n, double a, const double *__restrict__ x,
-                                                        double *__restrict__ y)
-{
-    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) y[i] = a * x[i];
-}
-
 __global__ void __launch_bounds__(256) scale_kernel(int n, const double *__restrict__ w, double *__restrict__ y)
 {
     for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) y[i] = w[i] * y[i];
@@ -121,10 +115,8 @@ __global__ void __launch_bounds__(256) mesh_axpy_kernel(const int *__restrict__ 
 // partial[j * gridDim.x + blockIdx.x] = sum over this block's slice of V_j . w
 // for j = 0..k-1 (blockIdx.y = j).  Deterministic: fixed grid, fixed tree.
 __global__ void __launch_bounds__(256) multi_dot_kernel(int n, const double *__restrict__ V, int64_t ldv,
-                                                       const double *__restrict__ w, double *__restrict__ partial,
-                                                       const double *__restrict__ gate)
+                                                       const double *__restrict__ w, double *__restrict__ partial)
 {
-    if (gate && *gate == 0.0) return;  // a pass the Arnoldi process did not ask for
     __shared__ double s[256];
     const double *v = V + static_cast<int64_t>(blockIdx.y) * ldv;
     double acc = 0.0;
@@ -158,116 +150,268 @@ __global__ void __launch_bounds__(256) combine_kernel(int n, int k, const double
 // Classical Gram-Schmidt with one reorthogonalisation pass when the projection
 // removes more than 3/4 of |w|^2 (CGS2), and Givens rotations of the
 // Hessenberg column, all without a host round trip.  Layout of the state for
-// restart m: R (m x m, row-major, column j written by step j), h and h2 (m+2),
-// cs, sn (m), g (m+1), then flag, hn and 1/hn.
+// restart m: R (m x m, row-major, column j written by step j), h (m+2), cs, sn
+// (m), g (m+1), then flag and hn.
+//
+// A step is three launches: the partial dot products; the projection, whose
+// blocks each add the partials up themselves and, when a second pass is due,
+// form its partial dot products from the rows they have just written; and that
+// second pass with the rotations.  As ten launches (the reductions, gates,
+// norm, rotations and scaling each on their own) a step was bound by launches
+// and by single-block serial sums: 9 + 8 + 7 us of them at 23,800 rows, 62 us
+// an iteration of the Laplace solve there against 26 now.  What bounds it still
+// is the latency of four dependent launches (3 to 7 us each).
 struct Arnoldi {
-    double *R, *h, *h2, *cs, *sn, *g, *flag, *hn, *inv;
-    static size_t size(int m) { return static_cast<size_t>(m) * m + 2 * (m + 2) + 2 * m + (m + 1) + 3; }
+    double *R, *h, *cs, *sn, *g, *flag, *hn;
+    static size_t size(int m) { return static_cast<size_t>(m) * m + (m + 2) + 2 * m + (m + 1) + 2; }
     static Arnoldi at(double *base, int m)
     {
         Arnoldi a;
         a.R = base;
         a.h = a.R + static_cast<size_t>(m) * m;
-        a.h2 = a.h + m + 2;
-        a.cs = a.h2 + m + 2;
+        a.cs = a.h + m + 2;
         a.sn = a.cs + m;
         a.g = a.sn + m;
         a.flag = a.g + m + 1;
         a.hn = a.flag + 1;
-        a.inv = a.hn + 1;
         return a;
     }
 };
+constexpr int kDotVectors = 8;               // vectors per block of partial dot products
+constexpr int kMaxDots = 1024 + kDotVectors;  // restart + 1 of them at most, rounded up
 
-// sum of the kReduceBlocks partials of dot product i, in block order
-__device__ __forceinline__ double partial_sum(const double *__restrict__ partial, int i)
+// the point-Jacobi and weight scaling z_i = iw_i (inv_i v_i) of a basis vector,
+// written with the vector itself when inv is given
+struct ScaledCopy {
+    const double *inv, *iw;
+    double *z;
+};
+__device__ __forceinline__ void basis_store(double *v, int i, double x, const ScaledCopy &sc)
+{
+    v[i] = x;
+    if (sc.inv) sc.z[i] = sc.iw[i] * (sc.inv[i] * x);
+}
+
+// eight sums over the wavefront in ten shuffles (halving the vectors kept per
+// lane three times, then a butterfly of one): lane l returns the total of v[l / 8]
+__device__ __forceinline__ double wave_sum8(double (&v)[8], int lane)
+{
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+        const bool up = lane & 32;
+        const double keep = up ? v[k + 4] : v[k], send = up ? v[k] : v[k + 4];
+        v[k] = keep + __shfl_xor(send, 32);
+    }
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {
+        const bool up = lane & 16;
+        const double keep = up ? v[k + 2] : v[k], send = up ? v[k] : v[k + 2];
+        v[k] = keep + __shfl_xor(send, 16);
+    }
+    const bool up = lane & 8;
+    double t = (up ? v[1] : v[0]) + __shfl_xor(up ? v[0] : v[1], 8);
+#pragma unroll
+    for (int o = 4; o > 0; o >>= 1) t += __shfl_xor(t, o);
+    return t;
+}
+
+// this block's partials of V_j0..V_{j0+7} . w (those below count) over the rows
+// it owns, i = blockIdx.x * kT + thread, stepping by gridDim.x * kT:
+// partial[j * kReduceBlocks + blockIdx.x].  s: kT / 64 * 8 doubles.
+template <int kT>
+__device__ __forceinline__ void block_dots(int n, int j0, int count, const double *V, int64_t ldv,
+                                           const double *w, double *s, double *__restrict__ partial)
+{
+    const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+    double acc[kDotVectors];
+#pragma unroll
+    for (int k = 0; k < kDotVectors; ++k) acc[k] = 0.0;
+    for (int i = blockIdx.x * kT + t; i < n; i += gridDim.x * kT) {
+        const double wi = w[i];
+        double v[kDotVectors];
+#pragma unroll
+        for (int k = 0; k < kDotVectors; ++k) v[k] = j0 + k < count ? V[static_cast<int64_t>(j0 + k) * ldv + i] : 0.0;
+#pragma unroll
+        for (int k = 0; k < kDotVectors; ++k) acc[k] += v[k] * wi;
+    }
+    const double tot = wave_sum8(acc, lane);
+    __syncthreads();  // s is free
+    if ((lane & 7) == 0) s[wave * kDotVectors + (lane >> 3)] = tot;
+    __syncthreads();
+    if (t < kDotVectors && j0 + t < count) {
+        double sum = 0.0;
+#pragma unroll
+        for (int q = 0; q < kT / 64; ++q) sum += s[q * kDotVectors + t];
+        partial[static_cast<size_t>(j0 + t) * kReduceBlocks + blockIdx.x] = sum;
+    }
+}
+
+// dots[j] = sum of the n_parts partials of dot product j < count, in the same
+// order in every block; a wavefront takes eight of them at a time
+template <int kT>
+__device__ __forceinline__ void reduce_partials(int count, int n_parts, const double *__restrict__ partial,
+                                                double *dots)
+{
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    for (int j0 = wave * kDotVectors; j0 < count; j0 += kT / 64 * kDotVectors) {
+        double v[kDotVectors];
+#pragma unroll
+        for (int k = 0; k < kDotVectors; ++k) {
+            double p[kReduceBlocks / 64];
+#pragma unroll
+            for (int q = 0; q < kReduceBlocks / 64; ++q)
+                p[q] = (j0 + k < count && lane + 64 * q < n_parts)
+                           ? partial[static_cast<size_t>(j0 + k) * kReduceBlocks + lane + 64 * q]
+                           : 0.0;
+            v[k] = p[0];
+#pragma unroll
+            for (int q = 1; q < kReduceBlocks / 64; ++q) v[k] += p[q];
+        }
+        const double tot = wave_sum8(v, lane);
+        if ((lane & 7) == 0) dots[j0 + (lane >> 3)] = tot;
+    }
+    __syncthreads();
+}
+
+// sum of squares of x[0..count), the same in every wavefront
+__device__ __forceinline__ double wave_square_sum(const double *x, int count)
+{
+    double q = 0.0;
+    for (int i = threadIdx.x & 63; i < count; i += 64) q += x[i] * x[i];
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) q += __shfl_xor(q, o);
+    return q;
+}
+
+// w_i - sum_{k<count} h_k V_k,i, k ascending, eight loads in flight
+__device__ __forceinline__ double projected(const double *__restrict__ V, int64_t ldv, int count, const double *h,
+                                            int i, double wi)
 {
     double acc = 0.0;
-    for (int b = 0; b < kReduceBlocks; ++b) acc += partial[static_cast<size_t>(i) * kReduceBlocks + b];
-    return acc;
+    int k = 0;
+    for (; k + 8 <= count; k += 8) {
+        double v[8];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) v[u] = V[static_cast<int64_t>(k + u) * ldv + i];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) acc += h[k + u] * v[u];
+    }
+    for (; k < count; ++k) acc += h[k] * V[static_cast<int64_t>(k) * ldv + i];
+    return wi - acc;
 }
 
-// g = (beta, 0, ..., 0)
-__global__ void __launch_bounds__(256) arnoldi_start_kernel(int m, double beta, Arnoldi a)
+// V_0 = r / beta, g = (beta, 0, ..., 0)
+__global__ void __launch_bounds__(256) arnoldi_start_kernel(int n, int m, double beta, const double *__restrict__ r,
+                                                           double *__restrict__ v, ScaledCopy sc, Arnoldi a)
 {
-    for (int i = threadIdx.x; i <= m; i += blockDim.x) a.g[i] = i == 0 ? beta : 0.0;
+    const double inv = 1.0 / beta;
+    for (int i = blockIdx.x * 256 + threadIdx.x; i < n; i += gridDim.x * 256) basis_store(v, i, inv * r[i], sc);
+    if (blockIdx.x == 0)
+        for (int i = threadIdx.x; i <= m; i += 256) a.g[i] = i == 0 ? beta : 0.0;
 }
 
-// step j, first pass: h_i = V_i . w (i <= j), |w|^2 = h_{j+1}; asks for the
-// second pass or takes |w - V h| by Pythagoras
-__global__ void __launch_bounds__(256) arnoldi_project_kernel(int j, const double *__restrict__ partial, Arnoldi a)
+// step j: partials of V_0..V_j . w and w . w, w being V_{j+1}; blockIdx.y takes
+// eight vectors
+__global__ void __launch_bounds__(256) arnoldi_dots_kernel(int n, int count, const double *__restrict__ V,
+                                                          const double *__restrict__ w, double *__restrict__ partial)
 {
-    for (int i = threadIdx.x; i < j + 2; i += blockDim.x) a.h[i] = partial_sum(partial, i);
+    __shared__ double s[4 * kDotVectors];
+    block_dots<256>(n, blockIdx.y * kDotVectors, count, V, n, w, s, partial);
+}
+
+// step j, first pass: h_i = V_i . w, w -= V h.  |w|^2 after it follows by
+// Pythagoras unless cancellation asks for a second pass: without one V_{j+1} is
+// written normalised, with one w stays as it is and the blocks form the
+// partials of V_0..V_j . w and w . w over their rows into partial2.
+template <int kT>
+__global__ void __launch_bounds__(kT) arnoldi_project_kernel(int n, int j, int n_parts, double *V,
+                                                            const double *__restrict__ partial,
+                                                            double *__restrict__ partial2, ScaledCopy sc, Arnoldi a)
+{
+    __shared__ double s_h[kMaxDots];
+    __shared__ double s_red[kT / 64 * kDotVectors];
+    const int t = threadIdx.x;
+    reduce_partials<kT>(j + 2, n_parts, partial, s_h);
+    const double wn2 = s_h[j + 1], left = wn2 - wave_square_sum(s_h, j + 1);
+    const bool again = left < 0.25 * wn2;
+    const double hn = again ? 0.0 : sqrt(left);
+    double *w = V + static_cast<int64_t>(j + 1) * n;
+    const double scale = hn > 0.0 ? 1.0 / hn : 1.0;
+    for (int i = blockIdx.x * kT + t; i < n; i += gridDim.x * kT) {
+        const double x = projected(V, n, j + 1, s_h, i, w[i]);
+        if (again) w[i] = x;
+        else basis_store(w, i, scale * x, sc);
+    }
+    if (again)  // a thread's rows are those it has just written
+        for (int j0 = 0; j0 < j + 2; j0 += kDotVectors) block_dots<kT>(n, j0, j + 2, V, n, w, s_red, partial2);
+    if (blockIdx.x == 0) {
+        for (int i = t; i <= j; i += kT) a.h[i] = s_h[i];
+        if (t == 0) {
+            *a.flag = again ? 1.0 : 0.0;
+            *a.hn = hn;
+        }
+    }
+}
+
+// step j, last: the second pass where the first asked for it (h2 = V . w,
+// w -= V h2, its norm by Pythagoras: h2 is the rounding left by the first pass,
+// so nothing cancels), V_{j+1} normalised; and, in the last block, which owns
+// no rows, the rotations: R's column j, g, and the residual estimate |g_{j+1}|
+// and hn into the host-visible slots 2j, 2j+1.
+template <int kT>
+__global__ void __launch_bounds__(kT) arnoldi_finish_kernel(int n, int j, int m, int n_parts, double *V,
+                                                           const double *__restrict__ partial2, ScaledCopy sc,
+                                                           Arnoldi a, double *__restrict__ host)
+{
+    __shared__ double s_h[kMaxDots];
+    __shared__ double s_r[3 * kMaxDots];
+    const int t = threadIdx.x;
+    const bool again = *a.flag != 0.0, rotate = blockIdx.x == gridDim.x - 1;
+    double hn = 0.0;
+    if (again) {
+        reduce_partials<kT>(j + 2, n_parts, partial2, s_h);
+        hn = sqrt(fmax(s_h[j + 1] - wave_square_sum(s_h, j + 1), 0.0));
+    }
+    if (!rotate) {
+        if (!again) return;
+        double *w = V + static_cast<int64_t>(j + 1) * n;
+        const double scale = hn > 0.0 ? 1.0 / hn : 1.0;
+        const int rows = (gridDim.x - 1) * kT;
+        for (int i = blockIdx.x * kT + t; i < n; i += rows)
+            basis_store(w, i, scale * projected(V, n, j + 1, s_h, i, w[i]), sc);
+        return;
+    }
+    double *s_x = s_r, *s_cs = s_r + kMaxDots, *s_sn = s_r + 2 * kMaxDots;
+    if (!again) hn = *a.hn;
+    for (int i = t; i <= j; i += kT) {
+        s_x[i] = again ? a.h[i] + s_h[i] : a.h[i];
+        if (i < j) {
+            s_cs[i] = a.cs[i];
+            s_sn[i] = a.sn[i];
+        }
+    }
     __syncthreads();
-    if (threadIdx.x == 0) {
-        const double wn2 = a.h[j + 1];
-        double proj2 = 0.0;
-        for (int i = 0; i <= j; ++i) proj2 += a.h[i] * a.h[i];
-        const bool again = wn2 - proj2 < 0.25 * wn2;
-        *a.flag = again ? 1.0 : 0.0;
-        *a.hn = again ? 0.0 : sqrt(wn2 - proj2);
+    if (t == 0) {
+        double hi = s_x[0];
+        for (int i = 0; i < j; ++i) {
+            const double hi1 = s_x[i + 1], c = s_cs[i], sn = s_sn[i];
+            s_x[i] = c * hi + sn * hi1;
+            hi = -sn * hi + c * hi1;
+        }
+        // hi is the rotated h_j; h_{j+1} = hn
+        const double den = hypot(hi, hn);
+        const double c = den > 0.0 ? hi / den : 1.0, sgn = den > 0.0 ? hn / den : 0.0;
+        a.cs[j] = c;
+        a.sn[j] = sgn;
+        s_x[j] = den;
+        const double gj = a.g[j];
+        a.g[j + 1] = -sgn * gj;
+        a.g[j] = c * gj;
+        host[2 * j] = fabs(sgn * gj);
+        host[2 * j + 1] = hn;
     }
-}
-
-// step j, second pass (only with the flag set): h2_i = V_i . w, h_i += h2_i
-__global__ void __launch_bounds__(256) arnoldi_correct_kernel(int j, const double *__restrict__ partial, Arnoldi a)
-{
-    if (*a.flag == 0.0) return;
-    for (int i = threadIdx.x; i <= j; i += blockDim.x) {
-        const double c = partial_sum(partial, i);
-        a.h2[i] = c;
-        a.h[i] += c;
-    }
-}
-
-// w += sign * sum_{j<k} coef_j V_j, coefficients in device memory
-__global__ void __launch_bounds__(256) combine_device_kernel(int n, int k, const double *__restrict__ V, int64_t ldv,
-                                                            const double *__restrict__ coef, double sign,
-                                                            double *__restrict__ w, const double *__restrict__ gate)
-{
-    if (gate && *gate == 0.0) return;
-    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
-        double acc = 0.0;
-        for (int j = 0; j < k; ++j) acc += coef[j] * V[static_cast<int64_t>(j) * ldv + i];
-        w[i] += sign * acc;
-    }
-}
-
-// step j, last: the norm of the orthogonalised vector (from the partials of
-// w . w after a second pass), the rotations, R's column j, g, and the
-// residual estimate |g_{j+1}| and hn into the host-visible slots 2j, 2j+1
-__global__ void __launch_bounds__(64) arnoldi_finalize_kernel(int j, int m, const double *__restrict__ partial,
-                                                            Arnoldi a, double *__restrict__ host)
-{
-    if (threadIdx.x != 0) return;
-    double hn = *a.hn;
-    if (*a.flag != 0.0) hn = sqrt(fmax(partial_sum(partial, 0), 0.0));
-    *a.inv = hn > 0.0 ? 1.0 / hn : 0.0;
-    double hi = a.h[0];
-    for (int i = 0; i < j; ++i) {
-        const double hi1 = a.h[i + 1];
-        a.R[static_cast<size_t>(i) * m + j] = a.cs[i] * hi + a.sn[i] * hi1;
-        hi = -a.sn[i] * hi + a.cs[i] * hi1;
-    }
-    // hi is the rotated h_j; h_{j+1} = hn
-    const double den = hypot(hi, hn);
-    const double c = den > 0.0 ? hi / den : 1.0, sgn = den > 0.0 ? hn / den : 0.0;
-    a.cs[j] = c;
-    a.sn[j] = sgn;
-    a.R[static_cast<size_t>(j) * m + j] = den;
-    const double gj = a.g[j];
-    a.g[j + 1] = -sgn * gj;
-    a.g[j] = c * gj;
-    host[2 * j] = fabs(a.g[j + 1]);
-    host[2 * j + 1] = hn;
-}
-
-// v *= 1/hn unless hn is zero
-__global__ void __launch_bounds__(256) arnoldi_scale_kernel(int n, const double *__restrict__ inv, double *__restrict__ v)
-{
-    const double a = *inv;
-    if (a == 0.0) return;
-    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) v[i] = a * v[i];
+    __syncthreads();
+    for (int i = t; i <= j; i += kT) a.R[static_cast<size_t>(i) * m + j] = s_x[i];
 }
 
 // ---- CSR SpMV of the weighted Dirichlet operator: y_r = w_r sum_k v_k x_c
@@ -824,7 +968,7 @@ struct Krylov {
     {
         Runtime &rt = runtime();
         dim3 grid(kReduceBlocks, k);
-        multi_dot_kernel<<<grid, 256, 0, rt.stream>>>(n, Vb, n, wv, s.partials.ptr, nullptr);
+        multi_dot_kernel<<<grid, 256, 0, rt.stream>>>(n, Vb, n, wv, s.partials.ptr);
         OC_HIP_CHECK(hipGetLastError());
         hpart.resize(static_cast<size_t>(k) * kReduceBlocks);
         OC_HIP_CHECK(hipMemcpyAsync(hpart.data(), s.partials.ptr, sizeof(double) * hpart.size(),
@@ -862,27 +1006,39 @@ struct Krylov {
 
     // One Arnoldi step j on the device: V_{j+1} = orthonormalised W A P^-1 W^-1 V_j,
     // R's column j and g rotated, |g_{j+1}| and hn into the host slots 2j, 2j+1.
+    // With point Jacobi z = W^-1 P^-1 V_j is written with V_j already.
     int arnoldi_step(int j)
     {
         Runtime &rt = runtime();
         double *vj = V + static_cast<int64_t>(j) * n, *vn = V + static_cast<int64_t>(j + 1) * n;
-        OC_CHECK(apply_preconditioner(vj, z));
+        if (!point_jacobi()) OC_CHECK(apply_preconditioner(vj, z));
         OC_CHECK(spmv(z, vn));
-        // classical Gram-Schmidt: one fused reduction gives V_0..V_j . w and
-        // w . w (V_{j+1} is w itself); the norm after projection follows by
-        // Pythagoras unless cancellation asks for a second pass and an
-        // explicit norm, whose kernels then run (they return at once otherwise)
-        multi_dot_kernel<<<dim3(kReduceBlocks, j + 2), 256, 0, rt.stream>>>(n, V, n, vn, s.partials.ptr, nullptr);
-        arnoldi_project_kernel<<<1, 256, 0, rt.stream>>>(j, s.partials.ptr, ar);
-        combine_device_kernel<<<grid_for(n), 256, 0, rt.stream>>>(n, j + 1, V, n, ar.h, -1.0, vn, nullptr);
-        multi_dot_kernel<<<dim3(kReduceBlocks, j + 1), 256, 0, rt.stream>>>(n, V, n, vn, s.partials.ptr, ar.flag);
-        arnoldi_correct_kernel<<<1, 256, 0, rt.stream>>>(j, s.partials.ptr, ar);
-        combine_device_kernel<<<grid_for(n), 256, 0, rt.stream>>>(n, j + 1, V, n, ar.h2, -1.0, vn, ar.flag);
-        multi_dot_kernel<<<dim3(kReduceBlocks, 1), 256, 0, rt.stream>>>(n, vn, n, vn, s.partials.ptr, ar.flag);
-        arnoldi_finalize_kernel<<<1, 64, 0, rt.stream>>>(j, m, s.partials.ptr, ar, s.arnoldi_host_dev);
-        arnoldi_scale_kernel<<<grid_for(n), 256, 0, rt.stream>>>(n, ar.inv, vn);
+        const int parts = row_blocks(256);
+        arnoldi_dots_kernel<<<dim3(parts, (j + 2 + kDotVectors - 1) / kDotVectors), 256, 0, rt.stream>>>(n, j + 2, V, vn,
+                                                                                                        s.partials.ptr);
+        // the fewest threads per block whose kReduceBlocks blocks cover the rows
+        if (n <= 256 * kReduceBlocks) orthogonalise<256>(j, parts);
+        else if (n <= 512 * kReduceBlocks) orthogonalise<512>(j, parts);
+        else orthogonalise<1024>(j, parts);
         OC_HIP_CHECK(hipGetLastError());
         return OC_NO_ERROR;
+    }
+    bool point_jacobi() const { return s.cls == OC_EQUATIONS_SET_LAPLACE || precond == OC_PRECONDITIONER_JACOBI; }
+    ScaledCopy scaled_copy() const
+    {
+        return point_jacobi() ? ScaledCopy{inv_u, s.iwgt.ptr, z} : ScaledCopy{nullptr, nullptr, nullptr};
+    }
+    // blocks of `threads` rows over the vector, at most kReduceBlocks
+    int row_blocks(int threads) const { return std::max(1, std::min(kReduceBlocks, (n + threads - 1) / threads)); }
+    template <int kT>
+    void orthogonalise(int j, int parts)
+    {
+        Runtime &rt = runtime();
+        const int blocks = row_blocks(kT);
+        double *partial2 = s.partials.ptr + static_cast<size_t>(kReduceBlocks) * (1024 + 1);
+        arnoldi_project_kernel<kT><<<blocks, kT, 0, rt.stream>>>(n, j, parts, V, s.partials.ptr, partial2, scaled_copy(), ar);
+        arnoldi_finish_kernel<kT><<<blocks + 1, kT, 0, rt.stream>>>(n, j, m, blocks, V, partial2, scaled_copy(), ar,
+                                                                   s.arnoldi_host_dev);
     }
 
     // Solves W A x = b (x starts at 0) to ||b - W A x|| <= tol_abs; b is zero
@@ -915,8 +1071,7 @@ struct Krylov {
                 res = beta;
                 if (res <= tol_abs) break;
             }
-            copy_scale_kernel<<<grid_for(n), 256, 0, rt.stream>>>(n, 1.0 / beta, r, V);
-            arnoldi_start_kernel<<<1, 256, 0, rt.stream>>>(m, beta, ar);
+            arnoldi_start_kernel<<<grid_for(n), 256, 0, rt.stream>>>(n, m, beta, r, V, scaled_copy(), ar);
             const int steps = std::min(m, max_iter - total);
             int cols = 0;
             for (int j = 0; j < steps && cols == 0; ++j) {
@@ -992,7 +1147,7 @@ static int solver_prepare(EquationsSet &s, int restart, Krylov &K)
     }
     if (!s.work.ptr) OC_CHECK(s.work.alloc(static_cast<size_t>(8) * n));
     if (!s.precond.ptr) OC_CHECK(s.precond.alloc(static_cast<size_t>(9) * s.n_nodes + 3 * static_cast<size_t>(n)));
-    const size_t npart = std::max<size_t>(static_cast<size_t>(kReduceBlocks) * (1024 + 1),
+    const size_t npart = std::max<size_t>(static_cast<size_t>(2) * kReduceBlocks * (1024 + 1),
                                           static_cast<size_t>(s.n_meshes) * 256);
     if (!s.partials.ptr || s.partials.n < npart) OC_CHECK(s.partials.alloc(npart));
     K.n = n;
