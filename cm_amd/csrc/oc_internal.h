@@ -221,6 +221,8 @@ struct EquationsSet {
     // position of element row e*8+i; element matrices in kbuf64 (E*64, rows
     // in gather order)
     DevBuf<uint8_t> slot_offsets8;
+    DevBuf<double> lap_xyz;     // node coordinates (x, y, z, 0) for the element kernels
+    DevBuf<int32_t> lap_erow;   // small meshes: gather position -> element * 8 + local node (one-launch assembly)
     // Laplace sets on a structured grid: elements per direction (zero when
     // the mesh is not one), and when the fused assembly serves it: 0 never,
     // 1 when the grid fills the GPU, 2 always (oc_laplace_fused_set)
