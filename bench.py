@@ -464,7 +464,7 @@ def main():
         secondary["mr_jacobian_fp32"] = {
             "error_vs_fp64_rel_frobenius": float(np.linalg.norm(v32 - v64) / np.linalg.norm(v64)),
             "elements_per_s": E * args.steps / (ms32 / 1e3),
-            "element_matrix": kernel_roofline("mr_element_matrix_kernel<float>", "mfma32", E * args.steps / l32,
+            "element_matrix": kernel_roofline("mr_element_matrix_f32_kernel", "mfma32", E * args.steps / l32,
                                               j32 / l32 / 1e3, "mr_element_matrix_fp32", wl),
             "row_gather": kernel_roofline("csr_row_gather_kernel<float>", "hbm", gather_bytes(eq, 4) * args.steps / k32,
                                           g32 / k32 / 1e3, "csr_row_gather_fp32", wl),

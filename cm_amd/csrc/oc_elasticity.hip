@@ -4,8 +4,8 @@
 //
 // Jacobian: mr_gauss_kernel (one thread per element Gauss point, all
 // elements) evaluates the FP64 kinematics and tangent into Gauss-point
-// records (field-major, see GpField); mr_element_matrix_f64_kernel (FP64) or
-// mr_element_matrix_kernel<float> (FP32) contracts the records of every
+// records (see GpField); mr_element_matrix_f64_kernel (FP64) or
+// mr_element_matrix_f32_kernel (FP32) contracts the records of every
 // element into its 89x89 element matrix on MFMA; and csr_row_gather_kernel
 // assembles each CSR row from the element rows that touch it in ascending
 // element order (deterministic, write-once), placing them through the
@@ -16,6 +16,7 @@
 #include <algorithm>
 #include <cmath>
 #include <cstdint>
+#include <type_traits>
 #include <vector>
 
 #include "oc_fe_device.h"
@@ -23,8 +24,9 @@
 
 namespace oc {
 
-// Gauss-point record fields.  Record of Gauss point q = e*27 + g stores
-// field f at rec[f * n_gp + q] (coalesced across Gauss points).
+// Gauss-point record fields.  Field f of Gauss point g of element e is at
+// rec[(e * GP_NFIELDS + f) * 27 + g]: an element's records are contiguous, so the
+// element-matrix kernels take them without address arithmetic.
 enum GpField : int {
     GP_DXIDZ = 0,   // 9: DXI_DX of the deformed metrics, column-major
     GP_JGW = 9,     // J_z * w_g
@@ -100,17 +102,16 @@ mr_gauss_kernel(int n_elements, const int *__restrict__ conn_q, const int *__res
     gauss_kinematics(s_tab, g, s_z[le], s_X[le], k);
     double P = 0.0;
     for (int n = 0; n < 8; ++n) P += T->lin27[(g * 8 + n) * 4] * s_p[le][n];
-    const int64_t n_gp = static_cast<int64_t>(n_elements) * 27;
-    const int64_t q = static_cast<int64_t>(e) * 27 + g;
+    rec += static_cast<int64_t>(e) * GP_NFIELDS * 27 + g;
 #pragma unroll
-    for (int i = 0; i < 9; ++i) rec[(GP_DXIDZ + i) * n_gp + q] = k.dxidz[i];
-    rec[GP_JGW * n_gp + q] = k.jz * T->w27[g];
+    for (int i = 0; i < 9; ++i) rec[(GP_DXIDZ + i) * 27] = k.dxidz[i];
+    rec[GP_JGW * 27] = k.jz * T->w27[g];
     double c[36], sigma[6];
     mr_elasticity_tensor(k.F, k.Jznu, P, mat[2 * e], mat[2 * e + 1], c, sigma);
 #pragma unroll
-    for (int i = 0; i < 36; ++i) rec[(GP_C + i) * n_gp + q] = c[i];
+    for (int i = 0; i < 36; ++i) rec[(GP_C + i) * 27] = c[i];
 #pragma unroll
-    for (int i = 0; i < 6; ++i) rec[(GP_SIGJ + i) * n_gp + q] = sigma[i];
+    for (int i = 0; i < 6; ++i) rec[(GP_SIGJ + i) * 27] = sigma[i];
 }
 
 // Scatter map.  A CSR row of node n (any of its three displacement rows, or
@@ -413,19 +414,18 @@ mr_residual_element_kernel(int n_elements, const int *__restrict__ conn_q, const
 // sums its elements' integrals of psi_m J_z w (its gather list: entries
 // e*89 + 81 + m, ascending elements); inv_p = -1 / S.
 __global__ void __launch_bounds__(256)
-schur_mass_kernel(int nl, const int *__restrict__ gptr, const int *__restrict__ gidx, int n_elements,
+schur_mass_kernel(int nl, const int *__restrict__ gptr, const int *__restrict__ gidx,
                   const double *__restrict__ rec, const BasisTables *__restrict__ T, const double *__restrict__ mat,
                   double *__restrict__ inv_p)
 {
     const int p = blockIdx.x * blockDim.x + threadIdx.x;
     if (p >= nl) return;
-    const int64_t n_gp = static_cast<int64_t>(n_elements) * 27;
     double sum = 0.0;
     for (int k = gptr[p]; k < gptr[p + 1]; ++k) {
         const int64_t e = gidx[k] / 89;
         const int m = gidx[k] % 89 - 81;
         double acc = 0.0;
-        for (int g = 0; g < 27; ++g) acc += T->lin27[(g * 8 + m) * 4] * rec[GP_JGW * n_gp + e * 27 + g];
+        for (int g = 0; g < 27; ++g) acc += T->lin27[(g * 8 + m) * 4] * rec[(e * GP_NFIELDS + GP_JGW) * 27 + g];
         sum += acc / (2.0 * (mat[2 * e] + mat[2 * e + 1]));
     }
     inv_p[p] = sum > 0.0 ? -1.0 / sum : -1.0;
@@ -485,7 +485,7 @@ int launch_mr_residual(EquationsSet &s)
 // Analytic Jacobian (FiniteElasticity_FiniteElementJacobianEvaluate,
 // finite_elasticity_routines.f90:842-1175) in two phases.
 //
-// Phase A (mr_element_matrix_f64_kernel for FP64, mr_element_matrix_kernel<float>
+// Phase A (mr_element_matrix_f64_kernel for FP64, mr_element_matrix_f32_kernel
 // for FP32; all elements, no colours): for each of the six lower displacement
 // blocks (a, b), b <= a,
 //   K_(a,m),(b,n) = sum_(g,j) U_g^{ab}[m][j] D_g[j][n],
@@ -494,37 +494,149 @@ int launch_mr_residual(EquationsSet &s)
 // i.e. the reference's TEMPVEC / DOT_PRODUCT contraction (:1001-1037)
 // re-associated as a 27x81 by 81x27 GEMM on MFMA; pressure rows
 // K_(p,m),(b,n) = sum_g (J_z w_g psi_m) D_g[b][n] (:1039-1054) as an 8x27 by
-// 27x81 GEMM.  Both kernels run a producer/consumer pipeline per block:
-// producer waves build D, W and the pressure operand of the next element in
-// double-buffered LDS while consumer waves contract the current one, with D in
-// registers and U formed in registers from D and W.  Lower triangle kept,
-// mirrored (:1149-1153); the element matrix goes to an HBM buffer, row-major.
+// 27x81 GEMM.  U is formed in registers from D and W and never stored.  Lower
+// triangle kept, mirrored (:1149-1153); the element matrix goes to an HBM
+// buffer, row-major.
 // Phase B (csr_row_gather_kernel<Real>): one wavefront per CSR row adds the
 // element rows that touch it, in ascending element order, into an LDS copy of
 // the row and writes the row once (no zero fill, no read-modify-write).
 typedef float mfma_f32x4 __attribute__((ext_vector_type(4)));
-typedef double mfma_f64x4 __attribute__((ext_vector_type(4)));
 
+// Both element-matrix kernels are persistent (one block of twelve waves per CU)
+// and run their elements through a three-stage pipeline.  In slot s
+//   * the producers, waves 4..7, build the operands D, W and the pressure
+//     operand of element s in one half of double-buffered LDS and load the
+//     Gauss-point records of element s + 2;
+//   * the consumers, waves 0..3, run the MFMA contraction of element s - 1 from
+//     the other half;
+//   * the storers, waves 8..11, copy the staged tiles of element s - 2 to its
+//     row-major matrix.
+// Between the slot's two barriers the consumers put their accumulators into the
+// staging area and the producers the records of element s + 1 into theirs.
+//
+// The staging area holds the lower blocks and the pressure rows only, as the
+// MFMA tiles give them; a storer thread keeps the LDS places of its entries (the
+// same for every element), so the mirror image costs no writes, and stores two
+// entries of consecutive addresses: the element matrix leaves in contiguous
+// kilobytes.  Stored tile by tile from the accumulators it left in requests of 29
+// bytes on average (73 million for 32,768 elements), which alone took 620 us.
+// 32,768 elements: FP64 805 -> 713 us, where MFMAs and vector instructions take
+// turns (see f64_units); 13,100 elements in FP32 307 -> 229 us.
+constexpr int kElementThreads = 768;
+constexpr int kRoleThreads = 256;  // threads of each of the three roles
+
+// Staging area: lower block q = a (a + 1) / 2 + b as 27 rows of 29 (an odd
+// stride: a column read is free of bank conflicts), the pressure rows, a zero
+constexpr int kStageRow = 29, kStageBlock = 27 * kStageRow, kStagePRow = 83;
+constexpr int kStageP = 6 * kStageBlock, kStageZero = kStageP + 8 * kStagePRow, kStageSize = kStageZero + 1;
+constexpr int kEntries = 89 * 89;
+constexpr int kStorePairs = ((kEntries + 1) / 2 + kRoleThreads - 1) / kRoleThreads;  // pairs of entries per storer thread
+
+// staging place of entry idx of the row-major 89x89 matrix: blocks above the
+// diagonal mirror those below (:1149-1153), the p-p block is zero
+__device__ __forceinline__ int stage_place(int idx)
+{
+    const int r = idx / 89, j = idx % 89;
+    const int hi = max(r, j), lo = min(r, j);
+    if (lo >= 81) return kStageZero;
+    if (hi >= 81) return kStageP + (hi - 81) * kStagePRow + lo;
+    // (a, m) row and (b, n) column of the lower block
+    int a = r / 27, m = r % 27, b = j / 27, n = j % 27;
+    if (a < b || (a == b && m < n)) {
+        int x = a;
+        a = b;
+        b = x;
+        x = m;
+        m = n;
+        n = x;
+    }
+    return (a * (a + 1) / 2 + b) * kStageBlock + m * kStageRow + n;
+}
+
+// The stores go through a buffer resource over the 89x89 block of one element:
+// the lane part of an offset is one register and the rest a constant, so a
+// store costs no address arithmetic.
+typedef unsigned int u32x2 __attribute__((ext_vector_type(2)));
+typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ void store_pair(__amdgpu_buffer_rsrc_t rs, double v0, double v1, int voff, int soff)
+{
+    const u32x2 a = __builtin_bit_cast(u32x2, v0), b = __builtin_bit_cast(u32x2, v1);
+    __builtin_amdgcn_raw_buffer_store_b128(u32x4{a.x, a.y, b.x, b.y}, rs, voff, soff, 0);
+}
+__device__ __forceinline__ void store_pair(__amdgpu_buffer_rsrc_t rs, float v0, float v1, int voff, int soff)
+{
+    __builtin_amdgcn_raw_buffer_store_b64(u32x2{__builtin_bit_cast(unsigned, v0), __builtin_bit_cast(unsigned, v1)}, rs,
+                                          voff, soff, 0);
+}
+
+// the storers' slots: thread st copies the pairs of entries st + 256 i
 template <typename Real>
-struct Mfma;
+__device__ __forceinline__ void element_storer(int st, int n_mine, int e0, int step, const Real *s_stage,
+                                               Real *__restrict__ kbuf)
+{
+    constexpr int kR = static_cast<int>(sizeof(Real));
+    int place[2 * kStorePairs];
+#pragma unroll
+    for (int i = 0; i < 2 * kStorePairs; ++i)
+        place[i] = stage_place(min(2 * (st + kRoleThreads * (i >> 1)) + (i & 1), kEntries - 1));
+    const int last = 2 * (st + kRoleThreads * (kStorePairs - 1));
+    for (int s = 0; s < n_mine + 2; ++s) {
+        if (s >= 2) {
+            Real *Ke = kbuf + (e0 + static_cast<int64_t>(s - 2) * step) * kEntries;
+            const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(Ke, 0, kEntries * kR, 0x00020000);
+#pragma unroll
+            for (int i = 0; i < kStorePairs; ++i) {
+                const Real v0 = s_stage[place[2 * i]], v1 = s_stage[place[2 * i + 1]];
+                if (i + 1 < kStorePairs || last + 1 < kEntries) store_pair(rs, v0, v1, 2 * kR * st, 2 * kR * kRoleThreads * i);
+                else if (last < kEntries) Ke[last] = v0;
+            }
+        }
+        __syncthreads();
+        __syncthreads();
+    }
+}
 
-template <>
-struct Mfma<float> {
-    using acc_t = mfma_f32x4;
-    __device__ static acc_t step(float a, float b, acc_t c) { return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0); }
-    // output row of accumulator register r for this lane (column = lane % 16)
-    __device__ static int row(int lane, int r) { return 4 * (lane >> 4) + r; }
-    static constexpr int kRowStep = 1;
+// The records of one element on their way to LDS: loaded two elements ahead
+constexpr int kRec = GP_NFIELDS * 27, kRecPerThread = (kRec + kRoleThreads - 1) / kRoleThreads;
+__device__ __forceinline__ void load_records(const double *__restrict__ rec, int64_t e, bool valid, int pt,
+                                             double (&v)[kRecPerThread])
+{
+    const double *r = rec + e * kRec;
+#pragma unroll
+    for (int i = 0; i < kRecPerThread; ++i)
+        v[i] = (valid && (i + 1 < kRecPerThread || pt + kRoleThreads * i < kRec)) ? r[pt + kRoleThreads * i] : 0.0;
+}
+__device__ __forceinline__ void put_records(double (*s_rec)[27], int pt, const double (&v)[kRecPerThread])
+{
+    double *r = &s_rec[0][0];
+#pragma unroll
+    for (int i = 0; i < kRecPerThread; ++i)
+        if (i + 1 < kRecPerThread || pt + kRoleThreads * i < kRec) r[pt + kRoleThreads * i] = v[i];
+}
+
+// Producer thread pt < 243 owns (j, n) = (rq / 27, rq % 27) of D_g, rq = pt % 81,
+// for g = pg + 3k, pg = pt / 81: D_g[j][n] = sum_mi DXI_DX(mi, j) dphi_n/dxi_mi
+// (:974-986).  Its table values dphi_n/dxi_mi at those g stay in registers.
+struct ProducerTable {
+    double d[9][3];
 };
+__device__ __forceinline__ ProducerTable producer_table(const BasisTables *__restrict__ T, int pt)
+{
+    const int n = (pt % 81) % 27, pg = pt / 81;
+    ProducerTable t;
+#pragma unroll
+    for (int k = 0; k < 9; ++k)
+#pragma unroll
+        for (int mi = 0; mi < 3; ++mi) t.d[k][mi] = pt < 243 ? T->quad27[((pg + 3 * k) * 27 + n) * 4 + 1 + mi] : 0.0;
+    return t;
+}
+__device__ __forceinline__ double producer_d(const double (*R)[27], const ProducerTable &t, int dj, int g, int k)
+{
+    return R[GP_DXIDZ + 0 + 3 * dj][g] * t.d[k][0] + R[GP_DXIDZ + 1 + 3 * dj][g] * t.d[k][1] +
+           R[GP_DXIDZ + 2 + 3 * dj][g] * t.d[k][2];
+}
 
-template <>
-struct Mfma<double> {
-    using acc_t = mfma_f64x4;
-    __device__ static acc_t step(double a, double b, acc_t c) { return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0); }
-    __device__ static int row(int lane, int r) { return (lane >> 4) + 4 * r; }
-    static constexpr int kRowStep = 4;
-};
-
+// ---- FP32 element matrices: v_mfma_f32_16x16x4f32 -----------------------------
 // Per-lane operand slices of D_g[j][n] = sum_mi DXI_DX(mi, j) dphi_n/dxi_mi
 // (:974-986).  The contraction index is k = (j, g) with g padded to 28, so
 // MFMA k-step ks covers j = ks / 7 and g = 4 (ks % 7) + kk (kk = lane / 16).
@@ -534,275 +646,237 @@ struct Mfma<double> {
 // and, contracted with W, form its A operand
 //   U^{ab}_g[m][j] = sum_i D_g[i][m] W_g[(a,i),(b,j)]
 // on the fly, so U never goes through LDS.
-// Element-matrix stores go through a buffer resource over the 89x89 block of
-// one element: the lane part of each offset is one register and the tile part
-// a constant, so a store costs no address arithmetic.
-typedef unsigned int u32x2 __attribute__((ext_vector_type(2)));
-template <typename Real>
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t element_rsrc(Real *Ke)
-{
-    return __builtin_amdgcn_make_buffer_rsrc(Ke, 0, 89 * 89 * static_cast<int>(sizeof(Real)), 0x00020000);
-}
-__device__ __forceinline__ void element_store(__amdgpu_buffer_rsrc_t rs, double v, int voff, int soff)
-{
-    __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u32x2, v), rs, voff, soff, 0);
-}
-__device__ __forceinline__ void element_store(__amdgpu_buffer_rsrc_t rs, float v, int voff, int soff)
-{
-    __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, v), rs, voff, soff, 0);
-}
-
-template <typename Real>
 struct DSlice {
-    Real v[2][7][3];
+    float v[2][7][3];
 };
 
-// One displacement block (a, b), row tile MT, column tiles 0 (and 1 if TWO):
-// 21 k-steps of mfma 16x16x4, then the tiles go to the element buffer, the
-// (b, a) block as the mirror image.  A diagonal block keeps its lower triangle
-// (:1149-1153).
-template <typename Real, int MT, bool TWO>
-__device__ __forceinline__ void mr_uu_block(int a, int b, int lane, const DSlice<Real> &D, const Real (*s_W)[81],
-                                            Real *__restrict__ Ke)
+// One displacement block (A, B), row tile MT, column tiles 0 (and 1 if TWO)
+template <int A, int B, int MT, bool TWO>
+struct F32Unit {
+    static constexpr int a = A, b = B, mt = MT;
+    static constexpr bool two = TWO;
+};
+
+// accumulator register r of a lane holds row 4 (lane / 16) + r, column lane % 16
+template <typename U>
+__device__ __forceinline__ void f32_unit(int lane, const DSlice &D, const float (*s_W)[81], mfma_f32x4 (&acc)[2])
 {
-    using M = Mfma<Real>;
-    const int kk = lane >> 4, l = lane & 15;
-    typename M::acc_t acc0 = {Real(0), Real(0), Real(0), Real(0)};
-    typename M::acc_t acc1 = {Real(0), Real(0), Real(0), Real(0)};
+    const int kk = lane >> 4;
+    acc[0] = acc[1] = mfma_f32x4{0.0f, 0.0f, 0.0f, 0.0f};
     // k-step s = 7 j + gp; software pipeline: the W loads of step s + 2 and
     // the A operand of step s + 1 are issued behind the MFMAs of step s, and a
     // scheduling barrier per step keeps that order (and the register count)
-    const Real *wbase = &s_W[kk][a * 27 + b * 3];
-    auto load_w = [&](int st, Real *w) {
-        const Real *p = wbase + (4 * (st % 7)) * 81 + st / 7;
+    const float *wbase = &s_W[kk][U::a * 27 + U::b * 3];
+    auto load_w = [&](int st, float *w) {
+        const float *p = wbase + (4 * (st % 7)) * 81 + st / 7;
         w[0] = p[0];
         w[1] = p[9];
         w[2] = p[18];
     };
-    auto a_operand = [&](int st, const Real *w) {
+    auto a_operand = [&](int st, const float *w) {
         const int gp = st % 7;
-        return D.v[MT][gp][0] * w[0] + D.v[MT][gp][1] * w[1] + D.v[MT][gp][2] * w[2];
+        return D.v[U::mt][gp][0] * w[0] + D.v[U::mt][gp][1] * w[1] + D.v[U::mt][gp][2] * w[2];
     };
-    Real wq[2][3];
+    float wq[2][3];
     load_w(0, wq[0]);
     load_w(1, wq[1]);
-    Real u = a_operand(0, wq[0]);
+    float u = a_operand(0, wq[0]);
 #pragma unroll
     for (int st = 0; st < 21; ++st) {
         const int j = st / 7, gp = st % 7;
         if (st + 2 < 21) load_w(st + 2, wq[st & 1]);
-        acc0 = M::step(u, D.v[0][gp][j], acc0);
-        if (TWO) acc1 = M::step(u, D.v[1][gp][j], acc1);
+        acc[0] = __builtin_amdgcn_mfma_f32_16x16x4f32(u, D.v[0][gp][j], acc[0], 0, 0, 0);
+        if (U::two) acc[1] = __builtin_amdgcn_mfma_f32_16x16x4f32(u, D.v[1][gp][j], acc[1], 0, 0, 0);
         if (st + 1 < 21) u = a_operand(st + 1, wq[(st + 1) & 1]);
         __builtin_amdgcn_sched_barrier(0);
     }
-    // entry (m, n) of the tile at (a*27 + m)*89 + b*27 + n and its mirror at
-    // (b*27 + n)*89 + a*27 + m, with m = MT*16 + row0 + kRowStep*r and
-    // n = nt*16 + l: lane part row0*89 + l (mirror l*89 + row0), the rest
-    // constant
-    const __amdgpu_buffer_rsrc_t rs = element_rsrc(Ke);
-    const int row0 = M::row(lane, 0);
-    const int vdir = (row0 * 89 + l) * static_cast<int>(sizeof(Real));
-    const int vmir = (l * 89 + row0) * static_cast<int>(sizeof(Real));
+}
+
+// entry (m, n), m = MT*16 + 4 (lane / 16) + r, n = nt*16 + lane % 16, of a
+// unit's tiles into the staging area
+template <typename U>
+__device__ __forceinline__ void f32_unit_stage(int lane, const mfma_f32x4 (&acc)[2], float *s_stage)
+{
+    const int l = lane & 15, row0 = U::mt * 16 + 4 * (lane >> 4);
+    float *o = s_stage + (U::a * (U::a + 1) / 2 + U::b) * kStageBlock + row0 * kStageRow + l;
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
-        const int m = MT * 16 + row0 + M::kRowStep * r;
-        if (m >= 27) continue;
+        if (row0 + r >= 27) continue;
 #pragma unroll
-        for (int nt = 0; nt < (TWO ? 2 : 1); ++nt) {
-            const int n = nt * 16 + l;
-            if (n >= 27 || (a == b && m < n)) continue;
-            const Real v = nt ? acc1[r] : acc0[r];
-            const int cdir = ((a * 27 + MT * 16 + M::kRowStep * r) * 89 + b * 27 + nt * 16) * static_cast<int>(sizeof(Real));
-            const int cmir = ((b * 27 + nt * 16) * 89 + a * 27 + MT * 16 + M::kRowStep * r) * static_cast<int>(sizeof(Real));
-            element_store(rs, v, vdir, cdir);
-            element_store(rs, v, vmir, cmir);
-        }
+        for (int nt = 0; nt < (U::two ? 2 : 1); ++nt)
+            if (nt == 0 || 16 + l < 27) o[r * kStageRow + 16 * nt] = acc[nt][r];
     }
 }
 
 // Pressure rows K_(p,m),(b,n) = sum_g (J_z w_g psi_m(g)) D_g[b][n]
 // (:1039-1054): k = g only, so k-step ks is g = 4 ks + kk and the B operand
-// is D[t][ks][b]; six 16x16 tiles (b, t), rows 8..15 padding.  Also writes
-// the zero p-p block.
-template <typename Real>
-__device__ __forceinline__ void mr_pressure_rows(int lane, const DSlice<Real> &D, const Real *s_Pa,
-                                                 Real *__restrict__ Ke)
+// is D[t][ks][b]; six 16x16 tiles acc[b][t], rows 8..15 padding
+__device__ __forceinline__ void f32_pressure(int lane, const DSlice &D, const float *s_Pa, mfma_f32x4 (&acc)[3][2])
 {
-    using M = Mfma<Real>;
     const int kk = lane >> 4, l = lane & 15;
-    Real pa[7];
 #pragma unroll
-    for (int ks = 0; ks < 7; ++ks) pa[ks] = s_Pa[(4 * ks + kk) * 16 + l];
-    const __amdgpu_buffer_rsrc_t rs = element_rsrc(Ke);
-    const int row0 = M::row(lane, 0);
-    const int vdir = (row0 * 89 + l) * static_cast<int>(sizeof(Real));
-    const int vmir = (l * 89 + row0) * static_cast<int>(sizeof(Real));
+    for (int b = 0; b < 3; ++b) acc[b][0] = acc[b][1] = mfma_f32x4{0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-    for (int b = 0; b < 3; ++b) {
+    for (int ks = 0; ks < 7; ++ks) {
+        const float pa = s_Pa[(4 * ks + kk) * 16 + l];
 #pragma unroll
-        for (int t = 0; t < 2; ++t) {
-            typename M::acc_t acc = {Real(0), Real(0), Real(0), Real(0)};
+        for (int b = 0; b < 3; ++b)
 #pragma unroll
-            for (int ks = 0; ks < 7; ++ks) acc = M::step(pa[ks], D.v[t][ks][b], acc);
-            const int n = t * 16 + l;
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const int m = row0 + M::kRowStep * r;
-                if (m >= 8 || n >= 27) continue;
-                const int cdir = ((81 + M::kRowStep * r) * 89 + b * 27 + t * 16) * static_cast<int>(sizeof(Real));
-                const int cmir = ((b * 27 + t * 16) * 89 + 81 + M::kRowStep * r) * static_cast<int>(sizeof(Real));
-                element_store(rs, acc[r], vdir, cdir);
-                element_store(rs, acc[r], vmir, cmir);
-            }
-        }
+            for (int t = 0; t < 2; ++t) acc[b][t] = __builtin_amdgcn_mfma_f32_16x16x4f32(pa, D.v[t][ks][b], acc[b][t], 0, 0, 0);
     }
-    Ke[(81 + lane / 8) * 89 + 81 + lane % 8] = Real(0);
 }
 
-// Producer/consumer element-matrix kernel: one block of eight waves walks its
-// elements in a two-stage pipeline.  Waves 4..7 (producers) build, for
-// element i + 1, the operands D, W and the pressure A operand in one half of
-// double-buffered LDS and load the Gauss-point records of element i + 2;
-// waves 0..3 (consumers) meanwhile load their D slices of element i from the
-// other half and run its MFMA contraction.  One block barrier per element.
-template <typename Real>
-__global__ void __launch_bounds__(512)
-mr_element_matrix_kernel(int n_elements, const double *__restrict__ rec, const BasisTables *__restrict__ T,
-                         Real *__restrict__ kbuf)
+__device__ __forceinline__ void f32_pressure_stage(int lane, const mfma_f32x4 (&acc)[3][2], float *s_stage)
 {
-    __shared__ double s_tab[27][3][27];  // dphi_n/dxi_mi at g: [g][mi][n]
-    __shared__ double s_psi[27][8];      // trilinear psi_m(g)
-    __shared__ double s_rec[2][52][27];  // Gauss-point records
-    __shared__ Real s_D[2][28][3][32];   // D_g[j][n]; g = 27 and n >= 27 zero
-    __shared__ Real s_W[2][28][81];      // W_g[(a,i),(b,j)] at [g][(3a+i)*9 + 3b+j]; g = 27 zero
-    __shared__ Real s_Pa[2][28 * 16];    // J_z w_g psi_m(g) at [g*16 + m]; m >= 8 and g = 27 zero
-    constexpr int kRec = 52 * 27, kRecPerThread = (kRec + 255) / 256;
-    const int t = threadIdx.x, lane = t & 63;
-    const bool producer = t >= 256;
-    const int pt = t - 256;
-    // producer thread pt < 243 owns column rq = pt % 81 of W_g (row (a,i),
-    // column (b,j)) and of D_g (j = rq / 27, n = rq % 27) for g = pg (mod 3)
-    const int rq = (pt >= 0 ? pt : 0) % 81, pg = (pt >= 0 ? pt : 0) / 81;
-    const int wa = rq / 27, wi = (rq / 9) % 3, wb = (rq % 9) / 3, wj = rq % 3;
-    const int wf1 = GP_C + t2v(wi, wa) + 6 * t2v(wj, wb), wf2 = GP_SIGJ + t2v(wi, wj);
-    const bool wdiag = wa == wb;
-    const int dj = rq / 27, dn = rq % 27;
-    const int64_t n_gp = static_cast<int64_t>(n_elements) * 27;
-    const int n_mine = static_cast<int>(blockIdx.x) < n_elements
-                           ? (n_elements - 1 - static_cast<int>(blockIdx.x)) / static_cast<int>(gridDim.x) + 1
-                           : 0;
-    for (int k = t; k < 27 * 27 * 3; k += 512) {
-        const int g = k / 81, mi = (k / 27) % 3, n = k % 27;
-        s_tab[g][mi][n] = T->quad27[(g * 27 + n) * 4 + 1 + mi];
-    }
-    for (int k = t; k < 27 * 8; k += 512) s_psi[k / 8][k % 8] = T->lin27[k * 4];
-    for (int k = t; k < 2 * 28 * 3 * 32; k += 512) (&s_D[0][0][0][0])[k] = Real(0);
-    for (int k = t; k < 2 * 28 * 81; k += 512) (&s_W[0][0][0])[k] = Real(0);
-    for (int k = t; k < 2 * 28 * 16; k += 512) (&s_Pa[0][0])[k] = Real(0);
-    if (producer && n_mine > 0) {
-        const int64_t q0 = static_cast<int64_t>(blockIdx.x) * 27;
-        for (int k = pt; k < kRec; k += 256) s_rec[0][k / 27][k % 27] = rec[(k / 27) * n_gp + q0 + (k % 27)];
-    }
-    __syncthreads();
+    const int l = lane & 15, row0 = 4 * (lane >> 4);
+    if (row0 >= 8) return;
+    float *o = s_stage + kStageP + row0 * kStagePRow + l;
+#pragma unroll
+    for (int b = 0; b < 3; ++b)
+#pragma unroll
+        for (int t = 0; t < 2; ++t)
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+                if (t == 0 || 16 + l < 27) o[r * kStagePRow + b * 27 + t * 16] = acc[b][t][r];
+}
 
-    for (int it = 0; it <= n_mine; ++it) {
-        if (producer) {
-            if (it < n_mine) {
-                const int p = it & 1;
-                // records of the element after this one: issued first, stored last
-                const int e_next = static_cast<int>(blockIdx.x) + (it + 1) * static_cast<int>(gridDim.x);
-                double pre[kRecPerThread];
-#pragma unroll
-                for (int i = 0; i < kRecPerThread; ++i) {
-                    const int k = pt + 256 * i;
-                    pre[i] = (it + 1 < n_mine && k < kRec)
-                                 ? rec[(k / 27) * n_gp + static_cast<int64_t>(e_next) * 27 + (k % 27)]
-                                 : 0.0;
-                }
-                const double(*R)[27] = s_rec[p];
-                // all LDS reads of the phase before its writes: one round trip
-                if (pt < 243) {  // column rq of W_g and of D_g for g = pg + 3k
-                    Real wv[9], dv[9];
-#pragma unroll
-                    for (int k = 0; k < 9; ++k) {
-                        const int g = pg + 3 * k;
-                        double v = R[wf1][g];
-                        if (wdiag) v = v + R[wf2][g];
-                        wv[k] = static_cast<Real>(R[GP_JGW][g] * v);
-                        dv[k] = static_cast<Real>(R[GP_DXIDZ + 0 + 3 * dj][g] * s_tab[g][0][dn] +
-                                                  R[GP_DXIDZ + 1 + 3 * dj][g] * s_tab[g][1][dn] +
-                                                  R[GP_DXIDZ + 2 + 3 * dj][g] * s_tab[g][2][dn]);
-                    }
-#pragma unroll
-                    for (int k = 0; k < 9; ++k) {
-                        s_W[p][pg + 3 * k][rq] = wv[k];
-                        s_D[p][pg + 3 * k][dj][dn] = dv[k];
-                    }
-                }
-                if (pt < 27 * 8) s_Pa[p][pt / 8 * 16 + pt % 8] = static_cast<Real>(R[GP_JGW][pt / 8] * s_psi[pt / 8][pt % 8]);
-                if (it + 1 < n_mine) {
-#pragma unroll
-                    for (int i = 0; i < kRecPerThread; ++i) {
-                        const int k = pt + 256 * i;
-                        if (k < kRec) s_rec[p ^ 1][k / 27][k % 27] = pre[i];
-                    }
-                }
-            }
-        } else if (it >= 1) {
-            const int p = (it - 1) & 1;
-            const int e = static_cast<int>(blockIdx.x) + (it - 1) * static_cast<int>(gridDim.x);
-            Real *Ke = kbuf + static_cast<int64_t>(e) * 89 * 89;
-            // the lane index is made opaque per element so that the W and store
-            // offsets derived from it are recomputed here rather than hoisted
-            // out of the element loop and held in registers across it
-            int ln = lane;
-            asm volatile("" : "+v"(ln));
-            const int kk = ln >> 4, l = ln & 15, wave = t >> 6;
-            DSlice<Real> D;
+// the slots of consumer wave kWave (0..3)
+template <int kWave>
+__device__ __forceinline__ void f32_consumer(int lane, int n_mine, const float (*s_D)[28][3][32], const float (*s_W)[28][81],
+                                             const float (*s_Pa)[28 * 16], float *s_stage)
+{
+    // 483 MFMA k-steps per element over four waves (126/126/126/105)
+    using U0 = std::conditional_t<kWave == 0, F32Unit<1, 0, 0, true>, std::conditional_t<kWave == 1, F32Unit<2, 0, 0, true>,
+               std::conditional_t<kWave == 2, F32Unit<2, 1, 0, true>, F32Unit<0, 0, 0, false>>>>;
+    using U1 = std::conditional_t<kWave == 0, F32Unit<1, 0, 1, true>, std::conditional_t<kWave == 1, F32Unit<2, 0, 1, true>,
+               std::conditional_t<kWave == 2, F32Unit<2, 1, 1, true>, F32Unit<1, 1, 0, false>>>>;
+    using U2 = std::conditional_t<kWave == 0, F32Unit<0, 0, 1, true>, std::conditional_t<kWave == 1, F32Unit<1, 1, 1, true>,
+               std::conditional_t<kWave == 2, F32Unit<2, 2, 1, true>, F32Unit<2, 2, 0, false>>>>;
+    for (int s = 0; s < n_mine + 2; ++s) {
+        // the lane index is made opaque per element so that the offsets
+        // derived from it are recomputed here rather than held across the loop
+        int ln = lane;
+        asm volatile("" : "+v"(ln));
+        const bool work = s >= 1 && s - 1 < n_mine;
+        mfma_f32x4 acc[3][2], accp[3][2];
+        if (work) {
+            const int p = (s - 1) & 1, kk = ln >> 4, l = ln & 15;
+            DSlice D;
 #pragma unroll
             for (int tt = 0; tt < 2; ++tt)
 #pragma unroll
                 for (int gp = 0; gp < 7; ++gp)
 #pragma unroll
                     for (int j = 0; j < 3; ++j) D.v[tt][gp][j] = s_D[p][4 * gp + kk][j][16 * tt + l];
-            const Real(*W)[81] = s_W[p];
-            // 483 MFMA k-steps per element over four waves (126/126/126/105)
-            if (wave == 0) {
-                mr_uu_block<Real, 0, true>(1, 0, ln, D, W, Ke);
-                mr_uu_block<Real, 1, true>(1, 0, ln, D, W, Ke);
-                mr_uu_block<Real, 1, true>(0, 0, ln, D, W, Ke);
-            } else if (wave == 1) {
-                mr_uu_block<Real, 0, true>(2, 0, ln, D, W, Ke);
-                mr_uu_block<Real, 1, true>(2, 0, ln, D, W, Ke);
-                mr_uu_block<Real, 1, true>(1, 1, ln, D, W, Ke);
-            } else if (wave == 2) {
-                mr_uu_block<Real, 0, true>(2, 1, ln, D, W, Ke);
-                mr_uu_block<Real, 1, true>(2, 1, ln, D, W, Ke);
-                mr_uu_block<Real, 1, true>(2, 2, ln, D, W, Ke);
-            } else {
-                mr_pressure_rows<Real>(ln, D, s_Pa[p], Ke);
-                mr_uu_block<Real, 0, false>(0, 0, ln, D, W, Ke);
-                mr_uu_block<Real, 0, false>(1, 1, ln, D, W, Ke);
-                mr_uu_block<Real, 0, false>(2, 2, ln, D, W, Ke);
-            }
+            const float(*W)[81] = s_W[p];
+            if (kWave == 3) f32_pressure(ln, D, s_Pa[p], accp);
+            __builtin_amdgcn_sched_barrier(0);
+            f32_unit<U0>(ln, D, W, acc[0]);
+            f32_unit<U1>(ln, D, W, acc[1]);
+            f32_unit<U2>(ln, D, W, acc[2]);
+        }
+        __syncthreads();
+        if (work) {
+            if (kWave == 3) f32_pressure_stage(ln, accp, s_stage);
+            f32_unit_stage<U0>(ln, acc[0], s_stage);
+            f32_unit_stage<U1>(ln, acc[1], s_stage);
+            f32_unit_stage<U2>(ln, acc[2], s_stage);
         }
         __syncthreads();
     }
 }
 
-// FP64 element matrices on v_mfma_f64_4x4x4f64 (four 4x4x4 blocks per
-// instruction; lane = c + 4 blk + 16 h holds A_blk[c][h], B_blk[h][c] and the
-// result D_blk[h][c]).  The FP64 16x16x4 instruction runs at about 60% of the
-// 4x4x4 rate here, and the 4-wide tiles also pad 27 to 28 instead of 32.
-// Same producer/consumer pipeline as mr_element_matrix_kernel.  A consumer
-// instruction covers the row tiles I = 4t + blk of one displacement block
-// (rows m = 16t + 4blk + i) against one column tile J (n = 4J + j):
-//   A = U^{ab}_g[16t + l][j_dim] from the lane's D slice and W (l = c + 4 blk),
-//   B = D_g[j_dim][4J + c], shared by the four row tiles, read from LDS;
-// k-step s covers j_dim = s / 7 and g = 4 (s % 7) + h.  Lower block (a, b)
-// is numbered q = a (a + 1) / 2 + b (F64Unit).
+__global__ void __launch_bounds__(kElementThreads)
+mr_element_matrix_f32_kernel(int n_elements, const double *__restrict__ rec, const BasisTables *__restrict__ T,
+                             float *__restrict__ kbuf)
+{
+    __shared__ double s_rec[52][27];     // Gauss-point records
+    __shared__ float s_D[2][28][3][32];  // D_g[j][n]; g = 27 and n >= 27 zero
+    __shared__ float s_W[2][28][81];     // W_g[(a,i),(b,j)] at [g][(3a+i)*9 + 3b+j]; g = 27 zero
+    __shared__ float s_Pa[2][28 * 16];   // J_z w_g psi_m(g) at [g*16 + m]; m >= 8 and g = 27 zero
+    __shared__ float s_stage[kStageSize];
+    const int t = threadIdx.x, lane = t & 63;
+    const int role = __builtin_amdgcn_readfirstlane(t >> 6);
+    const int e0 = static_cast<int>(blockIdx.x), step = static_cast<int>(gridDim.x);
+    const int n_mine = e0 < n_elements ? (n_elements - 1 - e0) / step + 1 : 0;
+    for (int k = t; k < 2 * 28 * 3 * 32; k += kElementThreads) (&s_D[0][0][0][0])[k] = 0.0f;
+    for (int k = t; k < 2 * 28 * 81; k += kElementThreads) (&s_W[0][0][0])[k] = 0.0f;
+    for (int k = t; k < 2 * 28 * 16; k += kElementThreads) (&s_Pa[0][0])[k] = 0.0f;
+    if (t == 0) s_stage[kStageZero] = 0.0f;
+    // every wave passes the barriers of each slot in a loop of its own role
+    if (role < 4 || role >= 8) {
+        __syncthreads();
+        switch (role) {
+        case 0: f32_consumer<0>(lane, n_mine, s_D, s_W, s_Pa, s_stage); break;
+        case 1: f32_consumer<1>(lane, n_mine, s_D, s_W, s_Pa, s_stage); break;
+        case 2: f32_consumer<2>(lane, n_mine, s_D, s_W, s_Pa, s_stage); break;
+        case 3: f32_consumer<3>(lane, n_mine, s_D, s_W, s_Pa, s_stage); break;
+        default: element_storer<float>(t - 2 * kRoleThreads, n_mine, e0, step, s_stage, kbuf); break;
+        }
+        return;
+    }
+    const int pt = t - kRoleThreads;
+    const ProducerTable tab = producer_table(T, pt);
+    const double psi = pt < 27 * 8 ? T->lin27[pt * 4] : 0.0;  // psi_m(g) at g = pt / 8, m = pt % 8
+    // thread pt < 243 also owns column rq of W_g (row (a,i), column (b,j))
+    const int rq = pt % 81, pg = pt / 81, dj = rq / 27, dn = rq % 27;
+    const int wa = rq / 27, wi = (rq / 9) % 3, wb = (rq % 9) / 3, wj = rq % 3;
+    const int wf1 = GP_C + t2v(wi, wa) + 6 * t2v(wj, wb), wf2 = GP_SIGJ + t2v(wi, wj);
+    const bool wdiag = wa == wb;
+    double pre[kRecPerThread];
+    load_records(rec, e0, n_mine > 0, pt, pre);
+    put_records(s_rec, pt, pre);
+    load_records(rec, e0 + step, n_mine > 1, pt, pre);
+    __syncthreads();
+    for (int s = 0; s < n_mine + 2; ++s) {
+        double nxt[kRecPerThread];
+        load_records(rec, e0 + static_cast<int64_t>(s + 2) * step, s + 2 < n_mine, pt, nxt);
+        if (s < n_mine) {
+            const int p = s & 1;
+            const double(*R)[27] = s_rec;
+            // all LDS reads of a phase before its writes: one round trip
+            if (pt < 243) {  // g = pg + 3k
+                float dv[9], wv[9];
+#pragma unroll
+                for (int k = 0; k < 9; ++k) dv[k] = static_cast<float>(producer_d(R, tab, dj, pg + 3 * k, k));
+#pragma unroll
+                for (int k = 0; k < 9; ++k) s_D[p][pg + 3 * k][dj][dn] = dv[k];
+#pragma unroll
+                for (int k = 0; k < 9; ++k) {
+                    const int g = pg + 3 * k;
+                    double v = R[wf1][g];
+                    if (wdiag) v = v + R[wf2][g];
+                    wv[k] = static_cast<float>(R[GP_JGW][g] * v);
+                }
+#pragma unroll
+                for (int k = 0; k < 9; ++k) s_W[p][pg + 3 * k][rq] = wv[k];
+            }
+            if (pt < 27 * 8) s_Pa[p][pt / 8 * 16 + pt % 8] = static_cast<float>(R[GP_JGW][pt / 8] * psi);
+        }
+        __syncthreads();
+        put_records(s_rec, pt, pre);
+#pragma unroll
+        for (int i = 0; i < kRecPerThread; ++i) pre[i] = nxt[i];
+        __syncthreads();
+    }
+}
 
+// ---- FP64 element matrices: v_mfma_f64_4x4x4f64 ---------------------------------
+// Four 4x4x4 blocks per instruction; lane = c + 4 blk + 16 h holds A_blk[c][h],
+// B_blk[h][c] and the result D_blk[h][c].  The FP64 16x16x4 instruction runs at
+// about 60% of the 4x4x4 rate here, and the 4-wide tiles also pad 27 to 28
+// instead of 32.  A consumer instruction covers the row tiles I = 4t + blk of one
+// displacement block (rows m = 16t + 4blk + i) against one column tile J
+// (n = 4J + j):
+//   A = U^{ab}_g[16t + l][j_dim] from D and W (l = c + 4 blk),
+//   B = D_g[j_dim][4J + c], shared by the four row tiles, read from LDS;
+// k-step s covers g = 4 (s / 3) + h and j_dim = s % 3.  Lower block (a, b) is
+// numbered q = a (a + 1) / 2 + b (F64Unit).
+// An FP64 MFMA and a vector instruction do not overlap here, not even from two
+// wavefronts of a SIMD (16 of the one and 64 of the other take the sum of their
+// times), and alternating them costs 13 cycles a switch: so the SIMD's time is
+// that of its MFMAs plus that of all its wavefronts' vector instructions, and
+// the kernel keeps those few and together.
 __device__ __forceinline__ double2 lds_pair(const double *p) { return *reinterpret_cast<const double2 *>(p); }
 
 template <int Q, int T, int NJ>
@@ -812,225 +886,233 @@ struct F64Unit {
     static constexpr int b = Q - (a * (a + 1)) / 2;
 };
 
-// stores the tiles of one unit: acc[J] at m = 16T + 4blk + h, n = 4J + c
+// the tiles of one unit into the staging area: acc[J] at m = 16T + 4blk + h,
+// n = 4J + c
 template <typename U>
-__device__ __forceinline__ void f64_unit_store(const double *acc, int blk, int h, int c, __amdgpu_buffer_rsrc_t rs)
+__device__ __forceinline__ void f64_unit_stage(int lane, const double *acc, double *s_stage)
 {
-    const int m = 16 * U::t + 4 * blk + h;
-    const int vdir = ((4 * blk + h) * 89 + c) * 8, vmir = (c * 89 + 4 * blk + h) * 8;
+    const int c = lane & 3, m = 16 * U::t + (lane & 12) + (lane >> 4);
+    if (m >= 27) return;
+    double *o = s_stage + U::q * kStageBlock + m * kStageRow + c;
 #pragma unroll
-    for (int J = 0; J < U::nj; ++J) {
-        const int n = 4 * J + c;
-        if (m >= 27 || n >= 27 || (U::a == U::b && m < n)) continue;
-        element_store(rs, acc[J], vdir, ((U::a * 27 + 16 * U::t) * 89 + U::b * 27 + 4 * J) * 8);
-        element_store(rs, acc[J], vmir, ((U::b * 27 + 4 * J) * 89 + U::a * 27 + 16 * U::t) * 8);
-    }
+    for (int J = 0; J < U::nj; ++J)
+        if (J < 6 || c < 3) o[4 * J] = acc[J];
 }
 
+// LDS layouts.  D_g[j][n] at [g][j][n % 4][n / 4], the Gauss points 98 doubles
+// apart: the four g of a 16-byte read then fall on different banks.  W_g[(a,i),
+// (b,j)] of lower block q at [g][q][j][i], i padded to 4.
+constexpr int kDStride = 98, kWStride = 72;
+
 // three units of one wave, all on row half T, sharing the B reads of every
-// k-step; the B and W operands of step s + 1 are loaded while the MFMAs of
+// k-step; the operands of step s + 1 are loaded and formed while the MFMAs of
 // step s run
 template <int T, typename U0, typename U1, typename U2>
-__device__ __forceinline__ void f64_units(int lane, const double (&DT)[7][3], const double *sD, const double *sW,
-                                          __amdgpu_buffer_rsrc_t rs)
+__device__ __forceinline__ void f64_units(int lane, const double *sD, const double *sW, double (&acc)[3][7])
 {
     const int c = lane & 3, blk = (lane >> 2) & 3, h = lane >> 4;
-    double acc0[7], acc1[7], acc2[7];
 #pragma unroll
-    for (int J = 0; J < 7; ++J) acc0[J] = acc1[J] = acc2[J] = 0.0;
-    double B[2][7], W[2][3][3];
-    auto load = [&](int st, double (&b)[7], double (&w)[3][3]) {
-        const int jd = st / 7, g = 4 * (st % 7) + h;
-        const double *bp = sD + ((g * 3 + jd) * 4 + c) * 8;  // D_g[jd][4J + c], J = 0..6
+    for (int x = 0; x < 3; ++x)
+#pragma unroll
+        for (int J = 0; J < 7; ++J) acc[x][J] = 0.0;
+    double B[2][7], W[2][3][3], DT[2][3], u[2][3];  // DT: D_g[i][16t + 4blk + c]
+    auto load_b = [&](int st, double (&b)[7]) {
+        const double *bp = sD + (4 * (st / 3) + h) * kDStride + (st % 3 * 4 + c) * 8;  // D_g[jd][4J + c], J = 0..6
         const double2 b01 = lds_pair(bp), b23 = lds_pair(bp + 2), b45 = lds_pair(bp + 4);
         b[0] = b01.x; b[1] = b01.y; b[2] = b23.x; b[3] = b23.y; b[4] = b45.x; b[5] = b45.y; b[6] = bp[6];
+    };
+    auto load_w = [&](int st, double (&w)[3][3]) {
         const int qs[3] = {U0::q, U1::q, U2::q};
 #pragma unroll
         for (int x = 0; x < 3; ++x) {
-            const double *wp = sW + ((g * 6 + qs[x]) * 3 + jd) * 4;  // W_g[(a,i),(b,jd)], i = 0..2
+            const double *wp = sW + (4 * (st / 3) + h) * kWStride + (qs[x] * 3 + st % 3) * 4;  // W_g[(a,i),(b,jd)], i = 0..2
             const double2 w01 = lds_pair(wp);
             w[x][0] = w01.x; w[x][1] = w01.y; w[x][2] = wp[2];
         }
     };
-    load(0, B[0], W[0]);
+    auto load_dt = [&](int gp, double (&d)[3]) {
+        const double *dp = sD + (4 * gp + h) * kDStride + c * 8 + 4 * T + blk;
+#pragma unroll
+        for (int i = 0; i < 3; ++i) d[i] = dp[i * 32];
+    };
+    auto a_operands = [](const double (&d)[3], const double (&w)[3][3], double (&o)[3]) {
+#pragma unroll
+        for (int x = 0; x < 3; ++x) o[x] = d[0] * w[x][0] + d[1] * w[x][1] + d[2] * w[x][2];
+    };
+    load_dt(0, DT[0]);
+    load_w(0, W[0]);
+    load_w(1, W[1]);
+    load_b(0, B[0]);
+    a_operands(DT[0], W[0], u[0]);
 #pragma unroll
     for (int st = 0; st < 21; ++st) {
-        const int cur = st & 1, gp = st % 7;
-        if (st + 1 < 21) load(st + 1, B[cur ^ 1], W[cur ^ 1]);
-        double u[3];
-#pragma unroll
-        for (int x = 0; x < 3; ++x)
-            u[x] = DT[gp][0] * W[cur][x][0] + DT[gp][1] * W[cur][x][1] + DT[gp][2] * W[cur][x][2];
+        const int cur = st & 1;
+        if (st + 1 < 21) a_operands(DT[((st + 1) / 3) & 1], W[cur ^ 1], u[cur ^ 1]);
+        if (st + 1 < 21) load_b(st + 1, B[cur ^ 1]);
+        if (st + 2 < 21) load_w(st + 2, W[cur]);
+        if (st % 3 == 0 && st / 3 + 1 < 7) load_dt(st / 3 + 1, DT[(st / 3 + 1) & 1]);
+        __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (int J = 0; J < 7; ++J) {
-            if (J < U0::nj) acc0[J] = __builtin_amdgcn_mfma_f64_4x4x4f64(u[0], B[cur][J], acc0[J], 0, 0, 0);
-            if (J < U1::nj) acc1[J] = __builtin_amdgcn_mfma_f64_4x4x4f64(u[1], B[cur][J], acc1[J], 0, 0, 0);
-            if (J < U2::nj) acc2[J] = __builtin_amdgcn_mfma_f64_4x4x4f64(u[2], B[cur][J], acc2[J], 0, 0, 0);
+            if (J < U0::nj) acc[0][J] = __builtin_amdgcn_mfma_f64_4x4x4f64(u[cur][0], B[cur][J], acc[0][J], 0, 0, 0);
+            if (J < U1::nj) acc[1][J] = __builtin_amdgcn_mfma_f64_4x4x4f64(u[cur][1], B[cur][J], acc[1][J], 0, 0, 0);
+            if (J < U2::nj) acc[2][J] = __builtin_amdgcn_mfma_f64_4x4x4f64(u[cur][2], B[cur][J], acc[2][J], 0, 0, 0);
         }
         __builtin_amdgcn_sched_barrier(0);
     }
-    f64_unit_store<U0>(acc0, blk, h, c, rs);
-    f64_unit_store<U1>(acc1, blk, h, c, rs);
-    f64_unit_store<U2>(acc2, blk, h, c, rs);
 }
 
-// pressure rows K_(p,m),(b,n), m = 4I + h, n = 16t + 4blk + c, for all b and
-// t; the B operand D_g[b][n] comes from LDS
-__device__ __forceinline__ void f64_pressure(int lane, const double *sD, const double *sPa, __amdgpu_buffer_rsrc_t rs)
+// pressure rows K_(p,m),(b,n): acc[b][I][t] at m = 4I + h, n = 16t + 4blk + c; the
+// B operand D_g[b][n] comes from LDS
+__device__ __forceinline__ void f64_pressure(int lane, const double *sD, const double *sPa, double (&acc)[3][2][2])
 {
     const int c = lane & 3, blk = (lane >> 2) & 3, h = lane >> 4;
 #pragma unroll
     for (int b = 0; b < 3; ++b) {
-        double acc[2][2] = {{0.0, 0.0}, {0.0, 0.0}};
+        acc[b][0][0] = acc[b][0][1] = acc[b][1][0] = acc[b][1][1] = 0.0;
 #pragma unroll
         for (int gp = 0; gp < 7; ++gp) {
             const int g = 4 * gp + h;
             const double *pp = sPa + g * 8 + c;
             const double a0 = pp[0], a1 = pp[4];
-            const double *bp = sD + ((g * 3 + b) * 4 + c) * 8 + blk;  // D_g[b][16t + 4blk + c] at +4t
+            const double *bp = sD + g * kDStride + (b * 4 + c) * 8 + blk;  // D_g[b][16t + 4blk + c] at +4t
             const double b0 = bp[0], b1 = bp[4];
-            acc[0][0] = __builtin_amdgcn_mfma_f64_4x4x4f64(a0, b0, acc[0][0], 0, 0, 0);
-            acc[1][0] = __builtin_amdgcn_mfma_f64_4x4x4f64(a1, b0, acc[1][0], 0, 0, 0);
-            acc[0][1] = __builtin_amdgcn_mfma_f64_4x4x4f64(a0, b1, acc[0][1], 0, 0, 0);
-            acc[1][1] = __builtin_amdgcn_mfma_f64_4x4x4f64(a1, b1, acc[1][1], 0, 0, 0);
+            acc[b][0][0] = __builtin_amdgcn_mfma_f64_4x4x4f64(a0, b0, acc[b][0][0], 0, 0, 0);
+            acc[b][1][0] = __builtin_amdgcn_mfma_f64_4x4x4f64(a1, b0, acc[b][1][0], 0, 0, 0);
+            acc[b][0][1] = __builtin_amdgcn_mfma_f64_4x4x4f64(a0, b1, acc[b][0][1], 0, 0, 0);
+            acc[b][1][1] = __builtin_amdgcn_mfma_f64_4x4x4f64(a1, b1, acc[b][1][1], 0, 0, 0);
         }
-        const int vdir = (h * 89 + 4 * blk + c) * 8, vmir = ((4 * blk + c) * 89 + h) * 8;
-#pragma unroll
-        for (int I = 0; I < 2; ++I)
-#pragma unroll
-            for (int t = 0; t < 2; ++t) {
-                if (16 * t + 4 * blk + c >= 27) continue;
-                element_store(rs, acc[I][t], vdir, ((81 + 4 * I) * 89 + b * 27 + 16 * t) * 8);
-                element_store(rs, acc[I][t], vmir, ((b * 27 + 16 * t) * 89 + 81 + 4 * I) * 8);
-            }
     }
 }
 
-__global__ void __launch_bounds__(512)
+__device__ __forceinline__ void f64_pressure_stage(int lane, const double (&acc)[3][2][2], double *s_stage)
+{
+    const int n0 = lane & 15, h = lane >> 4;
+    double *o = s_stage + kStageP + h * kStagePRow + n0;
+#pragma unroll
+    for (int b = 0; b < 3; ++b)
+#pragma unroll
+        for (int I = 0; I < 2; ++I)
+#pragma unroll
+            for (int t = 0; t < 2; ++t)
+                if (t == 0 || 16 + n0 < 27) o[4 * I * kStagePRow + b * 27 + 16 * t] = acc[b][I][t];
+}
+
+// the slots of consumer wave kWave (0..3): waves 0, 1 take row half t = 0 (and
+// the pressure rows), waves 2, 3 t = 1; 1659 k-steps per element: 378 / 399 /
+// 441 / 441
+template <int kWave>
+__device__ __forceinline__ void f64_consumer(int lane, int n_mine, const double (*s_D)[28 * kDStride],
+                                             const double (*s_W)[28 * kWStride], const double (*s_Pa)[28][8],
+                                             double *s_stage)
+{
+    constexpr int kT = kWave >> 1;
+    using U0 = F64Unit<(kWave & 1) ? 4 : 1, kT, 7>;
+    using U1 = F64Unit<(kWave & 1) ? 2 : 3, kT, kWave == 1 ? 4 : 7>;
+    using U2 = F64Unit<(kWave & 1) ? 5 : 0, kT, kT == 0 ? 4 : 7>;
+    for (int s = 0; s < n_mine + 2; ++s) {
+        // the lane index is made opaque per element so that offsets derived
+        // from it are recomputed here rather than held across the loop
+        int ln = lane;
+        asm volatile("" : "+v"(ln));
+        const bool work = s >= 1 && s - 1 < n_mine;
+        double acc[3][7], accp[3][2][2];
+        if (work) {
+            const int p = (s - 1) & 1;
+            if (kWave == 1) f64_pressure(ln, s_D[p], &s_Pa[p][0][0], accp);
+            f64_units<kT, U0, U1, U2>(ln, s_D[p], s_W[p], acc);
+        }
+        __syncthreads();
+        if (work) {
+            if (kWave == 1) f64_pressure_stage(ln, accp, s_stage);
+            f64_unit_stage<U0>(ln, acc[0], s_stage);
+            f64_unit_stage<U1>(ln, acc[1], s_stage);
+            f64_unit_stage<U2>(ln, acc[2], s_stage);
+        }
+        __syncthreads();
+    }
+}
+
+__global__ void __launch_bounds__(kElementThreads)
 mr_element_matrix_f64_kernel(int n_elements, const double *__restrict__ rec, const BasisTables *__restrict__ T,
                              double *__restrict__ kbuf)
 {
-    __shared__ double s_tab[27][3][27];          // dphi_n/dxi_mi at g: [g][mi][n]
-    __shared__ double s_psi[27][8];              // trilinear psi_m(g)
-    __shared__ double s_rec[2][52][27];          // Gauss-point records
-    __shared__ __align__(16) double s_D[2][28][3][4][8];  // D_g[j][n] at [g][j][n % 4][n / 4]; padding zero
-    __shared__ __align__(16) double s_W[2][28][6][3][4];  // W_g[(a,i),(b,j)], lower block q, at [g][q][j][i]; padding zero
-    __shared__ double s_Pa[2][28][8];            // J_z w_g psi_m(g); g = 27 zero
-    constexpr int kRec = 52 * 27, kRecPerThread = (kRec + 255) / 256;
+    __shared__ double s_rec[52][27];                        // Gauss-point records
+    __shared__ __align__(16) double s_D[2][28 * kDStride];  // padding zero
+    __shared__ __align__(16) double s_W[2][28 * kWStride];  // padding zero
+    __shared__ double s_Pa[2][28][8];                       // J_z w_g psi_m(g); g = 27 zero
+    __shared__ double s_stage[kStageSize];
     const int t = threadIdx.x, lane = t & 63;
-    const bool producer = t >= 256;
-    const int pt = producer ? t - 256 : 0;
-    // producer thread pt < 243 owns (j, n) = (rq / 27, rq % 27) of D_g for
-    // g = pg (mod 3); pt < 216 owns (q, j, i) = wq of W_g for g = pw (mod 4)
+    const int role = __builtin_amdgcn_readfirstlane(t >> 6);
+    const int e0 = static_cast<int>(blockIdx.x), step = static_cast<int>(gridDim.x);
+    const int n_mine = e0 < n_elements ? (n_elements - 1 - e0) / step + 1 : 0;
+    for (int k = t; k < 2 * 28 * kDStride; k += kElementThreads) (&s_D[0][0])[k] = 0.0;
+    for (int k = t; k < 2 * 28 * kWStride; k += kElementThreads) (&s_W[0][0])[k] = 0.0;
+    for (int k = t; k < 2 * 28 * 8; k += kElementThreads) (&s_Pa[0][0][0])[k] = 0.0;
+    if (t == 0) s_stage[kStageZero] = 0.0;
+    // every wave passes the barriers of each slot in a loop of its own role
+    if (role < 4 || role >= 8) {
+        __syncthreads();
+        switch (role) {
+        case 0: f64_consumer<0>(lane, n_mine, s_D, s_W, s_Pa, s_stage); break;
+        case 1: f64_consumer<1>(lane, n_mine, s_D, s_W, s_Pa, s_stage); break;
+        case 2: f64_consumer<2>(lane, n_mine, s_D, s_W, s_Pa, s_stage); break;
+        case 3: f64_consumer<3>(lane, n_mine, s_D, s_W, s_Pa, s_stage); break;
+        default: element_storer<double>(t - 2 * kRoleThreads, n_mine, e0, step, s_stage, kbuf); break;
+        }
+        return;
+    }
+    const int pt = t - kRoleThreads;
+    const ProducerTable tab = producer_table(T, pt);
+    const double psi = pt < 27 * 8 ? T->lin27[pt * 4] : 0.0;  // psi_m(g) at g = pt / 8, m = pt % 8
     const int rq = pt % 81, pg = pt / 81, dj = rq / 27, dn = rq % 27;
+    // pt < 216 owns (q, j, i) = wq of W_g for g = pw (mod 4)
     const int wq = pt % 54, pw = pt / 54;
     const int wqq = wq / 9, wj = (wq / 3) % 3, wi = wq % 3;
     const int wa = wqq == 0 ? 0 : (wqq <= 2 ? 1 : 2), wb = wqq - (wa * (wa + 1)) / 2;
     const int wf1 = GP_C + t2v(wi, wa) + 6 * t2v(wj, wb), wf2 = GP_SIGJ + t2v(wi, wj);
     const bool wdiag = wa == wb;
-    const int64_t n_gp = static_cast<int64_t>(n_elements) * 27;
-    const int n_mine = static_cast<int>(blockIdx.x) < n_elements
-                           ? (n_elements - 1 - static_cast<int>(blockIdx.x)) / static_cast<int>(gridDim.x) + 1
-                           : 0;
-    for (int k = t; k < 27 * 27 * 3; k += 512) {
-        const int g = k / 81, mi = (k / 27) % 3, n = k % 27;
-        s_tab[g][mi][n] = T->quad27[(g * 27 + n) * 4 + 1 + mi];
-    }
-    for (int k = t; k < 27 * 8; k += 512) s_psi[k / 8][k % 8] = T->lin27[k * 4];
-    for (int k = t; k < 2 * 28 * 3 * 4 * 8; k += 512) (&s_D[0][0][0][0][0])[k] = 0.0;
-    for (int k = t; k < 2 * 28 * 6 * 3 * 4; k += 512) (&s_W[0][0][0][0][0])[k] = 0.0;
-    for (int k = t; k < 2 * 28 * 8; k += 512) (&s_Pa[0][0][0])[k] = 0.0;
-    if (producer && n_mine > 0) {
-        const int64_t q0 = static_cast<int64_t>(blockIdx.x) * 27;
-        for (int k = pt; k < kRec; k += 256) s_rec[0][k / 27][k % 27] = rec[(k / 27) * n_gp + q0 + (k % 27)];
-    }
+    double pre[kRecPerThread];
+    load_records(rec, e0, n_mine > 0, pt, pre);
+    put_records(s_rec, pt, pre);
+    load_records(rec, e0 + step, n_mine > 1, pt, pre);
     __syncthreads();
-
-    for (int it = 0; it <= n_mine; ++it) {
-        if (producer) {
-            if (it < n_mine) {
-                const int p = it & 1;
-                const int e_next = static_cast<int>(blockIdx.x) + (it + 1) * static_cast<int>(gridDim.x);
-                double pre[kRecPerThread];
+    for (int s = 0; s < n_mine + 2; ++s) {
+        double nxt[kRecPerThread];
+        load_records(rec, e0 + static_cast<int64_t>(s + 2) * step, s + 2 < n_mine, pt, nxt);
+        if (s < n_mine) {
+            const int p = s & 1;
+            const double(*R)[27] = s_rec;
+            // every LDS read of a phase is issued before its writes (which
+            // the compiler may not move reads across), so a phase waits
+            // for one LDS round trip rather than one per Gauss point
+            if (pt < 243) {  // g = pg + 3k
+                double dv[9];
 #pragma unroll
-                for (int i = 0; i < kRecPerThread; ++i) {
-                    const int k = pt + 256 * i;
-                    pre[i] = (it + 1 < n_mine && k < kRec)
-                                 ? rec[(k / 27) * n_gp + static_cast<int64_t>(e_next) * 27 + (k % 27)]
-                                 : 0.0;
-                }
-                const double(*R)[27] = s_rec[p];
-                // every LDS read of a phase is issued before its writes (which
-                // the compiler may not move reads across), so a phase waits
-                // for one LDS round trip rather than one per Gauss point
-                if (pt < 243) {  // D_g[j][n] = sum_mi DXI_DX(mi, j) dphi_n/dxi_mi (:974-986), g = pg + 3k
-                    double dv[9];
+                for (int k = 0; k < 9; ++k) dv[k] = producer_d(R, tab, dj, pg + 3 * k, k);
 #pragma unroll
-                    for (int k = 0; k < 9; ++k) {
-                        const int g = pg + 3 * k;
-                        dv[k] = R[GP_DXIDZ + 0 + 3 * dj][g] * s_tab[g][0][dn] +
-                                R[GP_DXIDZ + 1 + 3 * dj][g] * s_tab[g][1][dn] +
-                                R[GP_DXIDZ + 2 + 3 * dj][g] * s_tab[g][2][dn];
-                    }
-#pragma unroll
-                    for (int k = 0; k < 9; ++k) s_D[p][pg + 3 * k][dj][dn % 4][dn / 4] = dv[k];
-                }
-                if (pt < 216) {  // W_g[(a,i),(b,j)] = J_z w_g (c + delta_ab sigma_ij), g = pw + 4k < 27
-                    double wv[7];
-#pragma unroll
-                    for (int k = 0; k < 7; ++k) {
-                        const int g = min(pw + 4 * k, 26);
-                        double v = R[wf1][g];
-                        if (wdiag) v = v + R[wf2][g];
-                        wv[k] = R[GP_JGW][g] * v;
-                    }
-                    const double pa = R[GP_JGW][pt / 8] * s_psi[pt / 8][pt % 8];
-#pragma unroll
-                    for (int k = 0; k < 7; ++k)
-                        if (pw + 4 * k < 27) s_W[p][pw + 4 * k][wqq][wj][wi] = wv[k];
-                    s_Pa[p][pt / 8][pt % 8] = pa;
-                }
-                if (it + 1 < n_mine) {
-#pragma unroll
-                    for (int i = 0; i < kRecPerThread; ++i) {
-                        const int k = pt + 256 * i;
-                        if (k < kRec) s_rec[p ^ 1][k / 27][k % 27] = pre[i];
-                    }
-                }
+                for (int k = 0; k < 9; ++k) s_D[p][(pg + 3 * k) * kDStride + (dj * 4 + dn % 4) * 8 + dn / 4] = dv[k];
             }
-        } else if (it >= 1) {
-            const int p = (it - 1) & 1;
-            const int e = static_cast<int>(blockIdx.x) + (it - 1) * static_cast<int>(gridDim.x);
-            // the lane index is made opaque per element so that offsets derived
-            // from it are recomputed here rather than held across the loop
-            int ln = lane;
-            asm volatile("" : "+v"(ln));
-            const int c = ln & 3, blk = (ln >> 2) & 3, h = ln >> 4, wave = t >> 6;
-            // waves 0, 1: row half t = 0 (and the pressure rows); waves 2, 3: t = 1.
-            // The lane keeps D_g[i][16t + 4blk + c] for its Gauss points g = 4gp + h.
-            const int tw = wave >> 1;
-            double DT[7][3];
+            if (pt < 216) {  // W_g[(a,i),(b,j)] = J_z w_g (c + delta_ab sigma_ij), g = pw + 4k < 27
+                double wv[7];
 #pragma unroll
-            for (int gp = 0; gp < 7; ++gp)
+                for (int k = 0; k < 7; ++k) {
+                    const int g = min(pw + 4 * k, 26);
+                    double v = R[wf1][g];
+                    if (wdiag) v = v + R[wf2][g];
+                    wv[k] = R[GP_JGW][g] * v;
+                }
+                const double pa = R[GP_JGW][pt / 8] * psi;
 #pragma unroll
-                for (int j = 0; j < 3; ++j) DT[gp][j] = s_D[p][4 * gp + h][j][c][4 * tw + blk];
-            const double *sD = &s_D[p][0][0][0][0], *sW = &s_W[p][0][0][0][0];
-            const __amdgpu_buffer_rsrc_t rs = element_rsrc(kbuf + static_cast<int64_t>(e) * 89 * 89);
-            // 1659 k-steps per element: 378 / 399 / 441 / 441
-            if (wave == 0) {
-                f64_units<0, F64Unit<1, 0, 7>, F64Unit<3, 0, 7>, F64Unit<0, 0, 4>>(ln, DT, sD, sW, rs);
-            } else if (wave == 1) {
-                f64_units<0, F64Unit<4, 0, 7>, F64Unit<2, 0, 4>, F64Unit<5, 0, 4>>(ln, DT, sD, sW, rs);
-                f64_pressure(ln, sD, &s_Pa[p][0][0], rs);
-            } else if (wave == 2) {
-                f64_units<1, F64Unit<1, 1, 7>, F64Unit<3, 1, 7>, F64Unit<0, 1, 7>>(ln, DT, sD, sW, rs);
-            } else {
-                f64_units<1, F64Unit<4, 1, 7>, F64Unit<2, 1, 7>, F64Unit<5, 1, 7>>(ln, DT, sD, sW, rs);
-                // zero p-p block
-                double *Ke = kbuf + static_cast<int64_t>(e) * 89 * 89;
-                Ke[(81 + ln / 8) * 89 + 81 + ln % 8] = 0.0;
+                for (int k = 0; k < 7; ++k)
+                    if (pw + 4 * k < 27) s_W[p][(pw + 4 * k) * kWStride + (wqq * 3 + wj) * 4 + wi] = wv[k];
+                s_Pa[p][pt / 8][pt % 8] = pa;
             }
         }
+        __syncthreads();
+        put_records(s_rec, pt, pre);
+#pragma unroll
+        for (int i = 0; i < kRecPerThread; ++i) pre[i] = nxt[i];
         __syncthreads();
     }
 }
@@ -1123,7 +1205,7 @@ int launch_schur_mass(EquationsSet &s, double *inv_p)
     OC_CHECK(ensure_tables(&T));
     const int nl = s.n_nodes_l;
     schur_mass_kernel<<<static_cast<unsigned>((nl + 255) / 256), 256, 0, runtime().stream>>>(
-        nl, s.gather_ptr.ptr + 3 * static_cast<int64_t>(s.n_nodes), s.gather_idx.ptr, s.n_elements, s.gp_records.ptr, T,
+        nl, s.gather_ptr.ptr + 3 * static_cast<int64_t>(s.n_nodes), s.gather_idx.ptr, s.gp_records.ptr, T,
         s.mat.ptr, inv_p);
     OC_HIP_CHECK(hipGetLastError());
     return OC_NO_ERROR;
@@ -1151,16 +1233,16 @@ int launch_mr_element_matrices(EquationsSet &s, int precision, int blocks_per_cu
     const BasisTables *T = nullptr;
     OC_CHECK(ensure_tables(&T));
     Runtime &rt = runtime();
-    // default: one resident block of eight waves per CU
+    // default: one resident block of twelve waves per CU
     const int bpc = blocks_per_cu > 0 ? blocks_per_cu : 1;
     const unsigned blocks = static_cast<unsigned>(std::min(s.n_elements, rt.num_cus * bpc));
     if (precision == OC_FP64) {
         KernelTimer timer("mr_element_matrix_fp64");
-        mr_element_matrix_f64_kernel<<<blocks, 512, 0, rt.stream>>>(s.n_elements, s.gp_records.ptr, T, s.kbuf64.ptr);
+        mr_element_matrix_f64_kernel<<<blocks, kElementThreads, 0, rt.stream>>>(s.n_elements, s.gp_records.ptr, T, s.kbuf64.ptr);
     } else {
         KernelTimer timer("mr_element_matrix_fp32");
-        mr_element_matrix_kernel<float><<<blocks, 512, 0, rt.stream>>>(s.n_elements, s.gp_records.ptr, T,
-                                                                      s.kbuf32.ptr);
+        mr_element_matrix_f32_kernel<<<blocks, kElementThreads, 0, rt.stream>>>(s.n_elements, s.gp_records.ptr, T,
+                                                                               s.kbuf32.ptr);
     }
     OC_HIP_CHECK(hipGetLastError());
     return OC_NO_ERROR;

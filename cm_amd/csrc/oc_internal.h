@@ -202,7 +202,7 @@ struct EquationsSet {
     DevBuf<float> uu_x4;  // the iterate the smoother gathers, per node (x, y, z, -) in FP32; two buffers
     DevBuf<double> dofs, residual, rhs;
 
-    // Mooney-Rivlin: per-Gauss-point records (field-major, see
+    // Mooney-Rivlin: per-Gauss-point records (see GpField,
     // oc_elasticity.hip) and the CSR scatter map: element column j of row
     // dof_i of element e sits at row_ptr[dof_i] + (j / 27) * row_nb[dof_i] +
     // col_rank[(e*35 + k)*35 + j % 27] for j < 81 (3 * row_nb + rank of
