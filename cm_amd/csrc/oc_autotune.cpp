@@ -100,10 +100,10 @@ extern "C" int oc_autotune(oc_equations_set h, int precision, char *report, int 
     OC_CHECK(tune(js, "element_matrix_ms", 6, 0, reps,
                   [&](int i) { return launch_mr_element_matrices(s, precision, bpcs[i]); },
                   [&](int i) { return num(bpcs[i]); }, &c_elem));
-    // CSR row gather prefetch depth (element rows per chunk; default 8)
+    // CSR row gather prefetch depth (element rows per chunk; default 4)
     const int chunks[] = {4, 8, 16};
     Choice c_gather{};
-    OC_CHECK(tune(js, "row_gather_ms", 3, 1, reps, [&](int i) { return launch_mr_row_gather(s, precision, chunks[i]); },
+    OC_CHECK(tune(js, "row_gather_ms", 3, 0, reps, [&](int i) { return launch_mr_row_gather(s, precision, chunks[i]); },
                   [&](int i) { return num(chunks[i]); }, &c_gather));
 
     // SpMV: lanes per row (per node for node rows) x neighbours in flight per

@@ -174,6 +174,24 @@ column_rank_kernel(int n_elements, const int *__restrict__ conn_q, const int *__
     rank[gid] = ok ? static_cast<uint8_t>(rk) : 0;
 }
 
+// Row of the element buffer that holds element matrix row i (0..80: component i
+// / 27 of node i % 27; pressure rows after them): a node's three rows lie next
+// to each other, as the row gather reads them.
+__device__ __forceinline__ int kbuf_row(int i) { return i < 81 ? 3 * (i % 27) + i / 27 : i; }
+
+// The row gather's lists, from the DOF -> element-entry lists: entry p < 27 E of
+// the component-0 rows (node m of element e) holds the element-buffer row of the
+// node's first component and the row of the rank table; the entries of the
+// pressure rows follow.
+__global__ void __launch_bounds__(256) row_lists_kernel(int n_elements, const int *__restrict__ gidx, int2 *__restrict__ lists)
+{
+    const int64_t q = static_cast<int64_t>(n_elements) * 27;
+    const int64_t t = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
+    if (t >= static_cast<int64_t>(n_elements) * 35) return;
+    const int ei = gidx[t < q ? t : t + 2 * q], e = ei / 89, i = ei % 89;
+    lists[t] = make_int2(e * 89 + kbuf_row(i), e * kRankNodes + (i < 81 ? i : i - 54));
+}
+
 int mr_prepare(EquationsSet &s)
 {
     if (s.col_rank.ptr) return OC_NO_ERROR;
@@ -229,6 +247,11 @@ int mr_prepare(EquationsSet &s)
         for (int i = 0; i < 89; ++i) idx[fillp[dof_of(e, i)]++] = static_cast<int32_t>(e * 89 + i);
     OC_CHECK(s.gather_ptr.upload(ptr.data(), ptr.size()));
     OC_CHECK(s.gather_idx.upload(idx.data(), idx.size()));
+    const int64_t nlist = static_cast<int64_t>(s.n_elements) * 35;
+    OC_CHECK(s.row_lists.alloc(static_cast<size_t>(2 * nlist)));
+    row_lists_kernel<<<static_cast<unsigned>((nlist + 255) / 256), 256, 0, rt.stream>>>(
+        s.n_elements, s.gather_idx.ptr, reinterpret_cast<int2 *>(s.row_lists.ptr));
+    OC_HIP_CHECK(hipGetLastError());
     return OC_NO_ERROR;
 }
 
@@ -399,7 +422,7 @@ mr_residual_element_kernel(int n_elements, const int *__restrict__ conn_q, const
             const int r = q < 27 ? a * 27 + q : 81 + (q - 27);
             if (kFD) {
                 const int64_t e = v / 89, col = v % 89;
-                kfd[(e * 89 + r) * 89 + col] = (acc[a] - relem[e * 89 + r]) / delta;
+                kfd[(e * 89 + kbuf_row(r)) * 89 + col] = (acc[a] - relem[e * 89 + r]) / delta;
             } else {
                 relem[static_cast<int64_t>(v) * 89 + r] = acc[a];
             }
@@ -510,7 +533,7 @@ typedef float mfma_f32x4 __attribute__((ext_vector_type(4)));
 //   * the consumers, waves 0..3, run the MFMA contraction of element s - 1 from
 //     the other half;
 //   * the storers, waves 8..11, copy the staged tiles of element s - 2 to its
-//     row-major matrix.
+//     place in the element buffer.
 // Between the slot's two barriers the consumers put their accumulators into the
 // staging area and the producers the records of element s + 1 into theirs.
 //
@@ -532,11 +555,12 @@ constexpr int kStageP = 6 * kStageBlock, kStageZero = kStageP + 8 * kStagePRow, 
 constexpr int kEntries = 89 * 89;
 constexpr int kStorePairs = ((kEntries + 1) / 2 + kRoleThreads - 1) / kRoleThreads;  // pairs of entries per storer thread
 
-// staging place of entry idx of the row-major 89x89 matrix: blocks above the
+// staging place of entry idx of the 89x89 element buffer: blocks above the
 // diagonal mirror those below (:1149-1153), the p-p block is zero
 __device__ __forceinline__ int stage_place(int idx)
 {
-    const int r = idx / 89, j = idx % 89;
+    const int br = idx / 89, j = idx % 89;
+    const int r = br < 81 ? (br % 3) * 27 + br / 3 : br;  // the inverse of kbuf_row
     const int hi = max(r, j), lo = min(r, j);
     if (lo >= 81) return kStageZero;
     if (hi >= 81) return kStageP + (hi - 81) * kStagePRow + lo;
@@ -1117,56 +1141,95 @@ mr_element_matrix_f64_kernel(int n_elements, const double *__restrict__ rec, con
     }
 }
 
-template <typename Real, int kChunk>
-__global__ void __launch_bounds__(64)
-csr_row_gather_kernel(int n_rows, const int64_t *__restrict__ row_ptr, const int *__restrict__ gptr,
-                      const int *__restrict__ gidx, const Real *__restrict__ kbuf,
-                      const uint8_t *__restrict__ rank, const uint16_t *__restrict__ row_nb,
-                      Real *__restrict__ values)
+// kN element rows of one CSR row: every global load before the LDS adds.  The
+// addresses are uniform and advance by scalar multiplies.
+template <int kN, typename Real>
+__device__ __forceinline__ void gather_rows(const int2 *__restrict__ list, int sub, int lane, bool hi, int m0, int m1,
+                                            int blk0, int blk1, const Real *__restrict__ kbuf,
+                                            const uint8_t *__restrict__ rank, Real *s_row)
+{
+    Real v0[kN], v1[kN];
+    int o0[kN], o1[kN];
+#pragma unroll
+    for (int c = 0; c < kN; ++c) {
+        const int2 at = list[c];
+        const Real *k = kbuf + static_cast<int64_t>(at.x + sub) * 89;
+        const uint8_t *rk = rank + static_cast<int64_t>(at.y) * kRankNodes;
+        v0[c] = k[lane];
+        o0[c] = rk[m0];
+        if (hi) {
+            v1[c] = k[lane + 64];
+            o1[c] = rk[m1];
+        }
+    }
+    // the adds of one element row complete before the next one's: a
+    // wavefront's LDS instructions run in order, and the barrier (no
+    // instruction) keeps all lanes together, so that the compiler does not
+    // take the lanes with and without a second column one after the other
+#pragma unroll
+    for (int c = 0; c < kN; ++c) {
+        s_row[blk0 + o0[c]] += v0[c];
+        if (hi) s_row[blk1 + o1[c]] += v1[c];
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+    }
+}
+
+// One wavefront per CSR row, three per block: block b < nq takes the three
+// displacement rows of node b, the blocks after them three pressure rows each.
+// A node's element rows lie next to each other in the element buffer and its
+// three rows share the lists and the neighbour ranks, which one row per block
+// fetched three times, from three XCDs (3.05 GB read then, 2.5 now, of 2.1 at
+// least, for 32,768 elements in FP64).  The element rows are taken in groups of
+// kMax, ..., 2, 1: with a test per row and the divisions that the shared lists
+// need, the scalar instructions took three times the vector ones' issue slots.
+// 32,768 elements FP64: 834 -> 788 us (4.0 GB, the rate of a copy; groups of 8,
+// which hold more registers, 801); 13,100 elements FP32: 343 -> 282 us.
+constexpr int kGatherRows = 3;
+
+template <typename Real, int kMax>
+__global__ void __launch_bounds__(64 * kGatherRows)
+csr_row_gather_kernel(int nq, int nl, int n_elements, int max_row, const int64_t *__restrict__ row_ptr,
+                      const int *__restrict__ gptr, const int2 *__restrict__ lists, const Real *__restrict__ kbuf,
+                      const uint8_t *__restrict__ rank, const uint16_t *__restrict__ row_nb, Real *__restrict__ values)
 {
     extern __shared__ unsigned char s_raw[];
-    Real *s_row = reinterpret_cast<Real *>(s_raw);
-    const int r = blockIdx.x, lane = threadIdx.x;
-    if (r >= n_rows) return;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+    Real *s_row = reinterpret_cast<Real *>(s_raw) + wave * max_row;  // a wavefront's own: no block barriers
+    const int b = blockIdx.x;
+    const bool disp = b < nq;
+    const int l = (b - nq) * kGatherRows + wave;
+    if (!disp && l >= nl) return;
+    const int r = disp ? wave * nq + b : 3 * nq + l;
+    const int gr = disp ? b : r;
+    const int g0 = gptr[gr], n = gptr[gr + 1] - g0;
+    const int2 *list = lists + (disp ? g0 : g0 - 54 * n_elements);
     const int64_t r0 = row_ptr[r];
     const int len = static_cast<int>(row_ptr[r + 1] - r0);
     const int nb = row_nb[r];
     for (int k = lane; k < len; k += 64) s_row[k] = Real(0);
-    __syncthreads();
+    __builtin_amdgcn_wave_barrier();
     // lane j holds element columns j and j + 64: component block and rank slot
-    const int blk0 = (lane / 27) * nb, m0 = lane % 27;
-    const bool hi = lane + 64 < 89;
     const int j1 = lane + 64;
+    const bool hi = j1 < 89;
+    const int blk0 = (lane / 27) * nb, m0 = lane % 27;
     const int blk1 = j1 < 81 ? (j1 / 27) * nb : 3 * nb, m1 = j1 < 81 ? j1 % 27 : 27 + j1 - 81;
-    // contributions in chunks of kChunk element rows: all global loads of a
-    // chunk are issued before its LDS accumulation
-    for (int c0 = gptr[r]; c0 < gptr[r + 1]; c0 += kChunk) {
-        const int nc = min(kChunk, gptr[r + 1] - c0);
-        Real v0[kChunk], v1[kChunk];
-        int o0[kChunk], o1[kChunk];
-#pragma unroll
-        for (int c = 0; c < kChunk; ++c) {
-            if (c < nc) {
-                const int ei = gidx[c0 + c];  // e*89 + i
-                const int e = ei / 89, i = ei % 89;
-                const int64_t base = static_cast<int64_t>(ei) * 89;
-                const uint8_t *rk = rank + (static_cast<int64_t>(e) * kRankNodes + (i < 81 ? i % 27 : i - 54)) *
-                                               kRankNodes;
-                v0[c] = kbuf[base + lane];
-                o0[c] = blk0 + rk[m0];
-                v1[c] = hi ? kbuf[base + j1] : Real(0);
-                o1[c] = hi ? blk1 + rk[m1] : -1;
-            }
-        }
-#pragma unroll
-        for (int c = 0; c < kChunk; ++c) {
-            if (c < nc) {
-                s_row[o0[c]] += v0[c];
-                if (o1[c] >= 0) s_row[o1[c]] += v1[c];
-            }
-            __syncthreads();
-        }
+    const int sub = disp ? wave : 0;
+    int c = 0;
+    for (; c + kMax <= n; c += kMax) gather_rows<kMax>(list + c, sub, lane, hi, m0, m1, blk0, blk1, kbuf, rank, s_row);
+    if (kMax > 8 && n - c >= 8) {
+        gather_rows<8>(list + c, sub, lane, hi, m0, m1, blk0, blk1, kbuf, rank, s_row);
+        c += 8;
     }
+    if (kMax > 4 && n - c >= 4) {
+        gather_rows<4>(list + c, sub, lane, hi, m0, m1, blk0, blk1, kbuf, rank, s_row);
+        c += 4;
+    }
+    if (n - c >= 2) {
+        gather_rows<2>(list + c, sub, lane, hi, m0, m1, blk0, blk1, kbuf, rank, s_row);
+        c += 2;
+    }
+    if (n - c >= 1) gather_rows<1>(list + c, sub, lane, hi, m0, m1, blk0, blk1, kbuf, rank, s_row);
     for (int k = lane; k < len; k += 64) values[r0 + k] = s_row[k];
 }
 
@@ -1174,25 +1237,18 @@ template <typename Real>
 static int launch_row_gather(EquationsSet &s, const Real *kbuf, Real *values, int chunk)
 {
     Runtime &rt = runtime();
-    const size_t row_lds = static_cast<size_t>(s.max_row_len) * sizeof(Real);
-    const unsigned grid = static_cast<unsigned>(s.n_rows);
+    const size_t lds = static_cast<size_t>(kGatherRows) * s.max_row_len * sizeof(Real);
+    const unsigned grid = static_cast<unsigned>(s.n_nodes + (s.n_nodes_l + kGatherRows - 1) / kGatherRows);
+#define OC_ROW_GATHER(C)                                                                                            \
+    csr_row_gather_kernel<Real, C><<<grid, 64 * kGatherRows, lds, rt.stream>>>(                                    \
+        s.n_nodes, s.n_nodes_l, s.n_elements, s.max_row_len, s.row_ptr.ptr, s.gather_ptr.ptr,                      \
+        reinterpret_cast<const int2 *>(s.row_lists.ptr), kbuf, s.col_rank.ptr, s.row_nb.ptr, values)
     switch (chunk) {
-    case 4:
-        csr_row_gather_kernel<Real, 4><<<grid, 64, row_lds, rt.stream>>>(s.n_rows, s.row_ptr.ptr, s.gather_ptr.ptr,
-                                                                        s.gather_idx.ptr, kbuf, s.col_rank.ptr, s.row_nb.ptr,
-                                                                        values);
-        break;
-    case 16:
-        csr_row_gather_kernel<Real, 16><<<grid, 64, row_lds, rt.stream>>>(s.n_rows, s.row_ptr.ptr, s.gather_ptr.ptr,
-                                                                         s.gather_idx.ptr, kbuf, s.col_rank.ptr, s.row_nb.ptr,
-                                                                         values);
-        break;
-    default:
-        csr_row_gather_kernel<Real, 8><<<grid, 64, row_lds, rt.stream>>>(s.n_rows, s.row_ptr.ptr, s.gather_ptr.ptr,
-                                                                        s.gather_idx.ptr, kbuf, s.col_rank.ptr, s.row_nb.ptr,
-                                                                        values);
-        break;
+    case 8: OC_ROW_GATHER(8); break;
+    case 16: OC_ROW_GATHER(16); break;
+    default: OC_ROW_GATHER(4); break;
     }
+#undef OC_ROW_GATHER
     OC_HIP_CHECK(hipGetLastError());
     return OC_NO_ERROR;
 }

@@ -210,12 +210,13 @@ struct EquationsSet {
     DevBuf<double> gp_records;
     DevBuf<uint8_t> col_rank;
     DevBuf<uint16_t> row_nb;
-    DevBuf<double> kbuf64;      // element matrices, E*89*89, row-major
+    DevBuf<double> kbuf64;      // element matrices, E*89*89, rows by nodes (kbuf_row, oc_elasticity.hip)
     DevBuf<float> kbuf32;
     int max_row_len = 0;
     // element residuals (E*89) and the DOF -> element-entry gather lists
     DevBuf<double> relem;
     DevBuf<int32_t> gather_ptr, gather_idx;
+    DevBuf<int32_t> row_lists;  // Mooney-Rivlin: the CSR row gather's pairs, see row_lists_kernel
     // Laplace: 8-bit offsets (in the row-gather order: entry p*8+j belongs to
     // the p-th element row of the gather lists); gather_idx holds the gather
     // position of element row e*8+i; element matrices in kbuf64 (E*64, rows

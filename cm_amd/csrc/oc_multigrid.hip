@@ -85,7 +85,7 @@ q1_galerkin_element_kernel(int n_elements, const Real *__restrict__ kbuf, const 
         const Real *Ke = kbuf + static_cast<int64_t>(e) * 89 * 89;
         for (int k = t; k < 81 * 81; k += 256) {
             const int i = k / 81, j = k % 81;
-            sK[i][j] = (sf[i] && sf[j]) ? Ke[i * 89 + j] : static_cast<Real>(0);
+            sK[i][j] = (sf[i] && sf[j]) ? Ke[(3 * (i % 27) + i / 27) * 89 + j] : static_cast<Real>(0);  // rows by nodes
         }
         __syncthreads();
         for (int k = t; k < 81 * 24; k += 256) {
