@@ -119,11 +119,19 @@ struct MgLevel {
     DevBuf<uint8_t> freed;                // nn*3: DOF not fixed
     DevBuf<double> x, b, r;               // nn*3 each
 };
+struct alignas(16) MgNode {               // a triquadratic node's place in A P0 (mg_nodes_kernel)
+    int64_t first;
+    int32_t lo;
+    uint32_t bits;
+};
 struct Multigrid {
     std::vector<int32_t> h_n;             // elements per direction of each mesh
-    DevBuf<int32_t> n, e_off;
+    DevBuf<int32_t> n;
     std::vector<MgLevel> levels;          // levels[0] holds only the per-mesh tables
-    DevBuf<double> ke1;                   // Galerkin trilinear element matrices, E*24*24
+    DevBuf<int64_t> ap_off;               // per mesh: its first block of A P0
+    DevBuf<double> ap;                    // A P0, 3x3 blocks by fine node (product_first, oc_multigrid.hip)
+    DevBuf<MgNode> nodes;
+    DevBuf<float> ap_sp;                  // the same in FP32, for an FP32 Jacobian's V-cycle
     DevBuf<double> t0, r0, x0;            // level-0 scratch (3*n_nodes each)
     DevBuf<double> coarse_inv;            // per mesh dense inverse of the coarsest level
     int coarse_stride = 0;                // (max DOFs per mesh at the coarsest level)^2
@@ -324,6 +332,7 @@ int launch_mr_gauss(EquationsSet &s);
 int launch_schur_mass(EquationsSet &s, double *inv_p);
 // multigrid (oc_multigrid.hip): setup after a Jacobian assembly in
 // `precision`; apply z_u = V-cycle(t) for the displacement block
+int mg_prepare(EquationsSet &s, int precision, bool *made);
 int mg_setup(EquationsSet &s, int precision);
 int mg_apply(EquationsSet &s, int precision, const double *t, double *z);
 // pressure-column starts and the node-row layout check (oc_solver.hip)

@@ -7,10 +7,8 @@
 //   level 0  triquadratic nodes (2n+1)^3: the assembled CSR itself (u-u part,
 //            columns left of the first pressure column of each row);
 //   level 1  trilinear nodes (n+1)^3 on the same elements (numbered like the
-//            pressure nodes); operator P0^T K P0 formed element by element
-//            from the element matrices of the last Jacobian assembly,
-//            K1_e = W^T M_e K_e M_e W (W: trilinear values at the 27 element
-//            nodes, M_e: free-DOF mask), assembled into a 27-point stencil;
+//            pressure nodes); operator P0^T (A P0) from the assembled rows, A
+//            masked by the free DOFs, as a 27-point stencil;
 //   level l+1 (ceil(n_l/2)+1)^3 nodes, linear interpolation in each lattice
 //            direction (even fine index -> coarse i/2, odd -> mean of its two
 //            coarse neighbours), operator P^T A_l P on the stencils.
@@ -45,101 +43,168 @@ __device__ __forceinline__ int find_mesh(const int *__restrict__ off, int M, int
 
 __device__ __forceinline__ double lin_weight(int delta) { return delta == 0 ? 1.0 : 0.5; }
 
-// ---- setup -----------------------------------------------------------------------------
-template <typename Real>
-__global__ void __launch_bounds__(256)
-q1_galerkin_element_kernel(int n_elements, const Real *__restrict__ kbuf, const int *__restrict__ conn_q, int nq,
-                           const uint8_t *__restrict__ free_mask, double *__restrict__ ke1)
+// ---- the product A P0 --------------------------------------------------------------------
+// Node i = (ix, iy, iz) of the (2n+1)^3 lattice couples to the trilinear nodes
+// lo .. lo + c - 1 per direction: c = 3 from i/2 - 1 for an even index, c = 2
+// from i/2 for an odd one, those outside the grid holding zeros.  Its S = cx cy
+// cz blocks stand in x, y, z order, entry rc of block s at 9 first + rc S + s;
+// X(i) blocks precede index i in a direction, X(2n + 1) = 5n + 3.
+__device__ __forceinline__ int product_count(int i) { return (i & 1) ? 2 : 3; }
+__device__ __forceinline__ int product_lo(int i) { return (i >> 1) - ((i & 1) ? 0 : 1); }
+__device__ __forceinline__ int64_t product_first(int n, const int (&i)[3])
 {
-    __shared__ Real sK[81][82];  // K_e in its own precision: an FP32 Jacobian halves the block's LDS
-    __shared__ double sT[81][25];
-    // W[a][c], the trilinear corner function c at quadratic node a, is nonzero
-    // at exactly the 2 x 2 x 2 nodes a on c's side of the element: both
-    // products below run over those eight (ascending a), which leaves out only
-    // exact zero terms and so gives the same sums as the full 27-term loops
-    __shared__ double sWn[8][8];
-    __shared__ int sA[8][8];
-    __shared__ uint8_t sf[81];
-    const int t = threadIdx.x;
-    if (t < 8) {
-        const int c = t;
-        int q = 0;
-        for (int a = 0; a < 27; ++a) {
-            double w = 1.0;
-            const int ad[3] = {a % 3, (a / 3) % 3, a / 9};
-            for (int d = 0; d < 3; ++d) {
-                const double x = 0.5 * ad[d];
-                w *= ((c >> d) & 1) ? x : 1.0 - x;
-            }
-            if (w != 0.0 && q < 8) {
-                sA[c][q] = a;
-                sWn[c][q] = w;
-                ++q;
+    const auto before = [](int k) { return static_cast<int64_t>((k >> 1) * 5 + (k & 1) * 3); };
+    const int64_t X = 5 * static_cast<int64_t>(n) + 3;
+    const int cy = product_count(i[1]), cz = product_count(i[2]);
+    return cz * cy * before(i[0]) + cz * X * before(i[1]) + X * X * before(i[2]);
+}
+// s / c for c = 2 or 3 and s < 27
+__device__ __forceinline__ int div_count(int s, int c) { return c == 3 ? (s * 43) >> 7 : s >> 1; }
+
+// What the kernels below need of a fine node, in one 16-byte load: with the
+// lattice coordinates found by division in each of them (and the mesh by
+// bisection) the correction kernel issued most of its instructions on those
+// and took 83 us at 32^3.  The MgNode of node q: first block, level-1 node at
+// (lo, lo, lo) (as an index, also where lo is outside), and bits: k the parity
+// of i_k, 3 + 2k lo_k outside, 4 + 2k lo_k + c_k - 1 outside, 16.. N = n + 1.
+__global__ void __launch_bounds__(256)
+mg_nodes_kernel(int M, const int *__restrict__ n_mesh, const int *__restrict__ q_off,
+                const int64_t *__restrict__ ap_off, const int *__restrict__ off1, int nq, MgNode *__restrict__ nodes)
+{
+    const int q = blockIdx.x * blockDim.x + threadIdx.x;
+    if (q >= nq) return;
+    const int m = find_mesh(q_off, M, q);
+    const int n = n_mesh[m], N = n + 1, T = 2 * n + 1, local = q - q_off[m];
+    const int i[3] = {local % T, (local / T) % T, local / (T * T)};
+    MgNode v;
+    v.first = ap_off[m] + product_first(n, i);
+    v.lo = off1[m] + product_lo(i[0]) + N * (product_lo(i[1]) + N * product_lo(i[2]));
+    v.bits = static_cast<uint32_t>(N) << 16;
+    for (int k = 0; k < 3; ++k) {
+        if (i[k] & 1) v.bits |= 1u << k;
+        if (i[k] == 0) v.bits |= 8u << (2 * k);
+        if (i[k] == 2 * n) v.bits |= 16u << (2 * k);
+    }
+    nodes[q] = v;
+}
+
+// ---- setup -----------------------------------------------------------------------------
+// A P0 of the masked displacement block (fixed rows and columns dropped), in
+// FP64, and in FP32 beside it for an FP32 Jacobian's correction kernel.  A
+// group of 32 lanes stages its node's nine runs of values in LDS, read once in
+// whole runs, and lane s adds the up to 27 neighbours that interpolate from
+// its trilinear node, in z, y, x order.  Every later use of the interpolated
+// operator reads this quarter of the matrix (15.6 blocks a node against 64).
+constexpr int kProductNodes = 4;  // per block: 36 KB of FP64 values, four blocks per CU
+
+template <typename VT>
+__global__ void __launch_bounds__(32 * kProductNodes)
+q1_product_kernel(int M, const int *__restrict__ n_mesh, const int *__restrict__ q_off,
+                  const int64_t *__restrict__ ap_off, int nq, const int64_t *__restrict__ row_ptr,
+                  const int *__restrict__ col_idx, const VT *__restrict__ vals, const uint8_t *__restrict__ free_mask,
+                  double *__restrict__ ap, float *__restrict__ ap_sp)
+{
+    __shared__ VT s_run[kProductNodes][9 * 125];
+    const int lane = threadIdx.x & 31, grp = threadIdx.x >> 5;
+    const int q = xcd_block(blockIdx.x, gridDim.x) * kProductNodes + grp;
+    const int64_t nq64 = nq;
+    VT *run = s_run[grp];
+    int m = 0, n = 0, deg = 0, i[3] = {0, 0, 0}, blo[3] = {0, 0, 0}, len[3] = {0, 0, 0};
+    if (q < nq) {
+        m = find_mesh(q_off, M, q);
+        n = n_mesh[m];
+        const int T = 2 * n + 1, local = q - q_off[m];
+        i[0] = local % T;
+        i[1] = (local / T) % T;
+        i[2] = local / (T * T);
+        for (int k = 0; k < 3; ++k) {  // the neighbours are this box of the lattice, x fastest
+            const int reach = (i[k] & 1) ? 1 : 2;
+            blo[k] = max(i[k] - reach, 0);
+            len[k] = min(i[k] + reach, 2 * n) - blo[k] + 1;
+        }
+        deg = len[0] * len[1] * len[2];
+        const int64_t sr[3] = {row_ptr[q], row_ptr[nq64 + q], row_ptr[2 * nq64 + q]};
+        for (int p = lane; p < deg; p += 32) {
+            const int j = col_idx[sr[0] + p];
+#pragma unroll
+            for (int c = 0; c < 3; ++c) {
+                const bool fc = free_mask[c * nq64 + j];
+#pragma unroll
+                for (int r = 0; r < 3; ++r) {
+                    const VT v = vals[sr[r] + c * deg + p];
+                    run[(3 * r + c) * deg + p] = fc && free_mask[r * nq64 + q] ? v : static_cast<VT>(0);
+                }
             }
         }
     }
-    for (int e = blockIdx.x; e < n_elements; e += gridDim.x) {
-        __syncthreads();
-        if (t < 81) sf[t] = free_mask[static_cast<int64_t>(t / 27) * nq + conn_q[static_cast<int64_t>(e) * 27 + t % 27]];
-        __syncthreads();
-        const Real *Ke = kbuf + static_cast<int64_t>(e) * 89 * 89;
-        for (int k = t; k < 81 * 81; k += 256) {
-            const int i = k / 81, j = k % 81;
-            sK[i][j] = (sf[i] && sf[j]) ? Ke[(3 * (i % 27) + i / 27) * 89 + j] : static_cast<Real>(0);  // rows by nodes
-        }
-        __syncthreads();
-        for (int k = t; k < 81 * 24; k += 256) {
-            const int i = k / 24, col = k % 24, cp = col / 8, kk = col % 8;
-            double acc = 0.0;
+    __syncthreads();
+    if (q >= nq) return;
+    const int cx = product_count(i[0]), cy = product_count(i[1]), S = cx * cy * product_count(i[2]);
+    if (lane >= S) return;
+    const int K[3] = {product_lo(i[0]) + lane % cx, product_lo(i[1]) + (lane / cx) % cy,
+                      product_lo(i[2]) + lane / (cx * cy)};
+    int lo[3], hi[3];
+    bool inside = true;
+    for (int k = 0; k < 3; ++k) {
+        lo[k] = max(2 * K[k] - 1, blo[k]);
+        hi[k] = min(2 * K[k] + 1, blo[k] + len[k] - 1);
+        inside = inside && K[k] >= 0 && K[k] <= n;
+    }
+    double acc[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
+    if (inside)
+        for (int z = lo[2]; z <= hi[2]; ++z)
+            for (int y = lo[1]; y <= hi[1]; ++y)
+                for (int x = lo[0]; x <= hi[0]; ++x) {
+                    const double w = lin_weight(x - 2 * K[0]) * lin_weight(y - 2 * K[1]) * lin_weight(z - 2 * K[2]);
+                    const VT *v = run + (x - blo[0]) + len[0] * ((y - blo[1]) + len[1] * (z - blo[2]));
 #pragma unroll
-            for (int q = 0; q < 8; ++q) acc += static_cast<double>(sK[i][cp * 27 + sA[kk][q]]) * sWn[kk][q];
-            sT[i][col] = acc;
-        }
-        __syncthreads();
-        for (int k = t; k < 24 * 24; k += 256) {
-            const int row = k / 24, col = k % 24, c = row / 8, kr = row % 8;
-            double acc = 0.0;
+                    for (int rc = 0; rc < 9; ++rc) acc[rc] += w * static_cast<double>(v[rc * deg]);
+                }
+    const int64_t at = 9 * (ap_off[m] + product_first(n, i)) + lane;
 #pragma unroll
-            for (int q = 0; q < 8; ++q) acc += sWn[kr][q] * sT[c * 27 + sA[kr][q]][col];
-            ke1[static_cast<int64_t>(e) * 576 + k] = acc;
-        }
+    for (int rc = 0; rc < 9; ++rc) {
+        ap[at + rc * S] = acc[rc];
+        if (sizeof(VT) == sizeof(float)) ap_sp[at + rc * S] = static_cast<float>(acc[rc]);
     }
 }
 
-// level-1 stencil: block (I, I+d) = sum over the elements holding both
-// corners (ascending element order) of K1_e[(c, corner I), (c', corner J)]
+// level-1 stencil P0^T (A P0): block (I, I+d) = sum over the fine nodes 2I + s
+// near I that couple to I+d, in z, y, x order; one 32-lane group per node,
+// lane d < 27 its block, so a fine node's blocks are read side by side
 __global__ void __launch_bounds__(256)
-q1_stencil_kernel(int M, const int *__restrict__ n_mesh, const int *__restrict__ e_off, const int *__restrict__ off1,
-                  int nn, const double *__restrict__ ke1, double *__restrict__ A)
+q1_stencil_kernel(int M, const int *__restrict__ n_mesh, const int64_t *__restrict__ ap_off,
+                  const int *__restrict__ off1, int nn, const double *__restrict__ ap, double *__restrict__ A)
 {
-    const int64_t total = static_cast<int64_t>(nn) * 27;
-    for (int64_t t = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x; t < total;
-         t += static_cast<int64_t>(gridDim.x) * blockDim.x) {
-        const int node = static_cast<int>(t / 27), d = static_cast<int>(t % 27);
-        const int m = find_mesh(off1, M, node);
-        const int n = n_mesh[m], N = n + 1, local = node - off1[m];
-        const int I[3] = {local % N, (local / N) % N, local / (N * N)};
-        const int J[3] = {I[0] + d % 3 - 1, I[1] + (d / 3) % 3 - 1, I[2] + d / 9 - 1};
-        double blk[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
-        if (J[0] >= 0 && J[0] < N && J[1] >= 0 && J[1] < N && J[2] >= 0 && J[2] < N) {
-            int lo[3], hi[3];
-            for (int k = 0; k < 3; ++k) {
-                lo[k] = max(max(I[k], J[k]) - 1, 0);
-                hi[k] = min(min(I[k], J[k]), n - 1);
-            }
-            for (int ez = lo[2]; ez <= hi[2]; ++ez)
-                for (int ey = lo[1]; ey <= hi[1]; ++ey)
-                    for (int ex = lo[0]; ex <= hi[0]; ++ex) {
-                        const int64_t e = e_off[m] + ex + static_cast<int64_t>(n) * (ey + static_cast<int64_t>(n) * ez);
-                        const int kI = (I[0] - ex) + 2 * (I[1] - ey) + 4 * (I[2] - ez);
-                        const int kJ = (J[0] - ex) + 2 * (J[1] - ey) + 4 * (J[2] - ez);
-                        const double *k1 = ke1 + e * 576;
-                        for (int c = 0; c < 3; ++c)
-                            for (int cp = 0; cp < 3; ++cp) blk[3 * c + cp] += k1[(c * 8 + kI) * 24 + cp * 8 + kJ];
-                    }
-        }
-        for (int k = 0; k < 9; ++k) A[t * 9 + k] = blk[k];
+    const int node = static_cast<int>((static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x) >> 5);
+    const int d = threadIdx.x & 31;
+    if (node >= nn || d >= 27) return;
+    const int m = find_mesh(off1, M, node);
+    const int n = n_mesh[m], N = n + 1, local = node - off1[m];
+    const int I[3] = {local % N, (local / N) % N, local / (N * N)}, e[3] = {d % 3 - 1, (d / 3) % 3 - 1, d / 9 - 1};
+    double blk[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
+    int lo[3], hi[3];
+    bool inside = true;
+    for (int k = 0; k < 3; ++k) {  // fine nodes of the grid near both I and I + e
+        inside = inside && I[k] + e[k] >= 0 && I[k] + e[k] < N;
+        lo[k] = max(e[k] <= 0 ? -1 : 0, -2 * I[k]);
+        hi[k] = min(e[k] >= 0 ? 1 : 0, 2 * n - 2 * I[k]);
     }
+    if (inside)
+        for (int s2 = lo[2]; s2 <= hi[2]; ++s2)
+            for (int s1 = lo[1]; s1 <= hi[1]; ++s1)
+                for (int s0 = lo[0]; s0 <= hi[0]; ++s0) {
+                    const int i[3] = {2 * I[0] + s0, 2 * I[1] + s1, 2 * I[2] + s2};
+                    const double w = lin_weight(s0) * lin_weight(s1) * lin_weight(s2);
+                    const int cx = product_count(i[0]), cy = product_count(i[1]), S = cx * cy * product_count(i[2]);
+                    const int slot = I[0] + e[0] - product_lo(i[0]) +
+                                     cx * (I[1] + e[1] - product_lo(i[1]) + cy * (I[2] + e[2] - product_lo(i[2])));
+                    const double *a = ap + 9 * (ap_off[m] + product_first(n, i)) + slot;
+#pragma unroll
+                    for (int rc = 0; rc < 9; ++rc) blk[rc] += w * a[rc * S];
+                }
+    double *o = A + (static_cast<int64_t>(node) * 27 + d) * 9;
+#pragma unroll
+    for (int rc = 0; rc < 9; ++rc) o[rc] = blk[rc];
 }
 
 // Galerkin coarsening of a stencil level (masked by the fine level's free
@@ -351,24 +416,6 @@ __global__ void __launch_bounds__(256) coarse_inverse_kernel(int M, const int *_
 }
 
 // ---- V-cycle kernels -------------------------------------------------------------------
-// level 0: r = b - K_uu x on free rows (columns left of the first pressure column)
-template <typename VT, int kLanes>
-__global__ void __launch_bounds__(256)
-uu_residual_kernel(int nu, const int64_t *__restrict__ row_ptr, const int64_t *__restrict__ pstart,
-                   const int *__restrict__ col_idx, const VT *__restrict__ vals, const uint8_t *__restrict__ free_mask,
-                   const double *__restrict__ b, const double *__restrict__ x, double *__restrict__ r)
-{
-    const int lane = threadIdx.x % kLanes;
-    const int row = static_cast<int>((static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x) / kLanes);
-    if (row >= nu) return;
-    const bool f = free_mask[row] != 0;
-    double acc = 0.0;
-    if (f) acc = csr_row_dot<VT, kLanes>(row_ptr[row], pstart[row], lane, col_idx, vals, x);
-#pragma unroll
-    for (int o = kLanes / 2; o > 0; o >>= 1) acc += __shfl_xor(acc, o, kLanes);
-    if (lane == 0) r[row] = f ? b[row] - acc : 0.0;
-}
-
 // bf16 values: the upper 16 bits of an FP32 value, rounded to nearest even
 // (NaN kept quiet)
 __device__ __forceinline__ uint16_t bf16_round(float f)
@@ -573,11 +620,11 @@ uu_node_residual_kernel(int nq, const int64_t *__restrict__ row_ptr, const int64
     }
 }
 
-// level 0: x = (first ? 0 : x) + omega Kblock^-1 r, component-major (and,
-// with x4, the result's FP32 node quadruples for the bf16 passes)
+// level 0: x = omega Kblock^-1 r, component-major (and, with x4, its FP32 node
+// quadruples for the bf16 passes)
 __global__ void __launch_bounds__(256) q2_jacobi_kernel(int nq, const double *__restrict__ inv_u,
                                                        const double *__restrict__ r, double *__restrict__ x,
-                                                       double omega, int first, float *__restrict__ x4)
+                                                       double omega, float *__restrict__ x4)
 {
     for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < nq; i += gridDim.x * blockDim.x) {
         const double *o = inv_u + static_cast<int64_t>(i) * 9;
@@ -585,9 +632,8 @@ __global__ void __launch_bounds__(256) q2_jacobi_kernel(int nq, const double *__
         const double d[3] = {o[0] * r0 + o[1] * r1 + o[2] * r2, o[3] * r0 + o[4] * r1 + o[5] * r2,
                              o[6] * r0 + o[7] * r1 + o[8] * r2};
         for (int c = 0; c < 3; ++c) {
-            const int64_t k = static_cast<int64_t>(c) * nq + i;
-            const double xn = (first ? 0.0 : x[k]) + omega * d[c];
-            x[k] = xn;
+            const double xn = omega * d[c];
+            x[static_cast<int64_t>(c) * nq + i] = xn;
             if (x4) x4[4 * static_cast<int64_t>(i) + c] = static_cast<float>(xn);
         }
     }
@@ -630,42 +676,73 @@ __global__ void __launch_bounds__(256) restrict_q2_kernel(int M, const int *__re
     }
 }
 
-// level 1 -> 0 prolongation x0 += P0 x1 on free DOFs (and, with x4, the
-// result's FP32 node quadruples for the bf16 passes)
-__global__ void __launch_bounds__(256) prolong_q2_kernel(int M, const int *__restrict__ n_mesh,
-                                                        const int *__restrict__ q_off, int nq_total,
-                                                        const int *__restrict__ off1,
-                                                        const uint8_t *__restrict__ free_mask,
-                                                        const double *__restrict__ x1, double *__restrict__ x0,
-                                                        float *__restrict__ x4)
+// Coarse correction of level 0 and the smoothing sweep after it, in place:
+//   x <- x + P0 e + omega Kblock^-1 (r0 - A P0 e),
+// which is the sweep at x + P0 e, as its residual is r0 - A P0 e with r0 the
+// residual that was restricted: the sweep reads A P0, a quarter of the matrix,
+// and the prolongation needs no pass of its own.  One group of 8 lanes per
+// node, lane by trilinear neighbour (8, 12, 18 or 27 of them: 2.5 rounds on
+// average); the loads of a round depend on the node's record alone.  At 32^3
+// with FP32 values 63 us (205 MB) where the sweep over the bf16 matrix and the
+// prolongation took 124 + 14; at 16^3 in FP64 17 us where they took 38 + 7.
+template <typename VT>
+__global__ void __launch_bounds__(256)
+q1_correct_kernel(int nq, const MgNode *__restrict__ nodes, const VT *__restrict__ ap, const double *__restrict__ e,
+                  const uint8_t *__restrict__ free_mask, const double *__restrict__ r0,
+                  const double *__restrict__ inv_u, double omega, double *__restrict__ x, float *__restrict__ x4)
 {
-    for (int q = blockIdx.x * blockDim.x + threadIdx.x; q < nq_total; q += gridDim.x * blockDim.x) {
-        const int m = find_mesh(q_off, M, q);
-        const int n = n_mesh[m], N = n + 1, T = 2 * n + 1, local = q - q_off[m];
-        const int i[3] = {local % T, (local / T) % T, local / (T * T)};
-        int p0[3], p1[3];
-        double w0[3], w1[3];
-        for (int k = 0; k < 3; ++k) {
-            p0[k] = i[k] >> 1;
-            p1[k] = (i[k] + 1) >> 1;
-            w0[k] = (i[k] & 1) ? 0.5 : 1.0;
-            w1[k] = (i[k] & 1) ? 0.5 : 0.0;
+    constexpr int kLanes = 8, kRounds = 4;  // 27 slots at most
+    const int lane = threadIdx.x % kLanes;
+    const int64_t xb = xcd_block(blockIdx.x, gridDim.x);
+    const int q = static_cast<int>((xb * blockDim.x + threadIdx.x) / kLanes);
+    if (q >= nq) return;  // whole groups
+    const int64_t nq64 = nq;
+    const MgNode nd = nodes[q];
+    const int N = static_cast<int>(nd.bits >> 16);
+    const bool odd[3] = {(nd.bits & 1) != 0, (nd.bits & 2) != 0, (nd.bits & 4) != 0};
+    const int cx = odd[0] ? 2 : 3, cy = odd[1] ? 2 : 3, cz = odd[2] ? 2 : 3, S = cx * cy * cz;
+    const VT *a = ap + 9 * nd.first;
+    double v[8] = {0, 0, 0, 0, 0, 0, 0, 0};  // A P0 e and P0 e
+#pragma unroll
+    for (int u = 0; u < kRounds; ++u) {
+        const int s = lane + u * kLanes;
+        if (s >= S) break;
+        const int yz = div_count(s, cx), sz = div_count(yz, cy), k[3] = {s - cx * yz, yz - cy * sz, sz};
+        double w = 1.0;
+        bool inside = true;
+#pragma unroll
+        for (int d = 0; d < 3; ++d) {
+            w *= odd[d] ? 0.5 : (k[d] == 1 ? 1.0 : 0.0);
+            inside = inside && !(k[d] == 0 && (nd.bits >> (3 + 2 * d) & 1)) && !(k[d] == 2 && (nd.bits >> (4 + 2 * d) & 1));
         }
-        double v[3] = {0.0, 0.0, 0.0};
-        for (int s = 0; s < 8; ++s) {
-            const int b0 = s & 1, b1 = (s >> 1) & 1, b2 = s >> 2;
-            const double w = (b0 ? w1[0] : w0[0]) * (b1 ? w1[1] : w0[1]) * (b2 ? w1[2] : w0[2]);
-            if (w == 0.0) continue;
-            const int64_t P = off1[m] + (b0 ? p1[0] : p0[0]) +
-                              static_cast<int64_t>(N) * ((b1 ? p1[1] : p0[1]) + static_cast<int64_t>(N) * (b2 ? p1[2] : p0[2]));
-            for (int c = 0; c < 3; ++c) v[c] += w * x1[P * 3 + c];
-        }
-        for (int c = 0; c < 3; ++c) {
-            const int64_t k = static_cast<int64_t>(c) * nq_total + q;
-            if (free_mask[k]) x0[k] += v[c];
-            if (x4) x4[4 * static_cast<int64_t>(q) + c] = static_cast<float>(x0[k]);
+        const double *ek = e + 3 * static_cast<int64_t>(inside ? nd.lo + k[0] + N * (k[1] + N * k[2]) : 0);
+        double b[9];
+#pragma unroll
+        for (int rc = 0; rc < 9; ++rc) b[rc] = static_cast<double>(a[rc * S + s]);  // zeros where outside
+        const double ev[3] = {inside ? ek[0] : 0.0, inside ? ek[1] : 0.0, inside ? ek[2] : 0.0};
+#pragma unroll
+        for (int r = 0; r < 3; ++r) {
+            v[r] += b[3 * r] * ev[0] + b[3 * r + 1] * ev[1] + b[3 * r + 2] * ev[2];
+            v[4 + r] += w * ev[r];
         }
     }
+    // lane l of the group is left with the total of v[l]
+    const bool h4 = lane & 4, h2 = lane & 2, h1 = lane & 1;
+    double f[4], t[2];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) f[k] = (h4 ? v[k + 4] : v[k]) + __shfl_xor(h4 ? v[k] : v[k + 4], 4, kLanes);
+#pragma unroll
+    for (int k = 0; k < 2; ++k) t[k] = (h2 ? f[k + 2] : f[k]) + __shfl_xor(h2 ? f[k] : f[k + 2], 2, kLanes);
+    const double sum = (h1 ? t[1] : t[0]) + __shfl_xor(h1 ? t[0] : t[1], 1, kLanes);
+    const int64_t row = (lane & 3) * nq64 + q;
+    const double d = lane < 3 ? r0[row] - sum : 0.0;
+    const double d0 = __shfl(d, 0, kLanes), d1 = __shfl(d, 1, kLanes), d2 = __shfl(d, 2, kLanes);
+    const double pe = __shfl(sum, 4 | lane, kLanes);
+    if (lane >= 3) return;
+    const double *o = inv_u + static_cast<int64_t>(q) * 9 + 3 * lane;
+    const double xn = x[row] + (free_mask[row] ? pe : 0.0) + omega * (o[0] * d0 + o[1] * d1 + o[2] * d2);
+    x[row] = xn;
+    if (x4) x4[4 * static_cast<int64_t>(q) + lane] = static_cast<float>(xn);
 }
 
 // As(node, d) = A(node, d) Dinv(neighbour d): the first Jacobi step from
@@ -901,27 +978,46 @@ __global__ void __launch_bounds__(256) coarse_apply_kernel(int M, const int *__r
     if (lane == 0) x[k] = acc;
 }
 
+unsigned group_grid(int nn) { return static_cast<unsigned>((static_cast<int64_t>(nn) * 32 + 255) / 256); }
 unsigned grid1(int64_t n) { return static_cast<unsigned>(std::max<int64_t>(1, std::min<int64_t>((n + 255) / 256, 16384))); }
 
 }  // namespace
+
+// What the V-cycle of a precision needs, made before its setup is recorded;
+// *made tells whether something was missing (a recorded setup then lacks it)
+int mg_prepare(EquationsSet &s, int precision, bool *made)
+{
+    *made = false;
+    if (s.node_rows != 1) return set_error(OC_ERR_UNSUPPORTED, "the multigrid preconditioner needs node rows");
+    if (precision != OC_FP32) return OC_NO_ERROR;
+    Multigrid &g = *s.mg;
+    *made = !s.uu_bf.ptr || !g.ap_sp.ptr;
+    if (!s.values_sp.ptr) OC_CHECK(s.values_sp.alloc(s.nnz));
+    OC_CHECK(prepare_uu_bf16(s));
+    if (!g.ap_sp.ptr) OC_CHECK(g.ap_sp.alloc(g.ap.n));
+    return OC_NO_ERROR;
+}
 
 int mg_setup(EquationsSet &s, int precision)
 {
     Multigrid &g = *s.mg;
     Runtime &rt = runtime();
     const int M = s.n_meshes;
-    const unsigned eb = static_cast<unsigned>(std::min(s.n_elements, rt.num_cus * (precision == OC_FP32 ? 3 : 2)));
-    if (precision == OC_FP64)
-        q1_galerkin_element_kernel<double><<<eb, 256, 0, rt.stream>>>(s.n_elements, s.kbuf64.ptr, s.conn.ptr,
-                                                                     s.n_nodes, s.free_mask.ptr, g.ke1.ptr);
-    else
-        q1_galerkin_element_kernel<float><<<eb, 256, 0, rt.stream>>>(s.n_elements, s.kbuf32.ptr, s.conn.ptr,
-                                                                    s.n_nodes, s.free_mask.ptr, g.ke1.ptr);
-    OC_HIP_CHECK(hipGetLastError());
-    if (precision == OC_FP32 && s.uu_bf.ptr) OC_CHECK(launch_uu_pack(s));
+    const int nq = s.n_nodes;
+    const unsigned gp = static_cast<unsigned>((nq + kProductNodes - 1) / kProductNodes);
     MgLevel &L1 = g.levels[1];
-    q1_stencil_kernel<<<grid1(static_cast<int64_t>(L1.nn) * 27), 256, 0, rt.stream>>>(
-        M, g.n.ptr, g.e_off.ptr, L1.off.ptr, L1.nn, g.ke1.ptr, L1.A.ptr);
+    if (precision == OC_FP64)
+        q1_product_kernel<double><<<gp, 32 * kProductNodes, 0, rt.stream>>>(
+            M, g.n.ptr, s.q_off.ptr, g.ap_off.ptr, nq, s.row_ptr.ptr, s.col_idx.ptr, s.values.ptr, s.free_mask.ptr,
+            g.ap.ptr, nullptr);
+    else
+        q1_product_kernel<float><<<gp, 32 * kProductNodes, 0, rt.stream>>>(
+            M, g.n.ptr, s.q_off.ptr, g.ap_off.ptr, nq, s.row_ptr.ptr, s.col_idx.ptr, s.values_sp.ptr, s.free_mask.ptr,
+            g.ap.ptr, g.ap_sp.ptr);
+    OC_HIP_CHECK(hipGetLastError());
+    if (precision == OC_FP32) OC_CHECK(launch_uu_pack(s));
+    q1_stencil_kernel<<<group_grid(L1.nn), 256, 0, rt.stream>>>(M, g.n.ptr, g.ap_off.ptr, L1.off.ptr, L1.nn, g.ap.ptr,
+                                                               L1.A.ptr);
     coincident_q2_kernel<<<grid1(L1.nn), 256, 0, rt.stream>>>(M, g.n.ptr, s.q_off.ptr, s.n_nodes, L1.off.ptr, L1.nn,
                                                               s.free_mask.ptr, L1.freed.ptr);
     level_freed_kernel<<<grid1(L1.nn), 256, 0, rt.stream>>>(L1.nn, L1.A.ptr, L1.freed.ptr);
@@ -954,8 +1050,6 @@ int mg_setup(EquationsSet &s, int precision)
     return OC_NO_ERROR;
 }
 
-
-static unsigned group_grid(int nn) { return static_cast<unsigned>((static_cast<int64_t>(nn) * 32 + 255) / 256); }
 
 // one Jacobi sweep of a stencil level: x <- x + omega Dinv (b - A x), through
 // the level's r buffer (the two buffers trade places)
@@ -1095,61 +1189,38 @@ int mg_apply(EquationsSet &s, int precision, const double *t, double *z)
 {
     Multigrid &g = *s.mg;
     Runtime &rt = runtime();
-    const int M = s.n_meshes, nq = s.n_nodes, nu = 3 * nq, nl = static_cast<int>(g.levels.size());
+    const int M = s.n_meshes, nq = s.n_nodes, nl = static_cast<int>(g.levels.size());
     const double *inv_u = s.precond.ptr;  // nodal block inverses of the set's block preconditioner
-    const unsigned gu = static_cast<unsigned>((static_cast<int64_t>(nu) * 32 + 255) / 256);
-    const bool bf = precision == OC_FP32 && s.node_rows == 1 && s.uu_bf.ptr;
+    const bool bf = precision == OC_FP32;  // an FP32 Jacobian's packed bf16 values (mg_prepare)
     // default shape: 16 lanes x 2 neighbours in flight for FP64 values (6%
-    // faster than 32 x 1 at 32^3), 32 x 1 for bf16 and FP32
+    // faster than 32 x 1 at 32^3), 16 lanes x one quad for bf16
     const int variant = s.tuned_smoother >= 0 ? s.tuned_smoother : (precision == OC_FP64 ? 2 : 0);
     // with the packed bf16 values the kernels that produce the iterate also
     // write its FP32 node quadruples, into the two halves of uu_x4 in turn
     // (a sweep gathers one half and writes the other); q4 is the current one
     float *q4 = bf ? s.uu_x4.ptr : nullptr, *q4_other = bf ? s.uu_x4.ptr + 4 * static_cast<int64_t>(nq) : nullptr;
-    auto residual0 = [&](const double *b, const double *x, double *r) -> int {
-        if (bf)
-            OC_CHECK(launch_uu_bf16<0>(variant, s, b, x, nullptr, 0.0, r, q4));
-        else if (s.node_rows == 1 && precision == OC_FP32)
-            OC_CHECK((launch_uu_node<float, 0>(variant, nq, s, s.values_sp.ptr, b, x, nullptr, 0.0, r)));
-        else if (s.node_rows == 1)
-            OC_CHECK((launch_uu_node<double, 0>(variant, nq, s, s.values.ptr, b, x, nullptr, 0.0, r)));
-        else if (precision == OC_FP32)
-            uu_residual_kernel<float, 32><<<gu, 256, 0, rt.stream>>>(nu, s.row_ptr.ptr, s.pstart.ptr, s.col_idx.ptr,
-                                                                    s.values_sp.ptr, s.free_mask.ptr, b, x, r);
-        else
-            uu_residual_kernel<double, 32><<<gu, 256, 0, rt.stream>>>(nu, s.row_ptr.ptr, s.pstart.ptr, s.col_idx.ptr,
-                                                                      s.values.ptr, s.free_mask.ptr, b, x, r);
-        OC_HIP_CHECK(hipGetLastError());
-        return OC_NO_ERROR;
-    };
-    // level 0 pre-smoothing from x = 0.  With node rows a sweep is one fused
-    // kernel writing the other of z and x0; the first Jacobi step picks the
-    // buffer that leaves the last post-smoothing sweep in z.
-    const bool fused = s.node_rows == 1;
+    // level 0 pre-smoothing from x = 0.  A sweep is one kernel writing the
+    // other of z and x0; the first Jacobi step picks the buffer that leaves
+    // the last post-smoothing sweep in z.  The first post-smoothing sweep
+    // comes with the coarse correction, in place.
     const int post = g.post;
     double *cur = z, *other = g.x0.ptr;
-    if (fused && ((std::max(g.pre - 1, 0) + post) & 1)) std::swap(cur, other);
+    if ((std::max(g.pre - 1, 0) + std::max(post - 1, 0)) & 1) std::swap(cur, other);
     auto sweep0 = [&]() -> int {
         if (bf)
             OC_CHECK(launch_uu_bf16<1>(variant, s, t, cur, inv_u, g.omega, other, q4, q4_other));
-        else if (precision == OC_FP32)
-            OC_CHECK((launch_uu_node<float, 1>(variant, nq, s, s.values_sp.ptr, t, cur, inv_u, g.omega, other)));
         else
             OC_CHECK((launch_uu_node<double, 1>(variant, nq, s, s.values.ptr, t, cur, inv_u, g.omega, other)));
         std::swap(cur, other);
         std::swap(q4, q4_other);
         return OC_NO_ERROR;
     };
-    q2_jacobi_kernel<<<grid1(nq), 256, 0, rt.stream>>>(nq, inv_u, t, cur, g.omega, 1, q4);
-    for (int k = 1; k < g.pre; ++k) {
-        if (fused) {
-            OC_CHECK(sweep0());
-            continue;
-        }
-        OC_CHECK(residual0(t, cur, g.r0.ptr));
-        q2_jacobi_kernel<<<grid1(nq), 256, 0, rt.stream>>>(nq, inv_u, g.r0.ptr, cur, g.omega, 0, q4);
-    }
-    OC_CHECK(residual0(t, cur, g.r0.ptr));
+    q2_jacobi_kernel<<<grid1(nq), 256, 0, rt.stream>>>(nq, inv_u, t, cur, g.omega, q4);
+    for (int k = 1; k < g.pre; ++k) OC_CHECK(sweep0());
+    if (bf)
+        OC_CHECK(launch_uu_bf16<0>(variant, s, t, cur, nullptr, 0.0, g.r0.ptr, q4));
+    else
+        OC_CHECK((launch_uu_node<double, 0>(variant, nq, s, s.values.ptr, t, cur, nullptr, 0.0, g.r0.ptr)));
     MgLevel &L1 = g.levels[1];
     restrict_q2_kernel<<<group_grid(L1.nn), 256, 0, rt.stream>>>(M, g.n.ptr, s.q_off.ptr, nq, L1.off.ptr, L1.nn,
                                                             L1.freed.ptr, g.r0.ptr, L1.b.ptr);
@@ -1183,18 +1254,16 @@ int mg_apply(EquationsSet &s, int precision, const double *t, double *z)
         for (int k = 0; k < g.stencil_post; ++k) OC_CHECK(stencil_sweep(M, F, g.omega));
         OC_HIP_CHECK(hipGetLastError());
     }
-    prolong_q2_kernel<<<grid1(nq), 256, 0, rt.stream>>>(M, g.n.ptr, s.q_off.ptr, nq, L1.off.ptr, s.free_mask.ptr,
-                                                        L1.x.ptr, cur, q4);
+    const unsigned gc = static_cast<unsigned>((static_cast<int64_t>(nq) * 8 + 255) / 256);
+    const double omega1 = post > 0 ? g.omega : 0.0;  // without post-smoothing only x + P0 e
+    if (bf)
+        q1_correct_kernel<float><<<gc, 256, 0, rt.stream>>>(nq, g.nodes.ptr, g.ap_sp.ptr, L1.x.ptr, s.free_mask.ptr,
+                                                            g.r0.ptr, inv_u, omega1, cur, q4);
+    else
+        q1_correct_kernel<double><<<gc, 256, 0, rt.stream>>>(nq, g.nodes.ptr, g.ap.ptr, L1.x.ptr, s.free_mask.ptr,
+                                                             g.r0.ptr, inv_u, omega1, cur, nullptr);
     OC_HIP_CHECK(hipGetLastError());
-    for (int k = 0; k < post; ++k) {
-        if (fused) {
-            OC_CHECK(sweep0());
-            continue;
-        }
-        OC_CHECK(residual0(t, cur, g.r0.ptr));
-        q2_jacobi_kernel<<<grid1(nq), 256, 0, rt.stream>>>(nq, inv_u, g.r0.ptr, cur, g.omega, 0, q4);
-    }
-    OC_HIP_CHECK(hipGetLastError());
+    for (int k = 1; k < post; ++k) OC_CHECK(sweep0());
     return OC_NO_ERROR;
 }
 
@@ -1243,7 +1312,6 @@ extern "C" int oc_multigrid_structure_set(oc_equations_set h, const int *n_per_m
     std::unique_ptr<Multigrid> guard(g);
     g->h_n.assign(n_per_mesh, n_per_mesh + M);
     OC_CHECK(g->n.upload(g->h_n.data(), M));
-    OC_CHECK(g->e_off.upload(s.h_e_off.data(), s.h_e_off.size()));
     // levels: [0] placeholder, [1] trilinear (n+1)^3, then coarsening until every dim <= 3
     g->levels.resize(2);
     std::vector<int32_t> dims(M);
@@ -1272,7 +1340,17 @@ extern "C" int oc_multigrid_structure_set(oc_equations_set h, const int *n_per_m
     if (maxnd > 81) return set_error(OC_ERR_UNSUPPORTED, "coarsest multigrid level too large");
     g->coarse_stride = maxnd * maxnd;
     OC_CHECK(g->coarse_inv.alloc(static_cast<size_t>(M) * g->coarse_stride));
-    OC_CHECK(g->ke1.alloc(static_cast<size_t>(s.n_elements) * 576));
+    std::vector<int64_t> ap_off(static_cast<size_t>(M) + 1, 0);
+    for (int m = 0; m < M; ++m) {
+        const int64_t X = 5 * static_cast<int64_t>(g->h_n[m]) + 3;
+        ap_off[m + 1] = ap_off[m] + X * X * X;
+    }
+    OC_CHECK(g->ap_off.upload(ap_off.data(), ap_off.size()));
+    OC_CHECK(g->ap.alloc(static_cast<size_t>(ap_off[M]) * 9));
+    OC_CHECK(g->nodes.alloc(s.n_nodes));
+    mg_nodes_kernel<<<static_cast<unsigned>((s.n_nodes + 255) / 256), 256, 0, runtime().stream>>>(
+        M, g->n.ptr, s.q_off.ptr, g->ap_off.ptr, g->levels[1].off.ptr, s.n_nodes, g->nodes.ptr);
+    OC_HIP_CHECK(hipGetLastError());
     OC_CHECK(g->r0.alloc(static_cast<size_t>(3) * s.n_nodes));
     OC_CHECK(g->t0.alloc(static_cast<size_t>(3) * s.n_nodes));
     OC_CHECK(g->x0.alloc(static_cast<size_t>(3) * s.n_nodes));

@@ -1416,14 +1416,14 @@ static int newton_core(EquationsSet &s, const oc_newton_options *opt, const doub
     K.precond = opt->preconditioner;
     K.fp32 = opt->jacobian_precision == OC_FP32;
     OC_CHECK(solver_prepare(s, opt->krylov_restart, K));
-    // an FP32 Jacobian's multigrid smoother reads a packed bf16 copy of K_uu
-    // (filled in the preconditioner setup) and gathers the iterate as FP32
-    // node quadruples: allocated here, outside the step graph, and a graph
-    // recorded before the copy existed is recorded again
-    if (K.fp32 && K.precond == OC_PRECONDITIONER_MULTIGRID && s.node_rows == 1 && !s.uu_bf.ptr) {
-        if (!s.values_sp.ptr) OC_CHECK(s.values_sp.alloc(s.nnz));
-        OC_CHECK(prepare_uu_bf16(s));
-        if (s.step_graph) {
+    // an FP32 Jacobian's V-cycle reads a packed bf16 copy of K_uu and an FP32
+    // copy of A P0 (filled in the preconditioner setup): allocated here,
+    // outside the step graph, and a graph recorded before they existed is
+    // recorded again
+    if (K.precond == OC_PRECONDITIONER_MULTIGRID) {
+        bool made = false;
+        OC_CHECK(mg_prepare(s, opt->jacobian_precision, &made));
+        if (made && s.step_graph) {
             (void)hipGraphExecDestroy(s.step_graph);
             s.step_graph = nullptr;
         }
