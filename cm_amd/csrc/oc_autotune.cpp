@@ -107,15 +107,15 @@ extern "C" int oc_autotune(oc_equations_set h, int precision, char *report, int 
                   [&](int i) { return num(chunks[i]); }, &c_gather));
 
     // SpMV: lanes per row (per node for node rows) x neighbours in flight per
-    // lane; default 32 x 1 (FP32 values) or 16 x 2 (FP64) on node rows
+    // lane; default 32 x 1 (FP32 values) or a wavefront per node (FP64, 64 x 1)
     OC_CHECK(prepare_node_rows(s));
     DevBuf<double> y;
     OC_CHECK(y.alloc(s.n_rows));
     std::vector<std::pair<int, int>> spmv;
     for (int l : {8, 16, 32, 64})
         for (int u = 1; u <= 2; ++u)
-            if (u == 1 || (s.node_rows == 1 && l >= 16)) spmv.push_back({l, u});  // unrolled form: node rows only
-    const std::pair<int, int> spmv_def = s.node_rows == 1 && !fp32 ? std::make_pair(16, 2) : std::make_pair(32, 1);
+            if (u == 1 || (s.node_rows == 1 && (l == 16 || l == 32))) spmv.push_back({l, u});  // unrolled: node rows only
+    const std::pair<int, int> spmv_def = s.flat_rows() && !fp32 ? std::make_pair(64, 1) : std::make_pair(32, 1);
     int spmv_def_i = 0;
     for (size_t i = 0; i < spmv.size(); ++i)
         if (spmv[i] == spmv_def) spmv_def_i = static_cast<int>(i);
@@ -131,7 +131,7 @@ extern "C" int oc_autotune(oc_equations_set h, int precision, char *report, int 
                   &c_spmv));
 
     // level-0 multigrid node kernel (residual form), when the rows have the
-    // node layout: FP64 values (default 16 x 2), or for an FP32 Jacobian the
+    // node layout: FP64 values (default a wavefront per node), or for an FP32 Jacobian the
     // packed bf16 copy its smoother reads (default 16 lanes x 1 quad)
     int best_smoother = -1;
     if (s.node_rows == 1 && !s.free_mask.ptr) {  // no boundary conditions yet: every DOF free
@@ -149,7 +149,7 @@ extern "C" int oc_autotune(oc_equations_set h, int precision, char *report, int 
             OC_CHECK(launch_uu_pack(s));
         }
         Choice c_sm{};
-        OC_CHECK(tune(js, "smoother_residual_ms", 5, fp32 ? 0 : 2, reps,
+        OC_CHECK(tune(js, "smoother_residual_ms", 5, fp32 || !s.flat_rows() ? 0 : 4, reps,
                       [&](int v) { return launch_smoother_residual(s, precision, v, s.dofs.ptr, s.dofs.ptr, r.ptr); },
                       [&](int v) { return std::string(names[v]); }, &c_sm));
         best_smoother = c_sm.index;

@@ -5,6 +5,7 @@
 // A[i + 3*j] == A(i+1, j+1) of the Fortran source.
 #pragma once
 
+#include "oc_internal.h"
 #include <hip/hip_runtime.h>
 
 namespace oc {
@@ -407,6 +408,136 @@ __device__ __forceinline__ void node_rows_uu(const int64_t (&s)[3], int deg, int
 #pragma unroll
             for (int r = 0; r < 3; ++r)
                 a[r] += v[u][3 * r] * xv[u][0] + v[u][3 * r + 1] * xv[u][1] + v[u][3 * r + 2] * xv[u][2];
+    }
+}
+
+// A double moved between the lanes of a row of 16 by a DPP control
+template <int kCtrl>
+__device__ __forceinline__ double dpp_move(double v)
+{
+    const uint64_t b = __double_as_longlong(v);
+    const int lo = __builtin_amdgcn_update_dpp(0, static_cast<int>(b), kCtrl, 0xf, 0xf, true);
+    const int hi = __builtin_amdgcn_update_dpp(0, static_cast<int>(b >> 32), kCtrl, 0xf, 0xf, true);
+    return __longlong_as_double(static_cast<long long>((static_cast<uint64_t>(static_cast<uint32_t>(hi)) << 32) |
+                                                       static_cast<uint32_t>(lo)));
+}
+
+// The wavefront's sums of a[0], a[1], a[2]: lane 16 c is left with the total
+// of a[c] (c < 3).  Halving the sums kept per lane twice, then rotations
+// within the rows of 16 lanes: 3 shuffles instead of 18.
+__device__ __forceinline__ double wave_total3(const double (&a)[3], int lane)
+{
+    const bool up = lane & 32, odd = lane & 16;
+    const double k0 = (up ? a[2] : a[0]) + __shfl_xor(up ? a[0] : a[2], 32);
+    const double k1 = (up ? 0.0 : a[1]) + __shfl_xor(up ? a[1] : 0.0, 32);
+    double t = (odd ? k1 : k0) + __shfl_xor(odd ? k0 : k1, 16);
+    t += dpp_move<0x128>(t);  // row_ror:8, 4, 2, 1
+    t += dpp_move<0x124>(t);
+    t += dpp_move<0x122>(t);
+    t += dpp_move<0x121>(t);
+    return t;
+}
+
+// A Mooney-Rivlin node's three displacement rows times x, one wavefront per
+// node: a[c] += this lane's part of row c's sum over all its columns or, without
+// kPressure, the displacement ones.
+//
+// A row is taken flat: entry k = c deg + p for component c of neighbour p, then
+// the pressure columns, the same in all three rows.  The columns are read once
+// and the iterate's entries gathered once (a lane a neighbour) into LDS; the
+// values come in 16-byte loads from the 16-byte boundary below the row's start,
+// each row at its own shift against the entries, and meet the iterate there:
+// entry k is in plane k % kE at k / kE + 1, so entry kE q + c is lane q's in a
+// plane and at a slot that only c decides.  Lanes past the end repeat the last
+// load, so that no branch holds a load back.  What bounds it is requests
+// waiting for lines that others of the wavefront have on their way
+// (TCP_PENDING_STALL): each line of a row and of the columns is asked for once.
+constexpr int kFlatEntries = kFlatRowLength;       // entries of a row at most
+constexpr int kFlatLds = kFlatEntries + 24;         // doubles of LDS per wavefront
+template <int kE>
+constexpr int kFlatPlane = kFlatEntries / kE + 4;
+
+template <typename VT, bool kPressure>
+__device__ __forceinline__ void node_rows_flat(int i, int nq, int lane, const int64_t *__restrict__ row_ptr,
+                                               const int64_t *__restrict__ pstart, const int *__restrict__ col_idx,
+                                               const VT *__restrict__ vals, const double *__restrict__ x,
+                                               double *s_x, double (&a)[3])
+{
+    constexpr int kE = 16 / sizeof(VT), kSteps = 4 / kE;  // 256 entries
+    struct alignas(16) Vec {
+        VT e[kE];
+    };
+    // equal rows: component c's starts c row_ptr[nq] after component 0's
+    const int64_t s0 = row_ptr[i], per = row_ptr[nq];
+    const int uu = static_cast<int>(pstart[i] - s0), deg = uu / 3;
+    const int n = kPressure ? static_cast<int>(row_ptr[i + 1] - s0) : uu;
+    const int *col = col_idx + s0;
+    // (a node is its own neighbour, so deg >= 1)
+    const uint32_t j0 = col[min(lane, deg - 1)], j1 = col[min(64 + lane, deg - 1)];
+    const uint32_t jp = kPressure ? col[min(uu + lane, n - 1)] : 0;
+    Vec v[3][kSteps];
+    int shift[3];
+#pragma unroll
+    for (int r = 0; r < 3; ++r) {
+        const int64_t first = s0 + r * per;
+        shift[r] = static_cast<int>(first & (kE - 1));
+        const Vec *row = reinterpret_cast<const Vec *>(vals + (first - shift[r]));
+        const int last = (shift[r] + n - 1) / kE;
+#pragma unroll
+        for (int u = 0; u < kSteps; ++u) v[r][u] = row[min(64 * u + lane, last)];
+    }
+    const auto at = [&](int k) -> double & { return s_x[(k % kE) * kFlatPlane<kE> + k / kE + 1]; };
+    const auto entry = [&](int c, uint32_t j) {  // a scalar base and a 32-bit offset
+        return *reinterpret_cast<const double *>(reinterpret_cast<const char *>(x + static_cast<int64_t>(c) * nq) + 8u * j);
+    };
+    double g[3], gp = 0.0;
+#pragma unroll
+    for (int c = 0; c < 3; ++c) g[c] = entry(c, j0);
+    if (kPressure) gp = entry(0, jp);
+    for (int p = 128 + lane; p < deg; p += 64)
+        for (int c = 0; c < 3; ++c) at(c * deg + p) = entry(c, col[p]);
+    if (deg > 64) {
+        double h[3];
+#pragma unroll
+        for (int c = 0; c < 3; ++c) h[c] = entry(c, j1);
+        if (64 + lane < deg)
+#pragma unroll
+            for (int c = 0; c < 3; ++c) at(c * deg + 64 + lane) = h[c];
+    }
+    if (lane < deg)
+#pragma unroll
+        for (int c = 0; c < 3; ++c) at(c * deg + lane) = g[c];
+    if (kPressure)
+        for (int k = uu + lane; k < n; k += 64) at(k) = k < uu + 64 ? gp : x[col[k]];
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    for (int base = 0;;) {
+#pragma unroll
+        for (int r = 0; r < 3; ++r)
+#pragma unroll
+            for (int e = 0; e < kE; ++e) {
+                const int c = e - shift[r];
+                const double *plane = s_x + (c & (kE - 1)) * kFlatPlane<kE> + (c < 0 ? 0 : 1) + base / kE;
+#pragma unroll
+                for (int u = 0; u < kSteps; ++u) {
+                    // lanes whose entry kE q + c is one of the row's
+                    const int lanes = (n - c + kE - 1) / kE - base / kE - 64 * u;
+                    uint64_t own = lanes >= 64 ? ~0ull : (lanes <= 0 ? 0ull : (1ull << lanes) - 1);
+                    if (base == 0 && u == 0 && c < 0) own &= ~1ull;
+                    const bool mine = __builtin_amdgcn_inverse_ballot_w64(own);
+                    const VT t = mine ? v[r][u].e[e] : static_cast<VT>(0);
+                    a[r] += static_cast<double>(t) * (mine ? plane[64 * u + lane] : 0.0);
+                }
+            }
+        base += 256;
+        if (base >= n + kE - 1) break;
+#pragma unroll
+        for (int r = 0; r < 3; ++r) {
+            const Vec *row = reinterpret_cast<const Vec *>(vals + (s0 + r * per - shift[r]));
+            const int last = (shift[r] + n - 1) / kE;
+#pragma unroll
+            for (int u = 0; u < kSteps; ++u) v[r][u] = row[min(base / kE + 64 * u + lane, last)];
+        }
     }
 }
 

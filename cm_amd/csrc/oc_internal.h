@@ -161,6 +161,8 @@ struct SolverSystem {
     DevBuf<double> vector;          // RHS with the fixed columns moved over (linear) or residual
 };
 
+constexpr int kFlatRowLength = 504;  // the longest CSR row of node_rows_flat (oc_fe_device.h); a regular mesh has 402
+
 // Per-equations-set state.  Element arrays are element-major; node and DOF
 // indices are 0-based; CSR col_idx 0-based int32, row offsets int64 on the
 // device (a batch of meshes can exceed 2^31 nonzeros).
@@ -221,6 +223,7 @@ struct EquationsSet {
     DevBuf<double> kbuf64;      // element matrices, E*89*89, rows by nodes (kbuf_row, oc_elasticity.hip)
     DevBuf<float> kbuf32;
     int max_row_len = 0;
+    bool flat_rows() const { return node_rows == 1 && max_row_len <= kFlatRowLength; }  // node_rows_flat's rows
     // element residuals (E*89) and the DOF -> element-entry gather lists
     DevBuf<double> relem;
     DevBuf<int32_t> gather_ptr, gather_idx;

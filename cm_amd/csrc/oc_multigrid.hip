@@ -620,6 +620,37 @@ uu_node_residual_kernel(int nq, const int64_t *__restrict__ row_ptr, const int64
     }
 }
 
+// the same by one wavefront per node (node_rows_flat): FP64 values' default
+// where the rows fit its LDS.  At 32^3 276 us against 332 with 16 lanes x 2
+// neighbours, at 16^3 30.8 against 38.6.
+template <typename VT, int kSweep>
+__global__ void __launch_bounds__(256)
+uu_flat_kernel(int nq, const int64_t *__restrict__ row_ptr, const int64_t *__restrict__ pstart,
+               const int *__restrict__ col_idx, const VT *__restrict__ vals, const uint8_t *__restrict__ free_mask,
+               const double *__restrict__ b, const double *__restrict__ x, const double *__restrict__ inv_u,
+               double omega, double *__restrict__ out)
+{
+    __shared__ double s_x[4][kFlatLds];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int i = xcd_block(blockIdx.x, gridDim.x) * 4 + wave;
+    if (i >= nq) return;  // whole wavefronts
+    double a[3] = {0.0, 0.0, 0.0};
+    node_rows_flat<VT, false>(i, nq, lane, row_ptr, pstart, col_idx, vals, x, s_x[wave], a);
+    const double t = wave_total3(a, lane);
+    const int c = lane >> 4;
+    const int64_t row = c * static_cast<int64_t>(nq) + i;
+    const bool mine = (lane & 15) == 0 && c < 3;
+    const double r = mine && free_mask[row] ? b[row] - t : 0.0;
+    if (kSweep == 0) {
+        if (mine) out[row] = r;
+        return;
+    }
+    const double r0 = __shfl(r, 0), r1 = __shfl(r, 16), r2 = __shfl(r, 32);
+    if (!mine) return;
+    const double *o = inv_u + static_cast<int64_t>(i) * 9 + 3 * c;
+    out[row] = x[row] + omega * (o[0] * r0 + o[1] * r1 + o[2] * r2);
+}
+
 // level 0: x = omega Kblock^-1 r, component-major (and, with x4, its FP32 node
 // quadruples for the bf16 passes)
 __global__ void __launch_bounds__(256) q2_jacobi_kernel(int nq, const double *__restrict__ inv_u,
@@ -1073,7 +1104,9 @@ static int launch_uu_node(int variant, int nq, const EquationsSet &s, const VT *
                           const double *x, const double *inv_u, double omega, double *out)
 {
     Runtime &rt = runtime();
-    if (variant < 0 || variant >= kNodeVariants) variant = 0;
+    // one wavefront per node for FP64 values where the rows fit
+    if (variant < 0 || variant >= kNodeVariants) variant = sizeof(VT) == sizeof(double) ? 4 : 0;
+    if (variant == 4 && !s.flat_rows()) variant = 0;
     const unsigned grid =
         static_cast<unsigned>((static_cast<int64_t>(nq) * kNodeVariantLanes[variant] + 255) / 256);
 #define OC_UU_NODE(L, U)                                                                                       \
@@ -1084,7 +1117,10 @@ static int launch_uu_node(int variant, int nq, const EquationsSet &s, const VT *
     case 1: OC_UU_NODE(32, 2); break;
     case 2: OC_UU_NODE(16, 2); break;
     case 3: OC_UU_NODE(16, 4); break;
-    case 4: OC_UU_NODE(64, 1); break;
+    case 4:
+        uu_flat_kernel<VT, kSweep><<<grid, 256, 0, rt.stream>>>(nq, s.row_ptr.ptr, s.pstart.ptr, s.col_idx.ptr, vals,
+                                                               s.free_mask.ptr, b, x, inv_u, omega, out);
+        break;
     default: OC_UU_NODE(32, 1); break;
     }
 #undef OC_UU_NODE
@@ -1192,9 +1228,7 @@ int mg_apply(EquationsSet &s, int precision, const double *t, double *z)
     const int M = s.n_meshes, nq = s.n_nodes, nl = static_cast<int>(g.levels.size());
     const double *inv_u = s.precond.ptr;  // nodal block inverses of the set's block preconditioner
     const bool bf = precision == OC_FP32;  // an FP32 Jacobian's packed bf16 values (mg_prepare)
-    // default shape: 16 lanes x 2 neighbours in flight for FP64 values (6%
-    // faster than 32 x 1 at 32^3), 16 lanes x one quad for bf16
-    const int variant = s.tuned_smoother >= 0 ? s.tuned_smoother : (precision == OC_FP64 ? 2 : 0);
+    const int variant = s.tuned_smoother;  // -1: a wavefront per node for FP64 values, 16 lanes x one quad for bf16
     // with the packed bf16 values the kernels that produce the iterate also
     // write its FP32 node quadruples, into the two halves of uu_x4 in turn
     // (a sweep gathers one half and writes the other); q4 is the current one

@@ -527,6 +527,46 @@ __global__ void __launch_bounds__(256) spmv_node_kernel(int nq, int nl, const in
     }
 }
 
+// The same by one wavefront per node or pressure row (node_rows_flat): FP64
+// values' default.  At 32^3 332 us (1.52 GB) against 397 with 16 lanes x 2
+// neighbours, at 16^3 34.6 against 44.7; with FP32 values it loses to 32 lanes
+// (342 us against 264), as half the bytes leave the wavefront's own chain of
+// columns, iterate and sum to bound it.
+template <typename VT>
+__global__ void __launch_bounds__(256) spmv_flat_kernel(int nq, int nl, const int64_t *__restrict__ row_ptr,
+                                                       const int64_t *__restrict__ pstart,
+                                                       const int *__restrict__ col_idx, const VT *__restrict__ vals,
+                                                       const double *__restrict__ w, const double *__restrict__ x,
+                                                       double *__restrict__ y)
+{
+    __shared__ double s_x[4][kFlatLds];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int64_t nq64 = nq, total = nq64 + nl;
+    const int g = xcd_block(blockIdx.x, gridDim.x) * 4 + wave;
+    if (g >= total) return;  // whole wavefronts
+    // the pressure rows spread evenly among the nodes' rows: wavefront g takes one
+    // where g nl / total steps up, so that every XCD gets its share of both kinds
+    const int l = static_cast<int>(g * static_cast<int64_t>(nl) / total);
+    if (static_cast<int>((g + int64_t{1}) * nl / total) > l) {
+        const int64_t row = 3 * nq64 + l;
+        const double wr = w == nullptr ? 1.0 : w[row];
+        double acc = 0.0;
+        if (wr != 0.0) acc = csr_row_dot<VT, 64>(row_ptr[row], row_ptr[row + 1], lane, col_idx, vals, x);
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1) acc += __shfl_xor(acc, o);
+        if (lane == 0) y[row] = wr * acc;
+        return;
+    }
+    const int i = g - l;
+    double a[3] = {0.0, 0.0, 0.0};
+    node_rows_flat<VT, true>(i, nq, lane, row_ptr, pstart, col_idx, vals, x, s_x[wave], a);
+    const double t = wave_total3(a, lane);
+    if ((lane & 15) == 0 && lane < 48) {
+        const int64_t row = (lane >> 4) * nq64 + i;
+        y[row] = w == nullptr ? t : (w[row] != 0.0 ? w[row] * t : 0.0);
+    }
+}
+
 // Pressure Jacobi z_p = inv_p .* r_p (written by the groups i < nl) and
 // t = r_u - B^T z_p on free displacement rows, 0 on fixed ones, by nodes; z_p
 // is formed again where B^T reads it, so one launch does both (nl <= nq)
@@ -819,8 +859,8 @@ struct Krylov {
         KernelTimer timer("spmv");
         const bool lap = s.cls == OC_EQUATIONS_SET_LAPLACE;
         // defaults: 8 lanes per Laplace row; per Mooney-Rivlin node 32 lanes
-        // (FP32) or 16 lanes with two neighbours in flight each (FP64)
-        const int lanes = s.tuned_spmv_lanes > 0 ? s.tuned_spmv_lanes : (lap ? 8 : (fp32 ? 32 : 16));
+        // (FP32) or a wavefront (FP64)
+        const int lanes = s.tuned_spmv_lanes > 0 ? s.tuned_spmv_lanes : (lap ? 8 : (fp32 ? 32 : 64));
         if (lap) return launch_spmv<double>(s.values.ptr, lanes, s.wgt.ptr, x, y);
         if (fp32) return launch_spmv<float>(s.values_sp.ptr, lanes, s.wgt.ptr, x, y);
         return launch_spmv<double>(s.values.ptr, lanes, s.wgt.ptr, x, y);
@@ -828,11 +868,11 @@ struct Krylov {
     template <typename VT>
     int launch_spmv(const VT *vals, int lanes, const double *wv, const double *x, double *y, int unroll = -1)
     {
-        if (unroll < 0) unroll = s.tuned_spmv_unroll > 0 ? s.tuned_spmv_unroll : (fp32 ? 1 : 2);
+        if (unroll < 0) unroll = s.tuned_spmv_unroll > 0 ? s.tuned_spmv_unroll : 1;
         Runtime &rt = runtime();
         if (s.cls == OC_EQUATIONS_SET_MOONEY_RIVLIN && s.node_rows == 1 && lanes >= 16) {
             const int nq = s.n_nodes, nl = s.n_nodes_l;
-            const unsigned gn = static_cast<unsigned>((static_cast<int64_t>(nq + nl) * lanes + 255) / 256);
+            const unsigned gn = static_cast<unsigned>((static_cast<int64_t>(nq + nl) * std::min(lanes, 32) + 255) / 256);
             const bool u2 = unroll == 2;
             // the Krylov operator gathers the iterate in FP64: FP32 node
             // quadruples, as the bf16 smoother reads, made the product about
@@ -842,9 +882,9 @@ struct Krylov {
             if (lanes == 16) {
                 if (u2) OC_SPMV_NODE(16, 2);
                 else OC_SPMV_NODE(16, 1);
-            } else if (lanes == 64) {
-                if (u2) OC_SPMV_NODE(64, 2);
-                else OC_SPMV_NODE(64, 1);
+            } else if (lanes == 64 && s.flat_rows()) {
+                spmv_flat_kernel<VT><<<static_cast<unsigned>((static_cast<int64_t>(nq) + nl + 3) / 4), 256, 0, rt.stream>>>(
+                    nq, nl, s.row_ptr.ptr, s.pstart.ptr, s.col_idx.ptr, vals, wv, x, y);
             } else {
                 if (u2) OC_SPMV_NODE(32, 2);
                 else OC_SPMV_NODE(32, 1);
