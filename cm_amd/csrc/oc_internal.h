@@ -109,38 +109,38 @@ struct DevBuf {
 // space on the same elements (its nodes are the element corners, numbered as
 // the pressure nodes); level l+1 coarsens level l by 2 per direction.  Levels
 // >= 1 store a 27-point 3x3-block stencil per node (node-major vectors).
+struct alignas(16) MgNode {               // a node's blocks among those by coarse node (mg_nodes_kernel)
+    int64_t first;
+    int32_t lo;
+    uint32_t bits;
+};
 struct MgLevel {
     int nn = 0;                           // nodes over all meshes
     std::vector<int32_t> h_dim, h_off;    // nodes per direction / first node, per mesh (h_off: M+1)
     DevBuf<int32_t> dim, off;
     DevBuf<double> A;                     // nn*27*9: A[(node*27 + d)*9 + 3c + c']
     DevBuf<double> Dinv;                  // nn*9 inverse diagonal blocks
-    DevBuf<double> As;                    // A(node, d) Dinv(neighbour d), levels with a coarser level
     DevBuf<uint8_t> freed;                // nn*3: DOF not fixed
-    DevBuf<double> x, b, r;               // nn*3 each
-};
-struct alignas(16) MgNode {               // a triquadratic node's place in A P0 (mg_nodes_kernel)
-    int64_t first;
-    int32_t lo;
-    uint32_t bits;
+    DevBuf<double> x, b;                  // nn*3 each
+    // levels with a coarser one: the node table, and the blocks by coarse node:
+    // A P0 on level 0, the V-cycle's V on the others (stencil_up_setup_kernel),
+    // with its U (own, 27*9 a node) and R (down, 125*9 a coarse node)
+    DevBuf<MgNode> nodes;
+    DevBuf<double> up, own, down;
 };
 struct Multigrid {
     std::vector<int32_t> h_n;             // elements per direction of each mesh
     DevBuf<int32_t> n;
-    std::vector<MgLevel> levels;          // levels[0] holds only the per-mesh tables
-    DevBuf<int64_t> ap_off;               // per mesh: its first block of A P0
-    DevBuf<double> ap;                    // A P0, 3x3 blocks by fine node (product_first, oc_multigrid.hip)
-    DevBuf<MgNode> nodes;
-    DevBuf<float> ap_sp;                  // the same in FP32, for an FP32 Jacobian's V-cycle
+    std::vector<MgLevel> levels;          // levels[0]: the triquadratic lattice, tables and A P0 only
+    DevBuf<float> ap_sp;                  // A P0 in FP32, for an FP32 Jacobian's V-cycle
     DevBuf<double> t0, r0, x0;            // level-0 scratch (3*n_nodes each)
     DevBuf<double> coarse_inv;            // per mesh dense inverse of the coarsest level
     int coarse_stride = 0;                // (max DOFs per mesh at the coarsest level)^2
-    int pre = 1, post = 2;                // level-0 sweeps (oc_multigrid_options_set)
-    // the trilinear and coarser stencil levels: one sweep each way (more
-    // sweeps there cost Krylov iterations rather than saving them)
-    int stencil_pre = 1, stencil_post = 1;
+    // level-0 sweeps (oc_multigrid_options_set); the trilinear and coarser
+    // stencil levels take one each way (more there cost Krylov iterations
+    // rather than saving them)
+    int pre = 1, post = 2;
     double omega = 0.8;
-    int coarse_sweeps = 0;                // 0: dense solve of the coarsest level
 };
 
 // Solver system (oc_solver_matrices.hip): the equations matrix or Jacobian

@@ -43,47 +43,53 @@ __device__ __forceinline__ int find_mesh(const int *__restrict__ off, int M, int
 
 __device__ __forceinline__ double lin_weight(int delta) { return delta == 0 ? 1.0 : 0.5; }
 
-// ---- the product A P0 --------------------------------------------------------------------
-// Node i = (ix, iy, iz) of the (2n+1)^3 lattice couples to the trilinear nodes
-// lo .. lo + c - 1 per direction: c = 3 from i/2 - 1 for an even index, c = 2
-// from i/2 for an odd one, those outside the grid holding zeros.  Its S = cx cy
-// cz blocks stand in x, y, z order, entry rc of block s at 9 first + rc S + s;
-// X(i) blocks precede index i in a direction, X(2n + 1) = 5n + 3.
+// ---- interpolation by blocks -------------------------------------------------------------
+// Node i = (ix, iy, iz) of a level's lattice couples, through its own row and
+// the interpolation, to the coarse nodes lo .. lo + c - 1 per direction: c = 3
+// from i/2 - 1 for an even index, c = 2 from i/2 for an odd one, those outside
+// the coarse grid holding zeros.  Its S = cx cy cz blocks stand in x, y, z
+// order, entry rc of block s at 9 first + rc S + s; before(i) blocks precede
+// index i in a direction.  Level 0 is the triquadratic lattice of 2n + 1 nodes.
 __device__ __forceinline__ int product_count(int i) { return (i & 1) ? 2 : 3; }
 __device__ __forceinline__ int product_lo(int i) { return (i >> 1) - ((i & 1) ? 0 : 1); }
-__device__ __forceinline__ int64_t product_first(int n, const int (&i)[3])
+__host__ __device__ __forceinline__ int64_t product_before(int k)
 {
-    const auto before = [](int k) { return static_cast<int64_t>((k >> 1) * 5 + (k & 1) * 3); };
-    const int64_t X = 5 * static_cast<int64_t>(n) + 3;
+    return static_cast<int64_t>((k >> 1) * 5 + (k & 1) * 3);
+}
+__device__ __forceinline__ int64_t product_first(int dim, const int (&i)[3])
+{
+    const int64_t X = product_before(dim);
     const int cy = product_count(i[1]), cz = product_count(i[2]);
-    return cz * cy * before(i[0]) + cz * X * before(i[1]) + X * X * before(i[2]);
+    return cz * cy * product_before(i[0]) + cz * X * product_before(i[1]) + X * X * product_before(i[2]);
 }
 // s / c for c = 2 or 3 and s < 27
 __device__ __forceinline__ int div_count(int s, int c) { return c == 3 ? (s * 43) >> 7 : s >> 1; }
 
-// What the kernels below need of a fine node, in one 16-byte load: with the
-// lattice coordinates found by division in each of them (and the mesh by
-// bisection) the correction kernel issued most of its instructions on those
-// and took 83 us at 32^3.  The MgNode of node q: first block, level-1 node at
-// (lo, lo, lo) (as an index, also where lo is outside), and bits: k the parity
-// of i_k, 3 + 2k lo_k outside, 4 + 2k lo_k + c_k - 1 outside, 16.. N = n + 1.
+// What the V-cycle needs of a fine node, in one 16-byte load: with the lattice
+// coordinates found by division (and the mesh by bisection) the correction
+// kernel issued most of its instructions on those and took 83 us at 32^3.  The
+// MgNode of node q: first block, coarse node at (lo, lo, lo) (as an index, also
+// where lo is outside), and bits: k the parity of i_k, 3 + 2k lo_k outside
+// (i_k = 0), 4 + 2k lo_k + c_k - 1 outside, 9 + k i_k the last, 12 an odd fine
+// dimension, 16.. the coarse dimension N.
 __global__ void __launch_bounds__(256)
-mg_nodes_kernel(int M, const int *__restrict__ n_mesh, const int *__restrict__ q_off,
-                const int64_t *__restrict__ ap_off, const int *__restrict__ off1, int nq, MgNode *__restrict__ nodes)
+mg_nodes_kernel(int M, const int *__restrict__ dim_f, const int *__restrict__ off_f, const int *__restrict__ dim_c,
+                const int *__restrict__ off_c, const int64_t *__restrict__ first, int nn, MgNode *__restrict__ nodes)
 {
     const int q = blockIdx.x * blockDim.x + threadIdx.x;
-    if (q >= nq) return;
-    const int m = find_mesh(q_off, M, q);
-    const int n = n_mesh[m], N = n + 1, T = 2 * n + 1, local = q - q_off[m];
+    if (q >= nn) return;
+    const int m = find_mesh(off_f, M, q);
+    const int T = dim_f[m], N = dim_c[m], local = q - off_f[m];
     const int i[3] = {local % T, (local / T) % T, local / (T * T)};
     MgNode v;
-    v.first = ap_off[m] + product_first(n, i);
-    v.lo = off1[m] + product_lo(i[0]) + N * (product_lo(i[1]) + N * product_lo(i[2]));
-    v.bits = static_cast<uint32_t>(N) << 16;
+    v.first = first[m] + product_first(T, i);
+    v.lo = off_c[m] + product_lo(i[0]) + N * (product_lo(i[1]) + N * product_lo(i[2]));
+    v.bits = static_cast<uint32_t>(N) << 16 | (T & 1 ? 1u << 12 : 0u);
     for (int k = 0; k < 3; ++k) {
         if (i[k] & 1) v.bits |= 1u << k;
         if (i[k] == 0) v.bits |= 8u << (2 * k);
-        if (i[k] == 2 * n) v.bits |= 16u << (2 * k);
+        if (product_lo(i[k]) + product_count(i[k]) > N) v.bits |= 16u << (2 * k);
+        if (i[k] == T - 1) v.bits |= 512u << k;
     }
     nodes[q] = v;
 }
@@ -100,7 +106,7 @@ constexpr int kProductNodes = 4;  // per block: 36 KB of FP64 values, four block
 template <typename VT>
 __global__ void __launch_bounds__(32 * kProductNodes)
 q1_product_kernel(int M, const int *__restrict__ n_mesh, const int *__restrict__ q_off,
-                  const int64_t *__restrict__ ap_off, int nq, const int64_t *__restrict__ row_ptr,
+                  const MgNode *__restrict__ nodes, int nq, const int64_t *__restrict__ row_ptr,
                   const int *__restrict__ col_idx, const VT *__restrict__ vals, const uint8_t *__restrict__ free_mask,
                   double *__restrict__ ap, float *__restrict__ ap_sp)
 {
@@ -160,7 +166,7 @@ q1_product_kernel(int M, const int *__restrict__ n_mesh, const int *__restrict__
 #pragma unroll
                     for (int rc = 0; rc < 9; ++rc) acc[rc] += w * static_cast<double>(v[rc * deg]);
                 }
-    const int64_t at = 9 * (ap_off[m] + product_first(n, i)) + lane;
+    const int64_t at = 9 * nodes[q].first + lane;
 #pragma unroll
     for (int rc = 0; rc < 9; ++rc) {
         ap[at + rc * S] = acc[rc];
@@ -168,18 +174,59 @@ q1_product_kernel(int M, const int *__restrict__ n_mesh, const int *__restrict__
     }
 }
 
-// level-1 stencil P0^T (A P0): block (I, I+d) = sum over the fine nodes 2I + s
+// A P of a stencil level (A's fixed rows dropped), by blocks as above: one
+// 32-lane group per node, lane s its slot, adding the up to 8 neighbours of an
+// odd and 27 of an even node that interpolate from the slot's coarse node
+__global__ void __launch_bounds__(256)
+stencil_product_kernel(int M, const int *__restrict__ dim, const int *__restrict__ off, int nn,
+                       const int *__restrict__ dim_c, const MgNode *__restrict__ nodes, const double *__restrict__ A,
+                       const uint8_t *__restrict__ freed, double *__restrict__ ap)
+{
+    const int node = static_cast<int>((static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x) >> 5);
+    const int s = threadIdx.x & 31;
+    if (node >= nn) return;
+    const int m = find_mesh(off, M, node);
+    const int N = dim[m], Nc = dim_c[m], local = node - off[m];
+    const int i[3] = {local % N, (local / N) % N, local / (N * N)};
+    const int cx = product_count(i[0]), cy = product_count(i[1]), S = cx * cy * product_count(i[2]);
+    if (s >= S) return;
+    const int K[3] = {product_lo(i[0]) + s % cx, product_lo(i[1]) + (s / cx) % cy, product_lo(i[2]) + s / (cx * cy)};
+    int lo[3], hi[3];
+    bool inside = true;
+    for (int k = 0; k < 3; ++k) {
+        inside = inside && K[k] >= 0 && K[k] < Nc;
+        lo[k] = max(max(2 * K[k] - 1, i[k] - 1), 0);
+        hi[k] = min(min(2 * K[k] + 1, i[k] + 1), N - 1);
+    }
+    double acc[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
+    if (inside)
+        for (int z = lo[2]; z <= hi[2]; ++z)
+            for (int y = lo[1]; y <= hi[1]; ++y)
+                for (int x = lo[0]; x <= hi[0]; ++x) {
+                    const double w = lin_weight(x - 2 * K[0]) * lin_weight(y - 2 * K[1]) * lin_weight(z - 2 * K[2]);
+                    const int d = (x - i[0] + 1) + 3 * (y - i[1] + 1) + 9 * (z - i[2] + 1);
+                    const double *a = A + (static_cast<int64_t>(node) * 27 + d) * 9;
+#pragma unroll
+                    for (int rc = 0; rc < 9; ++rc) acc[rc] += w * a[rc];
+                }
+    double *o = ap + 9 * nodes[node].first + s;
+#pragma unroll
+    for (int rc = 0; rc < 9; ++rc) o[rc * S] = freed[static_cast<int64_t>(node) * 3 + rc / 3] ? acc[rc] : 0.0;
+}
+
+// the coarse stencil P^T (A P): block (I, I+d) = sum over the fine nodes 2I + s
 // near I that couple to I+d, in z, y, x order; one 32-lane group per node,
 // lane d < 27 its block, so a fine node's blocks are read side by side
 __global__ void __launch_bounds__(256)
-q1_stencil_kernel(int M, const int *__restrict__ n_mesh, const int64_t *__restrict__ ap_off,
-                  const int *__restrict__ off1, int nn, const double *__restrict__ ap, double *__restrict__ A)
+coarse_stencil_kernel(int M, const int *__restrict__ dim_f, const int *__restrict__ off_f,
+                      const int *__restrict__ dim_c, const int *__restrict__ off_c, int nn,
+                      const MgNode *__restrict__ nodes, const double *__restrict__ ap, double *__restrict__ A)
 {
     const int node = static_cast<int>((static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x) >> 5);
     const int d = threadIdx.x & 31;
     if (node >= nn || d >= 27) return;
-    const int m = find_mesh(off1, M, node);
-    const int n = n_mesh[m], N = n + 1, local = node - off1[m];
+    const int m = find_mesh(off_c, M, node);
+    const int T = dim_f[m], N = dim_c[m], local = node - off_c[m];
     const int I[3] = {local % N, (local / N) % N, local / (N * N)}, e[3] = {d % 3 - 1, (d / 3) % 3 - 1, d / 9 - 1};
     double blk[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
     int lo[3], hi[3];
@@ -187,7 +234,7 @@ q1_stencil_kernel(int M, const int *__restrict__ n_mesh, const int64_t *__restri
     for (int k = 0; k < 3; ++k) {  // fine nodes of the grid near both I and I + e
         inside = inside && I[k] + e[k] >= 0 && I[k] + e[k] < N;
         lo[k] = max(e[k] <= 0 ? -1 : 0, -2 * I[k]);
-        hi[k] = min(e[k] >= 0 ? 1 : 0, 2 * n - 2 * I[k]);
+        hi[k] = min(e[k] >= 0 ? 1 : 0, T - 1 - 2 * I[k]);
     }
     if (inside)
         for (int s2 = lo[2]; s2 <= hi[2]; ++s2)
@@ -198,7 +245,7 @@ q1_stencil_kernel(int M, const int *__restrict__ n_mesh, const int64_t *__restri
                     const int cx = product_count(i[0]), cy = product_count(i[1]), S = cx * cy * product_count(i[2]);
                     const int slot = I[0] + e[0] - product_lo(i[0]) +
                                      cx * (I[1] + e[1] - product_lo(i[1]) + cy * (I[2] + e[2] - product_lo(i[2])));
-                    const double *a = ap + 9 * (ap_off[m] + product_first(n, i)) + slot;
+                    const double *a = ap + 9 * nodes[off_f[m] + i[0] + T * (i[1] + T * i[2])].first + slot;
 #pragma unroll
                     for (int rc = 0; rc < 9; ++rc) blk[rc] += w * a[rc * S];
                 }
@@ -207,73 +254,120 @@ q1_stencil_kernel(int M, const int *__restrict__ n_mesh, const int64_t *__restri
     for (int rc = 0; rc < 9; ++rc) o[rc] = blk[rc];
 }
 
-// Galerkin coarsening of a stencil level (masked by the fine level's free
-// DOFs): coarse block (I, J) = sum over fine nodes i near I and j near J of
-// w_i w_j A_f(i, j).  A block of 243 threads takes nine (coarse node,
-// direction) pairs; thread (pair, s) sums fine node s of I's neighbourhood
-// against every j, and the 27 partial blocks are added in s order, so the
-// sum is deterministic and one pair's work is spread over 27 threads (the
-// coarse levels have few nodes).
-constexpr int kGalPairs = 9;
+// The V-cycle's two halves on a stencil level as one linear map each.  With one
+// Jacobi step from zero, x1 = omega Dinv b, the residual restricted and one
+// sweep after the correction e,
+//   b_c = P^T (b - A x1)                       = R b,
+//   x   = x1 + P e + omega Dinv (b - A (x1 + P e)) = U b + V e,
+// with R = P^T (I - omega A Dinv) (125 blocks a coarse node), U = omega Dinv (2 I -
+// omega A Dinv) (27 a node) and V = P - omega Dinv (A P) (8 to 27 a node): as many
+// values as the stencil read twice, in two launches instead of four.  At 16^3 (three
+// such levels) 26 us a V-cycle against 54, at 32^3 (four) 66 us against 108.
 
-__global__ void __launch_bounds__(27 * kGalPairs)
-galerkin_coarsen_kernel(int M, const int *__restrict__ dim_f, const int *__restrict__ off_f,
-                        const double *__restrict__ Af, const uint8_t *__restrict__ freed_f,
-                        const int *__restrict__ dim_c, const int *__restrict__ off_c, int nn_c,
-                        double *__restrict__ Ac)
+// V from A P in place, and U; 32 lanes a node, lane by slot and by neighbour.
+__global__ void __launch_bounds__(256)
+stencil_up_setup_kernel(int M, const int *__restrict__ dim, const int *__restrict__ off, int nn,
+                        const MgNode *__restrict__ nodes, const double *__restrict__ A,
+                        const uint8_t *__restrict__ freed, const double *__restrict__ Dinv, double omega,
+                        double *__restrict__ U, double *__restrict__ V)
 {
-    __shared__ double s_part[kGalPairs][27][9];
-    const int p = threadIdx.x / 27, s = threadIdx.x % 27;
-    const int64_t total = static_cast<int64_t>(nn_c) * 27;
-    const int64_t t = static_cast<int64_t>(blockIdx.x) * kGalPairs + p;
-    double blk[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
-    if (t < total) {
-        const int node = static_cast<int>(t / 27), d = static_cast<int>(t % 27);
-        const int m = find_mesh(off_c, M, node);
-        const int Nc = dim_c[m], Nf = dim_f[m], local = node - off_c[m];
-        const int I[3] = {local % Nc, (local / Nc) % Nc, local / (Nc * Nc)};
-        const int J[3] = {I[0] + d % 3 - 1, I[1] + (d / 3) % 3 - 1, I[2] + d / 9 - 1};
-        const int i[3] = {2 * I[0] + s % 3 - 1, 2 * I[1] + (s / 3) % 3 - 1, 2 * I[2] + s / 9 - 1};
-        if (J[0] >= 0 && J[0] < Nc && J[1] >= 0 && J[1] < Nc && J[2] >= 0 && J[2] < Nc && i[0] >= 0 && i[0] < Nf &&
-            i[1] >= 0 && i[1] < Nf && i[2] >= 0 && i[2] < Nf) {
-            const double wi = lin_weight(s % 3 - 1) * lin_weight((s / 3) % 3 - 1) * lin_weight(s / 9 - 1);
-            const int64_t fi = off_f[m] + i[0] + static_cast<int64_t>(Nf) * (i[1] + static_cast<int64_t>(Nf) * i[2]);
-            // fine neighbours j = 2J + q - 1 of J inside the grid and within
-            // one node of i, per direction (the other q add nothing), in
-            // ascending q = q0 + 3 q1 + 9 q2
-            int qlo[3], qhi[3];
-            for (int k = 0; k < 3; ++k) {
-                qlo[k] = max(max(0, 1 - 2 * J[k]), i[k] - 2 * J[k]);
-                qhi[k] = min(min(2, Nf - 2 * J[k]), i[k] - 2 * J[k] + 2);
-            }
-            for (int q2 = qlo[2]; q2 <= qhi[2]; ++q2)
-                for (int q1 = qlo[1]; q1 <= qhi[1]; ++q1)
-                    for (int q0 = qlo[0]; q0 <= qhi[0]; ++q0) {
-                        const int j[3] = {2 * J[0] + q0 - 1, 2 * J[1] + q1 - 1, 2 * J[2] + q2 - 1};
-                        const int e0 = j[0] - i[0], e1 = j[1] - i[1], e2 = j[2] - i[2];
-                        const double w = wi * lin_weight(q0 - 1) * lin_weight(q1 - 1) * lin_weight(q2 - 1);
-                        const int64_t fj =
-                            off_f[m] + j[0] + static_cast<int64_t>(Nf) * (j[1] + static_cast<int64_t>(Nf) * j[2]);
-                        const double *a = Af + (fi * 27 + (e0 + 1) + 3 * (e1 + 1) + 9 * (e2 + 1)) * 9;
-                        for (int c = 0; c < 3; ++c) {
-                            if (!freed_f[fi * 3 + c]) continue;
-                            for (int cp = 0; cp < 3; ++cp)
-                                if (freed_f[fj * 3 + cp]) blk[3 * c + cp] += w * a[3 * c + cp];
-                        }
-                    }
-        }
+    const int node = static_cast<int>((static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x) >> 5);
+    const int d = threadIdx.x & 31;
+    if (node >= nn || d >= 27) return;
+    const int m = find_mesh(off, M, node);
+    const int N = dim[m], local = node - off[m];
+    const int i[3] = {local % N, (local / N) % N, local / (N * N)};
+    double D[9];
+#pragma unroll
+    for (int k = 0; k < 9; ++k) D[k] = Dinv[static_cast<int64_t>(node) * 9 + k];
+    const int J[3] = {i[0] + d % 3 - 1, i[1] + (d / 3) % 3 - 1, i[2] + d / 9 - 1};
+    double u[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
+    if (J[0] >= 0 && J[0] < N && J[1] >= 0 && J[1] < N && J[2] >= 0 && J[2] < N) {
+        const int64_t j = off[m] + J[0] + static_cast<int64_t>(N) * (J[1] + static_cast<int64_t>(N) * J[2]);
+        const double *a = A + (static_cast<int64_t>(node) * 27 + d) * 9, *q = Dinv + j * 9;
+        double w[9];  // 2 I - omega A Dinv
+        for (int c = 0; c < 3; ++c)
+            for (int cp = 0; cp < 3; ++cp)
+                w[3 * c + cp] = (d == 13 && c == cp ? 2.0 : 0.0) -
+                                omega * (a[3 * c] * q[cp] + a[3 * c + 1] * q[3 + cp] + a[3 * c + 2] * q[6 + cp]);
+        for (int c = 0; c < 3; ++c)
+            for (int cp = 0; cp < 3; ++cp)
+                u[3 * c + cp] = omega * (D[3 * c] * w[cp] + D[3 * c + 1] * w[3 + cp] + D[3 * c + 2] * w[6 + cp]);
     }
 #pragma unroll
-    for (int k = 0; k < 9; ++k) s_part[p][s][k] = blk[k];
-    __syncthreads();
-    if (threadIdx.x < kGalPairs * 9) {
-        const int pp = threadIdx.x / 9, k = threadIdx.x % 9;
-        const int64_t tt = static_cast<int64_t>(blockIdx.x) * kGalPairs + pp;
-        if (tt < total) {
-            double acc = 0.0;
-            for (int ss = 0; ss < 27; ++ss) acc += s_part[pp][ss][k];
-            Ac[tt * 9 + k] = acc;
+    for (int rc = 0; rc < 9; ++rc) U[(static_cast<int64_t>(node) * 9 + rc) * 27 + d] = u[rc];
+    const int cx = product_count(i[0]), cy = product_count(i[1]), S = cx * cy * product_count(i[2]);
+    if (d >= S) return;
+    const int k[3] = {d % cx, (d / cx) % cy, d / (cx * cy)};
+    double w = 1.0;
+    for (int a = 0; a < 3; ++a) w *= (i[a] & 1) ? 0.5 : (k[a] == 1 ? 1.0 : 0.0);
+    double *v = V + 9 * nodes[node].first + d;
+    double g[9];
+#pragma unroll
+    for (int rc = 0; rc < 9; ++rc) g[rc] = v[rc * S];
+    for (int c = 0; c < 3; ++c) {
+        const bool f = freed[static_cast<int64_t>(node) * 3 + c];
+        for (int cp = 0; cp < 3; ++cp) {
+            const double p = f && c == cp ? w : 0.0;
+            v[(3 * c + cp) * S] = p - omega * (D[3 * c] * g[cp] + D[3 * c + 1] * g[3 + cp] + D[3 * c + 2] * g[6 + cp]);
         }
+    }
+}
+
+// R: a thread a (coarse node, fine neighbour 2K + d - 2), entries rc of a node
+// in runs of 125
+__global__ void __launch_bounds__(256)
+stencil_down_setup_kernel(int M, const int *__restrict__ dim, const int *__restrict__ off,
+                          const int *__restrict__ dim_c, const int *__restrict__ off_c, int nn_c,
+                          const double *__restrict__ A, const uint8_t *__restrict__ freed,
+                          const double *__restrict__ Dinv, const uint8_t *__restrict__ freed_c, double omega,
+                          double *__restrict__ R)
+{
+    const int64_t total = static_cast<int64_t>(nn_c) * 125;
+    for (int64_t t = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x; t < total;
+         t += static_cast<int64_t>(gridDim.x) * blockDim.x) {
+        const int node = static_cast<int>(t / 125), d = static_cast<int>(t % 125);
+        const int m = find_mesh(off_c, M, node);
+        const int N = dim[m], Nc = dim_c[m], local = node - off_c[m];
+        const int e[3] = {d % 5 - 2, (d / 5) % 5 - 2, d / 25 - 2};
+        const int K[3] = {2 * (local % Nc), 2 * ((local / Nc) % Nc), 2 * (local / (Nc * Nc))};
+        double r[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
+        bool inside = true;
+        int lo[3], hi[3];
+        for (int k = 0; k < 3; ++k) {
+            inside = inside && K[k] + e[k] >= 0 && K[k] + e[k] < N;
+            lo[k] = max(max(-1, e[k] - 1), -K[k]);
+            hi[k] = min(min(1, e[k] + 1), N - 1 - K[k]);
+        }
+        if (inside) {
+            const int64_t N64 = N;
+            double acc[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
+            for (int z = lo[2]; z <= hi[2]; ++z)
+                for (int y = lo[1]; y <= hi[1]; ++y)
+                    for (int x = lo[0]; x <= hi[0]; ++x) {
+                        const double w = lin_weight(x) * lin_weight(y) * lin_weight(z);
+                        const int64_t i = off[m] + K[0] + x + N64 * (K[1] + y + N64 * (K[2] + z));
+                        const int b = (e[0] - x + 1) + 3 * (e[1] - y + 1) + 9 * (e[2] - z + 1);
+                        for (int c = 0; c < 3; ++c)
+                            if (freed[i * 3 + c])
+                                for (int cp = 0; cp < 3; ++cp) acc[3 * c + cp] += w * A[(i * 27 + b) * 9 + 3 * c + cp];
+                    }
+            const int64_t j = off[m] + K[0] + e[0] + N64 * (K[1] + e[1] + N64 * (K[2] + e[2]));
+            const double *q = Dinv + j * 9;
+            const bool near = e[0] * e[0] <= 1 && e[1] * e[1] <= 1 && e[2] * e[2] <= 1;
+            for (int c = 0; c < 3; ++c)
+                for (int cp = 0; cp < 3; ++cp) {
+                    const double p = near && c == cp && freed[j * 3 + c]
+                                         ? lin_weight(e[0]) * lin_weight(e[1]) * lin_weight(e[2])
+                                         : 0.0;
+                    r[3 * c + cp] = freed_c[static_cast<int64_t>(node) * 3 + c]
+                                        ? p - omega * (acc[3 * c] * q[cp] + acc[3 * c + 1] * q[3 + cp] +
+                                                       acc[3 * c + 2] * q[6 + cp])
+                                        : 0.0;
+                }
+        }
+#pragma unroll
+        for (int rc = 0; rc < 9; ++rc) R[(static_cast<int64_t>(node) * 9 + rc) * 125 + d] = r[rc];
     }
 }
 
@@ -776,214 +870,81 @@ q1_correct_kernel(int nq, const MgNode *__restrict__ nodes, const VT *__restrict
     if (x4) x4[4 * static_cast<int64_t>(q) + lane] = static_cast<float>(xn);
 }
 
-// As(node, d) = A(node, d) Dinv(neighbour d): the first Jacobi step from
-// x = 0 (x1 = omega Dinv b) folded into the stencil, so r = b - A x1 =
-// b - omega sum_d As(node, d) b(neighbour d) needs no x1 from other nodes
-__global__ void __launch_bounds__(256) scaled_stencil_kernel(int M, const int *__restrict__ dim,
-                                                            const int *__restrict__ off, int nn,
-                                                            const double *__restrict__ A,
-                                                            const double *__restrict__ Dinv, double *__restrict__ As)
+// b_c = R b: one wavefront per coarse node, lanes over its 125 fine neighbours
+__global__ void __launch_bounds__(256)
+stencil_down_kernel(int M, const int *__restrict__ dim, const int *__restrict__ off, const int *__restrict__ dim_c,
+                    const int *__restrict__ off_c, int nn_c, const double *__restrict__ R,
+                    const double *__restrict__ b, double *__restrict__ bc)
 {
-    const int64_t total = static_cast<int64_t>(nn) * 27;
-    for (int64_t t = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x; t < total;
-         t += static_cast<int64_t>(gridDim.x) * blockDim.x) {
-        const int node = static_cast<int>(t / 27), d = static_cast<int>(t % 27);
-        const int m = find_mesh(off, M, node);
-        const int N = dim[m], local = node - off[m];
-        const int J[3] = {local % N + d % 3 - 1, (local / N) % N + (d / 3) % 3 - 1, local / (N * N) + d / 9 - 1};
-        double *o = As + t * 9;
-        if (J[0] < 0 || J[0] >= N || J[1] < 0 || J[1] >= N || J[2] < 0 || J[2] >= N) {
-            for (int k = 0; k < 9; ++k) o[k] = 0.0;
-            continue;
-        }
-        const int64_t j = off[m] + J[0] + static_cast<int64_t>(N) * (J[1] + static_cast<int64_t>(N) * J[2]);
-        const double *a = A + t * 9, *q = Dinv + j * 9;
-        for (int c = 0; c < 3; ++c)
-            for (int cp = 0; cp < 3; ++cp) o[3 * c + cp] = a[3 * c] * q[cp] + a[3 * c + 1] * q[3 + cp] + a[3 * c + 2] * q[6 + cp];
-    }
-}
-
-// First smoothing step of a stencil level and its residual in one launch:
-// x = omega Dinv b, r = b - omega sum_d As(node, d) b(neighbour d) on free
-// DOFs (0 on fixed ones); one 32-lane group per node as in stencil_apply_kernel
-__global__ void __launch_bounds__(256) stencil_first_residual_kernel(int M, const int *__restrict__ dim,
-                                                                    const int *__restrict__ off, int nn,
-                                                                    const double *__restrict__ As,
-                                                                    const uint8_t *__restrict__ freed,
-                                                                    const double *__restrict__ b,
-                                                                    const double *__restrict__ Dinv, double omega,
-                                                                    double *__restrict__ x, double *__restrict__ r)
-{
-    const int node = static_cast<int>((static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x) >> 5);
-    const int d = threadIdx.x & 31;
-    if (node >= nn) return;  // whole 32-lane groups
-    const int m = find_mesh(off, M, node);
-    const int N = dim[m], local = node - off[m];
-    double p[3] = {0.0, 0.0, 0.0};
-    if (d < 27) {
-        const int J[3] = {local % N + d % 3 - 1, (local / N) % N + (d / 3) % 3 - 1, local / (N * N) + d / 9 - 1};
-        if (J[0] >= 0 && J[0] < N && J[1] >= 0 && J[1] < N && J[2] >= 0 && J[2] < N) {
-            const int64_t j = off[m] + J[0] + static_cast<int64_t>(N) * (J[1] + static_cast<int64_t>(N) * J[2]);
-            const double *a = As + (static_cast<int64_t>(node) * 27 + d) * 9;
-            const double b0 = b[j * 3], b1 = b[j * 3 + 1], b2 = b[j * 3 + 2];
-#pragma unroll
-            for (int c = 0; c < 3; ++c) p[c] = a[3 * c] * b0 + a[3 * c + 1] * b1 + a[3 * c + 2] * b2;
-        }
-    }
-#pragma unroll
-    for (int sh = 16; sh > 0; sh >>= 1)
-#pragma unroll
-        for (int c = 0; c < 3; ++c) p[c] += __shfl_xor(p[c], sh, 32);
-    if (d != 0) return;
-    const double *o = Dinv + static_cast<int64_t>(node) * 9;
-    const int64_t k0 = static_cast<int64_t>(node) * 3;
-    const double bn[3] = {b[k0], b[k0 + 1], b[k0 + 2]};
-#pragma unroll
-    for (int c = 0; c < 3; ++c) {
-        r[k0 + c] = freed[k0 + c] ? bn[c] - omega * p[c] : 0.0;
-        x[k0 + c] = omega * (o[3 * c] * bn[0] + o[3 * c + 1] * bn[1] + o[3 * c + 2] * bn[2]);
-    }
-}
-
-__global__ void __launch_bounds__(256) stencil_jacobi_kernel(int nn, const double *__restrict__ Dinv,
-                                                            const double *__restrict__ r, double *__restrict__ x,
-                                                            double omega, int first)
-{
-    for (int node = blockIdx.x * blockDim.x + threadIdx.x; node < nn; node += gridDim.x * blockDim.x) {
-        const double *o = Dinv + static_cast<int64_t>(node) * 9;
-        const double *rr = r + static_cast<int64_t>(node) * 3;
-        for (int c = 0; c < 3; ++c) {
-            const int64_t k = static_cast<int64_t>(node) * 3 + c;
-            const double d = o[3 * c] * rr[0] + o[3 * c + 1] * rr[1] + o[3 * c + 2] * rr[2];
-            x[k] = (first ? 0.0 : x[k]) + omega * d;
-        }
-    }
-}
-
-// levels >= 1, one 32-lane group per node (the coarse levels have few
-// nodes, so a node's 27 neighbour products run in parallel): lane d < 27
-// forms A(node, d) x(neighbour d), and a fixed butterfly adds the 27
-// products.  kSweep 0: out = r = b - A x on free DOFs.  kSweep 1: one Jacobi
-// sweep, out = x + omega Dinv r (out and x distinct buffers).
-template <int kSweep>
-__global__ void __launch_bounds__(256) stencil_apply_kernel(int M, const int *__restrict__ dim,
-                                                           const int *__restrict__ off, int nn,
-                                                           const double *__restrict__ A,
-                                                           const uint8_t *__restrict__ freed,
-                                                           const double *__restrict__ b,
-                                                           const double *__restrict__ x,
-                                                           const double *__restrict__ Dinv, double omega,
-                                                           double *__restrict__ out)
-{
-    const int node = static_cast<int>((static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x) >> 5);
-    const int d = threadIdx.x & 31;
-    if (node >= nn) return;  // whole 32-lane groups
-    const int m = find_mesh(off, M, node);
-    const int N = dim[m], local = node - off[m];
-    double p[3] = {0.0, 0.0, 0.0};
-    if (d < 27) {
-        const int J[3] = {local % N + d % 3 - 1, (local / N) % N + (d / 3) % 3 - 1, local / (N * N) + d / 9 - 1};
-        if (J[0] >= 0 && J[0] < N && J[1] >= 0 && J[1] < N && J[2] >= 0 && J[2] < N) {
-            const int64_t j = off[m] + J[0] + static_cast<int64_t>(N) * (J[1] + static_cast<int64_t>(N) * J[2]);
-            const double *a = A + (static_cast<int64_t>(node) * 27 + d) * 9;
-            const double x0 = x[j * 3], x1 = x[j * 3 + 1], x2 = x[j * 3 + 2];
-#pragma unroll
-            for (int c = 0; c < 3; ++c) p[c] = a[3 * c] * x0 + a[3 * c + 1] * x1 + a[3 * c + 2] * x2;
-        }
-    }
-#pragma unroll
-    for (int sh = 16; sh > 0; sh >>= 1)
-#pragma unroll
-        for (int c = 0; c < 3; ++c) p[c] += __shfl_xor(p[c], sh, 32);
-    if (d != 0) return;
-    double r[3];
-#pragma unroll
-    for (int c = 0; c < 3; ++c) {
-        const int64_t k = static_cast<int64_t>(node) * 3 + c;
-        r[c] = freed[k] ? b[k] - p[c] : 0.0;
-    }
-    if (kSweep == 0) {
-#pragma unroll
-        for (int c = 0; c < 3; ++c) out[static_cast<int64_t>(node) * 3 + c] = r[c];
-    } else {
-        const double *o = Dinv + static_cast<int64_t>(node) * 9;
-#pragma unroll
-        for (int c = 0; c < 3; ++c) {
-            const int64_t k = static_cast<int64_t>(node) * 3 + c;
-            out[k] = x[k] + omega * (o[3 * c] * r[0] + o[3 * c + 1] * r[1] + o[3 * c + 2] * r[2]);
-        }
-    }
-}
-
-__global__ void __launch_bounds__(256) restrict_stencil_kernel(int M, const int *__restrict__ dim_f,
-                                                              const int *__restrict__ off_f,
-                                                              const int *__restrict__ dim_c,
-                                                              const int *__restrict__ off_c, int nn_c,
-                                                              const uint8_t *__restrict__ freed_c,
-                                                              const double *__restrict__ rf, double *__restrict__ bc)
-{
-    // one 32-lane group per coarse node, as restrict_q2_kernel
-    const int node = static_cast<int>((static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x) >> 5);
-    const int s = threadIdx.x & 31;
-    if (node >= nn_c) return;  // whole 32-lane groups
+    const int node = static_cast<int>(blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6));
+    const int lane = threadIdx.x & 63;
+    if (node >= nn_c) return;  // whole wavefronts
     const int m = find_mesh(off_c, M, node);
-    const int Nc = dim_c[m], Nf = dim_f[m], local = node - off_c[m];
-    const int I[3] = {local % Nc, (local / Nc) % Nc, local / (Nc * Nc)};
-    double acc[3] = {0.0, 0.0, 0.0};
-    if (s < 27) {
-        const int i[3] = {2 * I[0] + s % 3 - 1, 2 * I[1] + (s / 3) % 3 - 1, 2 * I[2] + s / 9 - 1};
-        if (i[0] >= 0 && i[0] < Nf && i[1] >= 0 && i[1] < Nf && i[2] >= 0 && i[2] < Nf) {
-            const double w = lin_weight(s % 3 - 1) * lin_weight((s / 3) % 3 - 1) * lin_weight(s / 9 - 1);
-            const int64_t f = off_f[m] + i[0] + static_cast<int64_t>(Nf) * (i[1] + static_cast<int64_t>(Nf) * i[2]);
+    const int N = dim[m], Nc = dim_c[m], local = node - off_c[m];
+    const int K[3] = {2 * (local % Nc), 2 * ((local / Nc) % Nc), 2 * (local / (Nc * Nc))};
+    const double *r = R + static_cast<int64_t>(node) * (9 * 125);
+    double a[3] = {0.0, 0.0, 0.0};
 #pragma unroll
-            for (int c = 0; c < 3; ++c) acc[c] = w * rf[f * 3 + c];
-        }
+    for (int u = 0; u < 2; ++u) {
+        const int d = min(lane + 64 * u, 124);
+        double v[9];
+#pragma unroll
+        for (int rc = 0; rc < 9; ++rc) v[rc] = r[rc * 125 + d];
+        const int i[3] = {K[0] + d % 5 - 2, K[1] + (d / 5) % 5 - 2, K[2] + d / 25 - 2};
+        const bool ok = lane + 64 * u < 125 && i[0] >= 0 && i[0] < N && i[1] >= 0 && i[1] < N && i[2] >= 0 && i[2] < N;
+        const double *bj = b + 3 * static_cast<int64_t>(ok ? off[m] + i[0] + N * (i[1] + N * i[2]) : 0);
+        const double b0 = ok ? bj[0] : 0.0, b1 = ok ? bj[1] : 0.0, b2 = ok ? bj[2] : 0.0;
+#pragma unroll
+        for (int c = 0; c < 3; ++c) a[c] += v[3 * c] * b0 + v[3 * c + 1] * b1 + v[3 * c + 2] * b2;
     }
+    const double t = wave_total3(a, lane);
+    if ((lane & 15) == 0 && lane < 48) bc[static_cast<int64_t>(node) * 3 + (lane >> 4)] = t;
+}
+
+// x = U b + V e: one 32-lane group per node, lanes over its 27 neighbours and
+// its 8 to 27 coarse ones
+__global__ void __launch_bounds__(256)
+stencil_up_kernel(int nn, const MgNode *__restrict__ nodes, const double *__restrict__ U,
+                  const double *__restrict__ V, const double *__restrict__ b, const double *__restrict__ e,
+                  double *__restrict__ x)
+{
+    const int node = static_cast<int>((static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x) >> 5);
+    const int lane = threadIdx.x & 31;
+    if (node >= nn) return;  // whole 32-lane groups
+    const MgNode nd = nodes[node];
+    const int N = static_cast<int>(nd.bits >> 16), Nf = 2 * N - 2 + (nd.bits >> 12 & 1);
+    const int d = min(lane, 26);
+    double u[9];
+#pragma unroll
+    for (int rc = 0; rc < 9; ++rc) u[rc] = U[(static_cast<int64_t>(node) * 9 + rc) * 27 + d];
+    const bool odd[3] = {(nd.bits & 1) != 0, (nd.bits & 2) != 0, (nd.bits & 4) != 0};
+    const int cx = odd[0] ? 2 : 3, cy = odd[1] ? 2 : 3, cz = odd[2] ? 2 : 3, S = cx * cy * cz;
+    const int s = min(lane, S - 1);
+    double v[9];
+#pragma unroll
+    for (int rc = 0; rc < 9; ++rc) v[rc] = V[9 * nd.first + rc * S + s];
+    const int n[3] = {d % 3, (d / 3) % 3, d / 9};
+    const int yz = div_count(s, cx), sz = div_count(yz, cy), k[3] = {s - cx * yz, yz - cy * sz, sz};
+    bool okb = lane < 27, oke = lane < S;
+#pragma unroll
+    for (int a = 0; a < 3; ++a) {
+        okb = okb && !(n[a] == 0 && (nd.bits >> (3 + 2 * a) & 1)) && !(n[a] == 2 && (nd.bits >> (9 + a) & 1));
+        oke = oke && !(k[a] == 0 && (nd.bits >> (3 + 2 * a) & 1)) && !(k[a] == 2 && (nd.bits >> (4 + 2 * a) & 1));
+    }
+    const double *bj = b + 3 * static_cast<int64_t>(okb ? node + n[0] - 1 + Nf * (n[1] - 1 + Nf * (n[2] - 1)) : 0);
+    const double *ek = e + 3 * static_cast<int64_t>(oke ? nd.lo + k[0] + N * (k[1] + N * k[2]) : 0);
+    const double bv[3] = {okb ? bj[0] : 0.0, okb ? bj[1] : 0.0, okb ? bj[2] : 0.0};
+    const double ev[3] = {oke ? ek[0] : 0.0, oke ? ek[1] : 0.0, oke ? ek[2] : 0.0};
+    double p[3];
+#pragma unroll
+    for (int c = 0; c < 3; ++c)
+        p[c] = u[3 * c] * bv[0] + u[3 * c + 1] * bv[1] + u[3 * c + 2] * bv[2] + v[3 * c] * ev[0] +
+               v[3 * c + 1] * ev[1] + v[3 * c + 2] * ev[2];
 #pragma unroll
     for (int sh = 16; sh > 0; sh >>= 1)
 #pragma unroll
-        for (int c = 0; c < 3; ++c) acc[c] += __shfl_xor(acc[c], sh, 32);
-    if (s != 0) return;
-#pragma unroll
-    for (int c = 0; c < 3; ++c) {
-        const int64_t k = static_cast<int64_t>(node) * 3 + c;
-        bc[k] = freed_c[k] ? acc[c] : 0.0;
-    }
-}
-
-__global__ void __launch_bounds__(256) prolong_stencil_kernel(int M, const int *__restrict__ dim_f,
-                                                             const int *__restrict__ off_f, int nn_f,
-                                                             const int *__restrict__ dim_c,
-                                                             const int *__restrict__ off_c,
-                                                             const uint8_t *__restrict__ freed_f,
-                                                             const double *__restrict__ xc, double *__restrict__ xf)
-{
-    for (int node = blockIdx.x * blockDim.x + threadIdx.x; node < nn_f; node += gridDim.x * blockDim.x) {
-        const int m = find_mesh(off_f, M, node);
-        const int Nf = dim_f[m], Nc = dim_c[m], local = node - off_f[m];
-        const int i[3] = {local % Nf, (local / Nf) % Nf, local / (Nf * Nf)};
-        int p0[3], p1[3];
-        double w0[3], w1[3];
-        for (int k = 0; k < 3; ++k) {
-            p0[k] = i[k] >> 1;
-            p1[k] = (i[k] + 1) >> 1;
-            w0[k] = (i[k] & 1) ? 0.5 : 1.0;
-            w1[k] = (i[k] & 1) ? 0.5 : 0.0;
-        }
-        double v[3] = {0.0, 0.0, 0.0};
-        for (int s = 0; s < 8; ++s) {
-            const int b0 = s & 1, b1 = (s >> 1) & 1, b2 = s >> 2;
-            const double w = (b0 ? w1[0] : w0[0]) * (b1 ? w1[1] : w0[1]) * (b2 ? w1[2] : w0[2]);
-            if (w == 0.0) continue;
-            const int64_t P = off_c[m] + (b0 ? p1[0] : p0[0]) +
-                              static_cast<int64_t>(Nc) * ((b1 ? p1[1] : p0[1]) + static_cast<int64_t>(Nc) * (b2 ? p1[2] : p0[2]));
-            for (int c = 0; c < 3; ++c) v[c] += w * xc[P * 3 + c];
-        }
-        for (int c = 0; c < 3; ++c) {
-            const int64_t k = static_cast<int64_t>(node) * 3 + c;
-            if (freed_f[k]) xf[k] += v[c];
-        }
-    }
+        for (int c = 0; c < 3; ++c) p[c] += __shfl_xor(p[c], sh, 32);
+    if (lane < 3) x[static_cast<int64_t>(node) * 3 + lane] = lane == 0 ? p[0] : (lane == 1 ? p[1] : p[2]);
 }
 
 __global__ void __launch_bounds__(256) coarse_apply_kernel(int M, const int *__restrict__ dim,
@@ -1025,7 +986,7 @@ int mg_prepare(EquationsSet &s, int precision, bool *made)
     *made = !s.uu_bf.ptr || !g.ap_sp.ptr;
     if (!s.values_sp.ptr) OC_CHECK(s.values_sp.alloc(s.nnz));
     OC_CHECK(prepare_uu_bf16(s));
-    if (!g.ap_sp.ptr) OC_CHECK(g.ap_sp.alloc(g.ap.n));
+    if (!g.ap_sp.ptr) OC_CHECK(g.ap_sp.alloc(g.levels[0].up.n));
     return OC_NO_ERROR;
 }
 
@@ -1036,42 +997,43 @@ int mg_setup(EquationsSet &s, int precision)
     const int M = s.n_meshes;
     const int nq = s.n_nodes;
     const unsigned gp = static_cast<unsigned>((nq + kProductNodes - 1) / kProductNodes);
-    MgLevel &L1 = g.levels[1];
+    MgLevel &L0 = g.levels[0], &L1 = g.levels[1];
     if (precision == OC_FP64)
         q1_product_kernel<double><<<gp, 32 * kProductNodes, 0, rt.stream>>>(
-            M, g.n.ptr, s.q_off.ptr, g.ap_off.ptr, nq, s.row_ptr.ptr, s.col_idx.ptr, s.values.ptr, s.free_mask.ptr,
-            g.ap.ptr, nullptr);
+            M, g.n.ptr, s.q_off.ptr, L0.nodes.ptr, nq, s.row_ptr.ptr, s.col_idx.ptr, s.values.ptr, s.free_mask.ptr,
+            L0.up.ptr, nullptr);
     else
         q1_product_kernel<float><<<gp, 32 * kProductNodes, 0, rt.stream>>>(
-            M, g.n.ptr, s.q_off.ptr, g.ap_off.ptr, nq, s.row_ptr.ptr, s.col_idx.ptr, s.values_sp.ptr, s.free_mask.ptr,
-            g.ap.ptr, g.ap_sp.ptr);
+            M, g.n.ptr, s.q_off.ptr, L0.nodes.ptr, nq, s.row_ptr.ptr, s.col_idx.ptr, s.values_sp.ptr, s.free_mask.ptr,
+            L0.up.ptr, g.ap_sp.ptr);
     OC_HIP_CHECK(hipGetLastError());
     if (precision == OC_FP32) OC_CHECK(launch_uu_pack(s));
-    q1_stencil_kernel<<<group_grid(L1.nn), 256, 0, rt.stream>>>(M, g.n.ptr, g.ap_off.ptr, L1.off.ptr, L1.nn, g.ap.ptr,
-                                                               L1.A.ptr);
+    coarse_stencil_kernel<<<group_grid(L1.nn), 256, 0, rt.stream>>>(M, L0.dim.ptr, L0.off.ptr, L1.dim.ptr, L1.off.ptr,
+                                                                   L1.nn, L0.nodes.ptr, L0.up.ptr, L1.A.ptr);
     coincident_q2_kernel<<<grid1(L1.nn), 256, 0, rt.stream>>>(M, g.n.ptr, s.q_off.ptr, s.n_nodes, L1.off.ptr, L1.nn,
                                                               s.free_mask.ptr, L1.freed.ptr);
     level_freed_kernel<<<grid1(L1.nn), 256, 0, rt.stream>>>(L1.nn, L1.A.ptr, L1.freed.ptr);
     level_mask_kernel<<<grid1(static_cast<int64_t>(L1.nn) * 27), 256, 0, rt.stream>>>(
         M, L1.dim.ptr, L1.off.ptr, L1.nn, L1.A.ptr, L1.freed.ptr, L1.Dinv.ptr);
     OC_HIP_CHECK(hipGetLastError());
-    if (L1.As.ptr)
-        scaled_stencil_kernel<<<grid1(static_cast<int64_t>(L1.nn) * 27), 256, 0, rt.stream>>>(
-            M, L1.dim.ptr, L1.off.ptr, L1.nn, L1.A.ptr, L1.Dinv.ptr, L1.As.ptr);
     const int nl = static_cast<int>(g.levels.size());
     for (int l = 1; l + 1 < nl; ++l) {
         MgLevel &F = g.levels[l], &C = g.levels[l + 1];
-        galerkin_coarsen_kernel<<<static_cast<unsigned>((static_cast<int64_t>(C.nn) * 27 + kGalPairs - 1) / kGalPairs),
-                                  27 * kGalPairs, 0, rt.stream>>>(
-            M, F.dim.ptr, F.off.ptr, F.A.ptr, F.freed.ptr, C.dim.ptr, C.off.ptr, C.nn, C.A.ptr);
+        stencil_product_kernel<<<group_grid(F.nn), 256, 0, rt.stream>>>(M, F.dim.ptr, F.off.ptr, F.nn, C.dim.ptr,
+                                                                       F.nodes.ptr, F.A.ptr, F.freed.ptr, F.up.ptr);
+        coarse_stencil_kernel<<<group_grid(C.nn), 256, 0, rt.stream>>>(M, F.dim.ptr, F.off.ptr, C.dim.ptr, C.off.ptr,
+                                                                      C.nn, F.nodes.ptr, F.up.ptr, C.A.ptr);
         coincident_kernel<<<grid1(C.nn), 256, 0, rt.stream>>>(M, F.dim.ptr, F.off.ptr, F.freed.ptr, C.dim.ptr,
                                                              C.off.ptr, C.nn, C.freed.ptr);
         level_freed_kernel<<<grid1(C.nn), 256, 0, rt.stream>>>(C.nn, C.A.ptr, C.freed.ptr);
         level_mask_kernel<<<grid1(static_cast<int64_t>(C.nn) * 27), 256, 0, rt.stream>>>(
             M, C.dim.ptr, C.off.ptr, C.nn, C.A.ptr, C.freed.ptr, C.Dinv.ptr);
-        if (C.As.ptr)
-            scaled_stencil_kernel<<<grid1(static_cast<int64_t>(C.nn) * 27), 256, 0, rt.stream>>>(
-                M, C.dim.ptr, C.off.ptr, C.nn, C.A.ptr, C.Dinv.ptr, C.As.ptr);
+        stencil_up_setup_kernel<<<group_grid(F.nn), 256, 0, rt.stream>>>(M, F.dim.ptr, F.off.ptr, F.nn, F.nodes.ptr,
+                                                                        F.A.ptr, F.freed.ptr, F.Dinv.ptr, g.omega,
+                                                                        F.own.ptr, F.up.ptr);
+        stencil_down_setup_kernel<<<grid1(static_cast<int64_t>(C.nn) * 125), 256, 0, rt.stream>>>(
+            M, F.dim.ptr, F.off.ptr, C.dim.ptr, C.off.ptr, C.nn, F.A.ptr, F.freed.ptr, F.Dinv.ptr, C.freed.ptr,
+            g.omega, F.down.ptr);
         OC_HIP_CHECK(hipGetLastError());
     }
     MgLevel &Lc = g.levels[nl - 1];
@@ -1081,17 +1043,6 @@ int mg_setup(EquationsSet &s, int precision)
     return OC_NO_ERROR;
 }
 
-
-// one Jacobi sweep of a stencil level: x <- x + omega Dinv (b - A x), through
-// the level's r buffer (the two buffers trade places)
-static int stencil_sweep(int M, MgLevel &F, double omega)
-{
-    stencil_apply_kernel<1><<<group_grid(F.nn), 256, 0, runtime().stream>>>(
-        M, F.dim.ptr, F.off.ptr, F.nn, F.A.ptr, F.freed.ptr, F.b.ptr, F.x.ptr, F.Dinv.ptr, omega, F.r.ptr);
-    OC_HIP_CHECK(hipGetLastError());
-    std::swap(F.x, F.r);
-    return OC_NO_ERROR;
-}
 
 // Launch shapes of the level-0 node kernels: lanes per node (below) x
 // neighbours per lane in flight (1, 2, 2, 4, 1; the cases of launch_uu_node);
@@ -1255,25 +1206,15 @@ int mg_apply(EquationsSet &s, int precision, const double *t, double *z)
         OC_CHECK(launch_uu_bf16<0>(variant, s, t, cur, nullptr, 0.0, g.r0.ptr, q4));
     else
         OC_CHECK((launch_uu_node<double, 0>(variant, nq, s, s.values.ptr, t, cur, nullptr, 0.0, g.r0.ptr)));
-    MgLevel &L1 = g.levels[1];
+    MgLevel &L0 = g.levels[0], &L1 = g.levels[1];
     restrict_q2_kernel<<<group_grid(L1.nn), 256, 0, rt.stream>>>(M, g.n.ptr, s.q_off.ptr, nq, L1.off.ptr, L1.nn,
                                                             L1.freed.ptr, g.r0.ptr, L1.b.ptr);
     OC_HIP_CHECK(hipGetLastError());
     // down the stencil levels
     for (int l = 1; l + 1 < nl; ++l) {
         MgLevel &F = g.levels[l], &C = g.levels[l + 1];
-        if (g.stencil_pre <= 1 && F.As.ptr) {
-            stencil_first_residual_kernel<<<group_grid(F.nn), 256, 0, rt.stream>>>(
-                M, F.dim.ptr, F.off.ptr, F.nn, F.As.ptr, F.freed.ptr, F.b.ptr, F.Dinv.ptr, g.omega, F.x.ptr, F.r.ptr);
-        } else {
-            stencil_jacobi_kernel<<<grid1(F.nn), 256, 0, rt.stream>>>(F.nn, F.Dinv.ptr, F.b.ptr, F.x.ptr, g.omega, 1);
-            for (int k = 1; k < g.stencil_pre; ++k) OC_CHECK(stencil_sweep(M, F, g.omega));
-            stencil_apply_kernel<0><<<group_grid(F.nn), 256, 0, rt.stream>>>(M, F.dim.ptr, F.off.ptr, F.nn, F.A.ptr,
-                                                                            F.freed.ptr, F.b.ptr, F.x.ptr, nullptr,
-                                                                            0.0, F.r.ptr);
-        }
-        restrict_stencil_kernel<<<group_grid(C.nn), 256, 0, rt.stream>>>(M, F.dim.ptr, F.off.ptr, C.dim.ptr, C.off.ptr,
-                                                                   C.nn, C.freed.ptr, F.r.ptr, C.b.ptr);
+        stencil_down_kernel<<<static_cast<unsigned>((C.nn + 3) / 4), 256, 0, rt.stream>>>(
+            M, F.dim.ptr, F.off.ptr, C.dim.ptr, C.off.ptr, C.nn, F.down.ptr, F.b.ptr, C.b.ptr);
         OC_HIP_CHECK(hipGetLastError());
     }
     MgLevel &Lc = g.levels[nl - 1];
@@ -1283,18 +1224,17 @@ int mg_apply(EquationsSet &s, int precision, const double *t, double *z)
     // up
     for (int l = nl - 2; l >= 1; --l) {
         MgLevel &F = g.levels[l], &C = g.levels[l + 1];
-        prolong_stencil_kernel<<<grid1(F.nn), 256, 0, rt.stream>>>(M, F.dim.ptr, F.off.ptr, F.nn, C.dim.ptr,
-                                                                  C.off.ptr, F.freed.ptr, C.x.ptr, F.x.ptr);
-        for (int k = 0; k < g.stencil_post; ++k) OC_CHECK(stencil_sweep(M, F, g.omega));
+        stencil_up_kernel<<<group_grid(F.nn), 256, 0, rt.stream>>>(F.nn, F.nodes.ptr, F.own.ptr, F.up.ptr, F.b.ptr,
+                                                                  C.x.ptr, F.x.ptr);
         OC_HIP_CHECK(hipGetLastError());
     }
     const unsigned gc = static_cast<unsigned>((static_cast<int64_t>(nq) * 8 + 255) / 256);
     const double omega1 = post > 0 ? g.omega : 0.0;  // without post-smoothing only x + P0 e
     if (bf)
-        q1_correct_kernel<float><<<gc, 256, 0, rt.stream>>>(nq, g.nodes.ptr, g.ap_sp.ptr, L1.x.ptr, s.free_mask.ptr,
+        q1_correct_kernel<float><<<gc, 256, 0, rt.stream>>>(nq, L0.nodes.ptr, g.ap_sp.ptr, L1.x.ptr, s.free_mask.ptr,
                                                             g.r0.ptr, inv_u, omega1, cur, q4);
     else
-        q1_correct_kernel<double><<<gc, 256, 0, rt.stream>>>(nq, g.nodes.ptr, g.ap.ptr, L1.x.ptr, s.free_mask.ptr,
+        q1_correct_kernel<double><<<gc, 256, 0, rt.stream>>>(nq, L0.nodes.ptr, L0.up.ptr, L1.x.ptr, s.free_mask.ptr,
                                                              g.r0.ptr, inv_u, omega1, cur, nullptr);
     OC_HIP_CHECK(hipGetLastError());
     for (int k = 1; k < post; ++k) OC_CHECK(sweep0());
@@ -1346,45 +1286,57 @@ extern "C" int oc_multigrid_structure_set(oc_equations_set h, const int *n_per_m
     std::unique_ptr<Multigrid> guard(g);
     g->h_n.assign(n_per_mesh, n_per_mesh + M);
     OC_CHECK(g->n.upload(g->h_n.data(), M));
-    // levels: [0] placeholder, [1] trilinear (n+1)^3, then coarsening until every dim <= 3
+    // levels: [0] the triquadratic lattice (tables and A P0 only), [1] trilinear
+    // (n+1)^3, then coarsening until every dim <= 3
     g->levels.resize(2);
     std::vector<int32_t> dims(M);
-    for (int m = 0; m < M; ++m) dims[m] = g->h_n[m] + 1;
-    while (true) {
-        MgLevel &L = g->levels.back();
+    const auto tables = [&](MgLevel &L) -> int {
         L.h_dim = dims;
         L.h_off.assign(M + 1, 0);
         for (int m = 0; m < M; ++m) L.h_off[m + 1] = L.h_off[m] + dims[m] * dims[m] * dims[m];
         L.nn = L.h_off[M];
         OC_CHECK(L.dim.upload(L.h_dim.data(), M));
-        OC_CHECK(L.off.upload(L.h_off.data(), M + 1));
+        return L.off.upload(L.h_off.data(), M + 1);
+    };
+    for (int m = 0; m < M; ++m) dims[m] = 2 * g->h_n[m] + 1;
+    OC_CHECK(tables(g->levels[0]));
+    for (int m = 0; m < M; ++m) dims[m] = g->h_n[m] + 1;
+    while (true) {
+        MgLevel &L = g->levels.back();
+        OC_CHECK(tables(L));
         OC_CHECK(L.A.alloc(static_cast<size_t>(L.nn) * 27 * 9));
         OC_CHECK(L.Dinv.alloc(static_cast<size_t>(L.nn) * 9));
         OC_CHECK(L.freed.alloc(static_cast<size_t>(L.nn) * 3));
         OC_CHECK(L.x.alloc(static_cast<size_t>(L.nn) * 3));
         OC_CHECK(L.b.alloc(static_cast<size_t>(L.nn) * 3));
-        OC_CHECK(L.r.alloc(static_cast<size_t>(L.nn) * 3));
         if (*std::max_element(dims.begin(), dims.end()) <= 3) break;
-        OC_CHECK(L.As.alloc(static_cast<size_t>(L.nn) * 27 * 9));
         for (int m = 0; m < M; ++m) dims[m] = (dims[m] - 1 + 1) / 2 + 1;  // n -> ceil(n/2)
         g->levels.emplace_back();
+    }
+    for (size_t l = 0; l + 1 < g->levels.size(); ++l) {
+        MgLevel &F = g->levels[l], &C = g->levels[l + 1];
+        std::vector<int64_t> first(static_cast<size_t>(M) + 1, 0);
+        for (int m = 0; m < M; ++m) {
+            const int64_t X = product_before(F.h_dim[m]);
+            first[m + 1] = first[m] + X * X * X;
+        }
+        DevBuf<int64_t> first_d;
+        OC_CHECK(first_d.upload(first.data(), first.size()));
+        OC_CHECK(F.up.alloc(static_cast<size_t>(first[M]) * 9));
+        OC_CHECK(F.nodes.alloc(F.nn));
+        mg_nodes_kernel<<<static_cast<unsigned>((F.nn + 255) / 256), 256, 0, runtime().stream>>>(
+            M, F.dim.ptr, F.off.ptr, C.dim.ptr, C.off.ptr, first_d.ptr, F.nn, F.nodes.ptr);
+        OC_HIP_CHECK(hipGetLastError());
+        OC_HIP_CHECK(hipStreamSynchronize(runtime().stream));  // first_d is read
+        if (l == 0) continue;
+        OC_CHECK(F.own.alloc(static_cast<size_t>(F.nn) * 27 * 9));
+        OC_CHECK(F.down.alloc(static_cast<size_t>(C.nn) * 125 * 9));
     }
     int maxnd = 0;
     for (int m = 0; m < M; ++m) maxnd = std::max(maxnd, 3 * dims[m] * dims[m] * dims[m]);
     if (maxnd > 81) return set_error(OC_ERR_UNSUPPORTED, "coarsest multigrid level too large");
     g->coarse_stride = maxnd * maxnd;
     OC_CHECK(g->coarse_inv.alloc(static_cast<size_t>(M) * g->coarse_stride));
-    std::vector<int64_t> ap_off(static_cast<size_t>(M) + 1, 0);
-    for (int m = 0; m < M; ++m) {
-        const int64_t X = 5 * static_cast<int64_t>(g->h_n[m]) + 3;
-        ap_off[m + 1] = ap_off[m] + X * X * X;
-    }
-    OC_CHECK(g->ap_off.upload(ap_off.data(), ap_off.size()));
-    OC_CHECK(g->ap.alloc(static_cast<size_t>(ap_off[M]) * 9));
-    OC_CHECK(g->nodes.alloc(s.n_nodes));
-    mg_nodes_kernel<<<static_cast<unsigned>((s.n_nodes + 255) / 256), 256, 0, runtime().stream>>>(
-        M, g->n.ptr, s.q_off.ptr, g->ap_off.ptr, g->levels[1].off.ptr, s.n_nodes, g->nodes.ptr);
-    OC_HIP_CHECK(hipGetLastError());
     OC_CHECK(g->r0.alloc(static_cast<size_t>(3) * s.n_nodes));
     OC_CHECK(g->t0.alloc(static_cast<size_t>(3) * s.n_nodes));
     OC_CHECK(g->x0.alloc(static_cast<size_t>(3) * s.n_nodes));
@@ -1407,5 +1359,9 @@ extern "C" int oc_multigrid_options_set(oc_equations_set h, int pre_sweeps, int 
     h->s.mg->pre = pre_sweeps;
     h->s.mg->post = post_sweeps;
     h->s.mg->omega = omega;
+    if (h->s.step_graph) {  // its multigrid setup holds the former omega
+        (void)hipGraphExecDestroy(h->s.step_graph);
+        h->s.step_graph = nullptr;
+    }
     return OC_NO_ERROR;
 }
