@@ -133,6 +133,8 @@ struct Multigrid {
     DevBuf<int32_t> n;
     std::vector<MgLevel> levels;          // levels[0]: the triquadratic lattice, tables and A P0 only
     DevBuf<float> ap_sp;                  // A P0 in FP32, for an FP32 Jacobian's V-cycle
+    DevBuf<double> bt;                    // the displacement rows' pressure entries by the same slots, 3 rows a node,
+    DevBuf<float> bt_sp;                  // in the Jacobian's precision
     DevBuf<double> t0, r0, x0;            // level-0 scratch (3*n_nodes each)
     DevBuf<double> coarse_inv;            // per mesh dense inverse of the coarsest level
     int coarse_stride = 0;                // (max DOFs per mesh at the coarsest level)^2
@@ -337,7 +339,7 @@ int launch_schur_mass(EquationsSet &s, double *inv_p);
 // `precision`; apply z_u = V-cycle(t) for the displacement block
 int mg_prepare(EquationsSet &s, int precision, bool *made);
 int mg_setup(EquationsSet &s, int precision);
-int mg_apply(EquationsSet &s, int precision, const double *t, double *z);
+int mg_apply(EquationsSet &s, int precision, const double *r, const double *inv_p, const double *scale, double *z);
 // pressure-column starts and the node-row layout check (oc_solver.hip)
 int prepare_node_rows(EquationsSet &s);
 // the packed bf16 displacement block's structure (uu_off, uu_col) and value

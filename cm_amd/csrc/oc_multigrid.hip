@@ -101,14 +101,16 @@ mg_nodes_kernel(int M, const int *__restrict__ dim_f, const int *__restrict__ of
 // whole runs, and lane s adds the up to 27 neighbours that interpolate from
 // its trilinear node, in z, y, x order.  Every later use of the interpolated
 // operator reads this quarter of the matrix (15.6 blocks a node against 64).
+// The rows' pressure entries go beside it, packed by the same slots.
 constexpr int kProductNodes = 4;  // per block: 36 KB of FP64 values, four blocks per CU
 
 template <typename VT>
 __global__ void __launch_bounds__(32 * kProductNodes)
 q1_product_kernel(int M, const int *__restrict__ n_mesh, const int *__restrict__ q_off,
                   const MgNode *__restrict__ nodes, int nq, const int64_t *__restrict__ row_ptr,
-                  const int *__restrict__ col_idx, const VT *__restrict__ vals, const uint8_t *__restrict__ free_mask,
-                  double *__restrict__ ap, float *__restrict__ ap_sp)
+                  const int64_t *__restrict__ pstart, const int *__restrict__ col_idx, const VT *__restrict__ vals,
+                  const uint8_t *__restrict__ free_mask, double *__restrict__ ap, float *__restrict__ ap_sp,
+                  VT *__restrict__ bt)
 {
     __shared__ VT s_run[kProductNodes][9 * 125];
     const int lane = threadIdx.x & 31, grp = threadIdx.x >> 5;
@@ -166,7 +168,18 @@ q1_product_kernel(int M, const int *__restrict__ n_mesh, const int *__restrict__
 #pragma unroll
                     for (int rc = 0; rc < 9; ++rc) acc[rc] += w * static_cast<double>(v[rc * deg]);
                 }
-    const int64_t at = 9 * nodes[q].first + lane;
+    const int64_t first = nodes[q].first, at = 9 * first + lane;
+    // the pressure columns are the trilinear nodes of the grid among the slots,
+    // x fastest: slot s of row r at 3 first + r S + s of bt
+    int plo[3], plen[3];
+    for (int k = 0; k < 3; ++k) {
+        plo[k] = max(product_lo(i[k]), 0);
+        plen[k] = min(product_lo(i[k]) + product_count(i[k]), n + 1) - plo[k];
+    }
+    const int pp = (K[0] - plo[0]) + plen[0] * ((K[1] - plo[1]) + plen[1] * (K[2] - plo[2]));
+#pragma unroll
+    for (int r = 0; r < 3; ++r)
+        bt[3 * first + r * S + lane] = inside ? vals[pstart[r * nq64 + q] + pp] : static_cast<VT>(0);
 #pragma unroll
     for (int rc = 0; rc < 9; ++rc) {
         ap[at + rc * S] = acc[rc];
@@ -598,8 +611,8 @@ __global__ void __launch_bounds__(256)
 uu_node_bf16_kernel(int nq, const int64_t *__restrict__ uu_off, const int *__restrict__ uu_col,
                     const uint16_t *__restrict__ uu_bf, const uint8_t *__restrict__ free_mask,
                     const double *__restrict__ b, const float4 *__restrict__ x4, const double *__restrict__ x,
-                    const double *__restrict__ inv_u, double omega, double *__restrict__ out,
-                    float *__restrict__ out4)
+                    const double *__restrict__ inv_u, double omega, const double *__restrict__ scale,
+                    double *__restrict__ out, float *__restrict__ out4)
 {
     const int lane = threadIdx.x % kLanes;
     const int64_t xb = xcd_block(blockIdx.x, gridDim.x);
@@ -664,7 +677,7 @@ uu_node_bf16_kernel(int nq, const int64_t *__restrict__ uu_off, const int *__res
         const double *o = inv_u + static_cast<int64_t>(i) * 9 + 3 * lane;
         const int64_t row = lane * nq64 + i;
         const double xn = x[row] + omega * (o[0] * r0 + o[1] * r1 + o[2] * r2);
-        out[row] = xn;
+        out[row] = scale ? scale[row] * xn : xn;
         if (out4) out4[4 * static_cast<int64_t>(i) + lane] = static_cast<float>(xn);
     }
 }
@@ -680,7 +693,7 @@ uu_node_residual_kernel(int nq, const int64_t *__restrict__ row_ptr, const int64
                         const int *__restrict__ col_idx, const VT *__restrict__ vals,
                         const uint8_t *__restrict__ free_mask, const double *__restrict__ b,
                         const double *__restrict__ x, const double *__restrict__ inv_u, double omega,
-                        double *__restrict__ out)
+                        const double *__restrict__ scale, double *__restrict__ out)
 {
     const int lane = threadIdx.x % kLanes;
     const int64_t xb = xcd_block(blockIdx.x, gridDim.x);
@@ -710,7 +723,8 @@ uu_node_residual_kernel(int nq, const int64_t *__restrict__ row_ptr, const int64
         const double r2 = free_mask[2 * nq64 + i] ? b[2 * nq64 + i] - a2 : 0.0;
         const double *o = inv_u + static_cast<int64_t>(i) * 9 + 3 * lane;
         const int64_t row = lane * nq64 + i;
-        out[row] = x[row] + omega * (o[0] * r0 + o[1] * r1 + o[2] * r2);
+        const double xn = x[row] + omega * (o[0] * r0 + o[1] * r1 + o[2] * r2);
+        out[row] = scale ? scale[row] * xn : xn;
     }
 }
 
@@ -722,7 +736,7 @@ __global__ void __launch_bounds__(256)
 uu_flat_kernel(int nq, const int64_t *__restrict__ row_ptr, const int64_t *__restrict__ pstart,
                const int *__restrict__ col_idx, const VT *__restrict__ vals, const uint8_t *__restrict__ free_mask,
                const double *__restrict__ b, const double *__restrict__ x, const double *__restrict__ inv_u,
-               double omega, double *__restrict__ out)
+               double omega, const double *__restrict__ scale, double *__restrict__ out)
 {
     __shared__ double s_x[4][kFlatLds];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -742,26 +756,70 @@ uu_flat_kernel(int nq, const int64_t *__restrict__ row_ptr, const int64_t *__res
     const double r0 = __shfl(r, 0), r1 = __shfl(r, 16), r2 = __shfl(r, 32);
     if (!mine) return;
     const double *o = inv_u + static_cast<int64_t>(i) * 9 + 3 * c;
-    out[row] = x[row] + omega * (o[0] * r0 + o[1] * r1 + o[2] * r2);
+    const double xn = x[row] + omega * (o[0] * r0 + o[1] * r1 + o[2] * r2);
+    out[row] = scale ? scale[row] * xn : xn;
 }
 
-// level 0: x = omega Kblock^-1 r, component-major (and, with x4, its FP32 node
-// quadruples for the bf16 passes)
-__global__ void __launch_bounds__(256) q2_jacobi_kernel(int nq, const double *__restrict__ inv_u,
-                                                       const double *__restrict__ r, double *__restrict__ x,
-                                                       double omega, float *__restrict__ x4)
+// The V-cycle's start: z_p = scale inv_p .* r_p, t = r_u - B^T (inv_p .* r_p) on
+// free rows (0 on fixed ones) and the first smoothing step x = omega Kblock^-1 t
+// from zero (and, with x4, its FP32 node quadruples for the bf16 passes).  A
+// group of 8 lanes per node, lane by pressure neighbour as in q1_correct_kernel:
+// the packed B^T needs no columns and its lines hold nothing else, where the
+// CSR rows' ends are 16 entries in lines of 32.  At 32^3 with FP32 values 39 us
+// against 57 + 9 for the product from the CSR and the step (and 5 for the
+// scaling of z); 16^3 in FP64 9.1 against 10.3 + 4.6 (and 4.7).
+template <typename VT>
+__global__ void __launch_bounds__(256)
+mg_start_kernel(int nq, int nl, const MgNode *__restrict__ nodes, const VT *__restrict__ bt,
+                const double *__restrict__ inv_p, const double *__restrict__ r, const double *__restrict__ scale,
+                const uint8_t *__restrict__ free_mask, const double *__restrict__ inv_u, double omega,
+                double *__restrict__ z, double *__restrict__ t, double *__restrict__ x, float *__restrict__ x4)
 {
-    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < nq; i += gridDim.x * blockDim.x) {
-        const double *o = inv_u + static_cast<int64_t>(i) * 9;
-        const double r0 = r[i], r1 = r[nq + i], r2 = r[2 * static_cast<int64_t>(nq) + i];
-        const double d[3] = {o[0] * r0 + o[1] * r1 + o[2] * r2, o[3] * r0 + o[4] * r1 + o[5] * r2,
-                             o[6] * r0 + o[7] * r1 + o[8] * r2};
-        for (int c = 0; c < 3; ++c) {
-            const double xn = omega * d[c];
-            x[static_cast<int64_t>(c) * nq + i] = xn;
-            if (x4) x4[4 * static_cast<int64_t>(i) + c] = static_cast<float>(xn);
-        }
+    constexpr int kLanes = 8, kRounds = 4;  // 27 slots at most
+    const int lane = threadIdx.x % kLanes;
+    const int64_t xb = xcd_block(blockIdx.x, gridDim.x);
+    const int q = static_cast<int>((xb * blockDim.x + threadIdx.x) / kLanes);
+    if (q >= nq) return;  // whole groups
+    const int64_t nq64 = nq;
+    const double *rp = r + 3 * nq64;
+    if (q < nl && lane == kLanes - 1) z[3 * nq64 + q] = scale[3 * nq64 + q] * (inv_p[q] * rp[q]);
+    const MgNode nd = nodes[q];
+    const int N = static_cast<int>(nd.bits >> 16);
+    const bool odd[3] = {(nd.bits & 1) != 0, (nd.bits & 2) != 0, (nd.bits & 4) != 0};
+    const int cx = odd[0] ? 2 : 3, cy = odd[1] ? 2 : 3, cz = odd[2] ? 2 : 3, S = cx * cy * cz;
+    const VT *a = bt + 3 * nd.first;
+    double v[4] = {0, 0, 0, 0};
+#pragma unroll
+    for (int u = 0; u < kRounds; ++u) {
+        const int s = lane + u * kLanes;
+        if (s >= S) break;
+        const int yz = div_count(s, cx), sz = div_count(yz, cy), k[3] = {s - cx * yz, yz - cy * sz, sz};
+        bool inside = true;
+#pragma unroll
+        for (int d = 0; d < 3; ++d)
+            inside = inside && !(k[d] == 0 && (nd.bits >> (3 + 2 * d) & 1)) && !(k[d] == 2 && (nd.bits >> (4 + 2 * d) & 1));
+        const int l = inside ? nd.lo + k[0] + N * (k[1] + N * k[2]) : 0;
+        const double zp = inside ? inv_p[l] * rp[l] : 0.0;
+#pragma unroll
+        for (int c = 0; c < 3; ++c) v[c] += static_cast<double>(a[c * S + s]) * zp;
     }
+    // lanes 2c and 2c + 1 of the group are left with the total of v[c]
+    const bool h4 = lane & 4, h2 = lane & 2;
+    double f[2];
+#pragma unroll
+    for (int k = 0; k < 2; ++k) f[k] = (h4 ? v[k + 2] : v[k]) + __shfl_xor(h4 ? v[k] : v[k + 2], 4, kLanes);
+    double sum = (h2 ? f[1] : f[0]) + __shfl_xor(h2 ? f[0] : f[1], 2, kLanes);
+    sum += __shfl_xor(sum, 1, kLanes);
+    const int c = lane >> 1;
+    const int64_t row = c * nq64 + q;
+    const double tc = c < 3 && free_mask[row] ? r[row] - sum : 0.0;
+    const double t0 = __shfl(tc, 0, kLanes), t1 = __shfl(tc, 2, kLanes), t2 = __shfl(tc, 4, kLanes);
+    if (c >= 3 || (lane & 1)) return;
+    const double *o = inv_u + static_cast<int64_t>(q) * 9 + 3 * c;
+    const double xn = omega * (o[0] * t0 + o[1] * t1 + o[2] * t2);
+    t[row] = tc;
+    x[row] = xn;
+    if (x4) x4[4 * static_cast<int64_t>(q) + c] = static_cast<float>(xn);
 }
 
 // level 0 -> 1 restriction b1 = P0^T r0 (r0 is zero on fixed DOFs)
@@ -814,7 +872,8 @@ template <typename VT>
 __global__ void __launch_bounds__(256)
 q1_correct_kernel(int nq, const MgNode *__restrict__ nodes, const VT *__restrict__ ap, const double *__restrict__ e,
                   const uint8_t *__restrict__ free_mask, const double *__restrict__ r0,
-                  const double *__restrict__ inv_u, double omega, double *__restrict__ x, float *__restrict__ x4)
+                  const double *__restrict__ inv_u, double omega, const double *__restrict__ scale,
+                  double *__restrict__ x, float *__restrict__ x4)
 {
     constexpr int kLanes = 8, kRounds = 4;  // 27 slots at most
     const int lane = threadIdx.x % kLanes;
@@ -866,7 +925,7 @@ q1_correct_kernel(int nq, const MgNode *__restrict__ nodes, const VT *__restrict
     if (lane >= 3) return;
     const double *o = inv_u + static_cast<int64_t>(q) * 9 + 3 * lane;
     const double xn = x[row] + (free_mask[row] ? pe : 0.0) + omega * (o[0] * d0 + o[1] * d1 + o[2] * d2);
-    x[row] = xn;
+    x[row] = scale ? scale[row] * xn : xn;
     if (x4) x4[4 * static_cast<int64_t>(q) + lane] = static_cast<float>(xn);
 }
 
@@ -981,12 +1040,17 @@ int mg_prepare(EquationsSet &s, int precision, bool *made)
 {
     *made = false;
     if (s.node_rows != 1) return set_error(OC_ERR_UNSUPPORTED, "the multigrid preconditioner needs node rows");
-    if (precision != OC_FP32) return OC_NO_ERROR;
     Multigrid &g = *s.mg;
-    *made = !s.uu_bf.ptr || !g.ap_sp.ptr;
+    const size_t blocks = g.levels[0].up.n / 9;
+    if (precision != OC_FP32) {
+        *made = !g.bt.ptr;
+        return g.bt.ptr ? OC_NO_ERROR : g.bt.alloc(blocks * 3);
+    }
+    *made = !s.uu_bf.ptr || !g.ap_sp.ptr || !g.bt_sp.ptr;
     if (!s.values_sp.ptr) OC_CHECK(s.values_sp.alloc(s.nnz));
     OC_CHECK(prepare_uu_bf16(s));
-    if (!g.ap_sp.ptr) OC_CHECK(g.ap_sp.alloc(g.levels[0].up.n));
+    if (!g.ap_sp.ptr) OC_CHECK(g.ap_sp.alloc(blocks * 9));
+    if (!g.bt_sp.ptr) OC_CHECK(g.bt_sp.alloc(blocks * 3));
     return OC_NO_ERROR;
 }
 
@@ -1000,12 +1064,12 @@ int mg_setup(EquationsSet &s, int precision)
     MgLevel &L0 = g.levels[0], &L1 = g.levels[1];
     if (precision == OC_FP64)
         q1_product_kernel<double><<<gp, 32 * kProductNodes, 0, rt.stream>>>(
-            M, g.n.ptr, s.q_off.ptr, L0.nodes.ptr, nq, s.row_ptr.ptr, s.col_idx.ptr, s.values.ptr, s.free_mask.ptr,
-            L0.up.ptr, nullptr);
+            M, g.n.ptr, s.q_off.ptr, L0.nodes.ptr, nq, s.row_ptr.ptr, s.pstart.ptr, s.col_idx.ptr, s.values.ptr,
+            s.free_mask.ptr, L0.up.ptr, nullptr, g.bt.ptr);
     else
         q1_product_kernel<float><<<gp, 32 * kProductNodes, 0, rt.stream>>>(
-            M, g.n.ptr, s.q_off.ptr, L0.nodes.ptr, nq, s.row_ptr.ptr, s.col_idx.ptr, s.values_sp.ptr, s.free_mask.ptr,
-            L0.up.ptr, g.ap_sp.ptr);
+            M, g.n.ptr, s.q_off.ptr, L0.nodes.ptr, nq, s.row_ptr.ptr, s.pstart.ptr, s.col_idx.ptr, s.values_sp.ptr,
+            s.free_mask.ptr, L0.up.ptr, g.ap_sp.ptr, g.bt_sp.ptr);
     OC_HIP_CHECK(hipGetLastError());
     if (precision == OC_FP32) OC_CHECK(launch_uu_pack(s));
     coarse_stencil_kernel<<<group_grid(L1.nn), 256, 0, rt.stream>>>(M, L0.dim.ptr, L0.off.ptr, L1.dim.ptr, L1.off.ptr,
@@ -1052,7 +1116,7 @@ constexpr int kNodeVariantLanes[kNodeVariants] = {32, 32, 16, 16, 64};
 
 template <typename VT, int kSweep>
 static int launch_uu_node(int variant, int nq, const EquationsSet &s, const VT *vals, const double *b,
-                          const double *x, const double *inv_u, double omega, double *out)
+                          const double *x, const double *inv_u, double omega, const double *scale, double *out)
 {
     Runtime &rt = runtime();
     // one wavefront per node for FP64 values where the rows fit
@@ -1063,14 +1127,14 @@ static int launch_uu_node(int variant, int nq, const EquationsSet &s, const VT *
 #define OC_UU_NODE(L, U)                                                                                       \
     uu_node_residual_kernel<VT, L, kSweep, U><<<grid, 256, 0, rt.stream>>>(nq, s.row_ptr.ptr, s.pstart.ptr,   \
                                                                          s.col_idx.ptr, vals, s.free_mask.ptr, \
-                                                                         b, x, inv_u, omega, out)
+                                                                         b, x, inv_u, omega, scale, out)
     switch (variant) {
     case 1: OC_UU_NODE(32, 2); break;
     case 2: OC_UU_NODE(16, 2); break;
     case 3: OC_UU_NODE(16, 4); break;
     case 4:
         uu_flat_kernel<VT, kSweep><<<grid, 256, 0, rt.stream>>>(nq, s.row_ptr.ptr, s.pstart.ptr, s.col_idx.ptr, vals,
-                                                               s.free_mask.ptr, b, x, inv_u, omega, out);
+                                                               s.free_mask.ptr, b, x, inv_u, omega, scale, out);
         break;
     default: OC_UU_NODE(32, 1); break;
     }
@@ -1088,7 +1152,8 @@ template <int kSweep>
 // here, into the first of the set's two quadruple buffers); out4: where a
 // sweep also writes its result's quadruples (nullptr: not written)
 static int launch_uu_bf16(int variant, const EquationsSet &s, const double *b, const double *x, const double *inv_u,
-                          double omega, double *out, const float *x4_in = nullptr, float *out4 = nullptr)
+                          double omega, const double *scale, double *out, const float *x4_in = nullptr,
+                          float *out4 = nullptr)
 {
     Runtime &rt = runtime();
     if (variant < 0 || variant >= kNodeVariants) variant = 0;
@@ -1101,7 +1166,8 @@ static int launch_uu_bf16(int variant, const EquationsSet &s, const double *b, c
     }
 #define OC_UU_BF16(L, Q)                                                                                          \
     uu_node_bf16_kernel<L, kSweep, Q><<<grid, 256, 0, rt.stream>>>(nq, s.uu_off.ptr, s.uu_col.ptr, s.uu_bf.ptr, \
-                                                                 s.free_mask.ptr, b, x4, x, inv_u, omega, out, out4)
+                                                                 s.free_mask.ptr, b, x4, x, inv_u, omega, scale, \
+                                                                 out, out4)
     switch (variant) {
     case 1: OC_UU_BF16(8, 1); break;
     case 2: OC_UU_BF16(32, 1); break;
@@ -1166,13 +1232,15 @@ int launch_smoother_residual(EquationsSet &s, int precision, int variant, const 
                                             : static_cast<const void *>(s.values.ptr);
     if (!s.free_mask.ptr || !s.pstart.ptr || !vals || !b || !x || !r)
         return set_error(OC_ERR_INVALID_ARGUMENT, "smoother residual: free-DOF mask, pressure starts or values missing");
-    if (precision == OC_FP32 && s.uu_bf.ptr) return launch_uu_bf16<0>(variant, s, b, x, nullptr, 0.0, r);
-    if (precision == OC_FP32) return launch_uu_node<float, 0>(variant, s.n_nodes, s, s.values_sp.ptr, b, x, nullptr, 0.0, r);
-    return launch_uu_node<double, 0>(variant, s.n_nodes, s, s.values.ptr, b, x, nullptr, 0.0, r);
+    if (precision == OC_FP32 && s.uu_bf.ptr) return launch_uu_bf16<0>(variant, s, b, x, nullptr, 0.0, nullptr, r);
+    if (precision == OC_FP32) return launch_uu_node<float, 0>(variant, s.n_nodes, s, s.values_sp.ptr, b, x, nullptr, 0.0,
+                                                                     nullptr, r);
+    return launch_uu_node<double, 0>(variant, s.n_nodes, s, s.values.ptr, b, x, nullptr, 0.0, nullptr, r);
 }
 
-// z (displacement part, component-major) = V-cycle applied to t
-int mg_apply(EquationsSet &s, int precision, const double *t, double *z)
+// z = scale .* (P^-1 r): z_p = inv_p .* r_p and the displacement part, component-
+// major, the V-cycle applied to r_u - B^T z_p
+int mg_apply(EquationsSet &s, int precision, const double *r, const double *inv_p, const double *scale, double *z)
 {
     Multigrid &g = *s.mg;
     Runtime &rt = runtime();
@@ -1189,24 +1257,31 @@ int mg_apply(EquationsSet &s, int precision, const double *t, double *z)
     // the last post-smoothing sweep in z.  The first post-smoothing sweep
     // comes with the coarse correction, in place.
     const int post = g.post;
-    double *cur = z, *other = g.x0.ptr;
+    double *t = g.t0.ptr, *cur = z, *other = g.x0.ptr;
     if ((std::max(g.pre - 1, 0) + std::max(post - 1, 0)) & 1) std::swap(cur, other);
-    auto sweep0 = [&]() -> int {
+    auto sweep0 = [&](const double *sc) -> int {
         if (bf)
-            OC_CHECK(launch_uu_bf16<1>(variant, s, t, cur, inv_u, g.omega, other, q4, q4_other));
+            OC_CHECK(launch_uu_bf16<1>(variant, s, t, cur, inv_u, g.omega, sc, other, q4, q4_other));
         else
-            OC_CHECK((launch_uu_node<double, 1>(variant, nq, s, s.values.ptr, t, cur, inv_u, g.omega, other)));
+            OC_CHECK((launch_uu_node<double, 1>(variant, nq, s, s.values.ptr, t, cur, inv_u, g.omega, sc, other)));
         std::swap(cur, other);
         std::swap(q4, q4_other);
         return OC_NO_ERROR;
     };
-    q2_jacobi_kernel<<<grid1(nq), 256, 0, rt.stream>>>(nq, inv_u, t, cur, g.omega, q4);
-    for (int k = 1; k < g.pre; ++k) OC_CHECK(sweep0());
-    if (bf)
-        OC_CHECK(launch_uu_bf16<0>(variant, s, t, cur, nullptr, 0.0, g.r0.ptr, q4));
-    else
-        OC_CHECK((launch_uu_node<double, 0>(variant, nq, s, s.values.ptr, t, cur, nullptr, 0.0, g.r0.ptr)));
     MgLevel &L0 = g.levels[0], &L1 = g.levels[1];
+    const unsigned gc = static_cast<unsigned>((static_cast<int64_t>(nq) * 8 + 255) / 256);
+    if (bf)
+        mg_start_kernel<float><<<gc, 256, 0, rt.stream>>>(nq, s.n_nodes_l, L0.nodes.ptr, g.bt_sp.ptr, inv_p, r, scale,
+                                                          s.free_mask.ptr, inv_u, g.omega, z, t, cur, q4);
+    else
+        mg_start_kernel<double><<<gc, 256, 0, rt.stream>>>(nq, s.n_nodes_l, L0.nodes.ptr, g.bt.ptr, inv_p, r, scale,
+                                                           s.free_mask.ptr, inv_u, g.omega, z, t, cur, nullptr);
+    OC_HIP_CHECK(hipGetLastError());
+    for (int k = 1; k < g.pre; ++k) OC_CHECK(sweep0(nullptr));
+    if (bf)
+        OC_CHECK(launch_uu_bf16<0>(variant, s, t, cur, nullptr, 0.0, nullptr, g.r0.ptr, q4));
+    else
+        OC_CHECK((launch_uu_node<double, 0>(variant, nq, s, s.values.ptr, t, cur, nullptr, 0.0, nullptr, g.r0.ptr)));
     restrict_q2_kernel<<<group_grid(L1.nn), 256, 0, rt.stream>>>(M, g.n.ptr, s.q_off.ptr, nq, L1.off.ptr, L1.nn,
                                                             L1.freed.ptr, g.r0.ptr, L1.b.ptr);
     OC_HIP_CHECK(hipGetLastError());
@@ -1228,16 +1303,16 @@ int mg_apply(EquationsSet &s, int precision, const double *t, double *z)
                                                                   C.x.ptr, F.x.ptr);
         OC_HIP_CHECK(hipGetLastError());
     }
-    const unsigned gc = static_cast<unsigned>((static_cast<int64_t>(nq) * 8 + 255) / 256);
     const double omega1 = post > 0 ? g.omega : 0.0;  // without post-smoothing only x + P0 e
+    const double *sc = post > 1 ? nullptr : scale;   // the last step scales z
     if (bf)
         q1_correct_kernel<float><<<gc, 256, 0, rt.stream>>>(nq, L0.nodes.ptr, g.ap_sp.ptr, L1.x.ptr, s.free_mask.ptr,
-                                                            g.r0.ptr, inv_u, omega1, cur, q4);
+                                                            g.r0.ptr, inv_u, omega1, sc, cur, q4);
     else
         q1_correct_kernel<double><<<gc, 256, 0, rt.stream>>>(nq, L0.nodes.ptr, L0.up.ptr, L1.x.ptr, s.free_mask.ptr,
-                                                             g.r0.ptr, inv_u, omega1, cur, nullptr);
+                                                             g.r0.ptr, inv_u, omega1, sc, cur, nullptr);
     OC_HIP_CHECK(hipGetLastError());
-    for (int k = 1; k < post; ++k) OC_CHECK(sweep0());
+    for (int k = 1; k < post; ++k) OC_CHECK(sweep0(k + 1 == post ? scale : nullptr));
     return OC_NO_ERROR;
 }
 

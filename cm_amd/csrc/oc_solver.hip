@@ -567,48 +567,6 @@ __global__ void __launch_bounds__(256) spmv_flat_kernel(int nq, int nl, const in
     }
 }
 
-// Pressure Jacobi z_p = inv_p .* r_p (written by the groups i < nl) and
-// t = r_u - B^T z_p on free displacement rows, 0 on fixed ones, by nodes; z_p
-// is formed again where B^T reads it, so one launch does both (nl <= nq)
-template <typename VT, int kLanes>
-__global__ void __launch_bounds__(256) schur_rhs_node_kernel(int nq, int nl, const int64_t *__restrict__ row_ptr,
-                                                            const int64_t *__restrict__ pstart,
-                                                            const int *__restrict__ col_idx,
-                                                            const VT *__restrict__ vals,
-                                                            const uint8_t *__restrict__ free_mask,
-                                                            const double *__restrict__ inv_p,
-                                                            const double *__restrict__ r, double *__restrict__ z,
-                                                            double *__restrict__ t)
-{
-    const int lane = threadIdx.x % kLanes;
-    const int64_t xb = xcd_block(blockIdx.x, gridDim.x);
-    const int i = static_cast<int>((xb * blockDim.x + threadIdx.x) / kLanes);
-    if (i >= nq) return;  // whole groups
-    const int64_t nq64 = nq;
-    if (i < nl && lane == 0) z[3 * nq64 + i] = inv_p[i] * r[3 * nq64 + i];
-    const int64_t p0 = pstart[i], p1 = pstart[nq64 + i], p2 = pstart[2 * nq64 + i];
-    const int dp = static_cast<int>(row_ptr[i + 1] - p0);
-    double a0 = 0.0, a1 = 0.0, a2 = 0.0;
-    for (int p = lane; p < dp; p += kLanes) {
-        const int c = col_idx[p0 + p];
-        const double zp = inv_p[c - 3 * nq64] * r[c];
-        a0 += static_cast<double>(vals[p0 + p]) * zp;
-        a1 += static_cast<double>(vals[p1 + p]) * zp;
-        a2 += static_cast<double>(vals[p2 + p]) * zp;
-    }
-#pragma unroll
-    for (int o = kLanes / 2; o > 0; o >>= 1) {
-        a0 += __shfl_xor(a0, o, kLanes);
-        a1 += __shfl_xor(a1, o, kLanes);
-        a2 += __shfl_xor(a2, o, kLanes);
-    }
-    if (lane < 3) {
-        const int64_t row = lane * nq64 + i;
-        const double a = lane == 0 ? a0 : (lane == 1 ? a1 : a2);
-        t[row] = free_mask[row] ? r[row] - a : 0.0;
-    }
-}
-
 // ---- preconditioners ----------------------------------------------------------------
 template <typename VT>
 __device__ __forceinline__ double csr_entry_t(const int64_t *__restrict__ row_ptr, const int *__restrict__ col_idx,
@@ -748,30 +706,6 @@ __global__ void __launch_bounds__(256) triangular_u_kernel(int nq, const int64_t
     z[node] = o[0] * t[0] + o[1] * t[1] + o[2] * t[2];
     z[nq + node] = o[3] * t[0] + o[4] * t[1] + o[5] * t[2];
     z[2 * nq + node] = o[6] * t[0] + o[7] * t[1] + o[8] * t[2];
-}
-
-// t = r_u - B^T z_p on the free displacement rows (pressure columns start at
-// pstart[row]); 8 lanes per row, shuffle reduction in a fixed order
-template <typename VT>
-__global__ void __launch_bounds__(256) schur_rhs_kernel(int nu, const int64_t *__restrict__ row_ptr,
-                                                       const int64_t *__restrict__ pstart,
-                                                       const int *__restrict__ col_idx, const VT *__restrict__ vals,
-                                                       const uint8_t *__restrict__ free_mask,
-                                                       const double *__restrict__ r, const double *__restrict__ z,
-                                                       double *__restrict__ t)
-{
-    constexpr int kLanes = 8;
-    const int lane = threadIdx.x % kLanes;
-    const int row = static_cast<int>((static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x) / kLanes);
-    if (row >= nu) return;
-    const bool f = free_mask[row] != 0;
-    double acc = 0.0;
-    if (f)
-        for (int64_t k = pstart[row] + lane; k < row_ptr[row + 1]; k += kLanes)
-            acc += static_cast<double>(vals[k]) * z[col_idx[k]];
-#pragma unroll
-    for (int o = kLanes / 2; o > 0; o >>= 1) acc += __shfl_xor(acc, o, kLanes);
-    if (lane == 0) t[row] = f ? r[row] - acc : 0.0;
 }
 
 __global__ void __launch_bounds__(256) pressure_start_kernel(int n_u_rows, int first_p_col,
@@ -959,30 +893,7 @@ struct Krylov {
         } else {
             const int nq = s.n_nodes, nl = s.n_nodes_l;
             if (precond == OC_PRECONDITIONER_MULTIGRID) {
-                const bool nodes = s.node_rows == 1 && nl <= nq;
-                if (!nodes)
-                    apply_jacobi_kernel<<<grid_for(nl), 256, 0, rt.stream>>>(
-                        nl, inv_p, rin + 3 * static_cast<int64_t>(nq), zout + 3 * static_cast<int64_t>(nq));
-                const int nu = 3 * nq;
-                double *t = s.mg->t0.ptr;
-                const unsigned gs = grid_rows(static_cast<int64_t>(nu) * 8);
-                const unsigned gsn = grid_rows(static_cast<int64_t>(nq) * 16);
-                if (nodes && fp32)
-                    schur_rhs_node_kernel<float, 16><<<gsn, 256, 0, rt.stream>>>(
-                        nq, nl, s.row_ptr.ptr, pstart, s.col_idx.ptr, s.values_sp.ptr, s.free_mask.ptr, inv_p, rin,
-                        zout, t);
-                else if (nodes)
-                    schur_rhs_node_kernel<double, 16><<<gsn, 256, 0, rt.stream>>>(
-                        nq, nl, s.row_ptr.ptr, pstart, s.col_idx.ptr, s.values.ptr, s.free_mask.ptr, inv_p, rin,
-                        zout, t);
-                else if (fp32)
-                    schur_rhs_kernel<float><<<gs, 256, 0, rt.stream>>>(nu, s.row_ptr.ptr, pstart, s.col_idx.ptr,
-                                                                        s.values_sp.ptr, s.free_mask.ptr, rin, zout, t);
-                else
-                    schur_rhs_kernel<double><<<gs, 256, 0, rt.stream>>>(nu, s.row_ptr.ptr, pstart, s.col_idx.ptr,
-                                                                         s.values.ptr, s.free_mask.ptr, rin, zout, t);
-                OC_HIP_CHECK(hipGetLastError());
-                OC_CHECK(mg_apply(s, fp32 ? OC_FP32 : OC_FP64, t, zout));
+                return mg_apply(s, fp32 ? OC_FP32 : OC_FP64, rin, inv_p, s.iwgt.ptr, zout);
             } else if (precond == OC_PRECONDITIONER_BLOCK_TRIANGULAR) {
                 apply_jacobi_kernel<<<grid_for(nl), 256, 0, rt.stream>>>(nl, inv_p, rin + 3 * static_cast<int64_t>(nq),
                                                                          zout + 3 * static_cast<int64_t>(nq));
