@@ -37,71 +37,130 @@ enum GpField : int {
 
 constexpr int kGaussElemsPerBlock = 9;  // 9 elements x 27 Gauss points = 243 threads
 
-// Restates, per Gauss point, the interpolation/metrics/F/J block of the
-// Jacobian routine (:954-989) and FINITE_ELASTICITY_GAUSS_ELASTICITY_TENSOR
-// (:609-740).
-__global__ void __launch_bounds__(256)
-mr_gauss_kernel(int n_elements, const int *__restrict__ conn_q, const int *__restrict__ conn_l,
-                const double *__restrict__ coords, int nq, const double *__restrict__ dofs,
-                const double *__restrict__ mat, const BasisTables *__restrict__ T, double *__restrict__ rec)
+constexpr int kGaussThreads = 256;
+
+// The interpolation of nine elements at their Gauss points, one direction at a
+// time: a thread takes a field's 9 nodal values of one zeta plane of an element
+// to the 9 (xi, eta) points (value and both derivatives, in registers, with the
+// 1D functions as constants), then each Gauss point adds the three planes: 99
+// multiply-adds and 36 LDS reads a field and point row where the 27-node sums
+// of every point took 486 and 243 for all six fields.  Those reads bound both
+// kernels that use it (32,768 elements: residual 252 -> 63 us, records 120 -> 109
+// us of which the 368 MB they write take 70).
+struct ElementLds {
+    double nodal[kGaussElemsPerBlock * 6][27];      // X then z, by component
+    double plane[kGaussElemsPerBlock * 6 * 3][27];  // [.. 3 f + plane][kind * 9 + xi + 3 eta]: d/dxi, d/deta, value
+    double p[kGaussElemsPerBlock][8];
+};
+
+// Thread t = 27 le + g: kinematics and pressure of Gauss point g of the block's
+// element le; false where there is none.  With kFD launch element v is the pair
+// (v / 89, v % 89) and the column's DOF is raised by delta.
+template <bool kFD>
+__device__ __forceinline__ bool element_points(int n_elements, int e0, const int *__restrict__ conn_q,
+                                               const int *__restrict__ conn_l, const double *__restrict__ coords,
+                                               int nq, const double *__restrict__ dofs, double delta, ElementLds &s,
+                                               GaussKinematics &k, double *P)
 {
-    __shared__ double s_tab[kTabSize];
-    __shared__ double s_X[kGaussElemsPerBlock][81];
-    __shared__ double s_z[kGaussElemsPerBlock][81];
-    __shared__ double s_p[kGaussElemsPerBlock][8];
-    constexpr int kTabPer = (27 * 27 * 3 + 255) / 256;
-    constexpr int kNodePer = (kGaussElemsPerBlock * 81 + 255) / 256;
+    constexpr int kNodePer = (kGaussElemsPerBlock * 81 + kGaussThreads - 1) / kGaussThreads;
     const int t = threadIdx.x;
-    const int e0 = xcd_block(blockIdx.x, gridDim.x) * kGaussElemsPerBlock;
-    // all global loads are issued before the LDS writes: the table and the
-    // connectivity, then the nodal values they index
-    double tab[kTabPer];
-#pragma unroll
-    for (int i = 0; i < kTabPer; ++i) {  // [ni][n][g] <- quad27[(g*27 + n)*4 + 1 + ni]
-        const int k = t + 256 * i;
-        const int ni = k / 729, n = (k / 27) % 27, g = k % 27;
-        tab[i] = k < 27 * 27 * 3 ? T->quad27[(g * 27 + n) * 4 + 1 + ni] : 0.0;
-    }
+    // all global loads are issued before the LDS writes: the connectivity,
+    // then the nodal values it indexes
     int node[kNodePer];
 #pragma unroll
     for (int i = 0; i < kNodePer; ++i) {
-        const int k = t + 256 * i;
-        const int e = e0 + k / 81;
-        node[i] = (k < kGaussElemsPerBlock * 81 && e < n_elements) ? conn_q[e * 27 + k % 27] : -1;
+        const int j = t + kGaussThreads * i;
+        const int v = e0 + j / 81;
+        node[i] = (j < kGaussElemsPerBlock * 81 && v < n_elements) ? conn_q[(kFD ? v / 89 : v) * 27 + j % 27] : -1;
     }
-    const int pe = e0 + t / 8;
-    const int pnode = (t < kGaussElemsPerBlock * 8 && pe < n_elements) ? conn_l[pe * 8 + t % 8] : -1;
+    const int pv = e0 + t / 8;
+    const int pnode = (t < kGaussElemsPerBlock * 8 && pv < n_elements) ? conn_l[(kFD ? pv / 89 : pv) * 8 + t % 8] : -1;
     double xv[kNodePer], zv[kNodePer];
 #pragma unroll
     for (int i = 0; i < kNodePer; ++i) {
-        const int k = t + 256 * i, c = (k % 81) / 27;
+        const int c = ((t + kGaussThreads * i) % 81) / 27;
         xv[i] = node[i] >= 0 ? coords[static_cast<int64_t>(c) * nq + node[i]] : 0.0;
         zv[i] = node[i] >= 0 ? dofs[static_cast<int64_t>(c) * nq + node[i]] : 0.0;
     }
     const double pval = pnode >= 0 ? dofs[static_cast<int64_t>(3) * nq + pnode] : 0.0;
 #pragma unroll
-    for (int i = 0; i < kTabPer; ++i) {
-        const int k = t + 256 * i;
-        const int ni = k / 729, n = (k / 27) % 27, g = k % 27;
-        if (k < 27 * 27 * 3) s_tab[(ni * 27 + n) * kTabStride + g] = tab[i];
-    }
-#pragma unroll
     for (int i = 0; i < kNodePer; ++i) {
-        const int k = t + 256 * i;
+        const int j = t + kGaussThreads * i;
+        const int le = j / 81, r = j % 81;
         if (node[i] >= 0) {
-            s_X[k / 81][k % 81] = xv[i];
-            s_z[k / 81][k % 81] = zv[i];
+            s.nodal[6 * le + r / 27][r % 27] = xv[i];
+            s.nodal[6 * le + 3 + r / 27][r % 27] = zv[i] + ((kFD && (e0 + le) % 89 == r) ? delta : 0.0);
         }
     }
-    if (pnode >= 0) s_p[t / 8][t % 8] = pval;
+    if (pnode >= 0) s.p[t / 8][t % 8] = pval + ((kFD && pv % 89 == 81 + t % 8) ? delta : 0.0);
+    __syncthreads();
+    if (t < kGaussElemsPerBlock * 18) {
+        // only derivatives leave the planes: taken from the element's centre
+        // node the sums round with the element's size, not its distance from
+        // the origin
+        const double *u = s.nodal[t / 3] + 9 * (t % 3), centre = s.nodal[t / 3][13];
+        double v[3][3], d[3][3];  // [eta row][xi]: value, derivative
+#pragma unroll
+        for (int y = 0; y < 3; ++y) {
+            const double u0 = u[3 * y] - centre, u1 = u[3 * y + 1] - centre, u2 = u[3 * y + 2] - centre;
+#pragma unroll
+            for (int g = 0; g < 3; ++g) {
+                v[y][g] = kQuad[g][0] * u0 + kQuad[g][1] * u1 + kQuad[g][2] * u2;
+                d[y][g] = kQuadD[g][0] * u0 + kQuadD[g][1] * u1 + kQuadD[g][2] * u2;
+            }
+        }
+        double *o = s.plane[t];
+#pragma unroll
+        for (int h = 0; h < 3; ++h)
+#pragma unroll
+            for (int g = 0; g < 3; ++g) {
+                o[g + 3 * h] = kQuad[h][0] * d[0][g] + kQuad[h][1] * d[1][g] + kQuad[h][2] * d[2][g];
+                o[9 + g + 3 * h] = kQuadD[h][0] * v[0][g] + kQuadD[h][1] * v[1][g] + kQuadD[h][2] * v[2][g];
+                o[18 + g + 3 * h] = kQuad[h][0] * v[0][g] + kQuad[h][1] * v[1][g] + kQuad[h][2] * v[2][g];
+            }
+    }
     __syncthreads();
     const int le = t / 27, g = t % 27;
-    const int e = e0 + le;
-    if (t >= kGaussElemsPerBlock * 27 || e >= n_elements) return;
+    if (t >= kGaussElemsPerBlock * 27 || e0 + le >= n_elements) return false;
+    const int xy = g % 9, gz = g / 9;
+    double q[3], qd[3];
+#pragma unroll
+    for (int z = 0; z < 3; ++z) {
+        q[z] = pick3(gz, kQuad[0][z], kQuad[1][z], kQuad[2][z]);
+        qd[z] = pick3(gz, kQuadD[0][z], kQuadD[1][z], kQuadD[2][z]);
+    }
+    double dX[9], dz[9];
+#pragma unroll
+    for (int f = 0; f < 6; ++f) {
+        const double(*pl)[27] = s.plane + (6 * le + f) * 3;
+        double *o = (f < 3 ? dX : dz) + f % 3;
+        o[0] = q[0] * pl[0][xy] + q[1] * pl[1][xy] + q[2] * pl[2][xy];
+        o[3] = q[0] * pl[0][9 + xy] + q[1] * pl[1][9 + xy] + q[2] * pl[2][9 + xy];
+        o[6] = qd[0] * pl[0][18 + xy] + qd[1] * pl[1][18 + xy] + qd[2] * pl[2][18 + xy];
+    }
+    gauss_kinematics(dz, dX, k);
+    const double x1 = pick3(g % 3, kXi[0], kXi[1], kXi[2]), y1 = pick3(xy / 3, kXi[0], kXi[1], kXi[2]),
+                 z1 = pick3(gz, kXi[0], kXi[1], kXi[2]), x0 = 1.0 - x1, y0 = 1.0 - y1;
+    const double *p = s.p[le];
+    *P = (1.0 - z1) * (y0 * (x0 * p[0] + x1 * p[1]) + y1 * (x0 * p[2] + x1 * p[3])) +
+         z1 * (y0 * (x0 * p[4] + x1 * p[5]) + y1 * (x0 * p[6] + x1 * p[7]));
+    return true;
+}
+
+// Restates, per Gauss point, the interpolation/metrics/F/J block of the
+// Jacobian routine (:954-989) and FINITE_ELASTICITY_GAUSS_ELASTICITY_TENSOR
+// (:609-740).
+__global__ void __launch_bounds__(kGaussThreads)
+mr_gauss_kernel(int n_elements, const int *__restrict__ conn_q, const int *__restrict__ conn_l,
+                const double *__restrict__ coords, int nq, const double *__restrict__ dofs,
+                const double *__restrict__ mat, const BasisTables *__restrict__ T, double *__restrict__ rec)
+{
+    __shared__ ElementLds s;
+    const int e0 = xcd_block(blockIdx.x, gridDim.x) * kGaussElemsPerBlock;
+    const int e = e0 + static_cast<int>(threadIdx.x) / 27, g = threadIdx.x % 27;
     GaussKinematics k;
-    gauss_kinematics(s_tab, g, s_z[le], s_X[le], k);
-    double P = 0.0;
-    for (int n = 0; n < 8; ++n) P += T->lin27[(g * 8 + n) * 4] * s_p[le][n];
+    double P;
+    if (!element_points<false>(n_elements, e0, conn_q, conn_l, coords, nq, dofs, 0.0, s, k, &P)) return;
     rec += static_cast<int64_t>(e) * GP_NFIELDS * 27 + g;
 #pragma unroll
     for (int i = 0; i < 9; ++i) rec[(GP_DXIDZ + i) * 27] = k.dxidz[i];
@@ -262,7 +321,7 @@ int launch_mr_gauss(EquationsSet &s)
     Runtime &rt = runtime();
     const unsigned blocks = static_cast<unsigned>((s.n_elements + kGaussElemsPerBlock - 1) / kGaussElemsPerBlock);
     KernelTimer timer("mr_gauss_jacobian");
-    mr_gauss_kernel<<<blocks, 256, 0, rt.stream>>>(s.n_elements, s.conn.ptr, s.conn_l.ptr, s.coords.ptr, s.n_nodes,
+    mr_gauss_kernel<<<blocks, kGaussThreads, 0, rt.stream>>>(s.n_elements, s.conn.ptr, s.conn_l.ptr, s.coords.ptr, s.n_nodes,
                                                    s.dofs.ptr, s.mat.ptr, T, s.gp_records.ptr);
     OC_HIP_CHECK(hipGetLastError());
     return OC_NO_ERROR;
@@ -285,87 +344,35 @@ int launch_mr_gauss(EquationsSet &s)
 // column col of e's element matrix (R(x + delta e_col) - R(x)) / delta, R(x)
 // from relem (EquationsSet_FiniteElementJacobianEvaluateFD,
 // equations_set_routines.f90:3032-3150).
-// 320 threads: 243 evaluate the Gauss points, then each of the 9 x 35
-// residual work items has a thread of its own.
-constexpr int kResThreads = 320;
-
+// The sums over the Gauss points run one direction at a time as well: a thread
+// per (element, component, xi point, zeta node) adds the nine points of its xi
+// plane into the three eta nodes, one per (element, component, zeta and eta
+// node) adds the xi points; a thread per pressure entry.  48 LDS reads and 72
+// multiply-adds for three entries, where each entry's 27 terms took 12 and 9
+// apiece.
 template <bool kFD, int kSub>
-__global__ void __launch_bounds__(kResThreads)
+__global__ void __launch_bounds__(kGaussThreads)
 mr_residual_element_kernel(int n_elements, const int *__restrict__ conn_q, const int *__restrict__ conn_l,
                            const double *__restrict__ coords, int nq, const double *__restrict__ dofs,
                            const double *__restrict__ mat, const BasisTables *__restrict__ T,
                            double *__restrict__ relem, double delta, double *__restrict__ kfd)
 {
-    // The nodal values (X, z) are only read by the Gauss-point phase and the
-    // Gauss-point results (DXI_DX, JGW sigma, the pressure weight) only
-    // written after it, so they share LDS (the block stays under 64 KB).
-    constexpr int kNodal = 2 * kGaussElemsPerBlock * 81;
-    constexpr int kResults = 2 * kGaussElemsPerBlock * 9 * 27 + kGaussElemsPerBlock * 27;
-    __shared__ double s_tab[kTabSize];
-    __shared__ double s_p[kGaussElemsPerBlock][8];
-    __shared__ double s_u[kNodal > kResults ? kNodal : kResults];
-    double(*s_X)[81] = reinterpret_cast<double(*)[81]>(s_u);
-    double(*s_z)[81] = reinterpret_cast<double(*)[81]>(s_u + kGaussElemsPerBlock * 81);
-    double(*s_T)[9][27] = reinterpret_cast<double(*)[9][27]>(s_u);  // T(j, a): [3a + j][g]
-    double(*s_rp)[27] = reinterpret_cast<double(*)[27]>(s_u + kGaussElemsPerBlock * 9 * 27);
-    constexpr int kTabPer = (27 * 27 * 3 + kResThreads - 1) / kResThreads;
-    constexpr int kNodePer = (kGaussElemsPerBlock * 81 + kResThreads - 1) / kResThreads;
+    __shared__ ElementLds s;
+    // the Gauss points' results take the place of the planes they have read
+    double(*s_T)[27] = s.plane;                                    // [9 le + 3 a + j][g]
+    double(*s_rp)[27] = s.plane + kGaussElemsPerBlock * 9;         // [le][g]
+    double(*s_PQ)[6] = reinterpret_cast<double(*)[6]>(s.plane + kGaussElemsPerBlock * 10);
+    static_assert(kGaussElemsPerBlock * (10 * 27 + 27 * 6) <= kGaussElemsPerBlock * 18 * 27, "results fit the planes");
     const int t = threadIdx.x;
     const int e0 = xcd_block(blockIdx.x, gridDim.x) * kGaussElemsPerBlock;
-    // all global loads are issued before the LDS writes: the table and the
-    // connectivity, then the nodal values they index
-    double tab[kTabPer];
-#pragma unroll
-    for (int i = 0; i < kTabPer; ++i) {  // [ni][n][g] <- quad27[(g*27 + n)*4 + 1 + ni]
-        const int k = t + kResThreads * i;
-        const int ni = k / 729, n = (k / 27) % 27, g = k % 27;
-        tab[i] = k < 27 * 27 * 3 ? T->quad27[(g * 27 + n) * 4 + 1 + ni] : 0.0;
-    }
-    // n_elements counts launch elements (element-column pairs with kFD)
-    int node[kNodePer];
-#pragma unroll
-    for (int i = 0; i < kNodePer; ++i) {
-        const int k = t + kResThreads * i;
-        const int le = k / 81, n = k % 27, v = e0 + le;
-        node[i] = (k < kGaussElemsPerBlock * 81 && v < n_elements) ? conn_q[(kFD ? v / 89 : v) * 27 + n] : -1;
-    }
-    const int pv = e0 + t / 8;
-    const int pnode = (t < kGaussElemsPerBlock * 8 && pv < n_elements) ? conn_l[(kFD ? pv / 89 : pv) * 8 + t % 8] : -1;
-    double xv[kNodePer], zv[kNodePer];
-#pragma unroll
-    for (int i = 0; i < kNodePer; ++i) {
-        const int k = t + kResThreads * i, c = (k % 81) / 27;
-        xv[i] = node[i] >= 0 ? coords[static_cast<int64_t>(c) * nq + node[i]] : 0.0;
-        zv[i] = node[i] >= 0 ? dofs[static_cast<int64_t>(c) * nq + node[i]] : 0.0;
-    }
-    const double pval = pnode >= 0 ? dofs[static_cast<int64_t>(3) * nq + pnode] : 0.0;
-#pragma unroll
-    for (int i = 0; i < kTabPer; ++i) {
-        const int k = t + kResThreads * i;
-        const int ni = k / 729, n = (k / 27) % 27, g = k % 27;
-        if (k < 27 * 27 * 3) s_tab[(ni * 27 + n) * kTabStride + g] = tab[i];
-    }
-#pragma unroll
-    for (int i = 0; i < kNodePer; ++i) {
-        const int k = t + kResThreads * i;
-        const int le = k / 81, r = k % 81;
-        if (node[i] >= 0) {
-            s_X[le][r] = xv[i];
-            s_z[le][r] = zv[i] + ((kFD && (e0 + le) % 89 == r) ? delta : 0.0);
-        }
-    }
-    if (pnode >= 0) s_p[t / 8][t % 8] = pval + ((kFD && pv % 89 == 81 + t % 8) ? delta : 0.0);
-    __syncthreads();
+    const int le = t / 27, g = t % 27, v = e0 + le;
     {
-        const int le = t / 27, g = t % 27;
-        const int v = e0 + le, e = kFD ? v / 89 : v;
-        const bool active = t < kGaussElemsPerBlock * 27 && v < n_elements;
+        GaussKinematics k;
+        double P;
+        const bool active = element_points<kFD>(n_elements, e0, conn_q, conn_l, coords, nq, dofs, delta, s, k, &P);
         double rT[9], rrp = 0.0;
         if (active) {
-            GaussKinematics k;
-            gauss_kinematics(s_tab, g, s_z[le], s_X[le], k);
-            double P = 0.0;
-            for (int n = 0; n < 8; ++n) P += T->lin27[(g * 8 + n) * 4] * s_p[le][n];
+            const int e = kFD ? v / 89 : v;
             double sigma[6], jgw, J;
             if (kSub == OC_INCOMPRESSIBLE_MOONEY_RIVLIN_SUBTYPE) {
                 // the 4-component residual loop of the subtype (:1654-1761):
@@ -386,47 +393,88 @@ mr_residual_element_kernel(int n_elements, const int *__restrict__ conn_q, const
                 }
             rrp = k.jx * T->w27[g] * (J - 1.0);
         }
-        __syncthreads();  // X and z consumed: their LDS takes the results
+        __syncthreads();
         if (active) {
-            for (int i = 0; i < 9; ++i) s_T[le][i][g] = rT[i];
+#pragma unroll
+            for (int i = 0; i < 9; ++i) s_T[9 * le + i][g] = rT[i];
             s_rp[le][g] = rrp;
         }
     }
     __syncthreads();
-    // one work item per (element, displacement node m), for its three
-    // component rows; then one item per pressure row
-    for (int w = t; w < kGaussElemsPerBlock * 35; w += kResThreads) {
-        const int le = w / 35, q = w % 35;
-        const int v = e0 + le;
-        if (v >= n_elements) continue;
-        double acc[3] = {0.0, 0.0, 0.0};
-        if (q < 27) {
-            const int m = q;
-#pragma unroll 3
-            for (int g = 0; g < 27; ++g) {
-                const double f[3] = {s_tab[(0 * 27 + m) * kTabStride + g], s_tab[(1 * 27 + m) * kTabStride + g],
-                                     s_tab[(2 * 27 + m) * kTabStride + g]};
+    const bool mine = t < kGaussElemsPerBlock * 27 && v < n_elements;
+    const int a = g / 9;
+    if (mine) {  // xi point g / 3 % 3, zeta node g % 3
+        const int gx = (g / 3) % 3, mz = g % 3;
+        const double q[3] = {pick3(mz, kQuad[0][0], kQuad[0][1], kQuad[0][2]),
+                             pick3(mz, kQuad[1][0], kQuad[1][1], kQuad[1][2]),
+                             pick3(mz, kQuad[2][0], kQuad[2][1], kQuad[2][2])};
+        const double qd[3] = {pick3(mz, kQuadD[0][0], kQuadD[0][1], kQuadD[0][2]),
+                              pick3(mz, kQuadD[1][0], kQuadD[1][1], kQuadD[1][2]),
+                              pick3(mz, kQuadD[2][0], kQuadD[2][1], kQuadD[2][2])};
+        const double(*T3)[27] = s_T + 9 * le + 3 * a;
+        double pq[6] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
 #pragma unroll
-                for (int a = 0; a < 3; ++a) {
-                    const double dot = fma(f[2], s_T[le][3 * a + 2][g], fma(f[1], s_T[le][3 * a + 1][g], f[0] * s_T[le][3 * a][g]));
-                    acc[a] = acc[a] + dot;
-                }
+        for (int h = 0; h < 3; ++h) {
+            const int i = gx + 3 * h;
+            const double ax = q[0] * T3[0][i] + q[1] * T3[0][i + 9] + q[2] * T3[0][i + 18];
+            const double ay = q[0] * T3[1][i] + q[1] * T3[1][i + 9] + q[2] * T3[1][i + 18];
+            const double az = qd[0] * T3[2][i] + qd[1] * T3[2][i + 9] + qd[2] * T3[2][i + 18];
+#pragma unroll
+            for (int my = 0; my < 3; ++my) {
+                pq[my] += kQuad[h][my] * az + kQuadD[h][my] * ay;
+                pq[3 + my] += kQuad[h][my] * ax;
             }
+        }
+#pragma unroll
+        for (int i = 0; i < 6; ++i) s_PQ[t][i] = pq[i];
+    }
+    __syncthreads();
+    const auto put = [&](int u, int r, double value) {
+        if (kFD) {
+            const int64_t e = u / 89, col = u % 89;
+            kfd[(e * 89 + kbuf_row(r)) * 89 + col] = (value - relem[e * 89 + r]) / delta;
         } else {
-            const int m = q - 27;
-#pragma unroll 1
-            for (int g = 0; g < 27; ++g) acc[0] = acc[0] + s_rp[le][g] * T->lin27[(g * 8 + m) * 4];
+            relem[static_cast<int64_t>(u) * 89 + r] = value;
         }
-        const int nr = q < 27 ? 3 : 1;
-        for (int a = 0; a < nr; ++a) {
-            const int r = q < 27 ? a * 27 + q : 81 + (q - 27);
-            if (kFD) {
-                const int64_t e = v / 89, col = v % 89;
-                kfd[(e * 89 + kbuf_row(r)) * 89 + col] = (acc[a] - relem[e * 89 + r]) / delta;
-            } else {
-                relem[static_cast<int64_t>(v) * 89 + r] = acc[a];
+    };
+    if (mine) {  // zeta node g / 3 % 3, eta node g % 3
+        const int mz = (g / 3) % 3, my = g % 3;
+        double p[3], q[3];
+#pragma unroll
+        for (int gx = 0; gx < 3; ++gx) {
+            const double *pq = s_PQ[27 * le + 9 * a + 3 * gx + mz];
+            p[gx] = pq[my];
+            q[gx] = pq[3 + my];
+        }
+#pragma unroll
+        for (int mx = 0; mx < 3; ++mx) {
+            double r = 0.0;
+#pragma unroll
+            for (int gx = 0; gx < 3; ++gx) r += kQuad[gx][mx] * p[gx] + kQuadD[gx][mx] * q[gx];
+            put(v, 27 * a + mx + 3 * my + 9 * mz, r);
+        }
+    }
+    // pressure entries, by the last threads first: they have less to do above
+    const int w = kGaussThreads - 1 - t;
+    if (w < kGaussElemsPerBlock * 8 && e0 + w / 8 < n_elements) {
+        const int m = w % 8;
+        double lx[3], ly[3], lz[3];
+#pragma unroll
+        for (int i = 0; i < 3; ++i) {
+            lx[i] = (m & 1) ? kXi[i] : 1.0 - kXi[i];
+            ly[i] = (m & 2) ? kXi[i] : 1.0 - kXi[i];
+            lz[i] = (m & 4) ? kXi[i] : 1.0 - kXi[i];
+        }
+        const double *rp = s_rp[w / 8];
+        double r = 0.0;
+#pragma unroll
+        for (int z = 0; z < 3; ++z)
+#pragma unroll
+            for (int y = 0; y < 3; ++y) {
+                const double *row = rp + 3 * y + 9 * z;
+                r += lz[z] * ly[y] * (lx[0] * row[0] + lx[1] * row[1] + lx[2] * row[2]);
             }
-        }
+        put(e0 + w / 8, 81 + m, r);
     }
 }
 
@@ -475,10 +523,10 @@ static int launch_residual_elements(const EquationsSet &s, unsigned blocks, cons
     Runtime &rt = runtime();
     const int nv = kFD ? s.n_elements * 89 : s.n_elements;
     if (s.subtype == OC_INCOMPRESSIBLE_MOONEY_RIVLIN_SUBTYPE)
-        mr_residual_element_kernel<kFD, OC_INCOMPRESSIBLE_MOONEY_RIVLIN_SUBTYPE><<<blocks, kResThreads, 0, rt.stream>>>(
+        mr_residual_element_kernel<kFD, OC_INCOMPRESSIBLE_MOONEY_RIVLIN_SUBTYPE><<<blocks, kGaussThreads, 0, rt.stream>>>(
             nv, s.conn.ptr, s.conn_l.ptr, s.coords.ptr, s.n_nodes, dofs, s.mat.ptr, T, relem, delta, kfd);
     else
-        mr_residual_element_kernel<kFD, OC_MOONEY_RIVLIN_SUBTYPE><<<blocks, kResThreads, 0, rt.stream>>>(
+        mr_residual_element_kernel<kFD, OC_MOONEY_RIVLIN_SUBTYPE><<<blocks, kGaussThreads, 0, rt.stream>>>(
             nv, s.conn.ptr, s.conn_l.ptr, s.coords.ptr, s.n_nodes, dofs, s.mat.ptr, T, relem, delta, kfd);
     OC_HIP_CHECK(hipGetLastError());
     return OC_NO_ERROR;

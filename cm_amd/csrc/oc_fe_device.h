@@ -111,39 +111,20 @@ struct GaussKinematics {
     double dxidz[9];
 };
 
-// Triquadratic first derivatives at the 27 Gauss points, transposed for LDS:
-// dphi_n/dxi_ni at g is tab[(ni * 27 + n) * kTabStride + g].  The odd stride
-// keeps both access patterns nearly free of bank conflicts: lanes that differ
-// in g (one thread per Gauss point) and lanes that differ in n.
-constexpr int kTabStride = 29;
-constexpr int kTabSize = 3 * 27 * kTabStride;
+// Quadratic Lagrange functions of [0, 1] and their derivatives at the three
+// Gauss points xi_g = (1 + eta)/2, eta = -sqrt(0.6), 0, sqrt(0.6): [g][node]
+constexpr double kEta = 0.7745966692414834;
+constexpr double kQuad[3][3] = {{0.3 + 0.5 * kEta, 0.4, 0.3 - 0.5 * kEta}, {0.0, 1.0, 0.0},
+                                {0.3 - 0.5 * kEta, 0.4, 0.3 + 0.5 * kEta}};
+constexpr double kQuadD[3][3] = {{-2.0 * kEta - 1.0, 4.0 * kEta, 1.0 - 2.0 * kEta}, {-1.0, 0.0, 1.0},
+                                 {2.0 * kEta - 1.0, -4.0 * kEta, 2.0 * kEta + 1.0}};
+constexpr double kXi[3] = {0.5 - 0.5 * kEta, 0.5, 0.5 + 0.5 * kEta};
+__device__ __forceinline__ double pick3(int i, double a, double b, double c) { return i == 0 ? a : (i == 1 ? b : c); }
 
-// ze, Xe: element parameters [c*27 + n]; tab: the transposed derivative table.
-__device__ __forceinline__ void gauss_kinematics(const double *tab, int g, const double *ze, const double *Xe,
-                                                 GaussKinematics &k)
+// dz, dX: [x + 3 ni], the derivatives of z_x and X_x along xi_ni
+__device__ __forceinline__ void gauss_kinematics(const double (&dz)[9], const double (&dX)[9], GaussKinematics &k)
 {
-    double dz[9], dX[9], dxidnu[9];
-    // one derivative direction at a time, the three components together (each
-    // sum still runs over n in ascending order); the loops are kept rolled so
-    // that the unrolled loads do not take hundreds of registers
-#pragma unroll 1
-    for (int ni = 0; ni < 3; ++ni) {
-        double sz[3] = {0.0, 0.0, 0.0}, sX[3] = {0.0, 0.0, 0.0};
-#pragma unroll 3
-        for (int n = 0; n < 27; ++n) {
-            const double f = tab[(ni * 27 + n) * kTabStride + g];
-#pragma unroll
-            for (int x = 0; x < 3; ++x) {
-                sz[x] += f * ze[x * 27 + n];
-                sX[x] += f * Xe[x * 27 + n];
-            }
-        }
-#pragma unroll
-        for (int x = 0; x < 3; ++x) {
-            dz[x + 3 * ni] = sz[x];
-            dX[x + 3 * ni] = sX[x];
-        }
-    }
+    double dxidnu[9];
     // volume Jacobians of COORDINATE_METRICS_CALCULATE (coordinate_routines.f90:
     // 647-840), sqrt|det(dx^T dx)|, taken as |det dx| from the inversions
     k.jz = fabs(invert3_rcp(dz, k.dxidz));
