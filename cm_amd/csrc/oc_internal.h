@@ -261,11 +261,9 @@ struct EquationsSet {
     DevBuf<double> arnoldi;     // Hessenberg factor, rotations and coefficients of the Arnoldi process
     // Krylov progress read back without a stream synchronisation: pinned,
     // mapped, coherent host memory the Arnoldi kernels write (kArnoldiHostSlots
-    // doubles, host and device addresses), and two timing-free events marking
-    // alternate iterations; made at the first solve, per set
+    // doubles, host and device addresses); made at the first solve, per set
     double *arnoldi_host = nullptr;
     double *arnoldi_host_dev = nullptr;
-    hipEvent_t arnoldi_events[2] = {};
     // Mooney-Rivlin sets: 1 when the displacement rows c*nq + i (c < 3) of
     // every node i hold three blocks of the same sorted neighbour nodes
     // (components 0, 1, 2) and then one common list of pressure columns, so
@@ -298,8 +296,6 @@ struct EquationsSet {
     ~EquationsSet()
     {
         if (step_graph) (void)hipGraphExecDestroy(step_graph);
-        for (hipEvent_t e : arnoldi_events)
-            if (e) (void)hipEventDestroy(e);
         if (arnoldi_host) (void)hipHostFree(arnoldi_host);
         delete mg;
     }
