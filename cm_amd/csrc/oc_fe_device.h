@@ -392,6 +392,27 @@ __device__ __forceinline__ void node_rows_uu(const int64_t (&s)[3], int deg, int
     }
 }
 
+// o = A^-1 of a nodal 3x3 block by cofactors, the identity where it is singular
+__device__ __forceinline__ void invert_block(const double (&A)[9], double *__restrict__ o)
+{
+    const double c00 = A[4] * A[8] - A[5] * A[7], c01 = A[5] * A[6] - A[3] * A[8], c02 = A[3] * A[7] - A[4] * A[6];
+    const double det = A[0] * c00 + A[1] * c01 + A[2] * c02;
+    if (fabs(det) < 1e-300) {
+        for (int i = 0; i < 9; ++i) o[i] = (i % 4 == 0) ? 1.0 : 0.0;
+        return;
+    }
+    const double id = 1.0 / det;
+    o[0] = c00 * id;
+    o[1] = (A[2] * A[7] - A[1] * A[8]) * id;
+    o[2] = (A[1] * A[5] - A[2] * A[4]) * id;
+    o[3] = c01 * id;
+    o[4] = (A[0] * A[8] - A[2] * A[6]) * id;
+    o[5] = (A[2] * A[3] - A[0] * A[5]) * id;
+    o[6] = c02 * id;
+    o[7] = (A[1] * A[6] - A[0] * A[7]) * id;
+    o[8] = (A[0] * A[4] - A[1] * A[3]) * id;
+}
+
 // A double moved between the lanes of a row of 16 by a DPP control
 template <int kCtrl>
 __device__ __forceinline__ double dpp_move(double v)

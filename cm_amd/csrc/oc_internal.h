@@ -334,7 +334,7 @@ int launch_schur_mass(EquationsSet &s, double *inv_p);
 // multigrid (oc_multigrid.hip): setup after a Jacobian assembly in
 // `precision`; apply z_u = V-cycle(t) for the displacement block
 int mg_prepare(EquationsSet &s, int precision, bool *made);
-int mg_setup(EquationsSet &s, int precision);
+int mg_setup(EquationsSet &s, int precision, double *inv_u, double *diag_u);
 int mg_apply(EquationsSet &s, int precision, const double *r, const double *inv_p, const double *scale, double *z);
 // pressure-column starts and the node-row layout check (oc_solver.hip)
 int prepare_node_rows(EquationsSet &s);

@@ -43,6 +43,16 @@ __device__ __forceinline__ int find_mesh(const int *__restrict__ off, int M, int
 
 __device__ __forceinline__ double lin_weight(int delta) { return delta == 0 ? 1.0 : 0.5; }
 
+// bf16 values: the upper 16 bits of an FP32 value, rounded to nearest even
+// (NaN kept quiet)
+__device__ __forceinline__ uint16_t bf16_round(float f)
+{
+    uint32_t u = __float_as_uint(f);
+    if ((u & 0x7fffffffu) > 0x7f800000u) return static_cast<uint16_t>((u >> 16) | 0x40u);
+    u += 0x7fffu + ((u >> 16) & 1u);
+    return static_cast<uint16_t>(u >> 16);
+}
+
 // ---- interpolation by blocks -------------------------------------------------------------
 // Node i = (ix, iy, iz) of a level's lattice couples, through its own row and
 // the interpolation, to the coarse nodes lo .. lo + c - 1 per direction: c = 3
@@ -101,7 +111,10 @@ mg_nodes_kernel(int M, const int *__restrict__ dim_f, const int *__restrict__ of
 // whole runs, and lane s adds the up to 27 neighbours that interpolate from
 // its trilinear node, in z, y, x order.  Every later use of the interpolated
 // operator reads this quarter of the matrix (15.6 blocks a node against 64).
-// The rows' pressure entries go beside it, packed by the same slots.
+// The rows' pressure entries go beside it, packed by the same slots, and from
+// the same reading of the matrix the nodal blocks' inverses and an FP32
+// Jacobian's bf16 copy: passes of their own took 282 and 382 us at 32^3, this
+// one went from 758 to 946.
 constexpr int kProductNodes = 4;  // per block: 36 KB of FP64 values, four blocks per CU
 
 template <typename VT>
@@ -110,7 +123,8 @@ q1_product_kernel(int M, const int *__restrict__ n_mesh, const int *__restrict__
                   const MgNode *__restrict__ nodes, int nq, const int64_t *__restrict__ row_ptr,
                   const int64_t *__restrict__ pstart, const int *__restrict__ col_idx, const VT *__restrict__ vals,
                   const uint8_t *__restrict__ free_mask, double *__restrict__ ap, float *__restrict__ ap_sp,
-                  VT *__restrict__ bt)
+                  VT *__restrict__ bt, const int64_t *__restrict__ uu_off, uint16_t *__restrict__ uu_bf,
+                  double *__restrict__ inv_u, double *__restrict__ diag_u)
 {
     __shared__ VT s_run[kProductNodes][9 * 125];
     const int lane = threadIdx.x & 31, grp = threadIdx.x >> 5;
@@ -147,27 +161,63 @@ q1_product_kernel(int M, const int *__restrict__ n_mesh, const int *__restrict__
     }
     __syncthreads();
     if (q >= nq) return;
+    if (sizeof(VT) == sizeof(float)) {  // four neighbours a lane; fixed DOFs' iterate is zero, so the mask is no matter
+        const int n4 = (deg + 3) >> 2;
+        uint2 *o = reinterpret_cast<uint2 *>(uu_bf + 9 * uu_off[q]);
+        if (lane < n4)
+#pragma unroll
+            for (int rc = 0; rc < 9; ++rc) {
+                uint32_t b[4];
+#pragma unroll
+                for (int n = 0; n < 4; ++n)
+                    b[n] = 4 * lane + n < deg ? bf16_round(static_cast<float>(run[rc * deg + 4 * lane + n])) : 0u;
+                o[rc * n4 + lane] = make_uint2(b[0] | (b[1] << 16), b[2] | (b[3] << 16));
+            }
+    }
+    if (lane == 31) {  // no slot's lane: the node's own block, fixed DOFs as the identity
+        const int own = (i[0] - blo[0]) + len[0] * ((i[1] - blo[1]) + len[1] * (i[2] - blo[2]));
+        double D[9];
+#pragma unroll
+        for (int rc = 0; rc < 9; ++rc) D[rc] = static_cast<double>(run[rc * deg + own]);
+#pragma unroll
+        for (int c = 0; c < 3; ++c) {
+            if (!free_mask[c * nq64 + q]) D[4 * c] = 1.0;
+            diag_u[c * nq64 + q] = D[4 * c];
+        }
+        invert_block(D, inv_u + static_cast<int64_t>(q) * 9);
+    }
     const int cx = product_count(i[0]), cy = product_count(i[1]), S = cx * cy * product_count(i[2]);
     if (lane >= S) return;
     const int K[3] = {product_lo(i[0]) + lane % cx, product_lo(i[1]) + (lane / cx) % cy,
                       product_lo(i[2]) + lane / (cx * cy)};
-    int lo[3], hi[3];
+    // per direction the first of three neighbours 2K - 1 .. 2K + 1, moved into the
+    // box, and their weights, zero outside it (the box is at least three wide)
+    int lo[3];
+    double w[3][3];
     bool inside = true;
     for (int k = 0; k < 3; ++k) {
-        lo[k] = max(2 * K[k] - 1, blo[k]);
-        hi[k] = min(2 * K[k] + 1, blo[k] + len[k] - 1);
         inside = inside && K[k] >= 0 && K[k] <= n;
+        lo[k] = min(max(2 * K[k] - 1 - blo[k], 0), len[k] - 3);
+        for (int d = 0; d < 3; ++d) {
+            const int off = blo[k] + lo[k] + d - 2 * K[k];
+            w[k][d] = off == 0 ? 1.0 : (off == 1 || off == -1 ? 0.5 : 0.0);
+        }
     }
     double acc[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
     if (inside)
-        for (int z = lo[2]; z <= hi[2]; ++z)
-            for (int y = lo[1]; y <= hi[1]; ++y)
-                for (int x = lo[0]; x <= hi[0]; ++x) {
-                    const double w = lin_weight(x - 2 * K[0]) * lin_weight(y - 2 * K[1]) * lin_weight(z - 2 * K[2]);
-                    const VT *v = run + (x - blo[0]) + len[0] * ((y - blo[1]) + len[1] * (z - blo[2]));
+#pragma unroll 1
+        for (int yz = 0; yz < 9; ++yz) {
+            const int y = yz % 3, z = yz / 3;
+            const double wy = y == 0 ? w[1][0] : (y == 1 ? w[1][1] : w[1][2]);
+            const double wyz = wy * (z == 0 ? w[2][0] : (z == 1 ? w[2][1] : w[2][2]));
+            const VT *v = run + lo[0] + len[0] * (lo[1] + y + len[1] * (lo[2] + z));
 #pragma unroll
-                    for (int rc = 0; rc < 9; ++rc) acc[rc] += w * static_cast<double>(v[rc * deg]);
-                }
+            for (int rc = 0; rc < 9; ++rc) {
+                const VT *u = v + rc * deg;
+                acc[rc] += wyz * (w[0][0] * static_cast<double>(u[0]) + w[0][1] * static_cast<double>(u[1]) +
+                                  w[0][2] * static_cast<double>(u[2]));
+            }
+        }
     const int64_t first = nodes[q].first, at = 9 * first + lane;
     // the pressure columns are the trilinear nodes of the grid among the slots,
     // x fastest: slot s of row r at 3 first + r S + s of bt
@@ -540,15 +590,6 @@ __global__ void __launch_bounds__(1024) coarse_inverse_kernel(int M, const int *
 }
 
 // ---- V-cycle kernels -------------------------------------------------------------------
-// bf16 values: the upper 16 bits of an FP32 value, rounded to nearest even
-// (NaN kept quiet)
-__device__ __forceinline__ uint16_t bf16_round(float f)
-{
-    uint32_t u = __float_as_uint(f);
-    if ((u & 0x7fffffffu) > 0x7f800000u) return static_cast<uint16_t>((u >> 16) | 0x40u);
-    u += 0x7fffu + ((u >> 16) & 1u);
-    return static_cast<uint16_t>(u >> 16);
-}
 
 // The packed bf16 copy of K_uu (EquationsSet::uu_bf): padded neighbour
 // counts, then the padded column lists, once per set
@@ -1071,7 +1112,7 @@ int mg_prepare(EquationsSet &s, int precision, bool *made)
     return OC_NO_ERROR;
 }
 
-int mg_setup(EquationsSet &s, int precision)
+int mg_setup(EquationsSet &s, int precision, double *inv_u, double *diag_u)
 {
     Multigrid &g = *s.mg;
     Runtime &rt = runtime();
@@ -1082,13 +1123,12 @@ int mg_setup(EquationsSet &s, int precision)
     if (precision == OC_FP64)
         q1_product_kernel<double><<<gp, 32 * kProductNodes, 0, rt.stream>>>(
             M, g.n.ptr, s.q_off.ptr, L0.nodes.ptr, nq, s.row_ptr.ptr, s.pstart.ptr, s.col_idx.ptr, s.values.ptr,
-            s.free_mask.ptr, L0.up.ptr, nullptr, g.bt.ptr);
+            s.free_mask.ptr, L0.up.ptr, nullptr, g.bt.ptr, nullptr, nullptr, inv_u, diag_u);
     else
         q1_product_kernel<float><<<gp, 32 * kProductNodes, 0, rt.stream>>>(
             M, g.n.ptr, s.q_off.ptr, L0.nodes.ptr, nq, s.row_ptr.ptr, s.pstart.ptr, s.col_idx.ptr, s.values_sp.ptr,
-            s.free_mask.ptr, L0.up.ptr, g.ap_sp.ptr, g.bt_sp.ptr);
+            s.free_mask.ptr, L0.up.ptr, g.ap_sp.ptr, g.bt_sp.ptr, s.uu_off.ptr, s.uu_bf.ptr, inv_u, diag_u);
     OC_HIP_CHECK(hipGetLastError());
-    if (precision == OC_FP32) OC_CHECK(launch_uu_pack(s));
     coarse_stencil_kernel<<<group_grid(L1.nn), 256, 0, rt.stream>>>(M, L0.dim.ptr, L0.off.ptr, L1.dim.ptr, L1.off.ptr,
                                                                    L1.nn, L0.nodes.ptr, L0.up.ptr, L1.A.ptr);
     coincident_q2_kernel<<<grid1(L1.nn), 256, 0, rt.stream>>>(M, g.n.ptr, s.q_off.ptr, s.n_nodes, L1.off.ptr, L1.nn,

@@ -773,23 +773,7 @@ __global__ void __launch_bounds__(256) block_setup_kernel(int nq, const int64_t 
             A[a * 3 + b] = v;
         }
     for (int a = 0; a < 3; ++a) diag_u[a * nq + node] = A[a * 3 + a];
-    const double c00 = A[4] * A[8] - A[5] * A[7], c01 = A[5] * A[6] - A[3] * A[8], c02 = A[3] * A[7] - A[4] * A[6];
-    const double det = A[0] * c00 + A[1] * c01 + A[2] * c02;
-    double *o = inv + static_cast<int64_t>(node) * 9;
-    if (fabs(det) < 1e-300) {
-        for (int i = 0; i < 9; ++i) o[i] = (i % 4 == 0) ? 1.0 : 0.0;
-        return;
-    }
-    const double id = 1.0 / det;
-    o[0] = c00 * id;
-    o[1] = (A[2] * A[7] - A[1] * A[8]) * id;
-    o[2] = (A[1] * A[5] - A[2] * A[4]) * id;
-    o[3] = c01 * id;
-    o[4] = (A[0] * A[8] - A[2] * A[6]) * id;
-    o[5] = (A[2] * A[3] - A[0] * A[5]) * id;
-    o[6] = c02 * id;
-    o[7] = (A[1] * A[6] - A[0] * A[7]) * id;
-    o[8] = (A[0] * A[4] - A[1] * A[3]) * id;
+    invert_block(A, inv + static_cast<int64_t>(node) * 9);
 }
 
 // pressure rows: S_p = sum_j B_pj^2 / K_jj over free displacement columns
@@ -1010,10 +994,11 @@ struct Krylov {
             return OC_NO_ERROR;
         }
         const int nq = s.n_nodes, nl = s.n_nodes_l;
-        if (precond == OC_PRECONDITIONER_MULTIGRID) OC_CHECK(mg_setup(s, fp32 ? OC_FP32 : OC_FP64));
+        const bool mg = precond == OC_PRECONDITIONER_MULTIGRID;  // its setup forms the nodal blocks as well
+        if (mg) OC_CHECK(mg_setup(s, fp32 ? OC_FP32 : OC_FP64, inv_u, diag_u));
         const bool mass_schur = s.subtype == OC_MOONEY_RIVLIN_SUBTYPE && s.gp_records.ptr;
         if (fp32) {
-            block_setup_kernel<float><<<grid_rows(nq), 256, 0, rt.stream>>>(nq, s.row_ptr.ptr, s.col_idx.ptr,
+            if (!mg) block_setup_kernel<float><<<grid_rows(nq), 256, 0, rt.stream>>>(nq, s.row_ptr.ptr, s.col_idx.ptr,
                                                                             s.values_sp.ptr, s.free_mask.ptr, inv_u,
                                                                             diag_u);
             if (mass_schur)
@@ -1023,7 +1008,7 @@ struct Krylov {
                                                                                 s.values_sp.ptr, s.free_mask.ptr, diag_u,
                                                                                 inv_p);
         } else {
-            block_setup_kernel<double><<<grid_rows(nq), 256, 0, rt.stream>>>(nq, s.row_ptr.ptr, s.col_idx.ptr,
+            if (!mg) block_setup_kernel<double><<<grid_rows(nq), 256, 0, rt.stream>>>(nq, s.row_ptr.ptr, s.col_idx.ptr,
                                                                              s.values.ptr, s.free_mask.ptr, inv_u,
                                                                              diag_u);
             if (mass_schur)
