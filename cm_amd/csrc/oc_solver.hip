@@ -382,24 +382,26 @@ __global__ void __launch_bounds__(kT) arnoldi_project_kernel(int n, int j, int n
     }
 }
 
-// arnoldi_project_kernel for systems of one row a thread (n <= 256 *
+// arnoldi_project_kernel for systems of one row a thread (n <= kT *
 // kReduceBlocks) and j + 2 <= kRowVectors, where latency is all there is: the
 // basis rows are on their way while the partials are added up, and serve the
-// second pass's dot products from the registers.  At 23,800 rows 6.1 us against 7.3.
-__global__ void __launch_bounds__(256) arnoldi_project_row_kernel(int n, int j, int n_parts, double *V,
+// second pass's dot products from the registers.  At 23,800 rows 6.1 us against 7.3;
+// a step of the 16^3 load step (112,724 rows) to 218 us from 221.
+template <int kT>
+__global__ void __launch_bounds__(kT) arnoldi_project_row_kernel(int n, int j, int n_parts, double *V,
                                                                  const double *__restrict__ partial,
                                                                  double *__restrict__ partial2, ScaledCopy sc,
                                                                  Arnoldi a)
 {
     __shared__ double s_h[kMaxDots];
-    __shared__ double s_red[4][kRowVectors];
-    const int t = threadIdx.x, i = blockIdx.x * 256 + t, lane = t & 63, wave = t >> 6;
+    __shared__ double s_red[kT / 64][kRowVectors];
+    const int t = threadIdx.x, i = blockIdx.x * kT + t, lane = t & 63, wave = t >> 6;
     double *w = V + static_cast<int64_t>(j + 1) * n;
     const int row = min(i, n - 1);
     BasisRow b;
     b.load(V, n, j + 1, row);
     const double wi = w[row];
-    reduce_partials<256>(j + 2, n_parts, partial, s_h);
+    reduce_partials<kT>(j + 2, n_parts, partial, s_h);
     const double wn2 = s_h[j + 1], left = wn2 - wave_square_sum(s_h, j + 1);
     const bool again = left < 0.25 * wn2;
     const double hn = again ? 0.0 : sqrt(left);
@@ -420,12 +422,15 @@ __global__ void __launch_bounds__(256) arnoldi_project_row_kernel(int n, int j, 
             if ((lane & 7) == 0) s_red[wave][k0 + (lane >> 3)] = tot;
         }
         __syncthreads();
-        if (t < j + 2)
-            partial2[static_cast<size_t>(t) * kReduceBlocks + blockIdx.x] =
-                s_red[0][t] + s_red[1][t] + s_red[2][t] + s_red[3][t];
+        if (t < j + 2) {
+            double sum = 0.0;
+#pragma unroll
+            for (int q = 0; q < kT / 64; ++q) sum += s_red[q][t];
+            partial2[static_cast<size_t>(t) * kReduceBlocks + blockIdx.x] = sum;
+        }
     }
     if (blockIdx.x == 0) {
-        for (int k = t; k <= j; k += 256) a.h[k] = s_h[k];
+        for (int k = t; k <= j; k += kT) a.h[k] = s_h[k];
         if (t == 0) {
             *a.flag = again ? 1.0 : 0.0;
             *a.hn = hn;
@@ -1133,11 +1138,12 @@ struct Krylov {
         Runtime &rt = runtime();
         const int blocks = row_blocks(kT);
         double *partial2 = s.partials.ptr + static_cast<size_t>(kReduceBlocks) * (1024 + 1);
-        if (kT == 256 && j + 2 <= kRowVectors) {
-            arnoldi_project_row_kernel<<<blocks, 256, 0, rt.stream>>>(n, j, parts, V, s.partials.ptr, partial2,
-                                                                      scaled_copy(), ar);
-            arnoldi_finish_kernel<256, true><<<blocks + 1, 256, 0, rt.stream>>>(n, j, m, blocks, V, partial2,
-                                                                                scaled_copy(), ar, s.arnoldi_host_dev);
+        if (kT <= 512 && n <= kT * kReduceBlocks && j + 2 <= kRowVectors) {
+            constexpr int kR = std::min(kT, 512);  // a block of 1,024 would spill the row's registers
+            arnoldi_project_row_kernel<kR><<<blocks, kR, 0, rt.stream>>>(n, j, parts, V, s.partials.ptr, partial2,
+                                                                         scaled_copy(), ar);
+            arnoldi_finish_kernel<kR, true><<<blocks + 1, kR, 0, rt.stream>>>(n, j, m, blocks, V, partial2,
+                                                                              scaled_copy(), ar, s.arnoldi_host_dev);
             return;
         }
         arnoldi_project_kernel<kT><<<blocks, kT, 0, rt.stream>>>(n, j, parts, V, s.partials.ptr, partial2, scaled_copy(), ar);
