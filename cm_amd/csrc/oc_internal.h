@@ -138,6 +138,8 @@ struct Multigrid {
     DevBuf<double> t0, r0, x0;            // level-0 scratch (3*n_nodes each)
     DevBuf<double> coarse_inv;            // per mesh dense inverse of the coarsest level
     int coarse_stride = 0;                // (max DOFs per mesh at the coarsest level)^2
+    DevBuf<double> dense, dense_w;        // the last two levels as one matrix per mesh (few meshes; dense_kernel)
+    int dense_stride = 0, dense_w_stride = 0;
     // level-0 sweeps (oc_multigrid_options_set); the trilinear and coarser
     // stencil levels take one each way (more there cost Krylov iterations
     // rather than saving them)
