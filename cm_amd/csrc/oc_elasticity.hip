@@ -1189,10 +1189,10 @@ mr_element_matrix_f64_kernel(int n_elements, const double *__restrict__ rec, con
     }
 }
 
-// kN element rows of one CSR row: every global load before the LDS adds.  The
+// kN element rows of one pressure row: every global load before the LDS adds.  The
 // addresses are uniform and advance by scalar multiplies.
 template <int kN, typename Real>
-__device__ __forceinline__ void gather_rows(const int2 *__restrict__ list, int sub, int lane, bool hi, int m0, int m1,
+__device__ __forceinline__ void gather_rows(const int2 *__restrict__ list, int lane, bool hi, int m0, int m1,
                                             int blk0, int blk1, const Real *__restrict__ kbuf,
                                             const uint8_t *__restrict__ rank, Real *s_row)
 {
@@ -1201,7 +1201,7 @@ __device__ __forceinline__ void gather_rows(const int2 *__restrict__ list, int s
 #pragma unroll
     for (int c = 0; c < kN; ++c) {
         const int2 at = list[c];
-        const Real *k = kbuf + static_cast<int64_t>(at.x + sub) * 89;
+        const Real *k = kbuf + static_cast<int64_t>(at.x) * 89;
         const uint8_t *rk = rank + static_cast<int64_t>(at.y) * kRankNodes;
         v0[c] = k[lane];
         o0[c] = rk[m0];
@@ -1223,74 +1223,136 @@ __device__ __forceinline__ void gather_rows(const int2 *__restrict__ list, int s
     }
 }
 
-// One wavefront per CSR row, three per block: block b < nq takes the three
-// displacement rows of node b, the blocks after them three pressure rows each.
-// A node's element rows lie next to each other in the element buffer and its
-// three rows share the lists and the neighbour ranks, which one row per block
-// fetched three times, from three XCDs (3.05 GB read then, 2.5 now, of 2.1 at
-// least, for 32,768 elements in FP64).  The element rows are taken in groups of
-// kMax, ..., 2, 1: with a test per row and the divisions that the shared lists
-// need, the scalar instructions took three times the vector ones' issue slots.
-// 32,768 elements FP64: 834 -> 788 us (4.0 GB, the rate of a copy; groups of 8,
-// which hold more registers, 801); 13,100 elements FP32: 343 -> 282 us.
-constexpr int kGatherRows = 3;
+// The same for a displacement node's three rows, 267 consecutive entries of each
+// of its elements: lane l takes entries l + 64 u; pos[u] is an entry's LDS row
+// and component block, m[u] the element node whose rank places it.  The 35
+// ranks are loaded once, a lane a node, and handed round.
+constexpr int kNodeEntries = 3 * 89, kNodeLoads = (kNodeEntries + 63) / 64, kNodeLast = kNodeEntries - 64 * (kNodeLoads - 1);
+template <int kN, typename Real>
+__device__ __forceinline__ void gather_node(const int2 *__restrict__ list, int lane, const int (&pos)[kNodeLoads],
+                                            const int (&m)[kNodeLoads], const Real *__restrict__ kbuf,
+                                            const uint8_t *__restrict__ rank, Real *s_rows)
+{
+    Real v[kN][kNodeLoads];
+    int rk[kN];
+#pragma unroll
+    for (int c = 0; c < kN; ++c) {
+        const int2 at = list[c];
+        const Real *k = kbuf + static_cast<int64_t>(at.x) * 89;
+        rk[c] = rank[static_cast<int64_t>(at.y) * kRankNodes + min(lane, kRankNodes - 1)];
+#pragma unroll
+        for (int u = 0; u < kNodeLoads; ++u) v[c][u] = k[64 * u + (u + 1 < kNodeLoads ? lane : min(lane, kNodeLast - 1))];
+    }
+    // an element's entries have places of their own, so its reads all go before
+    // its writes: one LDS latency an element
+#pragma unroll
+    for (int c = 0; c < kN; ++c) {
+        int o[kNodeLoads];
+#pragma unroll
+        for (int u = 0; u < kNodeLoads; ++u) o[u] = pos[u] + __shfl(rk[c], m[u]);
+        Real t[kNodeLoads];
+#pragma unroll
+        for (int u = 0; u < kNodeLoads; ++u) t[u] = s_rows[o[u]];
+#pragma unroll
+        for (int u = 0; u < kNodeLoads; ++u)
+            if (u + 1 < kNodeLoads || lane < kNodeLast) s_rows[o[u]] = t[u] + v[c][u];
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+    }
+}
+
+// One wavefront per displacement node (its three CSR rows) and per pressure row,
+// kGatherWaves to a block.  A node's element rows lie next to each other in the
+// element buffer and share the lists and the neighbour ranks.  Requests waiting
+// for lines that others have on their way bounded one wavefront a row (73% of
+// its time in FP32): its two loads of an element row and its two rank loads met
+// in the same lines, as did the three rows'.  The element rows are taken in
+// groups of kMax, ..., 2, 1: with a test per row the scalar instructions took
+// three times the vector ones' issue slots.
+// 32,768 elements FP64: 788 -> 721 us (4.0 GB); 13,100 elements FP32 293 -> 185 us,
+// 4,301 elements 77 -> 54 us.  Two wavefronts a block: 769 us with four, 779 with one.
+constexpr int kGatherWaves = 2;
 
 template <typename Real, int kMax>
-__global__ void __launch_bounds__(64 * kGatherRows)
+__global__ void __launch_bounds__(64 * kGatherWaves)
 csr_row_gather_kernel(int nq, int nl, int n_elements, int max_row, const int64_t *__restrict__ row_ptr,
                       const int *__restrict__ gptr, const int2 *__restrict__ lists, const Real *__restrict__ kbuf,
                       const uint8_t *__restrict__ rank, const uint16_t *__restrict__ row_nb, Real *__restrict__ values)
 {
     extern __shared__ unsigned char s_raw[];
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
-    Real *s_row = reinterpret_cast<Real *>(s_raw) + wave * max_row;  // a wavefront's own: no block barriers
-    const int b = blockIdx.x;
+    Real *s_rows = reinterpret_cast<Real *>(s_raw) + wave * 3 * max_row;  // a wavefront's own: no block barriers
+    const int b = blockIdx.x * kGatherWaves + wave;
+    if (b >= nq + nl) return;
     const bool disp = b < nq;
-    const int l = (b - nq) * kGatherRows + wave;
-    if (!disp && l >= nl) return;
-    const int r = disp ? wave * nq + b : 3 * nq + l;
-    const int gr = disp ? b : r;
-    const int g0 = gptr[gr], n = gptr[gr + 1] - g0;
+    const int r = disp ? b : 3 * nq + (b - nq);
+    const int g0 = gptr[r], n = gptr[r + 1] - g0;
     const int2 *list = lists + (disp ? g0 : g0 - 54 * n_elements);
     const int64_t r0 = row_ptr[r];
     const int len = static_cast<int>(row_ptr[r + 1] - r0);
     const int nb = row_nb[r];
-    for (int k = lane; k < len; k += 64) s_row[k] = Real(0);
-    __builtin_amdgcn_wave_barrier();
-    // lane j holds element columns j and j + 64: component block and rank slot
-    const int j1 = lane + 64;
-    const bool hi = j1 < 89;
-    const int blk0 = (lane / 27) * nb, m0 = lane % 27;
-    const int blk1 = j1 < 81 ? (j1 / 27) * nb : 3 * nb, m1 = j1 < 81 ? j1 % 27 : 27 + j1 - 81;
-    const int sub = disp ? wave : 0;
+    const auto block = [&](int j) { return j < 81 ? (j / 27) * nb : 3 * nb; };
+    const auto node = [&](int j) { return j < 81 ? j % 27 : 27 + j - 81; };
     int c = 0;
-    for (; c + kMax <= n; c += kMax) gather_rows<kMax>(list + c, sub, lane, hi, m0, m1, blk0, blk1, kbuf, rank, s_row);
+    if (!disp) {
+        for (int k = lane; k < len; k += 64) s_rows[k] = Real(0);
+        __builtin_amdgcn_wave_barrier();
+        // lane j holds element columns j and j + 64: component block and rank slot
+        const bool hi = lane + 64 < 89;
+        const int blk0 = block(lane), m0 = node(lane), blk1 = block(min(lane + 64, 88)), m1 = node(min(lane + 64, 88));
+        for (; c + 4 <= n; c += 4) gather_rows<4>(list + c, lane, hi, m0, m1, blk0, blk1, kbuf, rank, s_rows);
+        if (n - c >= 2) {
+            gather_rows<2>(list + c, lane, hi, m0, m1, blk0, blk1, kbuf, rank, s_rows);
+            c += 2;
+        }
+        if (n - c >= 1) gather_rows<1>(list + c, lane, hi, m0, m1, blk0, blk1, kbuf, rank, s_rows);
+        for (int k = lane; k < len; k += 64) values[r0 + k] = s_rows[k];
+        return;
+    }
+    const int64_t r1 = row_ptr[nq + b], r2 = row_ptr[2 * static_cast<int64_t>(nq) + b];
+    for (int k = lane; k < len; k += 64) s_rows[k] = s_rows[max_row + k] = s_rows[2 * max_row + k] = Real(0);
+    __builtin_amdgcn_wave_barrier();
+    int pos[kNodeLoads], m[kNodeLoads];
+#pragma unroll
+    for (int u = 0; u < kNodeLoads; ++u) {
+        const int k = min(64 * u + lane, kNodeEntries - 1);
+        pos[u] = (k / 89) * max_row + block(k % 89);
+        m[u] = node(k % 89);
+    }
+    for (; c + kMax <= n; c += kMax) gather_node<kMax>(list + c, lane, pos, m, kbuf, rank, s_rows);
     if (kMax > 8 && n - c >= 8) {
-        gather_rows<8>(list + c, sub, lane, hi, m0, m1, blk0, blk1, kbuf, rank, s_row);
+        gather_node<8>(list + c, lane, pos, m, kbuf, rank, s_rows);
         c += 8;
     }
     if (kMax > 4 && n - c >= 4) {
-        gather_rows<4>(list + c, sub, lane, hi, m0, m1, blk0, blk1, kbuf, rank, s_row);
+        gather_node<4>(list + c, lane, pos, m, kbuf, rank, s_rows);
         c += 4;
     }
-    if (n - c >= 2) {
-        gather_rows<2>(list + c, sub, lane, hi, m0, m1, blk0, blk1, kbuf, rank, s_row);
+    if (kMax > 2 && n - c >= 2) {
+        gather_node<2>(list + c, lane, pos, m, kbuf, rank, s_rows);
         c += 2;
     }
-    if (n - c >= 1) gather_rows<1>(list + c, sub, lane, hi, m0, m1, blk0, blk1, kbuf, rank, s_row);
-    for (int k = lane; k < len; k += 64) values[r0 + k] = s_row[k];
+    if (n - c >= 1) gather_node<1>(list + c, lane, pos, m, kbuf, rank, s_rows);
+    for (int k = lane; k < len; k += 64) {
+        values[r0 + k] = s_rows[k];
+        values[r1 + k] = s_rows[max_row + k];
+        values[r2 + k] = s_rows[2 * max_row + k];
+    }
 }
 
 template <typename Real>
 static int launch_row_gather(EquationsSet &s, const Real *kbuf, Real *values, int chunk)
 {
     Runtime &rt = runtime();
-    const size_t lds = static_cast<size_t>(kGatherRows) * s.max_row_len * sizeof(Real);
-    const unsigned grid = static_cast<unsigned>(s.n_nodes + (s.n_nodes_l + kGatherRows - 1) / kGatherRows);
+    const size_t lds = static_cast<size_t>(3 * kGatherWaves) * s.max_row_len * sizeof(Real);
+    const unsigned grid = static_cast<unsigned>((static_cast<int64_t>(s.n_nodes) + s.n_nodes_l + kGatherWaves - 1) / kGatherWaves);
 #define OC_ROW_GATHER(C)                                                                                            \
-    csr_row_gather_kernel<Real, C><<<grid, 64 * kGatherRows, lds, rt.stream>>>(                                    \
+    csr_row_gather_kernel<Real, C><<<grid, 64 * kGatherWaves, lds, rt.stream>>>(                                   \
         s.n_nodes, s.n_nodes_l, s.n_elements, s.max_row_len, s.row_ptr.ptr, s.gather_ptr.ptr,                      \
         reinterpret_cast<const int2 *>(s.row_lists.ptr), kbuf, s.col_rank.ptr, s.row_nb.ptr, values)
+    // eight element rows in one round of loads where the mesh leaves wavefronts
+    // of the GPU idle: the round trips are all there is to wait for then
+    if (chunk <= 0 && s.n_nodes + s.n_nodes_l <= 8 * rt.num_cus) chunk = 8;
     switch (chunk) {
     case 8: OC_ROW_GATHER(8); break;
     case 16: OC_ROW_GATHER(16); break;
