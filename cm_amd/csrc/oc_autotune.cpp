@@ -107,7 +107,7 @@ extern "C" int oc_autotune(oc_equations_set h, int precision, char *report, int 
                   [&](int i) { return num(chunks[i]); }, &c_gather));
 
     // SpMV: lanes per row (per node for node rows) x neighbours in flight per
-    // lane; default 32 x 1 (FP32 values) or a wavefront per node (FP64, 64 x 1)
+    // lane; default 32 x 2 (FP32 values) or a wavefront per node (FP64, 64 x 1)
     OC_CHECK(prepare_node_rows(s));
     DevBuf<double> y;
     OC_CHECK(y.alloc(s.n_rows));
@@ -115,7 +115,7 @@ extern "C" int oc_autotune(oc_equations_set h, int precision, char *report, int 
     for (int l : {8, 16, 32, 64})
         for (int u = 1; u <= 2; ++u)
             if (u == 1 || (s.node_rows == 1 && (l == 16 || l == 32))) spmv.push_back({l, u});  // unrolled: node rows only
-    const std::pair<int, int> spmv_def = s.flat_rows() && !fp32 ? std::make_pair(64, 1) : std::make_pair(32, 1);
+    const std::pair<int, int> spmv_def = s.flat_rows() && !fp32 ? std::make_pair(64, 1) : std::make_pair(32, s.node_rows == 1 && fp32 ? 2 : 1);
     int spmv_def_i = 0;
     for (size_t i = 0; i < spmv.size(); ++i)
         if (spmv[i] == spmv_def) spmv_def_i = static_cast<int>(i);

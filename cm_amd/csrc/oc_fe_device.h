@@ -364,26 +364,37 @@ __device__ __forceinline__ void node_rows_uu(const int64_t (&s)[3], int deg, int
                                              const double *__restrict__ x, double (&a)[3])
 {
     for (int p0 = lane; p0 < deg; p0 += kLanes * kU) {
-        int j[kU];
+        // lanes past the end repeat the last neighbour's loads and select zeros,
+        // so that no branch holds a load back
+        int j[kU], q[kU];
         bool ok[kU];
 #pragma unroll
         for (int u = 0; u < kU; ++u) {
             ok[u] = p0 + u * kLanes < deg;
-            j[u] = ok[u] ? col_idx[s[0] + p0 + u * kLanes] : 0;
+            q[u] = min(p0 + u * kLanes, deg - 1);
+            j[u] = col_idx[s[0] + q[u]];
         }
-        double v[kU][9];
+        VT raw[kU][9];
 #pragma unroll
         for (int u = 0; u < kU; ++u)
 #pragma unroll
             for (int r = 0; r < 3; ++r)
 #pragma unroll
                 for (int c = 0; c < 3; ++c)
-                    v[u][3 * r + c] = ok[u] ? static_cast<double>(vals[s[r] + c * deg + p0 + u * kLanes]) : 0.0;
+                    raw[u][3 * r + c] = vals[s[r] + c * deg + q[u]];
         double xv[kU][3];
 #pragma unroll
         for (int u = 0; u < kU; ++u)
 #pragma unroll
-            for (int c = 0; c < 3; ++c) xv[u][c] = ok[u] ? x[c * nq64 + j[u]] : 0.0;
+            for (int c = 0; c < 3; ++c) {
+                const double t = x[c * nq64 + j[u]];
+                xv[u][c] = ok[u] ? t : 0.0;
+            }
+        double v[kU][9];
+#pragma unroll
+        for (int u = 0; u < kU; ++u)
+#pragma unroll
+            for (int k = 0; k < 9; ++k) v[u][k] = static_cast<double>(ok[u] ? raw[u][k] : static_cast<VT>(0));
 #pragma unroll
         for (int u = 0; u < kU; ++u)
 #pragma unroll

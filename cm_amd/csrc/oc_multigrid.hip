@@ -746,11 +746,15 @@ uu_node_bf16_kernel(int nq, const int64_t *__restrict__ uu_off, const int *__res
         uint2 v[kQ][9];
 #pragma unroll
         for (int u = 0; u < kQ; ++u) {
-            const int q = q0 + u * kLanes;
-            const bool ok = q < n4;
-            cj[u] = ok ? cols[q] : make_int4(i, i, i, i);
+            // lanes past the end repeat the last quad's loads and select zeros
+            const bool ok = q0 + u * kLanes < n4;
+            const int q = min(q0 + u * kLanes, n4 - 1);
+            cj[u] = cols[q];
 #pragma unroll
-            for (int rc = 0; rc < 9; ++rc) v[u][rc] = ok ? vals[rc * n4 + q] : make_uint2(0u, 0u);
+            for (int rc = 0; rc < 9; ++rc) {
+                const uint2 w = vals[rc * n4 + q];
+                v[u][rc] = make_uint2(ok ? w.x : 0u, ok ? w.y : 0u);
+            }
         }
 #pragma unroll
         for (int u = 0; u < kQ; ++u) {

@@ -690,7 +690,7 @@ __global__ void __launch_bounds__(256) spmv_node_kernel(int nq, int nl, const in
 // The same by one wavefront per node or pressure row (node_rows_flat): FP64
 // values' default.  At 32^3 332 us (1.52 GB) against 397 with 16 lanes x 2
 // neighbours, at 16^3 34.6 against 44.7; with FP32 values it loses to 32 lanes
-// (342 us against 264), as half the bytes leave the wavefront's own chain of
+// x 2 neighbours (342 us against 257), as half the bytes leave the wavefront's own chain of
 // columns, iterate and sum to bound it.
 template <typename VT>
 __global__ void __launch_bounds__(256) spmv_flat_kernel(int nq, int nl, const int64_t *__restrict__ row_ptr,
@@ -936,8 +936,9 @@ struct Krylov {
     {
         KernelTimer timer("spmv");
         const bool lap = s.cls == OC_EQUATIONS_SET_LAPLACE;
-        // defaults: 8 lanes per Laplace row; per Mooney-Rivlin node 32 lanes
-        // (FP32) or a wavefront (FP64)
+        // defaults: 8 lanes per Laplace row; per Mooney-Rivlin node 32 lanes with
+        // two neighbours in flight (FP32: 257 us at 32^3, 264 with one) or a
+        // wavefront (FP64)
         const int lanes = s.tuned_spmv_lanes > 0 ? s.tuned_spmv_lanes : (lap ? 8 : (fp32 ? 32 : 64));
         if (lap) return launch_spmv<double>(s.values.ptr, lanes, s.wgt.ptr, x, y);
         if (fp32) return launch_spmv<float>(s.values_sp.ptr, lanes, s.wgt.ptr, x, y);
@@ -946,7 +947,7 @@ struct Krylov {
     template <typename VT>
     int launch_spmv(const VT *vals, int lanes, const double *wv, const double *x, double *y, int unroll = -1)
     {
-        if (unroll < 0) unroll = s.tuned_spmv_unroll > 0 ? s.tuned_spmv_unroll : 1;
+        if (unroll < 0) unroll = s.tuned_spmv_unroll > 0 ? s.tuned_spmv_unroll : (fp32 ? 2 : 1);
         Runtime &rt = runtime();
         if (s.cls == OC_EQUATIONS_SET_MOONEY_RIVLIN && s.node_rows == 1 && lanes >= 16) {
             const int nq = s.n_nodes, nl = s.n_nodes_l;
