@@ -158,6 +158,7 @@ struct SolverSystem {
     int64_t nnz = 0;
     int precision = -1;             // precision of the last assembly
     DevBuf<int32_t> index, rows;
+    DevBuf<uint64_t> keep;          // free-column bits of the equations matrix's entries
     DevBuf<int64_t> row_ptr;
     DevBuf<int32_t> col_idx;
     DevBuf<double> values;
