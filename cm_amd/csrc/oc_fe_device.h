@@ -484,8 +484,9 @@ __device__ __forceinline__ void node_rows_flat(int i, int nq, int lane, const in
     const int64_t s0 = row_ptr[i], per = row_ptr[nq];
     const int uu = static_cast<int>(pstart[i] - s0), deg = uu / 3;
     const int n = kPressure ? static_cast<int>(row_ptr[i + 1] - s0) : uu;
+    if (n == 0) return;  // a node of no element: an empty row, which may stand at either end of the arrays
     const int *col = col_idx + s0;
-    // (a node is its own neighbour, so deg >= 1)
+    // (a row with entries holds the node itself, so deg >= 1)
     const uint32_t j0 = col[min(lane, deg - 1)], j1 = col[min(64 + lane, deg - 1)];
     const uint32_t jp = kPressure ? col[min(uu + lane, n - 1)] : 0;
     Vec v[3][kSteps];
