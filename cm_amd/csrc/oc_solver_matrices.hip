@@ -106,8 +106,9 @@ solver_matrix_kernel(int n, const int *__restrict__ rows, const int64_t *__restr
     T v[kWaveRows][kChunks];
 #pragma unroll
     for (int q = 0; q < kWaveRows; ++q)
+        if (len[q] > 0)  // a free DOF of no element has an empty row, which may stand at the end of the values
 #pragma unroll
-        for (int u = 0; u < kChunks; ++u) v[q][u] = values[k0[q] + max(min(64 * u + lane, len[q] - 1), 0)];
+            for (int u = 0; u < kChunks; ++u) v[q][u] = values[k0[q] + min(64 * u + lane, len[q] - 1)];
 #pragma unroll
     for (int q = 0; q < kWaveRows; ++q)
         for (int base = 0; base < len[q]; base += 64 * kChunks) {

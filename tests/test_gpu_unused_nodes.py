@@ -59,3 +59,59 @@ def test_newton(gpu, n, fix_unused):
         assert np.array_equal(got[unused], d[unused])
         eq.set_dofs(start)
     eq.destroy()
+
+
+def check_restriction(eq, fixed, precision):
+    """The solver matrix equals the equations matrix without the fixed rows and columns."""
+    eq.solver_matrices_assemble(precision)
+    rp, ci = eq.matrix_structure()
+    vals = eq.matrix_values_sp() if precision else eq.matrix_values()
+    free = np.ones(eq.n_rows, bool)
+    free[fixed] = False
+    rows = np.repeat(np.arange(eq.n_rows), np.diff(rp))
+    keep = free[rows] & free[ci]
+    number = np.cumsum(free) - 1
+    srp, sci = eq.solver_matrix_structure(0)
+    assert np.array_equal(eq.solver_matrix_values_sp() if precision else eq.solver_matrix_values(), vals[keep])
+    assert np.array_equal(sci, number[ci[keep]])
+    assert np.array_equal(np.diff(srp), np.bincount(number[rows[keep]], minlength=free.sum()))
+
+
+@pytest.mark.parametrize("precision", [0, 1])
+@pytest.mark.parametrize("n", [(1, 1, 1), (2, 3, 1)])
+def test_solver_matrix(gpu, n, precision):
+    """With the last rows free and empty, and without them; odd and even row counts."""
+    cm = gpu
+    _, u = with_unused_nodes(2, n, 7)
+    eq = cm.MooneyRivlinEquationsSet(u, 2.0, 6.0)
+    eq.set_dofs(eq.undeformed_dofs() * 1.01)
+    eq.residual_evaluate()
+    eq.jacobian_evaluate(precision)
+    for fixed in ([], [1], [0, 2, eq.n_rows - 1]):
+        eq.set_boundary_conditions(fixed, np.zeros(len(fixed)))
+        for _ in range(2):  # with the columns, then the values alone
+            check_restriction(eq, fixed, precision)
+    eq.destroy()
+
+
+@pytest.mark.parametrize("n", [(2, 2, 2), (5, 4, 3)])
+def test_laplace(gpu, n):
+    """Assembly, solver matrix and solve (bound as in test_gpu_arnoldi)."""
+    cm = gpu
+    m, u = with_unused_nodes(1, n, 3)
+    field = np.array([0.3, -0.7, 0.2]) @ u.coords + 0.1
+    boundary = 1 + np.unique(np.concatenate([m.face_nodes(a, side) for a in range(3) for side in (0, 1)]))
+    eq = cm.LaplaceEquationsSet(u)
+    eq.assemble()
+    rp, ci = orc.pattern([(u.n_nodes, u.elem_nodes)])
+    ref, _ = orc.laplace_assemble(u.elem_nodes, u.coords, rp, ci)
+    assert np.linalg.norm(eq.matrix_values() - ref) <= 1e-12 * np.linalg.norm(ref)
+    for fixed in (boundary, np.concatenate([[0], boundary, [u.n_nodes - 1]])):
+        eq.set_boundary_conditions(fixed, field[fixed])
+        for _ in range(2):
+            check_restriction(eq, fixed, cm.OC_FP64)
+        eq.solve(cm.newton_options(krylov_relative_tolerance=1e-12, absolute_tolerance=0.0))
+        want = field.copy()
+        want[np.setdiff1d([0, u.n_nodes - 1], fixed)] = 0.0
+        assert np.linalg.norm(eq.get_dofs() - want) < 8e-9 * np.linalg.norm(want)
+    eq.destroy()
