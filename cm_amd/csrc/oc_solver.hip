@@ -438,59 +438,16 @@ __global__ void __launch_bounds__(kT) arnoldi_project_row_kernel(int n, int j, i
     }
 }
 
-// step j, last: the second pass where the first asked for it (h2 = V . w,
-// w -= V h2, its norm by Pythagoras: h2 is the rounding left by the first pass,
-// so nothing cancels), V_{j+1} normalised; and, in the last block, which owns
-// no rows, the rotations: R's column j, g, and the residual estimate |g_{j+1}|
-// and hn into the host-visible slots 2j, 2j+1.
-// kRow: one row a thread, j + 2 <= kRowVectors (see arnoldi_project_row_kernel)
-template <int kT, bool kRow>
-__global__ void __launch_bounds__(kT) arnoldi_finish_kernel(int n, int j, int m, int n_parts, double *V,
-                                                           const double *__restrict__ partial2, ScaledCopy sc,
-                                                           Arnoldi a, double *__restrict__ host)
+// Step j's rotations, by one block: the column h_0..h_j in s_x is rotated into
+// R's column j, then the last rotation makes h_{j+1} = hn zero; g, and the
+// residual estimate |g_{j+1}| and hn into the host-visible slots 2j, 2j+1.
+// s_cs, s_sn: the rotations 0..j-1.  The block's LDS writes before the call need
+// no barrier of their own.
+__device__ __forceinline__ void arnoldi_rotate(int j, int m, double *s_x, const double *s_cs, const double *s_sn,
+                                               double hn, const Arnoldi &a, double *__restrict__ host)
 {
-    __shared__ double s_h[kMaxDots];
-    __shared__ double s_r[3 * kMaxDots];
-    const int t = threadIdx.x;
-    const bool rotate = blockIdx.x == gridDim.x - 1;
-    double *w = V + static_cast<int64_t>(j + 1) * n;
-    BasisRow b;
-    double wi = 0.0;
-    if (kRow && !rotate) {
-        const int row = min(static_cast<int>(blockIdx.x) * kT + t, n - 1);
-        b.load(V, n, j + 1, row);
-        wi = w[row];
-    }
-    const bool again = *a.flag != 0.0;
-    double hn = 0.0;
-    if (again) {
-        reduce_partials<kT>(j + 2, n_parts, partial2, s_h);
-        hn = sqrt(fmax(s_h[j + 1] - wave_square_sum(s_h, j + 1), 0.0));
-    }
-    if (!rotate) {
-        if (!again) return;
-        const double scale = hn > 0.0 ? 1.0 / hn : 1.0;
-        if (kRow) {
-            const int i = blockIdx.x * kT + t;
-            if (i < n) basis_store(w, i, scale * b.projected(j + 1, s_h, wi), sc);
-            return;
-        }
-        const int rows = (gridDim.x - 1) * kT;
-        for (int i = blockIdx.x * kT + t; i < n; i += rows)
-            basis_store(w, i, scale * projected(V, n, j + 1, s_h, i, w[i]), sc);
-        return;
-    }
-    double *s_x = s_r, *s_cs = s_r + kMaxDots, *s_sn = s_r + 2 * kMaxDots;
-    if (!again) hn = *a.hn;
-    for (int i = t; i <= j; i += kT) {
-        s_x[i] = again ? a.h[i] + s_h[i] : a.h[i];
-        if (i < j) {
-            s_cs[i] = a.cs[i];
-            s_sn[i] = a.sn[i];
-        }
-    }
     __syncthreads();
-    if (t == 0) {
+    if (threadIdx.x == 0) {
         double hi = s_x[0];
         for (int i = 0; i < j; ++i) {
             const double hi1 = s_x[i + 1], c = s_cs[i], sn = s_sn[i];
@@ -511,7 +468,104 @@ __global__ void __launch_bounds__(kT) arnoldi_finish_kernel(int n, int j, int m,
         __hip_atomic_store(host + 2 * j + 1, hn, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
     }
     __syncthreads();
-    for (int i = t; i <= j; i += kT) a.R[static_cast<size_t>(i) * m + j] = s_x[i];
+    for (int i = threadIdx.x; i <= j; i += blockDim.x) a.R[static_cast<size_t>(i) * m + j] = s_x[i];
+}
+
+// What a norm in the slots can not be: not written yet, and a second pass that
+// cancelled as well (arnoldi_finish_kernel)
+constexpr double kUnwritten = -1.0, kCancelled = -2.0;
+
+// step j, last: the second pass where the first asked for it (h2 = V . w,
+// w -= V h2), V_{j+1} normalised, and, in the last block, which owns no rows, the
+// rotations.  The norm follows by Pythagoras: as a rule h2 is the rounding the
+// first pass left and nothing cancels.  Where w lies almost in the basis (the
+// Krylov space is exhausted) the first pass leaves rounding alone, most of it
+// along V, and the difference is rounding of rounding, or zero, which would end
+// the cycle as solved.  There the vector stays unscaled, the column goes to R
+// unrotated and hn = kCancelled tells the host, which has the norm summed from
+// the vector (arnoldi_resume_kernel).
+// kRow: one row a thread, j + 2 <= kRowVectors (see arnoldi_project_row_kernel)
+template <int kT, bool kRow>
+__global__ void __launch_bounds__(kT) arnoldi_finish_kernel(int n, int j, int m, int n_parts, double *V,
+                                                           const double *__restrict__ partial2, ScaledCopy sc,
+                                                           Arnoldi a, double *__restrict__ host)
+{
+    __shared__ double s_h[kMaxDots];
+    __shared__ double s_r[3 * kMaxDots];
+    const int t = threadIdx.x;
+    const bool rotate = blockIdx.x == gridDim.x - 1;
+    double *w = V + static_cast<int64_t>(j + 1) * n;
+    BasisRow b;
+    double wi = 0.0;
+    if (kRow && !rotate) {
+        const int row = min(static_cast<int>(blockIdx.x) * kT + t, n - 1);
+        b.load(V, n, j + 1, row);
+        wi = w[row];
+    }
+    const bool again = *a.flag != 0.0;
+    bool cancelled = false;
+    double hn = 0.0;
+    if (again) {
+        reduce_partials<kT>(j + 2, n_parts, partial2, s_h);
+        const double left = s_h[j + 1] - wave_square_sum(s_h, j + 1);
+        cancelled = left < 0.25 * s_h[j + 1];
+        hn = sqrt(fmax(left, 0.0));
+    }
+    if (!rotate) {
+        if (!again) return;
+        const double scale = hn > 0.0 && !cancelled ? 1.0 / hn : 1.0;
+        if (kRow) {
+            const int i = blockIdx.x * kT + t;
+            if (i < n) basis_store(w, i, scale * b.projected(j + 1, s_h, wi), sc);
+            return;
+        }
+        const int rows = (gridDim.x - 1) * kT;
+        for (int i = blockIdx.x * kT + t; i < n; i += rows)
+            basis_store(w, i, scale * projected(V, n, j + 1, s_h, i, w[i]), sc);
+        return;
+    }
+    double *s_x = s_r, *s_cs = s_r + kMaxDots, *s_sn = s_r + 2 * kMaxDots;
+    if (!again) hn = *a.hn;
+    for (int i = t; i <= j; i += kT) {
+        s_x[i] = again ? a.h[i] + s_h[i] : a.h[i];
+        if (cancelled) a.R[static_cast<size_t>(i) * m + j] = s_x[i];
+        if (i < j) {
+            s_cs[i] = a.cs[i];
+            s_sn[i] = a.sn[i];
+        }
+    }
+    if (cancelled) {
+        if (t == 0) {
+            __hip_atomic_store(host + 2 * j, 0.0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+            __hip_atomic_store(host + 2 * j + 1, kCancelled, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+        }
+        return;
+    }
+    arnoldi_rotate(j, m, s_x, s_cs, s_sn, hn, a, host);
+}
+
+// What arnoldi_finish_kernel left of step j: V_{j+1} (length hn) normalised and,
+// in the last block, R's column rotated
+__global__ void __launch_bounds__(256) arnoldi_resume_kernel(int n, int j, int m, double hn, double *V, ScaledCopy sc,
+                                                            Arnoldi a, double *__restrict__ host)
+{
+    __shared__ double s_r[3 * kMaxDots];
+    if (blockIdx.x < gridDim.x - 1) {
+        double *w = V + static_cast<int64_t>(j + 1) * n;
+        const double scale = hn > 0.0 ? 1.0 / hn : 1.0;
+        for (int i = blockIdx.x * 256 + threadIdx.x; i < n; i += (gridDim.x - 1) * 256)
+            basis_store(w, i, scale * w[i], sc);
+        return;
+    }
+    double *s_x = s_r, *s_cs = s_r + kMaxDots, *s_sn = s_r + 2 * kMaxDots;
+    for (int i = threadIdx.x; i <= j; i += 256) {
+        s_x[i] = a.R[static_cast<size_t>(i) * m + j];
+        if (i < j) {
+            s_cs[i] = a.cs[i];
+            s_sn[i] = a.sn[i];
+        }
+    }
+    arnoldi_rotate(j, m, s_x, s_cs, s_sn, hn, a, host);
 }
 
 // ---- CSR SpMV of the weighted Dirichlet operator: y_r = w_r sum_k v_k x_c
@@ -1156,7 +1210,6 @@ struct Krylov {
     // mapped slots: polled, since an event after each step costs the stream a
     // barrier and the host two calls (a solve of 146 steps at 23,800 rows 3.47 ms
     // against 3.84).  Every 1,024 looks the stream is asked whether it still runs.
-    static constexpr double kUnwritten = -1.0;  // both are norms
     int wait_step(int k, double *res, double *hn)
     {
         const volatile double *slots = s.arnoldi_host + 2 * k;
@@ -1176,6 +1229,20 @@ struct Krylov {
         }
     }
 
+    // Step k's residual estimate and hn where its second pass cancelled too: the
+    // norm is summed from V_{k+1} itself.  A step queued after it has run on the
+    // unscaled vector; it is done when this returns, and is to be queued again.
+    int resume_step(int k, double *res, double *hn)
+    {
+        volatile double *slots = s.arnoldi_host + 2 * k;
+        OC_CHECK(norm(V + static_cast<int64_t>(k + 1) * n, hn));
+        for (int i = 0; i < (k + 1 < m ? 4 : 2); ++i) slots[i] = kUnwritten;
+        arnoldi_resume_kernel<<<row_blocks(256) + 1, 256, 0, runtime().stream>>>(n, k, m, *hn, V, scaled_copy(), ar,
+                                                                                 s.arnoldi_host_dev);
+        OC_HIP_CHECK(hipGetLastError());
+        return wait_step(k, res, hn);
+    }
+
     // Solves W A x = b (x starts at 0) to ||b - W A x|| <= tol_abs; b is zero
     // on fixed DOFs.  Right preconditioning: x = W^-1 P^-1 V y.  The host
     // stays one Arnoldi step ahead of the device: it queues step j, then
@@ -1192,23 +1259,27 @@ struct Krylov {
         double res = beta;
         std::vector<double> R(static_cast<size_t>(m) * m), g(m + 1), y(m);
         volatile double *slots = s.arnoldi_host;
-        bool first = true;
+        OC_HIP_CHECK(hipMemcpyAsync(r, b, sizeof(double) * n, hipMemcpyDeviceToDevice, rt.stream));
+        bool fresh = true;  // r = b - W A x and res = beta is its norm
+        auto true_residual = [&]() -> int {
+            OC_CHECK(spmv(x, w));
+            OC_HIP_CHECK(hipMemcpyAsync(r, b, sizeof(double) * n, hipMemcpyDeviceToDevice, rt.stream));
+            axpby_kernel<<<grid_for(n), 256, 0, rt.stream>>>(n, -1.0, w, 1.0, r);
+            OC_CHECK(norm(r, &beta));
+            res = beta;
+            fresh = true;
+            return OC_NO_ERROR;
+        };
         while (total < max_iter && res > tol_abs) {
-            // r = b - W A x
-            if (first) {
-                OC_HIP_CHECK(hipMemcpyAsync(r, b, sizeof(double) * n, hipMemcpyDeviceToDevice, rt.stream));
-                first = false;
-            } else {
-                OC_CHECK(spmv(x, w));
-                OC_HIP_CHECK(hipMemcpyAsync(r, b, sizeof(double) * n, hipMemcpyDeviceToDevice, rt.stream));
-                axpby_kernel<<<grid_for(n), 256, 0, rt.stream>>>(n, -1.0, w, 1.0, r);
-                OC_CHECK(norm(r, &beta));
-                res = beta;
-                if (res <= tol_abs) break;
+            if (!fresh) {
+                OC_CHECK(true_residual());
+                if (!(res > tol_abs)) break;
             }
+            fresh = false;
             arnoldi_start_kernel<<<grid_for(n), 256, 0, rt.stream>>>(n, m, beta, r, V, scaled_copy(), ar);
             const int steps = std::min(m, max_iter - total);
             int cols = 0;
+            bool breakdown = false;
             // nothing that writes them is in flight: a cycle ends with the stream drained
             for (int k = 0; k < 2 * steps; ++k) slots[k] = kUnwritten;
             for (int j = 0; j < steps && cols == 0; ++j) {
@@ -1218,8 +1289,13 @@ struct Krylov {
                     if (k < 0 || (k == j && j != steps - 1)) continue;
                     double rk, hk;
                     OC_CHECK(wait_step(k, &rk, &hk));
+                    if (hk == kCancelled) {
+                        OC_CHECK(resume_step(k, &rk, &hk));
+                        j = k;
+                    }
                     res = rk;
-                    if (rk <= tol_abs || hk == 0.0 || k == steps - 1) cols = k + 1;
+                    breakdown = hk == 0.0;
+                    if (rk <= tol_abs || breakdown || k == steps - 1) cols = k + 1;
                 }
             }
             total += cols;
@@ -1238,6 +1314,9 @@ struct Krylov {
             OC_CHECK(combine(V, cols, yc, 1.0, w));
             OC_CHECK(apply_preconditioner(w, z));
             axpby_kernel<<<grid_for(n), 256, 0, rt.stream>>>(n, 1.0, z, 1.0, x);
+            // a vector wholly in the basis makes the estimate zero, whether the
+            // system is solved or singular: the true residual tells
+            if (breakdown) OC_CHECK(true_residual());
         }
         *iters = total;
         *res_out = res;
