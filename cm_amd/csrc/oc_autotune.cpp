@@ -4,10 +4,14 @@
 //   * the CSR row gather's prefetch depth (element rows per chunk),
 //   * the SpMV's lanes per CSR row and neighbours in flight per lane,
 //   * the level-0 multigrid node kernel's shape,
-// keeps in the set (for later launches) the fastest of each when it beats the
-// default by more than the timing noise, and reports the timings as JSON.
+// keeps in the set, for later launches of that precision, the fastest of each
+// when it beats the default by more than the timing noise (else the default
+// rule stays in force), and reports the timings as JSON.
+#include <algorithm>
 #include <cstdio>
 #include <string>
+#include <tuple>
+#include <utility>
 #include <vector>
 
 #include "oc_internal.h"
@@ -100,14 +104,14 @@ extern "C" int oc_autotune(oc_equations_set h, int precision, char *report, int 
     OC_CHECK(tune(js, "element_matrix_ms", 6, 0, reps,
                   [&](int i) { return launch_mr_element_matrices(s, precision, bpcs[i]); },
                   [&](int i) { return num(bpcs[i]); }, &c_elem));
-    // CSR row gather prefetch depth (element rows per chunk; default 4)
+    // CSR row gather prefetch depth (element rows per chunk; default by the mesh's size)
     const int chunks[] = {4, 8, 16};
+    const int gather_def_i = row_gather_default(s) == 8 ? 1 : 0;
     Choice c_gather{};
-    OC_CHECK(tune(js, "row_gather_ms", 3, 0, reps, [&](int i) { return launch_mr_row_gather(s, precision, chunks[i]); },
+    OC_CHECK(tune(js, "row_gather_ms", 3, gather_def_i, reps, [&](int i) { return launch_mr_row_gather(s, precision, chunks[i]); },
                   [&](int i) { return num(chunks[i]); }, &c_gather));
 
-    // SpMV: lanes per row (per node for node rows) x neighbours in flight per
-    // lane; default 32 x 2 (FP32 values) or a wavefront per node (FP64, 64 x 1)
+    // SpMV: lanes per row (per node for node rows) x neighbours in flight per lane
     OC_CHECK(prepare_node_rows(s));
     DevBuf<double> y;
     OC_CHECK(y.alloc(s.n_rows));
@@ -115,10 +119,9 @@ extern "C" int oc_autotune(oc_equations_set h, int precision, char *report, int 
     for (int l : {8, 16, 32, 64})
         for (int u = 1; u <= 2; ++u)
             if (u == 1 || (s.node_rows == 1 && (l == 16 || l == 32))) spmv.push_back({l, u});  // unrolled: node rows only
-    const std::pair<int, int> spmv_def = s.flat_rows() && !fp32 ? std::make_pair(64, 1) : std::make_pair(32, s.node_rows == 1 && fp32 ? 2 : 1);
-    int spmv_def_i = 0;
-    for (size_t i = 0; i < spmv.size(); ++i)
-        if (spmv[i] == spmv_def) spmv_def_i = static_cast<int>(i);
+    std::pair<int, int> spmv_def = s.spmv_default(fp32);
+    if (s.node_rows != 1) spmv_def.second = 1;
+    const int spmv_def_i = static_cast<int>(std::find(spmv.begin(), spmv.end(), spmv_def) - spmv.begin());
     Choice c_spmv{};
     OC_CHECK(tune(js, "spmv_ms", static_cast<int>(spmv.size()), spmv_def_i, reps,
                   [&](int i) {
@@ -133,7 +136,7 @@ extern "C" int oc_autotune(oc_equations_set h, int precision, char *report, int 
     // level-0 multigrid node kernel (residual form), when the rows have the
     // node layout: FP64 values (default a wavefront per node), or for an FP32 Jacobian the
     // packed bf16 copy its smoother reads (default 16 lanes x 1 quad)
-    int best_smoother = -1;
+    int best_smoother = -1, smoother_def = -1;
     if (s.node_rows == 1 && !s.free_mask.ptr) {  // no boundary conditions yet: every DOF free
         OC_CHECK(s.free_mask.alloc(s.n_rows));
         OC_HIP_CHECK(hipMemset(s.free_mask.ptr, 1, s.n_rows));
@@ -149,25 +152,32 @@ extern "C" int oc_autotune(oc_equations_set h, int precision, char *report, int 
             OC_CHECK(launch_uu_pack(s));
         }
         Choice c_sm{};
-        OC_CHECK(tune(js, "smoother_residual_ms", 5, fp32 || !s.flat_rows() ? 0 : 4, reps,
+        smoother_def = fp32 || !s.flat_rows() ? 0 : 4;
+        OC_CHECK(tune(js, "smoother_residual_ms", 5, smoother_def, reps,
                       [&](int v) { return launch_smoother_residual(s, precision, v, s.dofs.ptr, s.dofs.ptr, r.ptr); },
                       [&](int v) { return std::string(names[v]); }, &c_sm));
         best_smoother = c_sm.index;
     }
     OC_HIP_CHECK(hipStreamSynchronize(runtime().stream));
-    const int best_bpc = bpcs[c_elem.index], best_chunk = chunks[c_gather.index];
-    const int best_lanes = spmv[static_cast<size_t>(c_spmv.index)].first;
-    const int best_unroll = spmv[static_cast<size_t>(c_spmv.index)].second;
-    s.tuned_element_blocks_per_cu = best_bpc;
-    s.tuned_gather_chunk = best_chunk;
-    s.tuned_spmv_lanes = best_lanes;
-    s.tuned_spmv_unroll = best_unroll;
-    if (best_smoother >= 0) s.tuned_smoother = best_smoother;
-    char buf[256];
-    std::snprintf(buf, sizeof buf, ", \"margin\": %.2f, \"chosen\": {\"element_blocks_per_cu\": %d, \"gather_chunk\": %d, "
-                                   "\"spmv_lanes\": %d, \"spmv_unroll\": %d, \"smoother_variant\": %d}}",
-                  kMargin, best_bpc, best_chunk, best_lanes, best_unroll, best_smoother);
+    // a default that stood is not stored: the launches then follow its rule
+    LaunchShapes &t = s.tuned[precision];
+    t = LaunchShapes{};
+    const std::pair<int, int> best_spmv = spmv[static_cast<size_t>(c_spmv.index)];
+    if (c_elem.index != 0) t.element_blocks_per_cu = bpcs[c_elem.index];
+    if (c_gather.index != gather_def_i) t.gather_chunk = chunks[c_gather.index];
+    if (c_spmv.index != spmv_def_i) std::tie(t.spmv_lanes, t.spmv_unroll) = best_spmv;
+    if (best_smoother != smoother_def) t.smoother = best_smoother;
+    char buf[512];
+    const char *shapes = "\"%s\": {\"element_blocks_per_cu\": %d, \"gather_chunk\": %d, \"spmv_lanes\": %d, "
+                         "\"spmv_unroll\": %d, \"smoother_variant\": %d}";
+    std::snprintf(buf, sizeof buf, ", \"margin\": %.2f, ", kMargin);
     js += buf;
+    std::snprintf(buf, sizeof buf, shapes, "default", bpcs[0], chunks[gather_def_i], spmv_def.first, spmv_def.second,
+                  smoother_def);
+    js += std::string(buf) + ", ";
+    std::snprintf(buf, sizeof buf, shapes, "chosen", bpcs[c_elem.index], chunks[c_gather.index], best_spmv.first,
+                  best_spmv.second, best_smoother);
+    js += std::string(buf) + "}";
     if (report && report_size > 0) std::snprintf(report, static_cast<size_t>(report_size), "%s", js.c_str());
     return OC_NO_ERROR;
 }

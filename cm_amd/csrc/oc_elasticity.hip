@@ -1355,6 +1355,11 @@ csr_row_gather_kernel(int nq, int nl, int n_elements, int max_row, const int64_t
     }
 }
 
+// The element rows a wavefront gathers at once: eight where the mesh leaves
+// wavefronts of the GPU idle, as the round trips are all there is to wait for
+// then, else four
+int row_gather_default(const EquationsSet &s) { return s.n_nodes + s.n_nodes_l <= 8 * runtime().num_cus ? 8 : 4; }
+
 template <typename Real>
 static int launch_row_gather(EquationsSet &s, const Real *kbuf, Real *values, int chunk)
 {
@@ -1365,10 +1370,7 @@ static int launch_row_gather(EquationsSet &s, const Real *kbuf, Real *values, in
     csr_row_gather_kernel<Real, C><<<grid, 64 * kGatherWaves, lds, rt.stream>>>(                                   \
         s.n_nodes, s.n_nodes_l, s.n_elements, s.max_row_len, s.row_ptr.ptr, s.gather_ptr.ptr,                      \
         reinterpret_cast<const int2 *>(s.row_lists.ptr), kbuf, s.col_rank.ptr, s.row_nb.ptr, values)
-    // eight element rows in one round of loads where the mesh leaves wavefronts
-    // of the GPU idle: the round trips are all there is to wait for then
-    if (chunk <= 0 && s.n_nodes + s.n_nodes_l <= 8 * rt.num_cus) chunk = 8;
-    switch (chunk) {
+    switch (chunk > 0 ? chunk : row_gather_default(s)) {
     case 8: OC_ROW_GATHER(8); break;
     case 16: OC_ROW_GATHER(16); break;
     default: OC_ROW_GATHER(4); break;
@@ -1463,7 +1465,7 @@ int launch_mr_jacobian_fd(EquationsSet &s)
         const unsigned fb = static_cast<unsigned>((nv + kGaussElemsPerBlock - 1) / kGaussElemsPerBlock);
         OC_CHECK(launch_residual_elements<true>(s, fb, s.dofs.ptr, T, s.relem.ptr, delta, s.kbuf64.ptr));
     }
-    return launch_mr_row_gather(s, OC_FP64, s.tuned_gather_chunk);
+    return launch_mr_row_gather(s, OC_FP64, s.tuned[OC_FP64].gather_chunk);
 }
 
 int launch_mr_jacobian(EquationsSet &s, int precision)
@@ -1477,8 +1479,8 @@ int launch_mr_jacobian(EquationsSet &s, int precision)
     }
     OC_CHECK(mr_jacobian_buffers(s, precision));
     OC_CHECK(launch_mr_gauss(s));
-    OC_CHECK(launch_mr_element_matrices(s, precision, s.tuned_element_blocks_per_cu));
-    return launch_mr_row_gather(s, precision, s.tuned_gather_chunk);
+    OC_CHECK(launch_mr_element_matrices(s, precision, s.tuned[precision].element_blocks_per_cu));
+    return launch_mr_row_gather(s, precision, s.tuned[precision].gather_chunk);
 }
 
 // ---------------------------------------------------------------------------

@@ -5,6 +5,7 @@
 
 #include <cstdint>
 #include <string>
+#include <utility>
 #include <vector>
 
 #include "../../include/oc_asm.h"
@@ -168,6 +169,15 @@ struct SolverSystem {
 
 constexpr int kFlatRowLength = 504;  // the longest CSR row of node_rows_flat (oc_fe_device.h); a regular mesh has 402
 
+// Launch shapes that oc_autotune found faster than the default on one set, for
+// Jacobians of one precision; 0 (smoother: -1) where the default rule holds
+struct LaunchShapes {
+    int element_blocks_per_cu = 0;
+    int gather_chunk = 0;
+    int spmv_lanes = 0, spmv_unroll = 0;  // lanes per row or node, neighbours in flight per lane
+    int smoother = -1;                    // level-0 node-kernel shape (oc_multigrid.hip)
+};
+
 // Per-equations-set state.  Element arrays are element-major; node and DOF
 // indices are 0-based; CSR col_idx 0-based int32, row offsets int64 on the
 // device (a batch of meshes can exceed 2^31 nonzeros).
@@ -275,12 +285,11 @@ struct EquationsSet {
     DevBuf<int64_t> pstart;     // first pressure column of each displacement row
     int krylov_capacity = 0;
 
-    // launch shapes (oc_autotune); 0 = default
-    int tuned_element_blocks_per_cu = 0;
-    int tuned_spmv_lanes = 0;
-    int tuned_gather_chunk = 0;
-    int tuned_smoother = -1;     // level-0 node-kernel shape (oc_multigrid.hip); -1 = default
-    int tuned_spmv_unroll = 0;   // neighbours per lane in flight in the node-wise SpMV
+    LaunchShapes tuned[2];  // by precision, OC_FP64 and OC_FP32
+    // the SpMV's default lanes per Mooney-Rivlin row or node and neighbours in
+    // flight per lane: FP32 values 32 x 2 (257 us at 32^3, 264 with one
+    // neighbour), FP64 a wavefront (332 us; 397 with 16 x 2)
+    std::pair<int, int> spmv_default(bool fp32) const { return fp32 ? std::make_pair(32, 2) : std::make_pair(64, 1); }
 
     // Newton-step graph: Jacobian assembly + preconditioner setup, recorded for
     // {precision, preconditioner, element blocks per CU, gather chunk,
@@ -330,6 +339,7 @@ int mr_node_materials(EquationsSet &s);  // fills node_mat from mat
 int mr_jacobian_buffers(EquationsSet &s, int precision);  // element-matrix and CSR value buffers
 int launch_mr_element_matrices(EquationsSet &s, int precision, int blocks_per_cu);
 int launch_mr_row_gather(EquationsSet &s, int precision, int chunk);
+int row_gather_default(const EquationsSet &s);
 int launch_mr_gauss(EquationsSet &s);
 // pressure-block Schur estimate from the pressure mass (analytic MR Jacobians:
 // it reads the Gauss records of the last Jacobian assembly)

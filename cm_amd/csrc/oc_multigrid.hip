@@ -1239,7 +1239,7 @@ int mg_setup(EquationsSet &s, int precision, double *inv_u, double *diag_u)
 
 // Launch shapes of the level-0 node kernels: lanes per node (below) x
 // neighbours per lane in flight (1, 2, 2, 4, 1; the cases of launch_uu_node);
-// the autotuner picks one (EquationsSet::tuned_smoother).
+// the autotuner may pick one (LaunchShapes::smoother).
 constexpr int kNodeVariants = 5;
 constexpr int kNodeVariantLanes[kNodeVariants] = {32, 32, 16, 16, 64};
 
@@ -1376,7 +1376,7 @@ int mg_apply(EquationsSet &s, int precision, const double *r, const double *inv_
     const int M = s.n_meshes, nq = s.n_nodes, nl = static_cast<int>(g.levels.size());
     const double *inv_u = s.precond.ptr;  // nodal block inverses of the set's block preconditioner
     const bool bf = precision == OC_FP32;  // an FP32 Jacobian's packed bf16 values (mg_prepare)
-    const int variant = s.tuned_smoother;  // -1: a wavefront per node for FP64 values, 16 lanes x one quad for bf16
+    const int variant = s.tuned[precision].smoother;  // -1: a wavefront per node for FP64 values, 16 lanes x one quad for bf16
     // with the packed bf16 values the kernels that produce the iterate also
     // write its FP32 node quadruples, into the two halves of uu_x4 in turn
     // (a sweep gathers one half and writes the other); q4 is the current one

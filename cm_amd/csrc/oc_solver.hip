@@ -990,18 +990,15 @@ struct Krylov {
     {
         KernelTimer timer("spmv");
         const bool lap = s.cls == OC_EQUATIONS_SET_LAPLACE;
-        // defaults: 8 lanes per Laplace row; per Mooney-Rivlin node 32 lanes with
-        // two neighbours in flight (FP32: 257 us at 32^3, 264 with one) or a
-        // wavefront (FP64)
-        const int lanes = s.tuned_spmv_lanes > 0 ? s.tuned_spmv_lanes : (lap ? 8 : (fp32 ? 32 : 64));
-        if (lap) return launch_spmv<double>(s.values.ptr, lanes, s.wgt.ptr, x, y);
-        if (fp32) return launch_spmv<float>(s.values_sp.ptr, lanes, s.wgt.ptr, x, y);
-        return launch_spmv<double>(s.values.ptr, lanes, s.wgt.ptr, x, y);
+        if (lap) return launch_spmv<double>(s.values.ptr, 8, s.wgt.ptr, x, y);
+        const LaunchShapes &t = s.tuned[fp32 ? OC_FP32 : OC_FP64];
+        const auto [lanes, unroll] = t.spmv_lanes > 0 ? std::make_pair(t.spmv_lanes, t.spmv_unroll) : s.spmv_default(fp32);
+        if (fp32) return launch_spmv<float>(s.values_sp.ptr, lanes, s.wgt.ptr, x, y, unroll);
+        return launch_spmv<double>(s.values.ptr, lanes, s.wgt.ptr, x, y, unroll);
     }
     template <typename VT>
-    int launch_spmv(const VT *vals, int lanes, const double *wv, const double *x, double *y, int unroll = -1)
+    int launch_spmv(const VT *vals, int lanes, const double *wv, const double *x, double *y, int unroll = 1)
     {
-        if (unroll < 0) unroll = s.tuned_spmv_unroll > 0 ? s.tuned_spmv_unroll : (fp32 ? 2 : 1);
         Runtime &rt = runtime();
         if (s.cls == OC_EQUATIONS_SET_MOONEY_RIVLIN && s.node_rows == 1 && lanes >= 16) {
             const int nq = s.n_nodes, nl = s.n_nodes_l;
@@ -1477,8 +1474,8 @@ static int step_assembly(EquationsSet &s, Krylov *K, int precision)
     }
     // the preconditioner kernels read the free-DOF mask, so a graph belongs to
     // one set of boundary conditions
-    const long long key[5] = {precision, K ? K->precond : -1, s.tuned_element_blocks_per_cu, s.tuned_gather_chunk,
-                              static_cast<long long>(s.bc_version)};
+    const long long key[5] = {precision, K ? K->precond : -1, s.tuned[precision].element_blocks_per_cu,
+                              s.tuned[precision].gather_chunk, static_cast<long long>(s.bc_version)};
     if (!s.step_graph || !std::equal(key, key + 5, s.step_graph_key)) {
         if (s.step_graph) {
             (void)hipGraphExecDestroy(s.step_graph);

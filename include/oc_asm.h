@@ -374,8 +374,10 @@ int oc_multigrid_options_set(oc_equations_set equations_set, int pre_sweeps, int
 /* Launch-shape autotuner (no counterpart in the reference): times the
  * element-matrix kernel's grid, the CSR row gather's prefetch depth, the
  * SpMV's lanes per row and the level-0 multigrid kernel's shape on this set at
- * its current DOFs, keeps the fastest of each for later launches, and writes
- * the timings as JSON into report. */
+ * its current DOFs, keeps the fastest of each for later launches with a
+ * Jacobian of that precision (where none beats the default by more than the
+ * timing noise, the default rule stays in force), and writes the timings as JSON
+ * into report. */
 int oc_autotune(oc_equations_set equations_set, int precision, char *report, int report_size);
 /* Euclidean norm of the residual over the free DOFs at the current DOFs. */
 int oc_residual_norm(oc_equations_set equations_set, double *norm);
