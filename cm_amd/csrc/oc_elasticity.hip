@@ -582,10 +582,11 @@ int launch_mr_residual(EquationsSet &s)
 // K_(p,m),(b,n) = sum_g (J_z w_g psi_m) D_g[b][n] (:1039-1054) as an 8x27 by
 // 27x81 GEMM.  U is formed in registers from D and W and never stored.  Lower
 // triangle kept, mirrored (:1149-1153); the element matrix goes to an HBM
-// buffer, row-major.
-// Phase B (csr_row_gather_kernel<Real>): one wavefront per CSR row adds the
-// element rows that touch it, in ascending element order, into an LDS copy of
-// the row and writes the row once (no zero fill, no read-modify-write).
+// buffer, its rows by nodes (kbuf_row).
+// Phase B (csr_row_gather_kernel<Real>): one wavefront per node (its three
+// displacement rows) or pressure row adds the element rows that touch it, in
+// ascending element order, into an LDS copy of the rows and writes them once (no
+// zero fill, no read-modify-write).
 typedef float mfma_f32x4 __attribute__((ext_vector_type(4)));
 
 // Both element-matrix kernels are persistent (one block of twelve waves per CU)

@@ -676,7 +676,8 @@ __global__ void __launch_bounds__(256) uu_cols_kernel(int nq, const int64_t *__r
     for (int p = lane; p < degp; p += kPackLanes) uu_col[off + p] = p < deg ? col_idx[s0 + p] : i;
 }
 
-// values of one FP32 Jacobian into the packed bf16 copy (each Newton step)
+// values of one FP32 Jacobian into the packed bf16 copy, without a multigrid setup
+// (whose q1_product_kernel forms it in passing): the autotuner times the smoother on it
 __global__ void __launch_bounds__(256) uu_pack_kernel(int nq, const int64_t *__restrict__ row_ptr,
                                                      const int64_t *__restrict__ pstart, const float *__restrict__ v,
                                                      const int64_t *__restrict__ uu_off, uint16_t *__restrict__ uu_bf)

@@ -385,7 +385,7 @@ __global__ void __launch_bounds__(kT) arnoldi_project_kernel(int n, int j, int n
 // arnoldi_project_kernel for systems of one row a thread (n <= kT *
 // kReduceBlocks) and j + 2 <= kRowVectors, where latency is all there is: the
 // basis rows are on their way while the partials are added up, and serve the
-// second pass's dot products from the registers.  At 23,800 rows 6.1 us against 7.3; In the 16^3
+// second pass's dot products from the registers.  At 23,800 rows 6.1 us against 7.3; in the 16^3
 // load step (112,724 rows, blocks of 512) 7.3 us against 9.
 template <int kT>
 __global__ void __launch_bounds__(kT) arnoldi_project_row_kernel(int n, int j, int n_parts, double *V,
