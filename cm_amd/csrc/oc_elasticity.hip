@@ -1285,7 +1285,7 @@ __device__ __forceinline__ void gather_node(const int2 *__restrict__ list, int l
 // in the same lines, as did the three rows'.  The element rows are taken in
 // groups of kMax, ..., 2, 1: with a test per row the scalar instructions took
 // three times the vector ones' issue slots.
-// 32,768 elements FP64: 788 -> 721 us (4.0 GB); 13,100 elements FP32 293 -> 185 us,
+// 32,768 elements FP64: 788 -> 721 us (3.8 GB); 13,100 elements FP32 293 -> 185 us,
 // 4,301 elements 77 -> 54 us.  Two wavefronts a block: 769 us with four, 779 with one.
 constexpr int kGatherWaves = 2;
 
